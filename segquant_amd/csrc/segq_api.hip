@@ -354,11 +354,11 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     }
     // int8 with several ranges keeps the big tiles if the caller lends a workspace to park
     // finished ranges in: one fp32 tile per workgroup
-    bool park = i8 && plain8 && fold && !groups && wide_ok && d->batch == 1 && d->out_dtype != SEGQ_ACC && ws && al(ws, 16);
+    bool park = i8 && plain8 && fold && !groups && wide_ok && d->out_dtype != SEGQ_ACC && ws && al(ws, 16);
     auto park_fits = [&](int c) {
         if (c < FIRST_WIDE_CFG || c >= NUM_TILE_CFG) return false;
         const TileCfg& t = TILE_CFGS[c];
-        const int64_t tiles = ((d->m + t.bm - 1) / t.bm) * ((d->n + t.bn - 1) / t.bn);
+        const int64_t tiles = ((d->m + t.bm - 1) / t.bm) * ((d->n + t.bn - 1) / t.bn) * d->batch;
         return ws_bytes >= tiles * t.bm * t.bn * 4;
     };
     if (d->tile == 0) {
@@ -522,7 +522,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     p.tiles_m = (int32_t)((d->m + c.bm - 1) / c.bm);
     p.tiles_n = (int32_t)((d->n + c.bn - 1) / c.bn);
     if (plan) {
-        plan->bytes = part_bytes + (park ? (int64_t)splits * p.tiles_m * p.tiles_n * c.bm * c.bn * 4 : 0);
+        plan->bytes = part_bytes + (park ? splits * d->batch * p.tiles_m * p.tiles_n * c.bm * c.bn * 4 : 0);
         plan->tile = cfg + 1;
         plan->splits = splits;
         plan->parked = park ? 1 : 0;

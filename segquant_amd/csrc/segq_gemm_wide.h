@@ -811,10 +811,10 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         if constexpr (PARK) {
             if (r < r_last) {
                 const int rl = r_last;
-                const float* sx = p.r[ph(r)].sx;
-                const float* sw = p.r[ph(r)].sw;
-                const float* sx2 = p.r[ph(rl)].sx;
-                const float* sw2 = p.r[ph(rl)].sw;
+                const float* sx = p.r[ph(r)].sx + z * p.bsSx;  // (a K split has no batch: its strides are 0)
+                const float* sw = p.r[ph(r)].sw + z * p.bsSw;
+                const float* sx2 = p.r[ph(rl)].sx + z * p.bsSx;
+                const float* sw2 = p.r[ph(rl)].sw + z * p.bsSw;
                 const int rs = p.r[ph(r)].sx_rs, cs = p.r[ph(r)].sw_cs, rs2 = p.r[ph(rl)].sx_rs, cs2 = p.r[ph(rl)].sw_cs;
                 float fx[TM];
 #pragma unroll

@@ -26,3 +26,28 @@ def test_fake_e4m3_sizes_and_offsets(dt, n, off):
     want = FakeQuantFp8Ext.fake_e4m3fy(x[off:])
     assert torch.isnan(got[0]) and got.dtype == want.dtype
     np.testing.assert_array_equal(got[1:].float().numpy(), want[1:].float().numpy())
+
+
+@pytest.mark.parametrize("fmt", [O.FMT_INT8, O.FMT_E4M3])
+@pytest.mark.parametrize("S,M,N,K", [(1, 5, 18, 128), (2, 300, 200, 384), (3, 130, 515, 256), (2, 77, 130, 208)])
+def test_dual_operator_batches(fmt, S, M, N, K):
+    """DualScale over several segments: two code tensors and parked sums per segment (K in whole steps), the merged
+    tensor otherwise; per-segment scales that differ, against the closed form in fp64."""
+    from segquant_amd import ops
+    g = torch.Generator().manual_seed(S * M + K)
+    x = torch.nn.functional.gelu(torch.randn(S, M, K, generator=g) * torch.tensor([1.0, 3.0, 0.5])[:S, None, None])
+    lim = (127.0, 128.0) if fmt == O.FMT_INT8 else (448.0, 448.0)
+    pos, neg = lim[0] / x.amax(dim=(1, 2)), lim[1] / (-x).amax(dim=(1, 2))
+    rng = np.random.default_rng(7)
+    w = rng.integers(-128, 128, size=(S, N, K)).astype(np.int8) if fmt == O.FMT_INT8 else \
+        np.where((c := rng.integers(0, 256, size=(S, N, K)).astype(np.uint8)) & 0x7F == 0x7F, 0x3A, c).astype(np.uint8)
+    sw = torch.rand(S, N, generator=g) * 30 + 10
+    out = ops.real_quantized_gemm_dual_scaled(fmt, fmt, x.to(DEV), torch.from_numpy(w).to(DEV), pos.to(DEV), neg.to(DEV), sw.to(DEV)).cpu().numpy()
+    for s in range(S):
+        yp, yn = O.quantize_act_dual(x[s:s + 1].numpy(), [pos[s].numpy()], [neg[s].numpy()], fmt)
+        wv = O.code_values(w[s], fmt)
+        p, n = O.code_values(yp[0], fmt), O.code_values(yn[0], fmt)
+        want = ((p @ wv.T) / np.float64(pos[s]) + (n @ wv.T) / np.float64(neg[s])) / sw[s].numpy().astype(np.float64)[None, :]
+        mag = ((np.abs(p) @ np.abs(wv).T) / np.float64(pos[s]) + (np.abs(n) @ np.abs(wv).T) / np.float64(neg[s])) / sw[s].numpy()[None, :]
+        # fp32 scaling of int32 sums; e4m3: the matrix cores' limited-width adder
+        assert (np.abs(out[s] - want) <= (4e-6 if fmt == O.FMT_INT8 else 3e-4) * mag + 1e-30).all()
