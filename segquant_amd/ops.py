@@ -115,6 +115,16 @@ def code_dtype(fmt: str) -> torch.dtype:
 # ---------------------------------------------------------------------------
 # quantise
 # ---------------------------------------------------------------------------
+def row_stride(x: torch.Tensor) -> int:
+    """Elements from one row of a 2-D tensor to the next, as a descriptor states it (one row: its length)."""
+    return x.stride(0) if x.shape[0] > 1 else x.shape[1]
+
+
+def rounded_col_div(col_div: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """The divisors as the quantise kernel takes them: rounded to ``dtype``, held in float32."""
+    return col_div.reshape(-1).to(dtype).to(torch.float32).contiguous()
+
+
 def quantize(x: torch.Tensor, fmt: str, scale: torch.Tensor, scale_neg: Optional[torch.Tensor] = None, **kw):
     """Quantise a 2-D float matrix ``x`` (rows, cols) to codes: :func:`quantize_desc` + one
     ``segq_quantize`` launch.  Returns the code tensor, or ``(Xp, Xn)`` when ``two_tensors``."""
@@ -149,7 +159,7 @@ def quantize_desc(x: torch.Tensor, fmt: str, scale: torch.Tensor, scale_neg: Opt
              dual: bool = False, dual_kseg_mask: int = 0xFFFFFFFF, dynamic: bool = False,
              two_tensors: bool = False, out: Optional[torch.Tensor] = None,
              out_neg: Optional[torch.Tensor] = None, pre_op: Optional[str] = None,
-             gate: Optional[torch.Tensor] = None, col_div: Optional[torch.Tensor] = None):
+             gate: Optional[torch.Tensor] = None, col_div: Optional[torch.Tensor] = None, col_div_rounded: bool = False):
     """The ``segq_quant_desc`` of a quantise launch, its output tensor(s), the launch's
     description for ``record_launches`` and the tensors the descriptor points into
     (keep them alive until the launch is enqueued).
@@ -162,7 +172,8 @@ def quantize_desc(x: torch.Tensor, fmt: str, scale: torch.Tensor, scale_neg: Opt
     x * op(gate) when ``gate`` (same shape and dtype as ``x``) is given.
     ``col_div``: one divisor per column (SmoothQuant's ``s``, any float dtype; it is
     used rounded to ``x.dtype`` as the reference's ``x.div_(s.to(x.dtype))`` does),
-    applied after the ``pre_op``.
+    applied after the ``pre_op``.  ``col_div_rounded``: ``col_div`` is what
+    :func:`rounded_col_div` returned for this dtype already.
     """
     _need_cuda(x, scale, scale_neg, gate)
     if x.dim() != 2 or x.stride(1) != 1:
@@ -199,7 +210,8 @@ def quantize_desc(x: torch.Tensor, fmt: str, scale: torch.Tensor, scale_neg: Opt
         _need_cuda(col_div)
         if col_div.numel() != cols:
             raise RuntimeError("col_div needs one entry per column")
-        col_div = col_div.reshape(-1).to(x.dtype).to(torch.float32).contiguous()
+        if not col_div_rounded:
+            col_div = rounded_col_div(col_div, x.dtype)
         d.col_div = col_div.data_ptr()
     if gate is not None:
         if pre_op is None or gate.shape != x.shape or gate.dtype != x.dtype or gate.stride(1) != 1:

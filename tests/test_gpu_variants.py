@@ -51,3 +51,31 @@ def test_dual_operator_batches(fmt, S, M, N, K):
         mag = ((np.abs(p) @ np.abs(wv).T) / np.float64(pos[s]) + (np.abs(n) @ np.abs(wv).T) / np.float64(neg[s])) / sw[s].numpy()[None, :]
         # fp32 scaling of int32 sums; e4m3: the matrix cores' limited-width adder
         assert (np.abs(out[s] - want) <= (4e-6 if fmt == O.FMT_INT8 else 3e-4) * mag + 1e-30).all()
+
+
+@pytest.mark.parametrize("off", [0, 8, 3])
+@pytest.mark.parametrize("rows", [1, 5, 130])
+def test_layers_read_column_slices_where_they_lie(rows, off):
+    """Inputs and gates that are column slices of a wider tensor (16-byte aligned: read in place; off the grid, with
+    rows that are no multiple of 16 bytes apart, repeated or reversed by a transposition: copied) give the bits of
+    their contiguous copies, on the first call of a token count and on later ones, plain and with a fused activation."""
+    from segquant_amd.layers.SegmentLinear import SegmentLinear
+    K, N = 256, 144
+    off = off & ~7 if rows == 1 else off  # (a single row is contiguous wherever it starts: unaligned, it is refused as ever)
+    g = torch.Generator().manual_seed(rows + off)
+    args = {"real_quant": True, "axis": -1, "dynamic": True}
+    layer = SegmentLinear(K, N, bias=True, custom_weight_tensor=torch.randn(N, K, generator=g) * 0.02,
+                          custom_bias_tensor=torch.randn(N, generator=g).to(torch.bfloat16), input_quant_type="int8", weight_quant_type="int8",
+                          input_quant_args=args, weight_quant_args={"real_quant": True, "axis": 1}, device=DEV)
+    layer.calibrate(torch.randn(64, K, generator=g).to(DEV))
+    layer.finish_calibrate()
+    for width in (2 * K + 16, 2 * K + 21):
+        wide = torch.randn(rows, width, generator=g).to(torch.bfloat16).to(DEV)
+        a, b = wide[:, off:off + K], wide[:, K + off:2 * K + off]
+        t = torch.randn(K, rows, generator=g).to(torch.bfloat16).to(DEV).t()
+        e = wide[:1, off:off + K].expand(rows, K)
+        for v in (a, b, t, e, a):
+            assert torch.equal(layer(v), layer(v.contiguous().clone()))
+            assert torch.equal(layer(v), layer(v.contiguous().clone()))
+        assert torch.equal(layer(a, pre_op="gelu", gate=b), layer(a.contiguous().clone(), pre_op="gelu", gate=b.contiguous().clone()))
+        assert torch.equal(layer(t, pre_op="silu", gate=a), layer(t.contiguous().clone(), pre_op="silu", gate=a.contiguous().clone()))
