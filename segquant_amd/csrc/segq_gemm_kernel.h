@@ -161,6 +161,16 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_kernel(const GemmParams p)
     static_assert(BM * 8 % NT == 0 && BN * 4 % NT == 0, "tile does not divide over the threads");
     static_assert((NT / 8) % 16 == 0, "row swizzle must not depend on the load iteration");
     static_assert(!B4 || FMT == GEMM_I8, "int4 weights pair with int8 activations");
+    // K steps whose loads are in flight in registers.  The dispatch gives the 64 x 128 tile at most two
+    // workgroups per CU, so that nothing else hides a step's wait for memory; 128 x 128 has room for two
+    // sets below the 256 registers at which two workgroups share a CU.  Whole passes, one step ahead and
+    // scales read in the epilogue -> this: 333 x 1000 x 1168 int8 19.8 -> 18.6 us, 154 x 5120 x 1280 int4
+    // 21.6 -> 19.7 us.  What is left is the serial chain of a step (LDS write, barrier, LDS read, MFMA).
+    // (Several ranges: a second accumulator set takes that room; e4m3, with twice the fragments, has none left.)
+    constexpr int DEPTH = BM * BN > 128 * 128 ? 1 : !FOLD ? (BM * BN <= 64 * 128 ? 4 : 2) : BM * BN <= 64 * 128 && FMT == GEMM_I8 ? 2 : 1;
+    // scales and bias are read before the K loop where registers allow it: read in the epilogue they are a
+    // chain of TN round trips to memory, as no load passes the stores of the columns before
+    constexpr bool EARLY = BM * BN <= 64 * 128;
     typedef typename AccT<FMT>::type acc_t;
     typedef typename AccT<FMT>::elem acc_e;
     const acc_t acc_zero = {0, 0, 0, 0};
@@ -214,50 +224,53 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_kernel(const GemmParams p)
     for (int i = 0; i < B_IT; ++i) b_goff[i] = (int64_t)min(n0 + b_r0 + i * B_RSTEP, p.N - 1) * p.ldb + b_ch * 16;
     const int b_sw = swz(b_r0);
 
-    uint4 ra[A_IT], rb[B_IT];
+    uint4 ra[DEPTH][A_IT], rb[DEPTH][B_IT];
 
-    auto load_tile = [&](int r, int k) {
-        const int k1 = p.r[r].k1;
+    // Loads one K step.  Pieces beyond the range's end read its first piece instead, which is there, and
+    // are cleared on the way to LDS: a load without a branch around it leaves the count of loads in flight
+    // known, so that a step is waited for alone.
+    auto load_tile = [&](int r, int k, uint4 (&qa)[A_IT], uint4 (&qb)[B_IT]) {
+        const int k0 = p.r[r].k0, k1 = p.r[r].k1;
         const uint8_t* ap = (p.r[r].a_sel == 1) ? A2b : Ab;
-        const bool a_ok = (k + a_ch * 16) < k1;
+        const int ka = (k + a_ch * 16) < k1 ? k : k0 - a_ch * 16;
 #pragma unroll
-        for (int i = 0; i < A_IT; ++i)
-            ra[i] = a_ok ? *reinterpret_cast<const uint4*>(ap + a_goff[i] + k) : make_uint4(0, 0, 0, 0);
+        for (int i = 0; i < A_IT; ++i) qa[i] = *reinterpret_cast<const uint4*>(ap + a_goff[i] + ka);
         if constexpr (B4) {
-            const bool b_ok = (k + b_ch * 32) < k1;
+            const int kb = (k + b_ch * 32) < k1 ? k >> 1 : (k0 >> 1) - b_ch * 16;
 #pragma unroll
-            for (int i = 0; i < B_IT; ++i)
-                rb[i] = b_ok ? *reinterpret_cast<const uint4*>(Bb + b_goff[i] + (k >> 1)) : make_uint4(0, 0, 0, 0);
+            for (int i = 0; i < B_IT; ++i) qb[i] = *reinterpret_cast<const uint4*>(Bb + b_goff[i] + kb);
         } else {
-            const bool b_ok = (k + b_ch * 16) < k1;
+            const int kb = (k + b_ch * 16) < k1 ? k : k0 - b_ch * 16;
 #pragma unroll
-            for (int i = 0; i < B_IT; ++i)
-                rb[i] = b_ok ? *reinterpret_cast<const uint4*>(Bb + b_goff[i] + k) : make_uint4(0, 0, 0, 0);
+            for (int i = 0; i < B_IT; ++i) qb[i] = *reinterpret_cast<const uint4*>(Bb + b_goff[i] + kb);
         }
     };
 
-    auto store_tile = [&](int buf, int a_sel) {
+    auto store_tile = [&](int buf, int r, int k, const uint4 (&qa)[A_IT], const uint4 (&qb)[B_IT]) {
+        const int k1 = p.r[r].k1, a_sel = p.r[r].a_sel;
+        const uint4 none = make_uint4(0, 0, 0, 0);
+        const bool a_ok = (k + a_ch * 16) < k1;
+        const bool b_ok = (k + b_ch * (B4 ? 32 : 16)) < k1;
         uint8_t* as = As + buf * BM * BK + a_lds;
 #pragma unroll
         for (int i = 0; i < A_IT; ++i)
-            *reinterpret_cast<uint4*>(as + i * (NT / 8) * BK) = select_sign(ra[i], a_sel);
+            *reinterpret_cast<uint4*>(as + i * (NT / 8) * BK) = select_sign(a_ok ? qa[i] : none, a_sel);
         uint8_t* bs = Bs + buf * BN * BK + b_r0 * BK;
-        if constexpr (B4) {
 #pragma unroll
-            for (int i = 0; i < B_IT; ++i) {
+        for (int i = 0; i < B_IT; ++i) {
+            const uint4 q = b_ok ? qb[i] : none;
+            if constexpr (B4) {
                 uint4 lo, hi;
-                unpack8_i4x16(rb[i].x, lo.x, lo.y);
-                unpack8_i4x16(rb[i].y, lo.z, lo.w);
-                unpack8_i4x16(rb[i].z, hi.x, hi.y);
-                unpack8_i4x16(rb[i].w, hi.z, hi.w);
+                unpack8_i4x16(q.x, lo.x, lo.y);
+                unpack8_i4x16(q.y, lo.z, lo.w);
+                unpack8_i4x16(q.z, hi.x, hi.y);
+                unpack8_i4x16(q.w, hi.z, hi.w);
                 uint8_t* row = bs + i * B_RSTEP * BK;
                 *reinterpret_cast<uint4*>(row + (((2 * b_ch) ^ b_sw) << 4)) = lo;
                 *reinterpret_cast<uint4*>(row + (((2 * b_ch + 1) ^ b_sw) << 4)) = hi;
+            } else {
+                *reinterpret_cast<uint4*>(bs + i * B_RSTEP * BK + ((b_ch ^ b_sw) << 4)) = q;
             }
-        } else {
-#pragma unroll
-            for (int i = 0; i < B_IT; ++i)
-                *reinterpret_cast<uint4*>(bs + i * B_RSTEP * BK + ((b_ch ^ b_sw) << 4)) = rb[i];
         }
     };
 
@@ -327,30 +340,59 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_kernel(const GemmParams p)
     const int m_base = m0 + wm * WM + lrow;
     const int n_base = n0 + wn * WN + 4 * lgrp;
 
-    // 1 / (sx * sw) factors of range r for this lane's rows and columns.
-    auto range_rx = [&](int r, float (&rx)[TM]) {
+    // Scales of range r for this lane's rows and columns, as they are stored, and their reciprocals.
+    auto load_sx = [&](int r, float (&q)[TM]) {
         const float* sx = p.r[r].sx + z * p.bsSx;
         const int rs = p.r[r].sx_rs;
 #pragma unroll
-        for (int b = 0; b < TM; ++b) rx[b] = 1.0f / sx[(int64_t)min(m_base + b * 16, p.M - 1) * rs];
+        for (int b = 0; b < TM; ++b) q[b] = sx[(int64_t)min(m_base + b * 16, p.M - 1) * rs];
     };
-    auto range_rw = [&](int r, int a, float (&rw)[4]) {
+    auto load_sw = [&](int r, int a, float (&q)[4]) {
         const float* sw = p.r[r].sw + z * p.bsSw;
         const int cs = p.r[r].sw_cs;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) q[v] = sw[(int64_t)min(n_base + a * 16 + v, p.N - 1) * cs];
+    };
+    auto inv_rx = [&](const float (&q)[TM], float (&rx)[TM]) {
+#pragma unroll
+        for (int b = 0; b < TM; ++b) rx[b] = 1.0f / q[b];
+    };
+    auto inv_rw = [&](const float (&q)[4], float (&rw)[4]) {
         // the factor 16 of the staged int4 weights is exact and removed here
         const float unscale = B4 ? 0.0625f : 1.0f;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) rw[v] = unscale / sw[(int64_t)min(n_base + a * 16 + v, p.N - 1) * cs];
+        for (int v = 0; v < 4; ++v) rw[v] = unscale / q[v];
+    };
+    // Bias of columns n_of(a0) .. as it is stored: one branch around all loads, converted when it is used
+    // (a branch and a conversion per element wait for memory once per element).
+    auto load_bias_raw = [&](int a0, int count, uint32_t (*q)[4]) {
+        if (!p.bias) return;
+        if (p.bias_dtype == SEGQ_F32) {
+#pragma unroll
+            for (int a = 0; a < count; ++a)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) q[a][v] = static_cast<const uint32_t*>(p.bias)[min(n_base + (a0 + a) * 16 + v, p.N - 1)];
+        } else {
+#pragma unroll
+            for (int a = 0; a < count; ++a)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) q[a][v] = static_cast<const uint16_t*>(p.bias)[min(n_base + (a0 + a) * 16 + v, p.N - 1)];
+        }
+    };
+    auto bias_value = [&](uint32_t q) {
+        return p.bias_dtype == SEGQ_F32 ? __uint_as_float(q) : p.bias_dtype == SEGQ_BF16 ? bf16_bits_to_f32(q) : f16_bits_to_f32(q & 0xffffu);
     };
 
     auto fold = [&](int r) {
         if constexpr (FOLD) {
-            float rx[TM];
-            range_rx(r, rx);
+            float sx[TM], rx[TM];
+            load_sx(r, sx);
+            inv_rx(sx, rx);
 #pragma unroll
             for (int a = 0; a < TN; ++a) {
-                float rw[4];
-                range_rw(r, a, rw);
+                float sw[4], rw[4];
+                load_sw(r, a, sw);
+                inv_rw(sw, rw);
 #pragma unroll
                 for (int b = 0; b < TM; ++b) {
 #pragma unroll
@@ -361,29 +403,61 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_kernel(const GemmParams p)
         }
     };
 
+    constexpr int KEPT = EARLY ? TN : 1;
+    float sx_raw[TM], sw_raw[KEPT][4];
+    uint32_t bias_raw[KEPT][4] = {};
+    if constexpr (EARLY) {
+        if (p.out_dtype != SEGQ_ACC) {  // raw accumulators have no scales
+            if constexpr (!FOLD) {
+                load_sx(0, sx_raw);
+#pragma unroll
+                for (int a = 0; a < TN; ++a) load_sw(0, a, sw_raw[a]);
+            }
+            load_bias_raw(0, TN, bias_raw);
+        }
+    }
+
     // ---- main loop over (range, k) steps
+    auto advance = [&](int& r_, int& k_) {  // r_ == nr: past the last step
+        k_ += BK;
+        if (k_ >= p.r[r_].k1) {
+            ++r_;
+            k_ = r_ < p.nr ? p.r[r_].k0 : 0;
+        }
+    };
+    int lr = 0, lk = p.r[0].k0;  // the step that is loaded next; past the end the last range's first, unused
+    auto load_next = [&](uint4 (&qa)[A_IT], uint4 (&qb)[B_IT]) {
+        load_tile(lr, lk, qa, qb);
+        advance(lr, lk);
+        if (lr >= p.nr) {
+            lr = p.nr - 1;
+            lk = p.r[lr].k0;
+        }
+    };
     int r = 0, k = p.r[0].k0;
-    load_tile(r, k);
-    store_tile(0, p.r[0].a_sel);
+#pragma unroll
+    for (int u = 0; u < DEPTH; ++u) load_next(ra[u], rb[u]);
+    store_tile(0, r, k, ra[0], rb[0]);
     __syncthreads();
     int buf = 0;
-    while (true) {
-        int rn = r, kn = k + BK;
-        const bool range_done = kn >= p.r[r].k1;
-        if (range_done) {
-            rn = r + 1;
-            kn = (rn < p.nr) ? p.r[rn].k0 : 0;
+    bool more = true;
+    while (more) {
+#pragma unroll
+        for (int u = 0; u < DEPTH; ++u) {
+            // the step in LDS came from set u, which takes the step DEPTH further on
+            load_next(ra[u], rb[u]);
+            compute(buf);
+            int rn = r, kn = k;
+            advance(rn, kn);
+            if (FOLD && rn != r) fold(r);
+            more = rn < p.nr;
+            if (!more) break;
+            store_tile(buf ^ 1, rn, kn, ra[(u + 1) % DEPTH], rb[(u + 1) % DEPTH]);
+            __syncthreads();
+            buf ^= 1;
+            r = rn;
+            k = kn;
         }
-        const bool more = rn < p.nr;
-        if (more) load_tile(rn, kn);
-        compute(buf);
-        if (FOLD && range_done) fold(r);
-        if (!more) break;
-        store_tile(buf ^ 1, p.r[rn].a_sel);
-        __syncthreads();
-        buf ^= 1;
-        r = rn;
-        k = kn;
     }
 
     // ---- epilogue
@@ -411,21 +485,21 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_kernel(const GemmParams p)
     }
 
     float rx[TM];
-    if constexpr (!FOLD) range_rx(0, rx);
+    if constexpr (!FOLD) {
+        if constexpr (!EARLY) load_sx(0, sx_raw);
+        inv_rx(sx_raw, rx);
+    }
 #pragma unroll
     for (int a = 0; a < TN; ++a) {
-        float rw[4];
-        if constexpr (!FOLD) range_rw(0, a, rw);
-        float bv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (p.bias) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int n = min(n_base + a * 16 + v, p.N - 1);
-                if (p.bias_dtype == SEGQ_F32) bv[v] = static_cast<const float*>(p.bias)[n];
-                else if (p.bias_dtype == SEGQ_BF16) bv[v] = bf16_bits_to_f32(static_cast<const uint16_t*>(p.bias)[n]);
-                else bv[v] = f16_bits_to_f32(static_cast<const uint16_t*>(p.bias)[n]);
-            }
+        const int kept = EARLY ? a : 0;
+        if constexpr (!EARLY) {
+            if constexpr (!FOLD) load_sw(0, a, sw_raw[0]);
+            load_bias_raw(a, 1, bias_raw);
         }
+        float rw[4], bv[4];
+        if constexpr (!FOLD) inv_rw(sw_raw[kept], rw);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) bv[v] = p.bias ? bias_value(bias_raw[kept][v]) : 0.0f;
 #pragma unroll
         for (int b = 0; b < TM; ++b) {
             const int m = m_base + b * 16, n = n_base + a * 16;

@@ -79,3 +79,44 @@ def test_layers_read_column_slices_where_they_lie(rows, off):
             assert torch.equal(layer(v), layer(v.contiguous().clone()))
         assert torch.equal(layer(a, pre_op="gelu", gate=b), layer(a.contiguous().clone(), pre_op="gelu", gate=b.contiguous().clone()))
         assert torch.equal(layer(t, pre_op="silu", gate=a), layer(t.contiguous().clone(), pre_op="silu", gate=a.contiguous().clone()))
+
+
+@pytest.mark.parametrize("fa,fb", [(O.FMT_INT8, O.FMT_INT8), (O.FMT_E4M3, O.FMT_E4M3), (O.FMT_INT8, O.FMT_INT4)])
+@pytest.mark.parametrize("lens", [(32,), (160,), (384,), (512,), (544,), (640,), (1184,), (96, 160, 544), (512, 32), (32, 32, 32, 1056)])
+def test_general_gemm_steps_in_flight(fa, fb, lens):
+    """One to ten K steps around the number the general kernel keeps in flight, ends inside a step, and ranges whose
+    steps are loaded while the range before is multiplied; odd N, each bias type, on the tiles of each depth."""
+    from segquant_amd import ops
+    M, N, K = 67, 131, sum(lens)
+    rng = np.random.default_rng(K + len(lens))
+    lo = -8 if fb == O.FMT_INT4 else -128
+
+    def codes(rows, fmt):
+        if fmt == O.FMT_E4M3:
+            c = rng.integers(0, 256, size=(rows, K)).astype(np.uint8)
+            return np.where(c & 0x7F == 0x7F, 0x3A, c).astype(np.uint8)
+        return rng.integers(lo if fmt == fb else -128, 8 if fmt == O.FMT_INT4 else 128, size=(rows, K)).astype(np.int8)
+
+    a, b = codes(M, fa), codes(N, fb)
+    ad = torch.from_numpy(a).to(DEV)
+    bd = torch.from_numpy(np.stack([O.pack_int4(r) for r in b]) if fb == O.FMT_INT4 else b).to(DEV)
+    sx = rng.uniform(0.5, 1.5, size=(len(lens), M)).astype(np.float32)
+    sw = rng.uniform(0.5, 1.5, size=(len(lens), N)).astype(np.float32)
+    sxd, swd = torch.from_numpy(sx).to(DEV), torch.from_numpy(sw).to(DEV)
+    va, vb = O.code_values(a, fa), O.code_values(b, fb)
+    want, mag, ranges, k = 0.0, 0.0, [], 0
+    for i, n in enumerate(lens):
+        f = 1.0 / (sx[i].astype(np.float64)[:, None] * sw[i].astype(np.float64)[None, :])
+        want = want + (va[:, k:k + n] @ vb[:, k:k + n].T) * f
+        mag = mag + (np.abs(va[:, k:k + n]) @ np.abs(vb[:, k:k + n]).T) * f
+        ranges.append(ops.Range(k, n, sxd[i], swd[i], 0, 1, 1))
+        k += n
+    for bt in (None, torch.float32, torch.bfloat16, torch.float16):
+        bias = None if bt is None else torch.from_numpy(rng.normal(size=N)).to(bt)
+        exact = want if bt is None else want + bias.double().numpy()[None, :]
+        for tile in (2, 3, 4):
+            y = ops.gemm(ad, bd, ranges, m=M, n=N, a_fmt=fa, b_fmt=fb, out_dtype=torch.float32, lda=K, ldb=bd.shape[1],
+                         bias=None if bias is None else bias.to(DEV), tile=tile)
+            # int8: fp32 scaling of exact sums, a few roundings of 2^-24 per range; e4m3: the matrix cores' limited-width adder
+            tol = 3e-4 if fa == O.FMT_E4M3 else 1e-6
+            assert (np.abs(y.cpu().numpy().astype(np.float64) - exact) <= tol * mag + 2.0 ** -22 * np.abs(exact)).all(), (lens, bt, tile)
