@@ -212,7 +212,12 @@ typedef struct segq_krange {
     int32_t a_sel;
     int32_t sx_row_stride;  /* 0: sx[0] for every row; 1: sx[m] */
     int32_t sw_col_stride;  /* 0: sw[0] for every column; 1: sw[n] */
-    int32_t reserved;
+    int32_t own_sum;        /* read in the first range, for e4m3 codes in plain tensors (a_sel 0 or 1); 0 otherwise.
+                             * 0: the sums are carried from range to range, multiplied by the ratio of their
+                             * scales, which has to be finite (scales that a calibrator clamps).  Non-zero: every
+                             * range is summed on its own and scaled by its own factors, as int8 ranges always
+                             * are, so that a scale may be infinite: limit / 0 of a DualScale side that holds
+                             * nothing, which adds nothing.  Not combined with a low-rank branch or a K split. */
     const float* sx;        /* device */
     const float* sw;        /* device */
 } segq_krange;
@@ -244,8 +249,8 @@ typedef struct segq_gemm_desc {
                          * a small kernel and the int8 GEMM kernels run on that (same accumulators, bit for bit;
                          * worth it when m is large and the GEMM is bound by the matrix cores, not by reading b).
                          * NULL or too small: int4 weights are unpacked on their way into LDS inside the GEMM.
-                         * With int8 codes on both sides, several ranges and batch * tiles * tile_rows *
-                         * tile_cols * 4 bytes here (4 batch (m + 288) (n + 288) always suffices), the sums of finished
+                         * With int8 codes on both sides, several ranges, batch == 1 and tiles * tile_rows *
+                         * tile_cols * 4 bytes here (4 (m + 288) (n + 288) always suffices), the sums of finished
                          * ranges are parked in the workspace as fp32 instead of in a second register set, which
                          * keeps the largest tiles available (same result up to fp32 rounding order).
                          * Contents are undefined afterwards.  Replaces nothing in the reference, whose CUTLASS

@@ -39,7 +39,7 @@ class QuantDesc(C.Structure):
 class KRange(C.Structure):
     _fields_ = [
         ("k_begin", C.c_int64), ("k_len", C.c_int64),
-        ("a_sel", C.c_int32), ("sx_row_stride", C.c_int32), ("sw_col_stride", C.c_int32), ("reserved", C.c_int32),
+        ("a_sel", C.c_int32), ("sx_row_stride", C.c_int32), ("sw_col_stride", C.c_int32), ("own_sum", C.c_int32),
         ("sx", C.c_void_p), ("sw", C.c_void_p),
     ]
 

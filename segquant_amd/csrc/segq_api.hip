@@ -69,8 +69,9 @@ static int choose_tile(int64_t m, int64_t n, int64_t batch, bool fold, bool wide
         return ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn) * batch;
     };
     // (plain 8-bit operands go to the 8-wave kernels from 32 tiles of 128 x 128 up: 64 x 9216 x 3072 runs
-    // 24.9 us there against 35.2 us on the general kernel)
-    if (wide_ok && tiles(FIRST_WIDE_CFG + 3) >= (plain8 && !fold ? 32 : 96)) {
+    // 24.9 us there against 35.2 us on the general kernel; with a second accumulator set, both ranges of a
+    // DualScale 512 x 1024 x 1024 17.9 against 25.8 us, quantising included, and 512 x 1024 x 256 10.5 against 14.2)
+    if (wide_ok && tiles(FIRST_WIDE_CFG + 3) >= (plain8 ? 32 : 96)) {
         // Short contractions of middling size: the plain 128 x 128 kernel needs ~100 registers, so two
         // workgroups share a CU and each one's prologue and epilogue (most of a tile's time at a dozen
         // K steps) run under the other's MFMAs.  Measured at K = 1280 .. 1536: 2048 x 10240 34.5 vs 45.5 us
@@ -343,8 +344,10 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     bool plain8 = i8 || f8;  // both operands straight to LDS: no sign selection, no int4 unpacking
     for (int i = 0; i < d->n_ranges; ++i) plain8 = plain8 && d->ranges[i].a_sel < 2;
     // several ranges cost a second (fp32) accumulator set, and with it the biggest tiles,
-    // unless the accumulators are fp32 already (plain e4m3: rescaled in place)
-    const bool fold2 = fold && !(f8 && plain8);
+    // unless the accumulators are fp32 already (plain e4m3: rescaled in place, which takes the ratio of two
+    // ranges' scales and is not for callers whose scales may be infinite: own_sum)
+    p.sep = f8 && fold && plain8 && d->ranges[0].own_sum != 0;
+    const bool fold2 = fold && !(f8 && plain8 && !p.sep);
     if (groups) {
         bool ok = wide_ok && plain8;
         for (int i = 0; i < d->n_ranges; ++i) ok = ok && d->ranges[i].a_sel < 2;
@@ -354,11 +357,11 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     }
     // int8 with several ranges keeps the big tiles if the caller lends a workspace to park
     // finished ranges in: one fp32 tile per workgroup
-    bool park = i8 && plain8 && fold && !groups && wide_ok && d->out_dtype != SEGQ_ACC && ws && al(ws, 16);
+    bool park = i8 && plain8 && fold && !groups && wide_ok && d->batch == 1 && d->out_dtype != SEGQ_ACC && ws && al(ws, 16);
     auto park_fits = [&](int c) {
         if (c < FIRST_WIDE_CFG || c >= NUM_TILE_CFG) return false;
         const TileCfg& t = TILE_CFGS[c];
-        const int64_t tiles = ((d->m + t.bm - 1) / t.bm) * ((d->n + t.bn - 1) / t.bn) * d->batch;
+        const int64_t tiles = ((d->m + t.bm - 1) / t.bm) * ((d->n + t.bn - 1) / t.bn);
         return ws_bytes >= tiles * t.bm * t.bn * 4;
     };
     if (d->tile == 0) {
@@ -370,7 +373,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         } else {
             cfg = park ? choose_tile(d->m, d->n, d->batch, false, wide_ok, plain8) : -1;
             park = park && park_fits(cfg);
-            if (!park) cfg = choose_tile(d->m, d->n, d->batch, fold2, wide_ok, plain8, ktotal / 128, (!fold || f8) && !lowrank);
+            if (!park) cfg = choose_tile(d->m, d->n, d->batch, fold2, wide_ok, plain8, ktotal / 128, (!fold || (f8 && !p.sep)) && !lowrank);
         }
     }
     else if (d->tile >= 1 && d->tile <= NUM_TILE_CFG) cfg = d->tile - 1;
@@ -408,7 +411,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     int splits = 1;
     int64_t part_bytes = 0;
     {
-        const bool can = plain8 && wide_ok && d->batch == 1 && !groups && !lowrank && d->out_dtype != SEGQ_ACC && ws && al(ws, 16) &&
+        const bool can = plain8 && wide_ok && d->batch == 1 && !groups && !lowrank && !p.sep && d->out_dtype != SEGQ_ACC && ws && al(ws, 16) &&
                          d->split_k != 1 && (d->tile == 0 || cfg >= FIRST_WIDE_CFG) && !codes_out;
         const int64_t total_steps = ktotal / 128;
         if (d->split_k > 1 && !can)
@@ -416,7 +419,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
                                               "a float output, an 8-wave tile and a workspace");
         if (can) {
             int want = 1, scfg = cfg;
-            const bool big_ok = !fold2 || park || f8;  // the 256 x 256 tile, or 256 x 128 with a second register set
+            const bool big_ok = !fold2 || park;  // the 256 x 256 tile, or 256 x 128 with a second register set
             const int64_t cus = device_cus();
             auto tiles_of = [&](int c) { return ((d->m + TILE_CFGS[c].bm - 1) / TILE_CFGS[c].bm) * ((d->n + TILE_CFGS[c].bn - 1) / TILE_CFGS[c].bn); };
             if (d->split_k > 1) {
@@ -522,7 +525,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     p.tiles_m = (int32_t)((d->m + c.bm - 1) / c.bm);
     p.tiles_n = (int32_t)((d->n + c.bn - 1) / c.bn);
     if (plan) {
-        plan->bytes = part_bytes + (park ? splits * d->batch * p.tiles_m * p.tiles_n * c.bm * c.bn * 4 : 0);
+        plan->bytes = part_bytes + (park ? (int64_t)splits * p.tiles_m * p.tiles_n * c.bm * c.bn * 4 : 0);
         plan->tile = cfg + 1;
         plan->splits = splits;
         plan->parked = park ? 1 : 0;
@@ -535,10 +538,10 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     // 140.7 -> 136.2 us; other heights between 2 and 16 measured the same or worse on the 4608-token shapes)
     p.group_m = (cfg == FIRST_WIDE_CFG + 9) ? 4 : 8;
     {
-        // e4m3 only (4608 x 15360 x 3072 in three ranges: 350 -> 338 us); int8, which parks its sums at the
-        // boundaries, loses more to the XCDs reading different operand columns at a time than it gains
+        // e4m3 rescaled in place only (4608 x 15360 x 3072 in three ranges: 350 -> 338 us); int8, which parks its
+        // sums at the boundaries, loses more to the XCDs reading different operand columns at a time than it gains
         // from spreading its stores (385 -> 397 us), and keeps the common order
-        p.rot = (d->n_ranges > 1 && splits == 1 && f8) ? 1 : 0;
+        p.rot = (d->n_ranges > 1 && splits == 1 && f8 && !p.sep) ? 1 : 0;
     }
     if ((int64_t)p.tiles_m * p.tiles_n > 0x7fffffff || d->batch > 65535) return fail(SEGQ_ERR_ARG, "segq_gemm: grid too large");
     const int64_t osz = (d->out_dtype == SEGQ_F32 || d->out_dtype == SEGQ_ACC) ? 4 : 2;

@@ -70,7 +70,7 @@ struct GemmParams {
     const float* oc_scale_neg;
     int32_t oc_fmt, oc_pre;  // segq_code (I8 / E4M3), segq_pre_op
     int32_t oc_vec;          // rows allow 8-byte stores
-    int32_t pad3_;
+    int32_t sep;             // e4m3, several ranges: every range is summed on its own (gemm_pipe_kernel)
     int32_t dry;             // host only: walk the dispatch down to the kernel instance, launch nothing (segq_gemm_plan)
     KRange r[SEGQ_MAX_RANGES];
 };

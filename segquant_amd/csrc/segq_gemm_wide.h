@@ -608,7 +608,8 @@ __device__ __forceinline__ void lowrank_accumulate(const GemmParams& p, v4f (&of
 constexpr int waitcnt_vm_lgkm0(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
 
 template <int BM, int BN, int WGM, int WGN, int FMT, bool FOLD, int NS, bool GRP = false, bool PARK = false, bool FINISH = false,
-          bool CODES = false>  // CODES: the epilogue writes the next linear's codes instead of floats (one range)
+          bool CODES = false,  // CODES: the epilogue writes the next linear's codes instead of floats (one range)
+          bool SEP = false>    // SEP (e4m3, several ranges): a second register set, as int8 has it, instead of rescaling in place
 __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmParams p) {
     static_assert(!CODES || (!FOLD && !GRP && !PARK && !FINISH), "codes out: plain operands, one range");
     constexpr int NW = WGM * WGN, NT = NW * 64;
@@ -642,17 +643,23 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     constexpr bool WS = !F8 && !GRP && BM * BN > 256 * 256;
     constexpr bool S8 = F8 || GRP || WS;  // whole-step fragments
     //
-    // PARK (int8, several ranges): no second register set at all.  When a range
-    // ends, its int32 sums are converted to the LAST range's units
-    // (x sx_L sw_L / (sx sw)) and added to this tile's fp32 slot of a workspace
-    // the caller lends; the accumulators restart from zero.  The epilogue adds the
-    // slot to the last range's sums and scales once.  Each thread only ever reads
-    // back what it wrote itself.  This keeps the big tiles for int8 with K
-    // segments or DualScale: a few hundred KB of traffic per tile and range
+    // PARK (int8, several ranges): no second register set at all.  When a range ends, its
+    // int32 sums are scaled by the range's own 1 / (sx sw), i.e. taken to output units, and
+    // added to this tile's fp32 slot of a workspace the caller lends; the accumulators
+    // restart from zero.  The epilogue scales the last range's sums and adds the slot.
+    // Each thread only ever reads back what it wrote itself.  This keeps the big tiles for
+    // int8 with K segments or DualScale: a few hundred KB of traffic per tile and range
     // boundary against ~14 MB of operands.
+    // Neither here nor in the second register set do a range's sums pass through another
+    // range's scales: a side of a DualScale tensor that holds nothing may have the scale
+    // limit / 0 = inf and adds exact zeros, where a ratio of the two scales would make
+    // infinities and NaNs of the other side's sums.  For e4m3 that is SEP, taken where the
+    // scales come from outside (segq_krange.own_sum): 2 x 2048 x 1536 x 3072 DualScale 61.9 us
+    // rescaled in place, 62.2 us with the second set, and 256 x 256 tiles out of reach.
     static_assert(!PARK || (FOLD && !F8 && !GRP), "parking: int8 with several ranges");
     static_assert(!WS || (!FOLD && !PARK), "int8 above 256 x 256: one range");
-    constexpr bool ACCF = FOLD && !F8 && !GRP && !PARK;
+    static_assert(!SEP || (FOLD && F8 && !PARK && !FINISH), "SEP: e4m3 with several ranges");
+    constexpr bool ACCF = FOLD && (!F8 || SEP) && !GRP && !PARK;
     constexpr bool HASF = ACCF || GRP;
     const acc_t acc_zero = {0, 0, 0, 0};
     // Split K (p.splits > 1): workgroup (tile, y) multiplies the y-th share of the K steps,
@@ -810,26 +817,17 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     auto park = [&](int r) __attribute__((always_inline)) {
         if constexpr (PARK) {
             if (r < r_last) {
-                const int rl = r_last;
-                const float* sx = p.r[ph(r)].sx + z * p.bsSx;  // (a K split has no batch: its strides are 0)
-                const float* sw = p.r[ph(r)].sw + z * p.bsSw;
-                const float* sx2 = p.r[ph(rl)].sx + z * p.bsSx;
-                const float* sw2 = p.r[ph(rl)].sw + z * p.bsSw;
-                const int rs = p.r[ph(r)].sx_rs, cs = p.r[ph(r)].sw_cs, rs2 = p.r[ph(rl)].sx_rs, cs2 = p.r[ph(rl)].sw_cs;
-                float fx[TM];
+                const float* sx = p.r[ph(r)].sx;  // (one problem: parking serves no batch)
+                const float* sw = p.r[ph(r)].sw;
+                const int rs = p.r[ph(r)].sx_rs, cs = p.r[ph(r)].sw_cs;
+                float rx[TM];
 #pragma unroll
-                for (int b = 0; b < TM; ++b) {
-                    const int64_t m = min(m_base + b * 16, p.M - 1);
-                    fx[b] = sx2[m * rs2] * __builtin_amdgcn_rcpf(sx[m * rs]);
-                }
+                for (int b = 0; b < TM; ++b) rx[b] = __builtin_amdgcn_rcpf(sx[(int64_t)min(m_base + b * 16, p.M - 1) * rs]);
 #pragma unroll
                 for (int a = 0; a < TN; ++a) {
-                    v4f fw;
+                    v4f rw;
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const int64_t n = min(n_base + a * 16 + v, p.N - 1);
-                        fw[v] = sw2[n * cs2] * __builtin_amdgcn_rcpf(sw[n * cs]);
-                    }
+                    for (int v = 0; v < 4; ++v) rw[v] = __builtin_amdgcn_rcpf(sw[(int64_t)min(n_base + a * 16 + v, p.N - 1) * cs]);
                     v4f old[TM];
                     if (r > r_begin) {
 #pragma unroll
@@ -837,7 +835,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
                     }
 #pragma unroll
                     for (int b = 0; b < TM; ++b) {
-                        v4f t = __builtin_convertvector(acc[a][b], v4f) * (fw * fx[b]);
+                        v4f t = __builtin_convertvector(acc[a][b], v4f) * rx[b] * rw;
                         if (r > r_begin) t += old[b];
                         slot[(a * TM + b) * NT] = t;
                         acc[a][b] = acc_zero;
@@ -847,7 +845,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         }
     };
     auto fold = [&](int r) __attribute__((always_inline)) {
-        if constexpr (FOLD && (F8 || GRP)) {
+        if constexpr (FOLD && !ACCF && (F8 || GRP)) {
             auto& facc = [&]() -> auto& { if constexpr (GRP) return accf; else return acc; }();
             if (r < r_last) {  // rescale to the next range's units
                 const float* sx = p.r[ph(r)].sx + z * p.bsSx;
@@ -1262,9 +1260,12 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
                     v4f t;
                     if constexpr (HASF) t = accf[a][b];
                     else t = __builtin_convertvector(acc[a][b], v4f);
-                    if constexpr (PARK) t += old[i];
-                    if constexpr (!ACCF)
-                        t = t * (*reinterpret_cast<const v4f*>(epi + BM + wn * WN + a * 16 + 4 * lgrp) * epi[wm * WM + b * 16 + lrow]);
+                    if constexpr (!ACCF) {
+                        const v4f rw = *reinterpret_cast<const v4f*>(epi + BM + wn * WN + a * 16 + 4 * lgrp);
+                        const float rx = epi[wm * WM + b * 16 + lrow];
+                        if constexpr (PARK) t = t * rx * rw + old[i];
+                        else t = t * (rw * rx);
+                    }
                     of[a][b] = t;
                 }
             }
@@ -1320,7 +1321,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         v4f none[1][1];
         wide_epilogue<BM, BN, WGM, WGN, GEMM_F8, false, false>(p, accf, none, smem, z, m0, n0, wave, lane, r_epi, epi);
     } else if constexpr (PARK) {
-        // the earlier ranges' sums come back in two halves, each with all its loads in flight at once
+        // the earlier ranges' sums come back, in output units, in two halves, each with all its loads in flight at once
         v4f accp[TN][TM];
         constexpr int H = (TN + 1) / 2;
         const bool parked = r_begin < r_last;  // (a split's share can lie inside one range)
@@ -1334,10 +1335,11 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
 #pragma unroll
             for (int a = h * H; a < min(TN, (h + 1) * H); ++a)
 #pragma unroll
-                for (int b = 0; b < TM; ++b) accp[a][b] = __builtin_convertvector(acc[a][b], v4f) + old[a - h * H][b];
+                for (int b = 0; b < TM; ++b)
+                    accp[a][b] = __builtin_convertvector(acc[a][b], v4f) * epi[wm * WM + b * 16 + lrow] *
+                                     *reinterpret_cast<const v4f*>(epi + BM + wn * WN + a * 16 + 4 * lgrp) + old[a - h * H][b];
         }
-        v4f none[1][1];
-        wide_epilogue<BM, BN, WGM, WGN, GEMM_F8, false, false>(p, accp, none, smem, z, m0, n0, wave, lane, r_epi, epi);
+        wide_epilogue<BM, BN, WGM, WGN, GEMM_F8, false, true>(p, accp, accp, smem, z, m0, n0, wave, lane, r_epi, epi);
     } else if constexpr (CODES) {
         codes_epilogue<BM, BN, WGM, WGN, FMT>(p, acc, smem, m0, n0, wave, lane, epi);
     } else {
@@ -1359,9 +1361,9 @@ int launch_wide_instance(const GemmParams& p, int64_t batch, hipStream_t st) {
 
 // wide tile ids (after the generic ones): 256x256 | 256x128 | 128x256 | 128x128, eight waves each
 template <int BM, int BN, int WGM, int WGN, int FMT, bool FOLD, int NS, bool GRP = false, bool PARK = false, bool FINISH = false,
-          bool CODES = false>
+          bool CODES = false, bool SEP = false>
 int launch_pipe_instance(const GemmParams& p, int64_t batch, hipStream_t st) {
-    auto kern = gemm_pipe_kernel<BM, BN, WGM, WGN, FMT, FOLD, NS, GRP, PARK, FINISH, CODES>;
+    auto kern = gemm_pipe_kernel<BM, BN, WGM, WGN, FMT, FOLD, NS, GRP, PARK, FINISH, CODES, SEP>;
     // the stages, the epilogue's vectors, and the ring of group factors
     constexpr int lds = NS * (BM + BN) * BK + (BM + 2 * BN) * 4 + (GRP ? 4 * BN * 4 : 0);
     if (p.dry) return SEGQ_OK;
@@ -1440,18 +1442,6 @@ int launch_wide(const GemmParams& p, int wcfg, bool fold, bool asel, int64_t bat
                         }
                         break;
                 }
-            } else if constexpr (F8W) {  // fp32 accumulators are rescaled in place: every tile serves several ranges
-                switch (wcfg) {
-                    case 0: SEGQ_PIPE2(256, 256, 4, 2, true, false);
-                    case 1: SEGQ_PIPE2(256, 128, 4, 2, true, false);
-                    case 2: SEGQ_PIPE1(128, 256, 2, 4, true, false);
-                    case 3: SEGQ_PIPE2(128, 128, 4, 2, true, false);
-                    case 4: SEGQ_PIPE1(192, 288, 4, 2, true, false);
-                    case 5: SEGQ_PIPE1(288, 192, 2, 4, true, false);
-                    case 6: SEGQ_PIPE2(256, 192, 4, 2, true, false);
-                    case 7: SEGQ_PIPE2(192, 256, 2, 4, true, false);
-                    case 9: SEGQ_PIPE1(384, 192, 4, 2, true, false);
-                }
             } else if (p.park) {  // int8, several ranges, a workspace to park finished ranges in: every tile
                 if constexpr (!F8W) {
                     switch (wcfg) {
@@ -1463,6 +1453,28 @@ int launch_wide(const GemmParams& p, int wcfg, bool fold, bool asel, int64_t bat
                         case 5: SEGQ_PIPE1(288, 192, 2, 4, true, true);
                         case 6: SEGQ_PIPE2(256, 192, 4, 2, true, true);
                         case 7: SEGQ_PIPE2(192, 256, 2, 4, true, true);
+                    }
+                }
+            } else if constexpr (F8W) {
+                if (p.sep) {  // independent sums without a workspace: a second register set
+                    if (!tail) {
+                        switch (wcfg) {
+                            case 0: case 1: return launch_pipe_instance<256, 128, 4, 2, FMT, true, 2, false, false, false, false, F8W>(p, batch, st);
+                            case 2: return launch_pipe_instance<128, 256, 2, 4, FMT, true, 2, false, false, false, false, F8W>(p, batch, st);
+                            case 3: return launch_pipe_instance<128, 128, 4, 2, FMT, true, 2, false, false, false, false, F8W>(p, batch, st);
+                        }
+                    }
+                } else {  // fp32 accumulators are rescaled in place: every tile serves several ranges
+                    switch (wcfg) {
+                        case 0: SEGQ_PIPE2(256, 256, 4, 2, true, false);
+                        case 1: SEGQ_PIPE2(256, 128, 4, 2, true, false);
+                        case 2: SEGQ_PIPE1(128, 256, 2, 4, true, false);
+                        case 3: SEGQ_PIPE2(128, 128, 4, 2, true, false);
+                        case 4: SEGQ_PIPE1(192, 288, 4, 2, true, false);
+                        case 5: SEGQ_PIPE1(288, 192, 2, 4, true, false);
+                        case 6: SEGQ_PIPE2(256, 192, 4, 2, true, false);
+                        case 7: SEGQ_PIPE2(192, 256, 2, 4, true, false);
+                        case 9: SEGQ_PIPE1(384, 192, 4, 2, true, false);
                     }
                 }
             } else {

@@ -341,7 +341,7 @@ def gemm_desc(a: torch.Tensor, b: torch.Tensor, ranges: Sequence[Range], *, m: i
          batch_stride_sx: int = 0, batch_stride_sw: int = 0, out: Optional[torch.Tensor] = None,
          tile: int = 0, workspace: Optional[torch.Tensor] = None,
          group_dequant: Optional[torch.Tensor] = None, split_k: int = 0,
-         addend: Optional[torch.Tensor] = None, lowrank=None, out_codes: Optional[dict] = None):
+         addend: Optional[torch.Tensor] = None, lowrank=None, out_codes: Optional[dict] = None, own_sums: bool = False):
     """The ``segq_gemm_desc`` of a segmented GEMM with fused de-quantisation and bias, its output
     tensor, the launch's description and the tensors the descriptor points into.
 
@@ -358,7 +358,8 @@ def gemm_desc(a: torch.Tensor, b: torch.Tensor, ranges: Sequence[Range], *, m: i
     ``out_dtype`` is a torch float dtype, or the string ``"acc"`` for the raw
     accumulators (int32 for integer codes, float32 for e4m3).  ``workspace``: a
     byte tensor the library may expand int4 weights into, or park the sums of
-    finished int8 ranges in (see ``int4_workspace``, ``park_bytes``).
+    finished int8 ranges in (see ``int4_workspace``, ``park_bytes``).  ``own_sums``: sum every
+    e4m3 range on its own, for scales that may be infinite (``segq_krange.own_sum``).
     """
     _need_cuda(a, b, a_neg, bias)
     raw = out_dtype == "acc"
@@ -443,6 +444,7 @@ def gemm_desc(a: torch.Tensor, b: torch.Tensor, ranges: Sequence[Range], *, m: i
                 raise RuntimeError("scales must be float32")
         kr.sx = r.sx.data_ptr() if r.sx is not None else None
         kr.sw = r.sw.data_ptr() if r.sw is not None else None
+    d.ranges[0].own_sum = 1 if own_sums else 0
     info = dict(m=m, n=n, batch=batch, k_alg=sum(r.k_len for r in ranges if r.a_sel in (0, 2)),
                 k_exec=sum(r.k_len for r in ranges), a_fmt=a_fmt, b_fmt=b_fmt)
     if oc is not None:
@@ -513,6 +515,23 @@ def real_quantized_gemm_scaled(fmt_a: str, fmt_w: str, inputs: torch.Tensor, wei
     return out
 
 
+def _dual_in_two_tensors(tiles: int, K: int, int4: bool) -> bool:
+    """Whether the DualScale operator writes two code tensors, which stream straight into LDS, or one
+    merged tensor, whose signs the GEMM selects on the way there.  ``tiles``: 128 x 128 tiles of the output.
+
+    Two where the GEMM then runs on the 8-wave kernels (plain 8-bit codes from 32 tiles, int4 weights from 96, K in
+    whole 128-byte steps) and its K loop repays the second tensor.  Both launches, merged / two, us: 512 x 1024,
+    32 tiles, K 256 13.9 / 10.5 (merged runs on the general kernel up to 95 tiles); 2 x 1000 x 1000, 128 tiles,
+    K 256 12.4 / 13.2, K 512 16.0 / 16.5, K 2048 40 / 34; 2 x 3000 x 3000, 1152 tiles, K 256 40.5 / 39.5,
+    K 512 56.6 / 49.5, K 4096 261 / 186.  int4, 256 tiles, K 1536 33.8 / 35.8, K 2048 42.8 / 41.5;
+    1152 tiles, K 512 59.6 / 54.4."""
+    if K % 128 or tiles < (96 if int4 else 32):
+        return False
+    if int4:  # (256 tiles: one for every compute unit)
+        return K >= (512 if tiles > 256 else 2048)
+    return tiles < 96 or K >= 512
+
+
 def real_quantized_gemm_dual_scaled(fmt_a: str, fmt_w: str, inputs: torch.Tensor, weights: torch.Tensor,
                                     pos_scale_x: torch.Tensor, neg_scale_x: torch.Tensor,
                                     scale_w: torch.Tensor) -> torch.Tensor:
@@ -520,11 +539,11 @@ def real_quantized_gemm_dual_scaled(fmt_a: str, fmt_w: str, inputs: torch.Tensor
 
     One quantise launch over all segments and one batched GEMM that reads every
     segment as two ranges, the non-negative codes with the positive scale and the
-    negative ones with the negative scale.  K in whole 128-byte steps: two code
-    tensors, which stream straight into LDS (int8 also parks the first range's sums
-    in the workspace and keeps the big tiles; (2, 2048, 3072) x 1536, fp16, the whole
-    pass: 76.7 us with the sign selected in registers, 65.2 us like this).  Any
-    other K runs on the general kernel, where one merged tensor is a third less to write.
+    negative ones with the negative scale.  Each range is summed on its own (a
+    second register set): the scales come from the caller, and a side that holds
+    nothing may have ``limit / 0 = inf``, whose zeros add nothing.  No workspace:
+    the operator shares no buffer with any other launch.  (2, 2048, 3072) x 1536,
+    fp16, the whole pass: 76.7 us from one merged tensor, 62.2 us from two.
     """
     _check_contract(inputs, weights, fmt_w, pos_scale_x, neg_scale_x, scale_w)
     S, M, N, K = _shapes(inputs, weights, fmt_w)
@@ -534,7 +553,7 @@ def real_quantized_gemm_dual_scaled(fmt_a: str, fmt_w: str, inputs: torch.Tensor
         raise RuntimeError("pos/neg scale_x must both have S or S*M entries")
     if not per_seg_w and scale_w.numel() != S * N:
         raise RuntimeError(f"scale_w has {scale_w.numel()} entries, expected {S} or {S * N}")
-    two = K % 128 == 0
+    two = _dual_in_two_tensors(S * -(-M // 128) * -(-N // 128), K, fmt_w == FMT_INT4)
     codes = quantize(inputs.view(S * M, K), fmt_a, pos_scale_x, neg_scale_x, seg_rows=M,
                      seg_stride=1 if per_seg_x else M, row_stride=0 if per_seg_x else 1, dual=True, two_tensors=two)
     codes, codes_neg = codes if two else (codes, None)
@@ -542,13 +561,11 @@ def real_quantized_gemm_dual_scaled(fmt_a: str, fmt_w: str, inputs: torch.Tensor
     kb = K // 2 if fmt_w == FMT_INT4 else K
     rs, cs = (0 if per_seg_x else 1), (0 if per_seg_w else 1)
     sel = (0, 1) if two else (2, 3)
-    g = gemm_desc(codes, weights,
-                  [Range(0, K, pos_scale_x, scale_w, sel[0], rs, cs), Range(0, K, neg_scale_x, scale_w, sel[1], rs, cs)],
-                  m=M, n=N, a_fmt=fmt_a, b_fmt=fmt_w, out_dtype=inputs.dtype, lda=K, ldb=kb, a_neg=codes_neg,
-                  batch=S, batch_stride_a=M * K, batch_stride_b=N * kb,
-                  batch_stride_sx=1 if per_seg_x else M, batch_stride_sw=1 if per_seg_w else N, out=out)
-    need = gemm_workspace_bytes(g) if two and fmt_w != FMT_INT4 else 0
-    gemm_launch(g, int4_workspace(inputs.device, need) if need else None)
+    gemm(codes, weights,
+         [Range(0, K, pos_scale_x, scale_w, sel[0], rs, cs), Range(0, K, neg_scale_x, scale_w, sel[1], rs, cs)],
+         m=M, n=N, a_fmt=fmt_a, b_fmt=fmt_w, out_dtype=inputs.dtype, lda=K, ldb=kb, a_neg=codes_neg,
+         batch=S, batch_stride_a=M * K, batch_stride_b=N * kb,
+         batch_stride_sx=1 if per_seg_x else M, batch_stride_sw=1 if per_seg_w else N, out=out, own_sums=True)
     return out
 
 

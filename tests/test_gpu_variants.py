@@ -120,3 +120,122 @@ def test_general_gemm_steps_in_flight(fa, fb, lens):
             # int8: fp32 scaling of exact sums, a few roundings of 2^-24 per range; e4m3: the matrix cores' limited-width adder
             tol = 3e-4 if fa == O.FMT_E4M3 else 1e-6
             assert (np.abs(y.cpu().numpy().astype(np.float64) - exact) <= tol * mag + 2.0 ** -22 * np.abs(exact)).all(), (lens, bt, tile)
+
+
+class _Plans:
+    """What each GEMM launched through ``ops.gemm`` from here on runs as (``gemm_plan`` of its descriptor)."""
+
+    def __init__(self, monkeypatch):
+        from segquant_amd import ops
+        self.seen = []
+        desc = ops.gemm_desc
+
+        def record(*args, **kw):
+            g = desc(*args, **kw)
+            self.seen.append(dict(ops.gemm_plan(g), two=g[0].a_neg is not None, workspace=g[0].workspace))
+            return g
+        monkeypatch.setattr(ops, "gemm_desc", record)
+
+
+def _dual_case(fmt, S, M, N, K, per_token, sides, seed, int4=False):
+    """Inputs, unclamped scales and the fp64 result of the DualScale operator; ``sides``: which signs each segment (or
+    token, in turn) holds, an empty one having the scale limit / 0 = inf.  Column 1 of the weights is zero, its scale too."""
+    g = torch.Generator().manual_seed(seed)
+    x = torch.nn.functional.gelu(torch.randn(S, M, K, generator=g)) * 10.0 ** torch.randint(-2, 3, (S, 1, 1), generator=g)
+    for i in range(S * (M if per_token else 1)):
+        part = x.view(S * M, K)[i] if per_token else x[i]
+        side = sides[i % len(sides)]
+        if side == "+":
+            part.clamp_(min=0.0)
+        elif side == "-":
+            part.copy_(-(part.abs() + 1e-3))
+    lim = (127.0, 128.0) if fmt == O.FMT_INT8 else (448.0, 448.0)
+    over = 2 if per_token else (1, 2)
+    pos, neg = lim[0] / x.amax(dim=over).clamp(min=0.0), lim[1] / (-x).amax(dim=over).clamp(min=0.0)
+    rng = np.random.default_rng(seed)
+    lo = -8 if int4 else -128
+    w = rng.integers(lo, -lo, size=(S, N, K)).astype(np.int8) if fmt == O.FMT_INT8 else \
+        np.where((c := rng.integers(0, 256, size=(S, N, K)).astype(np.uint8)) & 0x7F == 0x7F, 0x3A, c).astype(np.uint8)
+    sw = torch.rand(S, N, generator=g) * 30 + 10
+    w[:, 1], sw[:, 1] = 0, float("inf")
+    want, mag = np.empty((S, M, N)), np.empty((S, M, N))
+    for s in range(S):
+        rows = lambda t: t[s].numpy().astype(np.float64).reshape(-1, 1) + np.zeros((M, 1))
+        with np.errstate(invalid="ignore"):
+            yp, yn = O.quantize_act_dual(x[s:s + 1].numpy(), pos[s].numpy().reshape(-1), neg[s].numpy().reshape(-1), fmt)
+        wv, p, n = O.code_values(w[s], fmt), O.code_values(yp[0], fmt), O.code_values(yn[0], fmt)
+        col = sw[s].numpy().astype(np.float64)[None, :]
+        want[s] = ((p @ wv.T) / rows(pos) + (n @ wv.T) / rows(neg)) / col
+        mag[s] = ((np.abs(p) @ np.abs(wv).T) / rows(pos) + (np.abs(n) @ np.abs(wv).T) / rows(neg)) / col
+    return x, w, pos, neg, sw, want, mag
+
+
+@pytest.mark.parametrize("fmt", [O.FMT_INT8, O.FMT_E4M3])
+@pytest.mark.parametrize("S,M,N,K,tile,two", [(2, 300, 200, 256, "64x128", False), (1, 1100, 1000, 208, "64x128", False),
+                                              (2, 600, 700, 256, "128x128", True), (3, 400, 600, 384, "128x128", True), (3, 500, 900, 384, "128x128", False),
+                                              (1, 3000, 1500, 384, "256x128", False), (2, 2000, 2000, 512, "256x128", True),
+                                              (1, 300, 20000, 512, "128x256", True)])
+@pytest.mark.parametrize("per_token,sides", [(False, ["+-"]), (False, ["+", "-", "+-"]), (False, ["-"]), (True, ["+-", "+", "-"])])
+def test_dual_operator_sides(monkeypatch, fmt, S, M, N, K, tile, two, per_token, sides):
+    """The DualScale operator on every kernel that serves it, from one merged code tensor and from two: batches, ragged
+    edges, scales far apart from segment to segment or token to token, and sides that hold nothing, whose scale is
+    infinite and whose contribution is zero.  It borrows no workspace and shares no tile's K steps."""
+    from segquant_amd import ops
+    x, w, pos, neg, sw, want, mag = _dual_case(fmt, S, M, N, K, per_token, sides, S + M + N + K)
+    plans = _Plans(monkeypatch)
+    out = ops.real_quantized_gemm_dual_scaled(fmt, fmt, x.to(DEV), torch.from_numpy(w).to(DEV), pos.reshape(-1).to(DEV),
+                                              neg.reshape(-1).to(DEV), sw.to(DEV)).cpu().numpy()
+    assert [(p["shape"], p["two"], p["parked"], p["splits"], p["workspace"]) for p in plans.seen] == [(tile, two, False, 1, None)]
+    # int8: per range an exact sum, its conversion, two reciprocals (1 ulp each) and two products, then the addition:
+    # 8 x 2^-24 = 4.8e-7; e4m3: the matrix cores' limited-width adder
+    assert (np.abs(out - want) <= (5e-7 if fmt == O.FMT_INT8 else 3e-4) * mag).all()
+
+
+@pytest.mark.parametrize("S,M,N,K,two", [(1, 700, 500, 512, False), (2, 1000, 1000, 256, False), (1, 2100, 2100, 512, True)])
+def test_dual_operator_sides_int4(monkeypatch, S, M, N, K, two):
+    """The same with int4 weights, which are unpacked on their way into LDS."""
+    from segquant_amd import ops
+    x, w, pos, neg, sw, want, mag = _dual_case(O.FMT_INT8, S, M, N, K, True, ["+-", "+", "-"], S + M + N + K, int4=True)
+    packed = np.stack([np.stack([O.pack_int4(r) for r in ws]).reshape(-1) for ws in w])
+    plans = _Plans(monkeypatch)
+    out = ops.real_quantized_gemm_dual_scaled(O.FMT_INT8, O.FMT_INT4, x.to(DEV), torch.from_numpy(packed).to(DEV), pos.reshape(-1).to(DEV),
+                                              neg.reshape(-1).to(DEV), sw.to(DEV)).cpu().numpy()
+    assert [(p["two"], p["workspace"]) for p in plans.seen] == [(two, None)]
+    assert (np.abs(out - want) <= 5e-7 * mag).all()
+
+
+@pytest.mark.parametrize("empty", [0, 1, 2])
+@pytest.mark.parametrize("split_k", [1, 2, 3])
+@pytest.mark.parametrize("tile", [11, 12, 13, 14, 15, 16, 17, 18])
+def test_parked_ranges_with_an_infinite_scale(tile, split_k, empty):
+    """int8 ranges whose sums are parked, whole tiles and K shares: a range of zero codes with an infinite scale (the
+    first, the middle or the last one) adds nothing to the others, whose scales lie nine orders of magnitude apart."""
+    from segquant_amd import ops
+    M, N, lens = 300, 333, (256, 128, 384)
+    K = sum(lens)
+    rng = np.random.default_rng(tile * 10 + split_k)
+    a, b = rng.integers(-128, 128, size=(M, K)).astype(np.int8), rng.integers(-128, 128, size=(N, K)).astype(np.int8)
+    sx, sw = rng.uniform(1, 2, size=(3, M)).astype(np.float32), rng.uniform(1, 2, size=(3, N)).astype(np.float32)
+    sx[1] *= 1e9
+    sx[empty, ::2] = np.inf
+    sw[empty, 5] = np.inf
+    k0 = sum(lens[:empty])
+    a[::2, k0:k0 + lens[empty]] = 0
+    b[5, k0:k0 + lens[empty]] = 0
+    ad, bd = torch.from_numpy(a).to(DEV), torch.from_numpy(b).to(DEV)
+    sxd, swd = torch.from_numpy(sx).to(DEV), torch.from_numpy(sw).to(DEV)
+    want, mag, ranges, k = 0.0, 0.0, [], 0
+    for i, n in enumerate(lens):
+        f = 1.0 / (sx[i].astype(np.float64)[:, None] * sw[i].astype(np.float64)[None, :])
+        va, vb = a[:, k:k + n].astype(np.float64), b[:, k:k + n].astype(np.float64)
+        want, mag = want + (va @ vb.T) * f, mag + (np.abs(va) @ np.abs(vb).T) * f
+        ranges.append(ops.Range(k, n, sxd[i], swd[i], 0, 1, 1))
+        k += n
+    ws = torch.full((ops.split_bytes(M, N, split_k, park=True),), 0xFF, dtype=torch.uint8, device=DEV)
+    kw = dict(m=M, n=N, a_fmt=O.FMT_INT8, b_fmt=O.FMT_INT8, out_dtype=torch.float32, lda=K, ldb=K, tile=tile, split_k=split_k)
+    g = ops.gemm_desc(ad, bd, ranges, workspace=ws, **kw)
+    if split_k == 1 or tile not in (13, 12, 14):  # (the smaller tiles' K shares keep a second register set)
+        assert ops.gemm_plan(g)["parked"]
+    out = ops.gemm_launch(g).cpu().numpy()
+    # 8 roundings of 2^-24 per term as above, one more per K share
+    assert (np.abs(out - want) <= 8e-7 * mag).all()

@@ -596,3 +596,34 @@ def test_plan_refuses_what_the_launch_would_refuse():
     assert status(4608, 9216, [(0, 3072, 0)], I8, 15, lowrank=32) == 2   # 192 x 288 has no low-rank finish
     assert status(4608, 9216, [(0, 3072, 0)], I8, 11, lowrank=32) == 0
     assert status(4608, 9216, [(0, 3072, 0)], I8, 0, lowrank=32) == 0    # the library's own choice always has a kernel
+
+
+def test_plan_of_ranges_summed_on_their_own():
+    """own_sum: e4m3 ranges in a second register set, as int8 ranges without a workspace have it, on the tiles built for
+    it; a workspace is not used; neither a K split nor a low-rank branch is combined with it."""
+    import ctypes as C
+    from segquant_amd import _lib as L
+    lib = L.lib()
+
+    def plan(m, n, fmt=1, tile=0, split_k=0, lowrank=0, own=1):
+        d = L.GemmDesc()
+        d.a_fmt = d.b_fmt = fmt
+        d.out_dtype = d.bias_dtype = 2
+        d.m, d.n, d.lda, d.ldb, d.ldo, d.batch = m, n, 512, 512, n, 1
+        d.a, d.a_neg, d.b, d.out = 0x10000000, 0x20000000, 0x30000000, 0x40000000
+        d.n_ranges, d.tile, d.split_k = 2, tile, split_k
+        for i in range(2):
+            d.ranges[i].k_len, d.ranges[i].a_sel, d.ranges[i].sx, d.ranges[i].sw = 512, i, 0x60000000, 0x70000000
+        d.ranges[0].own_sum = own
+        if lowrank:
+            d.lowrank_t, d.lowrank_l2t, d.lowrank_rank, d.ld_lowrank_t, d.ld_lowrank_l2t = 0x80000000, 0x90000000, lowrank, lowrank, lowrank
+        if fmt == 1:
+            d.workspace, d.workspace_bytes = 0xA0000000, 1 << 34
+        t, s, p = C.c_int32(0), C.c_int32(0), C.c_int32(0)
+        return lib.segq_gemm_plan(C.byref(d), C.byref(t), C.byref(s), C.byref(p)), t.value, s.value, p.value
+
+    for m, n, tile in ((496, 1000, 14), (384, 1280, 4), (3000, 3000, 14), (2000, 4000, 12)):
+        # (int8 without a workspace takes the same tile: the two formats follow one rule)
+        assert plan(m, n) == (0, tile, 1, 0) and plan(m, n, fmt=0) == (0, tile, 1, 0)
+    assert plan(496, 1000, split_k=2)[0] == 2 and plan(2000, 4000, lowrank=32)[0] == 2
+    assert plan(2000, 4000, tile=15)[0] == 2 and plan(2000, 4000, tile=15, own=0)[0] == 0
