@@ -607,6 +607,20 @@ __device__ __forceinline__ void lowrank_accumulate(const GemmParams& p, v4f (&of
 // s_waitcnt immediate for "vmcnt(n) lgkmcnt(0)" on gfx9-family encodings
 constexpr int waitcnt_vm_lgkm0(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
 
+// 1 / x for the second register set of int8 ranges: v_rcp_f32 (1 ulp) and one Newton step, with which the sums lie as
+// close to the exact ones as with correctly rounded quotients, which the general kernel takes for the same launches when
+// they are small or ragged; v_rcp_f32 through a ratio of two scales put them 1.4 times as far (rms).  0, infinities and
+// NaN have no finite residual and keep v_rcp_f32's value.  512 x 1024 x 512, two ranges, with the quantise launch: v_rcp_f32 13.4 us, this
+// 13.8, divisions 14.6.  e4m3 keeps v_rcp_f32: the matrix cores' own sums are off by hundreds of times as much; parked
+// sums too, whose launches are the layers' long ones (9216 x 15360 x 3072: 0.2 % more with the Newton step).
+template <int FMT>
+__device__ __forceinline__ float recip(float x) {
+    const float y = __builtin_amdgcn_rcpf(x);
+    if constexpr (FMT == GEMM_F8) return y;
+    const float e = __builtin_fmaf(-x, y, 1.0f);
+    return __builtin_fabsf(e) < 1.0f ? __builtin_fmaf(y, e, y) : y;
+}
+
 template <int BM, int BN, int WGM, int WGN, int FMT, bool FOLD, int NS, bool GRP = false, bool PARK = false, bool FINISH = false,
           bool CODES = false,  // CODES: the epilogue writes the next linear's codes instead of floats (one range)
           bool SEP = false>    // SEP (e4m3, several ranges): a second register set, as int8 has it, instead of rescaling in place
@@ -878,12 +892,12 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
             const int rs = p.r[ph(r)].sx_rs, cs = p.r[ph(r)].sw_cs;
             float rx[TM];
 #pragma unroll
-            for (int b = 0; b < TM; ++b) rx[b] = __builtin_amdgcn_rcpf(sx[(int64_t)min(m_base + b * 16, p.M - 1) * rs]);
+            for (int b = 0; b < TM; ++b) rx[b] = recip<FMT>(sx[(int64_t)min(m_base + b * 16, p.M - 1) * rs]);
 #pragma unroll
             for (int a = 0; a < TN; ++a) {
                 float rw[4];
 #pragma unroll
-                for (int v = 0; v < 4; ++v) rw[v] = __builtin_amdgcn_rcpf(sw[(int64_t)min(n_base + a * 16 + v, p.N - 1) * cs]);
+                for (int v = 0; v < 4; ++v) rw[v] = recip<FMT>(sw[(int64_t)min(n_base + a * 16 + v, p.N - 1) * cs]);
 #pragma unroll
                 for (int b = 0; b < TM; ++b) {
 #pragma unroll

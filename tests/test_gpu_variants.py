@@ -239,3 +239,22 @@ def test_parked_ranges_with_an_infinite_scale(tile, split_k, empty):
     out = ops.gemm_launch(g).cpu().numpy()
     # 8 roundings of 2^-24 per term as above, one more per K share
     assert (np.abs(out - want) <= 8e-7 * mag).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(500, 1100, 2048), (900, 2100, 512), (2100, 4000, 512), (130, 70, 512)])
+def test_dual_operator_lies_as_close_as_single_precision_allows(M, N, K):
+    """int8, fp32 out: no further from the exact result than the same sums scaled in single precision with correctly
+    rounded reciprocals."""
+    from segquant_amd import ops
+    rng = np.random.default_rng(K + M)
+    codes, b = rng.integers(-128, 128, size=(M, K)).astype(np.int8), rng.integers(-128, 128, size=(N, K)).astype(np.int8)
+    sx, sw = rng.uniform(1, 2, size=(2, M)).astype(np.float32), rng.uniform(1, 2, size=N).astype(np.float32)
+    x = codes / np.where(codes >= 0, sx[0][:, None], sx[1][:, None])  # (x times its scale lies within 1e-5 of the code)
+    out = ops.real_quantized_gemm_dual_scaled(O.FMT_INT8, O.FMT_INT8, torch.from_numpy(x[None].astype(np.float32)).to(DEV), torch.from_numpy(b[None]).to(DEV),
+                                              *(torch.from_numpy(t).to(DEV) for t in (sx[0], sx[1], sw)))[0].cpu().numpy()
+    sums = [f(codes, 0).astype(np.float64) @ b.T.astype(np.float64) for f in (np.maximum, np.minimum)]
+    exact = sum(s / (v[:, None].astype(np.float64) * sw[None, :].astype(np.float64)) for s, v in zip(sums, sx))
+    one = np.float32(1)
+    single = sum(s.astype(np.float32) * (one / v)[:, None] * (one / sw)[None, :] for s, v in zip(sums, sx))
+    rms = lambda e: np.sqrt(np.mean(np.square(e)))
+    assert rms(out - exact) <= 1.02 * rms(single - exact)
