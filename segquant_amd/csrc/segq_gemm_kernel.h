@@ -151,7 +151,8 @@ template <int FMT> struct AccT;
 template <> struct AccT<GEMM_I8> { typedef v4i type; typedef int32_t elem; };
 template <> struct AccT<GEMM_F8> { typedef v4f type; typedef float elem; };
 
-template <int BM, int BN, int WGM, int WGN, int FMT, bool B4, bool FOLD>
+// DEPTH: K steps whose loads are in flight in registers (deep_steps() says which launches take which)
+template <int BM, int BN, int WGM, int WGN, int FMT, bool B4, bool FOLD, int DEPTH>
 __global__ void __launch_bounds__(WGM* WGN * 64) gemm_kernel(const GemmParams p) {
     constexpr int NT = WGM * WGN * 64;
     constexpr int WM = BM / WGM, WN = BN / WGN;
@@ -161,13 +162,6 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_kernel(const GemmParams p)
     static_assert(BM * 8 % NT == 0 && BN * 4 % NT == 0, "tile does not divide over the threads");
     static_assert((NT / 8) % 16 == 0, "row swizzle must not depend on the load iteration");
     static_assert(!B4 || FMT == GEMM_I8, "int4 weights pair with int8 activations");
-    // K steps whose loads are in flight in registers.  The dispatch gives the 64 x 128 tile at most two
-    // workgroups per CU, so that nothing else hides a step's wait for memory; 128 x 128 has room for two
-    // sets below the 256 registers at which two workgroups share a CU.  Whole passes, one step ahead and
-    // scales read in the epilogue -> this: 333 x 1000 x 1168 int8 19.8 -> 18.6 us, 154 x 5120 x 1280 int4
-    // 21.6 -> 19.7 us.  What is left is the serial chain of a step (LDS write, barrier, LDS read, MFMA).
-    // (Several ranges: a second accumulator set takes that room; e4m3, with twice the fragments, has none left.)
-    constexpr int DEPTH = BM * BN > 128 * 128 ? 1 : !FOLD ? (BM * BN <= 64 * 128 ? 4 : 2) : BM * BN <= 64 * 128 && FMT == GEMM_I8 ? 2 : 1;
     // scales and bias are read before the K loop where registers allow it: read in the epilogue they are a
     // chain of TN round trips to memory, as no load passes the stores of the columns before
     constexpr bool EARLY = BM * BN <= 64 * 128;
@@ -426,10 +420,15 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_kernel(const GemmParams p)
         }
     };
     int lr = 0, lk = p.r[0].k0;  // the step that is loaded next; past the end the last range's first, unused
+    bool past = false;
     auto load_next = [&](uint4 (&qa)[A_IT], uint4 (&qb)[B_IT]) {
+        // (one step ahead every wait is for all loads, so that a branch costs one range nothing, and saves short ones
+        // 2 %; with several ranges it costs e4m3 5 %)
+        if (DEPTH == 1 && !FOLD && past) return;
         load_tile(lr, lk, qa, qb);
         advance(lr, lk);
         if (lr >= p.nr) {
+            past = true;
             lr = p.nr - 1;
             lk = p.r[lr].k0;
         }
@@ -545,9 +544,25 @@ constexpr TileCfg TILE_CFGS[NUM_TILE_CFG] = {
     {256, 192, 4, 2}, {192, 256, 2, 4}, {128, 128, 2, 4}, {384, 192, 4, 2}, {128, 96, 4, 2},
 };
 
-template <int BM, int BN, int WGM, int WGN, int FMT, bool B4, bool FOLD>
+// Steps in flight of the general kernel's 64 x 128 and 128 x 128 tiles, one range (every other launch: one step ahead;
+// with several ranges a second accumulator set takes the registers of it: at two steps 64 x 128 int8 passes the 256 at
+// which two workgroups share a CU, 2048 x 1500 x 400 in two ranges 17.1 -> 29.6 us).  Past its last step a workgroup of
+// a deep launch loads DEPTH steps that it does not use, so that no load hangs on a branch and each step is waited for
+// alone; that has to be repaid (us, one step ahead -> this):
+//   64 x 128, four steps in flight, at most one workgroup per CU (nothing else hides its waits), six K steps or more:
+//     700 x 2560 x 2064 int8 25.0 -> 20.2, 333 x 1000 x 1168 14.2 -> 13.5; three K steps 8.2 -> 8.4; 384 tiles,
+//     2048 x 1500 x 656 12.6 -> 13.9
+//   128 x 128, two steps in flight, four K steps or more: 4000 x 3000 x 2064 int8 62.5 -> 58.3, x 784 36.2 -> 35.4;
+//     two K steps 22.8 -> 23.4
+inline bool deep_steps(const GemmParams& p, int bm, int64_t batch) {
+    int64_t steps = 0;
+    for (int i = 0; i < p.nr; ++i) steps += (p.r[i].k1 - p.r[i].k0 + BK - 1) / BK;
+    return bm > 64 ? steps >= 4 : steps >= 6 && (int64_t)p.tiles_m * p.tiles_n * batch <= device_cus();
+}
+
+template <int BM, int BN, int WGM, int WGN, int FMT, bool B4, bool FOLD, int DEPTH = 1>
 int launch_instance(const GemmParams& p, int64_t batch, hipStream_t st) {
-    auto kern = gemm_kernel<BM, BN, WGM, WGN, FMT, B4, FOLD>;
+    auto kern = gemm_kernel<BM, BN, WGM, WGN, FMT, B4, FOLD, DEPTH>;
     constexpr int lds = 2 * (BM + BN) * BK;
     if (p.dry) return SEGQ_OK;
     static unsigned long long attr_done = 0;
@@ -573,9 +588,13 @@ int launch_format(const GemmParams& p, int cfg, bool fold, int64_t batch, hipStr
         case 0: return launch_instance<256, 256, 2, 2, FMT, B4, false>(p, batch, st);
         case 2: return launch_instance<256, 128, 2, 2, FMT, B4, false>(p, batch, st);
         case 3: return launch_instance<256, 128, 2, 2, FMT, B4, true>(p, batch, st);
-        case 4: return launch_instance<128, 128, 2, 2, FMT, B4, false>(p, batch, st);
+        case 4:
+            return deep_steps(p, 128, batch) ? launch_instance<128, 128, 2, 2, FMT, B4, false, 2>(p, batch, st)
+                                             : launch_instance<128, 128, 2, 2, FMT, B4, false>(p, batch, st);
         case 5: return launch_instance<128, 128, 2, 2, FMT, B4, true>(p, batch, st);
-        case 6: return launch_instance<64, 128, 2, 2, FMT, B4, false>(p, batch, st);
+        case 6:
+            return deep_steps(p, 64, batch) ? launch_instance<64, 128, 2, 2, FMT, B4, false, 4>(p, batch, st)
+                                            : launch_instance<64, 128, 2, 2, FMT, B4, false>(p, batch, st);
         case 7: return launch_instance<64, 128, 2, 2, FMT, B4, true>(p, batch, st);
         case 8: return launch_instance<128, 256, 2, 2, FMT, B4, false>(p, batch, st);
         case 9: return launch_instance<128, 256, 2, 2, FMT, B4, true>(p, batch, st);

@@ -627,3 +627,35 @@ def test_plan_of_ranges_summed_on_their_own():
         assert plan(m, n) == (0, tile, 1, 0) and plan(m, n, fmt=0) == (0, tile, 1, 0)
     assert plan(496, 1000, split_k=2)[0] == 2 and plan(2000, 4000, lowrank=32)[0] == 2
     assert plan(2000, 4000, tile=15)[0] == 2 and plan(2000, 4000, tile=15, own=0)[0] == 0
+
+
+def _kernel_registers():
+    """Mangled kernel name -> vector registers per lane, from the metadata the compiler leaves in the library built here."""
+    import struct
+    msgpack = pytest.importorskip("msgpack")
+    from segquant_amd import _lib
+    blob = open(_lib.LIB_PATH, "rb").read()
+    found, at = {}, blob.find(b"\x7fELF\x02\x01\x01\x40")  # the device code objects
+    while at >= 0:
+        sections, = struct.unpack_from("<Q", blob, at + 0x28)
+        count, = struct.unpack_from("<H", blob, at + 0x3C)
+        for i in range(count):
+            head = at + sections + 64 * i
+            if struct.unpack_from("<I", blob, head + 4)[0] != 7:  # SHT_NOTE
+                continue
+            note = at + struct.unpack_from("<Q", blob, head + 24)[0]
+            name, size, kind = struct.unpack_from("<III", blob, note)
+            if kind == 32:  # NT_AMDGPU_METADATA
+                start = note + 12 + (name + 3) // 4 * 4
+                for k in msgpack.unpackb(blob[start:start + size])["amdhsa.kernels"]:
+                    found[k[".name"]] = k[".vgpr_count"]
+        at = blob.find(b"\x7fELF\x02\x01\x01\x40", at + 64)
+    return found
+
+
+def test_two_workgroups_of_the_general_kernel_share_a_compute_unit():
+    """The dispatch gives the 64 x 128 tile up to two workgroups of four waves per compute unit, and the 128 x 128 tile
+    with one range any number: more than 256 registers per lane would halve what runs at a time."""
+    regs = {k: v for k, v in _kernel_registers().items()
+            if "gemm_kernelILi64ELi128E" in k or ("gemm_kernelILi128ELi128E" in k and re.match(r".*ILi128ELi128ELi2ELi2ELi\dELb\dELb0E", k))}
+    assert len(regs) >= 9 and max(regs.values()) <= 256, regs
