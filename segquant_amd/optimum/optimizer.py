@@ -319,11 +319,8 @@ class DefaultOptimizer(BaseOptimizer):
         if col_div is not None and plan.get("col_div") is not None:
             raise RuntimeError("this layer already divides by its own smoothing factors: an external col_div is not combined with them")
         own_div = col_div is None and plan.get("col_div") is not None
-        if own_div:  # a smoothed layer's own divisors, rounded to the input's dtype once instead of on every call
-            casts = plan.setdefault("col_div_cast", {})
-            col_div = casts.get(x.dtype)
-            if col_div is None:
-                col_div = casts[x.dtype] = ops.rounded_col_div(plan["col_div"], x.dtype)
+        if own_div:  # a smoothed layer's own divisors, rounded to each input dtype when the plan was built
+            col_div = plan["col_div_cast"].get(x.dtype)
         if "l2t" in plan and (pre_op is not None or gate is not None):
             # the low-rank operand T = x (L1 / s) is built from the tensor handed in here, so that
             # tensor must be the layer's input itself, not what is in front of its activation function

@@ -155,8 +155,12 @@ class SmoothOptimizer(DefaultOptimizer):
         bounds = [0]
         for c in (self.chunksizes if self.seg_mode == "input" else [K]):
             bounds.append(bounds[-1] + c)
+        col_div = torch.cat([s.to(device) for s in self.s]).contiguous()
+        # rounded here for every input dtype, not on the first call that brings one: that call may be on another
+        # stream than the next, or under a capture, which would leave the later calls a tensor without contents
+        casts = {dt: ops.rounded_col_div(col_div, dt) for dt in (torch.float32, torch.float16, torch.bfloat16)}
         self._plan = dict(fa=fa, fw=fw, w=wcodes, sw=sw_list[0], sw_list=sw_list, sw_cs=1 if sw_list[0].numel() > 1 else 0,
-                          bounds=bounds, N=N, K=K, col_div=torch.cat([s.to(device) for s in self.s]).contiguous())
+                          bounds=bounds, N=N, K=K, col_div=col_div, col_div_cast=casts)
         return self._plan
 
     supports_parts = False  # SegmentLinear.forward_parts concatenates and takes forward() instead

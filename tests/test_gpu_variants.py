@@ -284,3 +284,40 @@ def test_general_gemm_on_more_tiles_than_compute_units(fa, fb, M, N, K):
     # aligns the products to the largest one: of these 2.2 million sums of 96 products one lies 3.3e-4 of sum |a||b| off,
     # on this tile as on 128 x 128 (1184 products: 4.8e-5)
     assert (np.abs(y - (va @ vb.T) * f) <= (5e-4 if fa == O.FMT_E4M3 else 5e-7) * (np.abs(va) @ np.abs(vb).T) * f).all()
+
+
+def _smoothed(opt_type, K=256, N=144, M=40):
+    from segquant_amd.layers.SegmentLinear import SegmentLinear
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(M, K, generator=g) * (torch.rand(K, generator=g) * 4 + 0.2)
+    layer = SegmentLinear(K, N, bias=True, custom_weight_tensor=torch.randn(N, K, generator=g) * 0.02, custom_bias_tensor=torch.randn(N, generator=g),
+                          input_quant_type="int8", weight_quant_type="int8", input_quant_args={"real_quant": True, "axis": -1, "dynamic": True},
+                          weight_quant_args={"real_quant": True, "axis": 1}, opt_type=opt_type,
+                          opt_kwargs={"low_rank": 32, "precision": "float32"} if opt_type == "svd" else None, device=DEV)
+    x = x.to(DEV)
+    layer.trace(x)
+    layer.smooth()
+    layer.calibrate(x)
+    layer.finish_calibrate()
+    return layer, x
+
+
+def test_a_smoothed_layer_first_seen_in_a_dtype_under_capture():
+    """The first call in fp16 of a layer in use in bf16 is one that is only recorded: eager calls before the graph's
+    first replay, and the replays, give what a layer that was never captured gives."""
+    layer, x = _smoothed("smooth")
+    want = _smoothed("smooth")[0](x.half())
+    layer(x.bfloat16())
+    buf = torch.zeros_like(x.half())
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = layer(buf)
+    assert torch.equal(layer(x.half()), want)
+    for _ in range(3):
+        buf.copy_(x.half())
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(layer(x.half()), want)
+        buf.zero_()
+    assert set(layer.optimizer._plan["col_div_cast"]) == set(TDT.values())
