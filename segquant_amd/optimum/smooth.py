@@ -234,16 +234,15 @@ class SVDOptimizer(SmoothOptimizer):
         l1 = [(self.l1s[i].to(device=device, dtype=torch.float32) / self.s[i].to(device)[:, None]) for i in range(self.chunks)]
         plan["l1s"] = l1                                                        # (k_i, r) each, fp32
         plan["l2t"] = torch.cat([self.l2s[i].to(device=device, dtype=torch.float32) for i in range(self.chunks)], dim=0).t().contiguous()  # (N, S r)
-        plan["l12_cast"] = {}
+        # (cast here for every input dtype, as the divisors are)
+        plan["l12_cast"] = {dt: ([l.to(dt) for l in l1], plan["l2t"].to(dt).contiguous())
+                            for dt in (torch.float32, torch.float16, torch.bfloat16)}
         return plan
 
     def _lowrank_operands(self, plan, x2):
         """(T, L2T) for the GEMM's epilogue, in the input's dtype."""
         dt = x2.dtype
-        cast = plan["l12_cast"].get(dt)
-        if cast is None:
-            cast = plan["l12_cast"][dt] = ([l.to(dt) for l in plan["l1s"]], plan["l2t"].to(dt).contiguous())
-        l1, l2t = cast
+        l1, l2t = plan["l12_cast"][dt]
         r = self.low_rank
         bounds = plan["bounds"]
         t = torch.empty((x2.shape[0], r * self.chunks), dtype=dt, device=x2.device)

@@ -321,3 +321,16 @@ def test_a_smoothed_layer_first_seen_in_a_dtype_under_capture():
         assert torch.equal(out, want) and torch.equal(layer(x.half()), want)
         buf.zero_()
     assert set(layer.optimizer._plan["col_div_cast"]) == set(TDT.values())
+
+
+def test_low_rank_factors_are_cast_before_the_first_call():
+    """A layer with a low-rank branch makes nothing on the first call of a dtype that later calls read: that call may be
+    recorded into a graph, or run on another stream."""
+    layer, x = _smoothed("svd")
+    out = layer(x.bfloat16())
+    kept = {dt: [t.data_ptr() for t in l1] + [l2.data_ptr()] for dt, (l1, l2) in layer.optimizer._plan["l12_cast"].items()}
+    assert set(kept) == set(TDT.values())
+    for dt in (torch.float16, torch.float32, torch.bfloat16):
+        again = layer(x.to(dt))
+        assert (again.float() - out.float()).norm() <= 2e-2 * out.float().norm()
+    assert kept == {dt: [t.data_ptr() for t in l1] + [l2.data_ptr()] for dt, (l1, l2) in layer.optimizer._plan["l12_cast"].items()}
