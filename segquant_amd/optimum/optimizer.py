@@ -353,7 +353,8 @@ class DefaultOptimizer(BaseOptimizer):
         # DualScale: two code tensors (Xp, Xn).  Reading plain codes lets both
         # operands stream straight into LDS; the single merged tensor would save a
         # third of the quantise traffic but costs the GEMM ~50 % (sign selection in
-        # registers), measured on the 4608 x 15360 x 3072 shape.
+        # registers), measured on the 4608 x 15360 x 3072 shape.  (The operator, whose
+        # shapes can be short and small, has a rule: ops._dual_in_two_tensors.)
         q = ops.quantize_desc(x2, plan["fa"], pos, neg, row_stride=1 if per_tok else 0,
                               kseg_bounds=bounds if S > 1 else None, kseg_stride=kstride, dual=dual,
                               dual_kseg_mask=mask, dynamic=dyn, two_tensors=dual, pre_op=pre_op, gate=gate,
