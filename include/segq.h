@@ -217,7 +217,7 @@ typedef struct segq_krange {
                              * scales, which has to be finite (scales that a calibrator clamps).  Non-zero: every
                              * range is summed on its own and scaled by its own factors, as int8 ranges always
                              * are, so that a scale may be infinite: limit / 0 of a DualScale side that holds
-                             * nothing, which adds nothing.  Not combined with a low-rank branch or a K split. */
+                             * nothing, which adds nothing.  Not combined with a low-rank branch. */
     const float* sx;        /* device */
     const float* sw;        /* device */
 } segq_krange;

@@ -408,10 +408,12 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     //  * More shares: each workgroup writes an fp32 partial result, a second kernel sums them in the
     //    order of the shares.  Workspace: the partial results.
     // Either way the parking slots of all those workgroups follow (int8 with several ranges).
+    // (No instance with a second register set of e4m3 sums meets in the launch: two shares of it take the second kernel.)
     int splits = 1;
     int64_t part_bytes = 0;
+    auto meet = [&](int s_, int c) { return s_ == 2 && tail_tile(c) && !p.sep; };
     {
-        const bool can = plain8 && wide_ok && d->batch == 1 && !groups && !lowrank && !p.sep && d->out_dtype != SEGQ_ACC && ws && al(ws, 16) &&
+        const bool can = plain8 && wide_ok && d->batch == 1 && !groups && !lowrank && d->out_dtype != SEGQ_ACC && ws && al(ws, 16) &&
                          d->split_k != 1 && (d->tile == 0 || cfg >= FIRST_WIDE_CFG) && !codes_out;
         const int64_t total_steps = ktotal / 128;
         if (d->split_k > 1 && !can)
@@ -447,8 +449,8 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
                 // 19 us against 25 us whole)
                 const int cands[4] = {FIRST_WIDE_CFG + 6, FIRST_WIDE_CFG, FIRST_WIDE_CFG + 7, FIRST_WIDE_CFG + 3};
                 double best = cost(cfg, 1);
-                for (int i = 0; i < (big_ok ? 4 : 1); ++i) {
-                    const int c = big_ok ? cands[i] : FIRST_WIDE_CFG + 1;
+                for (int i = 0; i < (big_ok ? 4 : p.sep ? 2 : 1); ++i) {
+                    const int c = big_ok ? cands[i] : FIRST_WIDE_CFG + (i == 0 ? 1 : 3);
                     if (c == FIRST_WIDE_CFG + 3 && (d->m > 128 || (i8 && fold))) continue;
                     int64_t s_ = cus / tiles_of(c);
                     if (s_ > total_steps / 8) s_ = total_steps / 8;
@@ -461,7 +463,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
             const int64_t tiles = tiles_of(scfg);
             const bool need_park = i8 && fold && scfg != FIRST_WIDE_CFG + 1 && scfg != FIRST_WIDE_CFG + 2 && scfg != FIRST_WIDE_CFG + 3;
             auto shares_for = [&](int s_) {
-                if (s_ == 2 && tail_tile(scfg)) return tiles * 2 * t.bm * t.bn * 4 + ((tiles * 4 + 255) & ~(int64_t)255);
+                if (meet(s_, scfg)) return tiles * 2 * t.bm * t.bn * 4 + ((tiles * 4 + 255) & ~(int64_t)255);
                 return (((int64_t)s_ * d->m * d->n * 4) + 255) & ~(int64_t)255;
             };
             auto bytes_for = [&](int s_) { return shares_for(s_) + (need_park || park ? (int64_t)s_ * tiles * t.bm * t.bn * 4 : 0); };
@@ -547,7 +549,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     const int64_t osz = (d->out_dtype == SEGQ_F32 || d->out_dtype == SEGQ_ACC) ? 4 : 2;
     p.vec_store = ((d->ldo * osz) % (4 * osz) == 0) && ((d->batch_stride_out * osz) % (4 * osz) == 0) && al(d->out, 4 * osz);
     p.vec_store16 = osz == 2 && d->ldo % 8 == 0 && d->batch_stride_out % 8 == 0 && al(d->out, 16);
-    if (splits == 2 && tail_tile(cfg)) {
+    if (meet(splits, cfg)) {
         p.splits = 2;
         p.part = static_cast<float*>(d->workspace);
         const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;

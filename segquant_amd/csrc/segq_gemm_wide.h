@@ -1013,7 +1013,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     // at a time they never queue.  DMA_ and MORE_ are compile-time so that the
     // steady-state loop body has no branches.
     int cr = r_first, ck = k_first, ck1 = p.r[ph(r_first)].k1;  // the tile being multiplied
-    bool dirty = false;  // int32 sums not yet folded into the fp32 set (a split can end inside a range)
+    bool dirty = false;  // sums not yet folded into the second set (a split can end inside a range)
     int buf = 0;                                   // its buffer, s % NS
     constexpr int NMF = TM * TN, NRD = TM + TN, NDM = A_IT + B_IT;
     constexpr int RD_EVERY = (NMF >= 2 * NRD + 4) ? 2 : 1;
@@ -1157,8 +1157,10 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         if constexpr (DMA_) advance_load();
         ck += BK;
         cslot = (cslot + 1) & 3;
+        dirty = true;
         if (ck >= ck1) {
             if constexpr (FOLD) fold(cr);
+            dirty = false;
             ++cr;
             const int rr = min(cr, p.nr - 1);
             ck = p.r[ph(rr)].k0;

@@ -17,6 +17,7 @@ Two layers:
 from __future__ import annotations
 
 import ctypes as C
+import functools
 from dataclasses import dataclass
 from typing import Optional, Sequence
 
@@ -532,6 +533,28 @@ def _dual_in_two_tensors(tiles: int, K: int, int4: bool) -> bool:
     return tiles < 96 or K >= 512
 
 
+@functools.lru_cache(maxsize=256)
+def _dual_share_bytes(device: int, M: int, N: int, K: int, fmt: str, dtype: torch.dtype) -> int:
+    """Workspace with which the DualScale operator's GEMM on two code tensors would share the K steps of its tiles
+    between workgroups; 0 if it would not.  Asked of the library once per shape (and device): the descriptor's
+    addresses are made up, nothing is launched."""
+    d = L.GemmDesc()
+    d.a_fmt = d.b_fmt = _CODE[fmt]
+    d.out_dtype = _dt(dtype)
+    d.m, d.n, d.lda, d.ldb, d.ldo, d.batch, d.n_ranges = M, N, K, K, N, 1, 2
+    d.a = d.a_neg = d.b = d.out = 4096
+    for i in range(2):
+        r = d.ranges[i]
+        r.k_len, r.a_sel, r.sx, r.sw, r.own_sum = K, i, 4096, 4096, 1 - i
+    need, tile, splits, parked = C.c_int64(0), C.c_int32(0), C.c_int32(0), C.c_int32(0)
+    L.check(L.lib().segq_gemm_workspace_bytes(C.byref(d), C.byref(need)))
+    d.workspace, d.workspace_bytes = 4096, need.value
+    L.check(L.lib().segq_gemm_plan(C.byref(d), C.byref(tile), C.byref(splits), C.byref(parked)))
+    # (two shares gain nothing over whole tiles, 3000 x 2000 x 4096 69.1 us either way, and would meet through words
+    # in the workspace: shares that a second kernel adds read nothing but what the launch wrote)
+    return need.value if splits.value > 2 else 0
+
+
 def real_quantized_gemm_dual_scaled(fmt_a: str, fmt_w: str, inputs: torch.Tensor, weights: torch.Tensor,
                                     pos_scale_x: torch.Tensor, neg_scale_x: torch.Tensor,
                                     scale_w: torch.Tensor) -> torch.Tensor:
@@ -541,9 +564,15 @@ def real_quantized_gemm_dual_scaled(fmt_a: str, fmt_w: str, inputs: torch.Tensor
     segment as two ranges, the non-negative codes with the positive scale and the
     negative ones with the negative scale.  Each range is summed on its own (a
     second register set): the scales come from the caller, and a side that holds
-    nothing may have ``limit / 0 = inf``, whose zeros add nothing.  No workspace:
-    the operator shares no buffer with any other launch.  (2, 2048, 3072) x 1536,
-    fp16, the whole pass: 76.7 us from one merged tensor, 62.2 us from two.
+    nothing may have ``limit / 0 = inf``, whose zeros add nothing.  (2, 2048, 3072)
+    x 1536, fp16, the whole pass: 76.7 us from one merged tensor, 62.2 us from two.
+
+    One segment, few tiles, a long K and 16-bit outputs: the K steps of a tile are
+    shared by several workgroups (bf16, K 4096, both launches, whole tiles and in
+    shares: 1024 x 1024 int8 49.4 and 41.1 us, e4m3 49.5 and 32.9; 200 x 1000 int8
+    68.3 and 24.7).  The room for the shares is the call's own, so that a second host thread on the stream cannot come between the
+    launch and the sum.  fp32 outputs would show the shares' roundings and keep
+    whole tiles.
     """
     _check_contract(inputs, weights, fmt_w, pos_scale_x, neg_scale_x, scale_w)
     S, M, N, K = _shapes(inputs, weights, fmt_w)
@@ -553,7 +582,10 @@ def real_quantized_gemm_dual_scaled(fmt_a: str, fmt_w: str, inputs: torch.Tensor
         raise RuntimeError("pos/neg scale_x must both have S or S*M entries")
     if not per_seg_w and scale_w.numel() != S * N:
         raise RuntimeError(f"scale_w has {scale_w.numel()} entries, expected {S} or {S * N}")
-    two = _dual_in_two_tensors(S * -(-M // 128) * -(-N // 128), K, fmt_w == FMT_INT4)
+    need = 0
+    if S == 1 and K % 128 == 0 and K >= 1024 and fmt_w != FMT_INT4 and inputs.dtype != torch.float32:
+        need = _dual_share_bytes(inputs.device.index, M, N, K, fmt_w, inputs.dtype)
+    two = need > 0 or _dual_in_two_tensors(S * -(-M // 128) * -(-N // 128), K, fmt_w == FMT_INT4)
     codes = quantize(inputs.view(S * M, K), fmt_a, pos_scale_x, neg_scale_x, seg_rows=M,
                      seg_stride=1 if per_seg_x else M, row_stride=0 if per_seg_x else 1, dual=True, two_tensors=two)
     codes, codes_neg = codes if two else (codes, None)
@@ -565,7 +597,8 @@ def real_quantized_gemm_dual_scaled(fmt_a: str, fmt_w: str, inputs: torch.Tensor
          [Range(0, K, pos_scale_x, scale_w, sel[0], rs, cs), Range(0, K, neg_scale_x, scale_w, sel[1], rs, cs)],
          m=M, n=N, a_fmt=fmt_a, b_fmt=fmt_w, out_dtype=inputs.dtype, lda=K, ldb=kb, a_neg=codes_neg,
          batch=S, batch_stride_a=M * K, batch_stride_b=N * kb,
-         batch_stride_sx=1 if per_seg_x else M, batch_stride_sw=1 if per_seg_w else N, out=out, own_sums=True)
+         batch_stride_sx=1 if per_seg_x else M, batch_stride_sw=1 if per_seg_w else N, out=out, own_sums=True,
+         workspace=torch.empty(need, dtype=torch.uint8, device=inputs.device) if need else None)
     return out
 
 

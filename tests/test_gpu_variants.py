@@ -149,7 +149,7 @@ class _Plans:
         monkeypatch.setattr(ops, "gemm_desc", record)
 
 
-def _dual_case(fmt, S, M, N, K, per_token, sides, seed, int4=False):
+def _dual_case(fmt, S, M, N, K, per_token, sides, seed, int4=False, dtype=torch.float32):
     """Inputs, unclamped scales and the fp64 result of the DualScale operator; ``sides``: which signs each segment (or
     token, in turn) holds, an empty one having the scale limit / 0 = inf.  Column 1 of the weights is zero, its scale too."""
     g = torch.Generator().manual_seed(seed)
@@ -163,6 +163,7 @@ def _dual_case(fmt, S, M, N, K, per_token, sides, seed, int4=False):
             part.copy_(-(part.abs() + 1e-3))
     lim = (127.0, 128.0) if fmt == O.FMT_INT8 else (448.0, 448.0)
     over = 2 if per_token else (1, 2)
+    x = x.to(dtype).float()
     pos, neg = lim[0] / x.amax(dim=over).clamp(min=0.0), lim[1] / (-x).amax(dim=over).clamp(min=0.0)
     rng = np.random.default_rng(seed)
     lo = -8 if int4 else -128
@@ -179,7 +180,7 @@ def _dual_case(fmt, S, M, N, K, per_token, sides, seed, int4=False):
         col = sw[s].numpy().astype(np.float64)[None, :]
         want[s] = ((p @ wv.T) / rows(pos) + (n @ wv.T) / rows(neg)) / col
         mag[s] = ((np.abs(p) @ np.abs(wv).T) / rows(pos) + (np.abs(n) @ np.abs(wv).T) / rows(neg)) / col
-    return x, w, pos, neg, sw, want, mag
+    return x.to(dtype), w, pos, neg, sw, want, mag
 
 
 @pytest.mark.parametrize("fmt", [O.FMT_INT8, O.FMT_E4M3])
@@ -201,6 +202,35 @@ def test_dual_operator_sides(monkeypatch, fmt, S, M, N, K, tile, two, per_token,
     # int8: per range an exact sum, its conversion, two reciprocals (1 ulp each) and two products, then the addition:
     # 8 x 2^-24 = 4.8e-7; e4m3: the matrix cores' limited-width adder
     assert (np.abs(out - want) <= (5e-7 if fmt == O.FMT_INT8 else 3e-4) * mag).all()
+
+
+@pytest.mark.parametrize("fmt", [O.FMT_INT8, O.FMT_E4M3])
+@pytest.mark.parametrize("M,N,K", [(3, 300, 4096), (64, 520, 2048), (200, 1000, 4096), (520, 1032, 4096), (1500, 1500, 4096)])
+@pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("per_token,sides", [(False, ["+-"]), (False, ["+"]), (True, ["+-", "+", "-"])])
+def test_dual_operator_in_k_shares(monkeypatch, fmt, M, N, K, dt, per_token, sides):
+    """One segment, few tiles, a long K: with 16-bit outputs the K steps are shared, in a workspace of the call's own
+    that no other launch ever sees; fp32 outputs keep whole tiles.  Sides that hold nothing have an infinite scale."""
+    from segquant_amd import ops
+    x, w, pos, neg, sw, want, mag = _dual_case(fmt, 1, M, N, K, per_token, sides, M + N + K, dtype=TDT[dt])
+    sw, want, mag = sw * 1024, want / 1024, mag / 1024  # (within fp16)
+    plans = _Plans(monkeypatch)
+    monkeypatch.setattr(ops, "int4_workspace", None)  # the buffer that layers share is not asked for
+    args = (x.to(DEV), torch.from_numpy(w).to(DEV), pos.reshape(-1).to(DEV), neg.reshape(-1).to(DEV), sw.to(DEV))
+    junk = torch.full((1 << 26,), 0x7FC00000, dtype=torch.int32, device=DEV)  # what the workspace finds in its memory: NaNs
+    del junk
+    outs = [ops.real_quantized_gemm_dual_scaled(fmt, fmt, *args) for _ in range(3)]
+    for p in plans.seen:
+        assert (p["splits"] > 2) == (p["workspace"] is not None)
+        if dt == "fp32":
+            assert p["splits"] == 1
+        elif K == 4096 and M > 100 or (fmt == O.FMT_E4M3 and M == 64):
+            assert p["splits"] > 2
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])  # the shares are added in their order
+    # the sums as in whole tiles, one more fp32 rounding per share; the output's one rounding
+    rounding = {"bf16": 2.0 ** -8, "fp16": 2.0 ** -11, "fp32": 0.0}[dt]
+    bound = (2e-6 if fmt == O.FMT_INT8 else 3e-4) * mag + rounding * np.abs(want) + (2.0 ** -24 if dt == "fp16" else 0.0)
+    assert (np.abs(outs[0].cpu().float().numpy().astype(np.float64) - want) <= bound).all()
 
 
 @pytest.mark.parametrize("S,M,N,K,two", [(1, 700, 500, 512, False), (2, 1000, 1000, 256, False), (1, 2100, 2100, 512, True)])

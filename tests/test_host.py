@@ -600,7 +600,7 @@ def test_plan_refuses_what_the_launch_would_refuse():
 
 def test_plan_of_ranges_summed_on_their_own():
     """own_sum: e4m3 ranges in a second register set, as int8 ranges without a workspace have it, on the tiles built for
-    it; a workspace is not used; neither a K split nor a low-rank branch is combined with it."""
+    it, in K shares where a workspace is lent for them; a low-rank branch is not combined with it."""
     import ctypes as C
     from segquant_amd import _lib as L
     lib = L.lib()
@@ -625,7 +625,7 @@ def test_plan_of_ranges_summed_on_their_own():
     for m, n, tile in ((496, 1000, 14), (384, 1280, 4), (3000, 3000, 14), (2000, 4000, 12)):
         # (int8 without a workspace takes the same tile: the two formats follow one rule)
         assert plan(m, n) == (0, tile, 1, 0) and plan(m, n, fmt=0) == (0, tile, 1, 0)
-    assert plan(496, 1000, split_k=2)[0] == 2 and plan(2000, 4000, lowrank=32)[0] == 2
+    assert plan(496, 1000, split_k=2) == (0, 12, 2, 0) and plan(2000, 4000, lowrank=32)[0] == 2
     assert plan(2000, 4000, tile=15)[0] == 2 and plan(2000, 4000, tile=15, own=0)[0] == 0
 
 
