@@ -670,7 +670,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     // infinities and NaNs of the other side's sums.  For e4m3 that is SEP, taken where the
     // scales come from outside (segq_krange.own_sum): 2 x 2048 x 1536 x 3072 DualScale 61.9 us
     // rescaled in place, 62.2 us with the second set, and 256 x 256 tiles out of reach.
-    static_assert(!PARK || (FOLD && !F8 && !GRP), "parking: int8 with several ranges");
+    static_assert(!PARK || (FOLD && !F8 && !GRP && FINISH), "parking: int8 with several ranges, finished in output units");
     static_assert(!WS || (!FOLD && !PARK), "int8 above 256 x 256: one range");
     static_assert(!SEP || (FOLD && F8 && !PARK && !FINISH), "SEP: e4m3 with several ranges");
     constexpr bool ACCF = FOLD && (!F8 || SEP) && !GRP && !PARK;
@@ -1253,14 +1253,18 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     }
     if constexpr (FINISH) {
         // FINISH instances serve the launches that finish in output units (the others do not pay for
-        // the registers of it): the low-rank branch and a tile split in two along K.  The sums are
-        // scaled first (1 / (sx sw) of the range they are in units of, from the vectors parked in LDS); then
+        // the registers of it): parked ranges, the low-rank branch and a tile split in two along K.  The sums are
+        // scaled first (1 / (sx sw) of the range they are in units of, from the vectors parked in LDS) and what is
+        // parked is added; then
         //  * a tile split in two along K: the two workgroups meet in the workspace (below);
         //  * low-rank branch (out += T L2): the product joins in fp32 on the matrix cores;
         // and the epilogue only adds the bias and the addend and rounds once.
         v4f of[TN][TM];
         [[maybe_unused]] const bool parked = r_begin < r_last;
-        constexpr int CH = 8;  // blocks whose loads are in flight at once (registers: the sums are still live)
+        // blocks whose loads are in flight at once (registers: the sums are still live).  What is parked comes back in two
+        // halves: 256 x 256 tiles 600 x 15360 x 3072 143 -> 135 us a pass, 2100 274 -> 260, 9216 (288 x 192) 843 -> 834
+        // against an instance without the finish; 351 rows in ten shares 75 -> 78
+        constexpr int CH = PARK ? (TN * TM + 1) / 2 : 8;
 #pragma unroll
         for (int c0 = 0; c0 < TN * TM; c0 += CH) {
             [[maybe_unused]] v4f old[CH];
@@ -1336,26 +1340,6 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     if constexpr (GRP) {
         v4f none[1][1];
         wide_epilogue<BM, BN, WGM, WGN, GEMM_F8, false, false>(p, accf, none, smem, z, m0, n0, wave, lane, r_epi, epi);
-    } else if constexpr (PARK) {
-        // the earlier ranges' sums come back, in output units, in two halves, each with all its loads in flight at once
-        v4f accp[TN][TM];
-        constexpr int H = (TN + 1) / 2;
-        const bool parked = r_begin < r_last;  // (a split's share can lie inside one range)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            v4f old[H][TM];
-#pragma unroll
-            for (int a = h * H; a < min(TN, (h + 1) * H); ++a)
-#pragma unroll
-                for (int b = 0; b < TM; ++b) old[a - h * H][b] = parked ? slot[(a * TM + b) * NT] : v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int a = h * H; a < min(TN, (h + 1) * H); ++a)
-#pragma unroll
-                for (int b = 0; b < TM; ++b)
-                    accp[a][b] = __builtin_convertvector(acc[a][b], v4f) * epi[wm * WM + b * 16 + lrow] *
-                                     *reinterpret_cast<const v4f*>(epi + BM + wn * WN + a * 16 + 4 * lgrp) + old[a - h * H][b];
-        }
-        wide_epilogue<BM, BN, WGM, WGN, GEMM_F8, false, true>(p, accp, accp, smem, z, m0, n0, wave, lane, r_epi, epi);
     } else if constexpr (CODES) {
         codes_epilogue<BM, BN, WGM, WGN, FMT>(p, acc, smem, m0, n0, wave, lane, epi);
     } else {
@@ -1417,6 +1401,7 @@ int launch_wide(const GemmParams& p, int wcfg, bool fold, bool asel, int64_t bat
 #define SEGQ_PIPE1(BM_, BN_, WGM_, WGN_, FOLD_, PARK_)                                                               \
     if (tail) break;                                                                                                 \
     return launch_pipe_instance<BM_, BN_, WGM_, WGN_, FMT, FOLD_, 2, false, PARK_, false>(p, batch, st)
+#define SEGQ_PARK(BM_, BN_, WGM_, WGN_) return launch_pipe_instance<BM_, BN_, WGM_, WGN_, FMT, true, 2, false, true, true>(p, batch, st)
     if (p.oc) {  // the epilogue writes codes: instances of their own, so that the others carry no trace of it
         if constexpr (!B4) {
             if (!asel && !fold && !tail && !p.park) {
@@ -1461,14 +1446,14 @@ int launch_wide(const GemmParams& p, int wcfg, bool fold, bool asel, int64_t bat
             } else if (p.park) {  // int8, several ranges, a workspace to park finished ranges in: every tile
                 if constexpr (!F8W) {
                     switch (wcfg) {
-                        case 0: SEGQ_PIPE2(256, 256, 4, 2, true, true);
-                        case 1: SEGQ_PIPE2(256, 128, 4, 2, true, true);
-                        case 2: SEGQ_PIPE1(128, 256, 2, 4, true, true);
-                        case 3: SEGQ_PIPE2(128, 128, 2, 4, true, true);
-                        case 4: SEGQ_PIPE1(192, 288, 4, 2, true, true);
-                        case 5: SEGQ_PIPE1(288, 192, 2, 4, true, true);
-                        case 6: SEGQ_PIPE2(256, 192, 4, 2, true, true);
-                        case 7: SEGQ_PIPE2(192, 256, 2, 4, true, true);
+                        case 0: SEGQ_PARK(256, 256, 4, 2);
+                        case 1: SEGQ_PARK(256, 128, 4, 2);
+                        case 2: if (tail) break; SEGQ_PARK(128, 256, 2, 4);
+                        case 3: SEGQ_PARK(128, 128, 2, 4);
+                        case 4: if (tail) break; SEGQ_PARK(192, 288, 4, 2);
+                        case 5: if (tail) break; SEGQ_PARK(288, 192, 2, 4);
+                        case 6: SEGQ_PARK(256, 192, 4, 2);
+                        case 7: SEGQ_PARK(192, 256, 2, 4);
                     }
                 }
             } else if constexpr (F8W) {
@@ -1504,6 +1489,7 @@ int launch_wide(const GemmParams& p, int wcfg, bool fold, bool asel, int64_t bat
     }
 #undef SEGQ_PIPE1
 #undef SEGQ_PIPE2
+#undef SEGQ_PARK
     if (tail)
         return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: tile %d finishes neither a low-rank branch nor a two-way K split", wcfg + FIRST_WIDE_CFG + 1);
 #define SEGQ_WIDE(BM_, BN_, WGM_, WGN_, FOLD_)                                                          \
