@@ -276,13 +276,26 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     if (w4 && ktotal > 131071) return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: K too large for int4 weights");
     if (kmax > 0x7fffff00) return fail(SEGQ_ERR_ARG, "segq_gemm: K too large");
 
+    const int few = [&]() -> int {
+        const int64_t reach = (int64_t)1 << 31;  // a tile's rows are addressed with 31 bits
+        const segq_krange& r = d->ranges[0];
+        const bool ok = d->n_ranges == 1 && r.a_sel < 2 && d->m < reach >> 4 && d->n < reach >> 4 && !lowrank && !codes_out && d->split_k <= 1 && 64 * d->lda + kmax < reach && 64 * d->ldb + kmax < reach &&
+                        (!groups || (w4 && r.k_begin % 128 == 0 && r.k_len % 128 == 0 && d->n % 4 == 0 && d->group_dequant_stride % 4 == 0 &&
+                                     al(d->group_dequant, 16) && kmax / 128 * d->group_dequant_stride < reach / 4));
+        if (d->tile != 0) return d->tile > FIRST_FEW_CFG && d->tile <= NUM_TILE_CFG ? (ok ? (int)d->tile - 1 : -2) : -1;
+        // (raw accumulators are for checks of the integers and keep the route, and the workspace, that they had)
+        return ok && d->out_dtype != SEGQ_ACC ? choose_few(d->m, d->n, d->batch, r.k_len, f8 ? GEMM_F8 : GEMM_I8, w4, groups) : -1;
+    }();
+    if (few == -2)
+        return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: tiles %d to %d serve one range without a sign selection, a low-rank branch, codes out or split_k "
+                                          "(and group factors of int4 weights)", FIRST_FEW_CFG + 1, NUM_TILE_CFG);
     if (groups && w4) {
         const int64_t kp = (kmax + 31) & ~(int64_t)31;
         if (!ws || !al(ws, 16) || ws_bytes < d->n * kp)
             return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: group factors with int4 weights need %lld bytes of workspace",
                         (long long)(d->n * kp));
     }
-    if (w4 && ws) {
+    if (few < 0 && w4 && ws) {
         // expand b to int8 in the caller's workspace and run the int8 kernels on it
         const int64_t kp = (kmax + 31) & ~(int64_t)31;  // whole 16-byte packed chunks
         if (al(ws, 16) && ws_bytes >= d->batch * d->n * kp && kp / 2 <= d->ldb) {
@@ -336,7 +349,25 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         p.ldadd = d->ld_addend;
         p.vec_add = d->addend && (d->ld_addend * asz) % (4 * asz) == 0 && (d->batch_stride_out * asz) % (4 * asz) == 0 && al(d->addend, 4 * asz);
     }
+    const int64_t osz = (d->out_dtype == SEGQ_F32 || d->out_dtype == SEGQ_ACC) ? 4 : 2;
+    p.vec_store = ((d->ldo * osz) % (4 * osz) == 0) && ((d->batch_stride_out * osz) % (4 * osz) == 0) && al(d->out, 4 * osz);
+    p.vec_store16 = osz == 2 && d->ldo % 8 == 0 && d->batch_stride_out % 8 == 0 && al(d->out, 16);
     p.nr = d->n_ranges;
+    if (few >= 0) {
+        const TileCfg& c = TILE_CFGS[few];
+        const int64_t tm = (d->m + c.bm - 1) / c.bm, tn = (d->n + c.bn - 1) / c.bn;
+        if (tm * tn > 0x7fffffff || d->batch > 65535) return fail(SEGQ_ERR_ARG, "segq_gemm: grid too large");
+        p.tiles_m = (int32_t)tm;
+        p.tiles_n = (int32_t)tn;
+        p.grw = d->group_dequant;
+        p.grw_gs = d->group_dequant_stride;
+        if (plan) {
+            plan->tile = few + 1;
+            if (groups) plan->bytes = d->n * ((kmax + 31) & ~(int64_t)31);  // asked for above, whatever the tile
+            p.dry = 1;
+        }
+        return launch_gemm_few(p, f8 ? GEMM_F8 : GEMM_I8, w4, few, d->batch, st);
+    }
     const bool fold = d->n_ranges > 1;
     bool wide_ok = d->m * d->lda < (int64_t)1 << 32 && d->n * d->ldb < (int64_t)1 << 32;
     for (int i = 0; i < d->n_ranges; ++i) wide_ok = wide_ok && d->ranges[i].k_begin % 128 == 0 && d->ranges[i].k_len % 128 == 0;
@@ -546,9 +577,6 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         p.rot = (d->n_ranges > 1 && splits == 1 && f8 && !p.sep) ? 1 : 0;
     }
     if ((int64_t)p.tiles_m * p.tiles_n > 0x7fffffff || d->batch > 65535) return fail(SEGQ_ERR_ARG, "segq_gemm: grid too large");
-    const int64_t osz = (d->out_dtype == SEGQ_F32 || d->out_dtype == SEGQ_ACC) ? 4 : 2;
-    p.vec_store = ((d->ldo * osz) % (4 * osz) == 0) && ((d->batch_stride_out * osz) % (4 * osz) == 0) && al(d->out, 4 * osz);
-    p.vec_store16 = osz == 2 && d->ldo % 8 == 0 && d->batch_stride_out % 8 == 0 && al(d->out, 16);
     if (meet(splits, cfg)) {
         p.splits = 2;
         p.part = static_cast<float*>(d->workspace);

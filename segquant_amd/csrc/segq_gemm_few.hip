@@ -1,0 +1,67 @@
+// Instances of the GEMM kernel for launches of few tiles.
+#include <type_traits>
+#include "segq_gemm_few.h"
+namespace segq {
+
+// Tile for a launch of few tiles, or -1 where the other kernels serve it better.  Both sides are estimated in us from
+// launches with weights from memory; K in steps of 128.  The constants were fitted over 110 shapes of 1 to 5000 rows and 100 to
+// 18432 columns; the choice is within 12 % of the best tile on nine of ten of them.
+int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4, bool grp) {
+    const int64_t cus = device_cus(), steps = (k + 127) / 128;
+    auto tiles = [&](int64_t bm, int64_t bn) { return (m + bm - 1) / bm * ((n + bn - 1) / bn) * batch; };
+    if (tiles(32, 64) > 32 * cus) return -1;
+    // this kernel: 3.5 us of launch, first loads and the meeting of the shares (1.1 us for each workgroup a CU takes beyond
+    // its first), then the tile's operand bytes at what a CU takes in with two workgroups on it (52 KB per us) or one (38);
+    // int4 weights add their unpacking, group factors the sums
+    int best = -1;
+    double cost = 0;
+    for (int c = FIRST_FEW_CFG; c < NUM_TILE_CFG; ++c) {
+        const int tm = TILE_CFGS[c].bm / 16, tn = TILE_CFGS[c].bn / 16;
+        const int64_t t = tiles(TILE_CFGS[c].bm, TILE_CFGS[c].bn), per_wave = (steps + FEW_WAVES - 1) / FEW_WAVES;
+        const bool two = few_two(tm, tn, b4, grp, per_wave <= few_depth(tm, tn, b4, grp) ? (int)per_wave : 0);
+        const double bytes = (TILE_CFGS[c].bm + TILE_CFGS[c].bn * (b4 ? 0.5 : 1.0)) * 128.0 * steps;
+        const double rate = (two ? 52e3 : 38e3) * (b4 ? 0.75 : 1.0) * (grp ? 0.9 : 1.0);
+        const double us = t > cus ? 2.8 + (double)t / cus * (bytes / rate + 1.1) : 3.5 + 0.9 * bytes / rate;
+        if (best < 0 || us < cost) {
+            best = c;
+            cost = us;
+        }
+    }
+    // the others: so much per K step and round of the CUs
+    const int64_t t128 = tiles(128, 128), rounds = (t128 + cus - 1) / cus;
+    if (b4 && grp)  // with the expansion of the weights in front
+        return cost < 7.0 + 0.85 * steps * (double)((t128 + 2 * cus - 1) / (2 * cus)) + (double)n * k / 8e6 ? best : -1;
+    if (b4) return cost < 6.5 + 0.8 * steps * rounds ? best : -1;
+    const double full = (double)tiles(64, 128) / (1.5 * cus);
+    double other = 6.5 + 0.75 * steps * (full > 1.0 ? full : 1.0);  // the general kernel, 64 x 128
+    if (k % 128 == 0) {
+        bool theirs = t128 >= 32;  // the 8-wave kernels ...
+        if (theirs) other = 4.5 + (fmt == GEMM_F8 ? 0.5 : 0.45) * steps * rounds;
+        auto shares = [&](int64_t t, double per_step) {  // ... also in K shares
+            const int64_t s = cus / t < steps / 8 ? cus / t : steps / 8;
+            if (batch > 1 || steps < 16 || t * 10 >= cus * 9 || s < 2) return;
+            const double us = 10.5 + per_step * steps / s + (double)n * k / 5.5e6;
+            if (us < other) other = us;
+            theirs = true;
+        };
+        if (m <= 128) shares(t128, 0.45);
+        else shares(tiles(256, 192), 0.9);
+        // They have tiles and shares of their own by size, asserted in the host tests, and keep what is not clearly
+        // ahead here (64 x 9216 x 3072 stays at 20.3 us in three shares: 13.9 here; 256 x 2176 x 1536 at 9.0: 8.3 here)
+        if (theirs) other *= 0.65;
+    }
+    return cost < other ? best : -1;
+}
+
+int launch_gemm_few(const GemmParams& g, int fmt, bool b4, int cfg, int64_t batch, hipStream_t st) {
+    if (g.dry) return SEGQ_OK;
+    const KRange& r = g.r[0];
+    const FewParams p = {r.a_sel == 1 ? g.A2 : g.A, g.B, g.C, r.sx, r.sw, g.bias, g.addend, g.grw,
+                         g.lda, g.ldb, g.ldc, g.ldadd, g.grw_gs, g.bsA, g.bsB, g.bsC, g.bsSx, g.bsSw,
+                         g.M, g.N, r.k0, r.k1, r.sx_rs, r.sw_cs, g.tiles_m, g.tiles_n, g.out_dtype, g.bias_dtype, g.vec_store, g.vec_add};
+    const int f = cfg - FIRST_FEW_CFG;
+    if (fmt == GEMM_F8) return launch_few_format<GEMM_F8, false, false>(p, f, batch, st);
+    if (!b4) return launch_few_format<GEMM_I8, false, false>(p, f, batch, st);
+    return p.grw ? launch_few_format<GEMM_I8, true, true>(p, f, batch, st) : launch_few_format<GEMM_I8, true, false>(p, f, batch, st);
+}
+}  // namespace segq

@@ -78,7 +78,8 @@ struct GemmParams {
 enum { GEMM_I8 = 0, GEMM_F8 = 1 };
 
 // o[0..3] += addend[z][m][n .. n + 3] (columns beyond N skipped)
-__device__ __forceinline__ void add_addend4(const GemmParams& p, int64_t z, int m, int n, float (&o)[4]) {
+template <class Params>
+__device__ __forceinline__ void add_addend4(const Params& p, int64_t z, int m, int n, float (&o)[4]) {
     if (!p.addend) return;
     const int64_t e = z * p.bsC + (int64_t)m * p.ldadd + n;
     if (p.out_dtype == SEGQ_F32) {
@@ -534,14 +535,16 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_kernel(const GemmParams p)
 
 // ---- host-side launch of one (format, tile, fold) instance -------------------
 struct TileCfg { int bm, bn, wgm, wgn; };
-constexpr int NUM_TILE_CFG = 21;
+constexpr int NUM_TILE_CFG = 25;
 constexpr int FIRST_BIG_CFG = 8;    // two retired ids (a 4-wave 256 x 256 kernel that no shape profited from)
 constexpr int FIRST_WIDE_CFG = 10;  // the 8-wave kernels from here on (segq_gemm_wide.h)
+constexpr int FIRST_FEW_CFG = 21;   // tiles whose waves share K (segq_gemm_few.h)
 constexpr TileCfg TILE_CFGS[NUM_TILE_CFG] = {
     {256, 256, 2, 2}, {256, 128, 2, 2}, {128, 128, 2, 2}, {64, 128, 2, 2}, {128, 256, 2, 2},
     {256, 256, 2, 4}, {256, 256, 4, 2}, {256, 128, 4, 2}, {256, 256, 2, 2}, {256, 256, 2, 2},
     {256, 256, 4, 2}, {256, 128, 4, 2}, {128, 256, 2, 4}, {128, 128, 2, 4}, {192, 288, 4, 2}, {288, 192, 2, 4},
     {256, 192, 4, 2}, {192, 256, 2, 4}, {128, 128, 2, 4}, {384, 192, 4, 2}, {128, 96, 4, 2},
+    {16, 32, 1, 1}, {16, 64, 1, 1}, {32, 32, 1, 1}, {32, 64, 1, 1},
 };
 
 // Steps in flight of the general kernel's 64 x 128 and 128 x 128 tiles, one range (every other launch: one step ahead;
@@ -610,5 +613,7 @@ int launch_format(const GemmParams& p, int cfg, bool fold, int64_t batch, hipStr
 int launch_gemm_i8(const GemmParams& p, int cfg, bool fold, int64_t batch, hipStream_t st);
 int launch_gemm_f8(const GemmParams& p, int cfg, bool fold, int64_t batch, hipStream_t st);
 int launch_gemm_w4(const GemmParams& p, int cfg, bool fold, int64_t batch, hipStream_t st);
+int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4, bool grp);
+int launch_gemm_few(const GemmParams& p, int fmt, bool b4, int cfg, int64_t batch, hipStream_t st);
 
 }  // namespace segq

@@ -272,7 +272,8 @@ def gemm_workspace_bytes(g) -> int:
 
 # tile ids of the 8-wave kernels (segq_gemm_desc.tile) -> rows x columns of the output tile
 TILE_SHAPES = {1: "256x256", 2: "256x128", 3: "128x128", 4: "64x128", 5: "128x256", 6: "256x256", 7: "256x256", 8: "256x128",
-               11: "256x256", 12: "256x128", 13: "128x256", 14: "128x128", 15: "192x288", 16: "288x192", 17: "256x192", 18: "192x256", 19: "128x128", 20: "384x192", 21: "128x96"}
+               11: "256x256", 12: "256x128", 13: "128x256", 14: "128x128", 15: "192x288", 16: "288x192", 17: "256x192", 18: "192x256", 19: "128x128", 20: "384x192", 21: "128x96",
+               22: "16x32", 23: "16x64", 24: "32x32", 25: "32x64"}
 
 
 def gemm_plan(g, workspace: Optional[torch.Tensor] = None) -> dict:
@@ -284,7 +285,7 @@ def gemm_plan(g, workspace: Optional[torch.Tensor] = None) -> dict:
         d.workspace = workspace.data_ptr(); d.workspace_bytes = workspace.numel() * workspace.element_size()
     tile, splits, parked = C.c_int32(0), C.c_int32(0), C.c_int32(0)
     L.check(L.lib().segq_gemm_plan(C.byref(d), C.byref(tile), C.byref(splits), C.byref(parked)))
-    family = "gemm_pipe_kernel" if tile.value >= 11 else "gemm_kernel"
+    family = "gemm_few_kernel" if tile.value >= 22 else "gemm_pipe_kernel" if tile.value >= 11 else "gemm_kernel"
     return dict(tile=tile.value, shape=TILE_SHAPES.get(tile.value, "?"), splits=splits.value, parked=bool(parked.value),
                 kernel=f"segq::{family}<{TILE_SHAPES.get(tile.value, '?').replace('x', ',')}>")
 

@@ -1,0 +1,130 @@
+"""The GEMM kernel for launches of few tiles against the closed form: the edges of its tiles, of the units its waves share K
+in, of its short-K instances (one to four units per wave) and of the loop behind them."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import segq_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+FORMATS = {"int8": (O.FMT_INT8, O.FMT_INT8), "e4m3": (O.FMT_E4M3, O.FMT_E4M3), "int4": (O.FMT_INT8, O.FMT_INT4)}
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from segquant_amd import ops as _ops
+    _ops.L.lib()
+    return _ops
+
+
+def _codes(g, shape, fmt):
+    if fmt == O.FMT_INT4:
+        return g.integers(-8, 8, size=shape).astype(np.int8)
+    if fmt == O.FMT_INT8:
+        return g.integers(-128, 128, size=shape).astype(np.int8)
+    c = g.integers(0, 256, size=shape).astype(np.uint8)
+    c[(c & 0x7F) == 0x7F] = 0x3A  # no NaN codes
+    return c
+
+
+def _dev(c, fmt, pad=0):
+    t = torch.from_numpy(np.stack([O.pack_int4(r) for r in c]) if fmt == O.FMT_INT4 else c).to(DEV)
+    if not pad:
+        return t
+    wide = torch.full((t.shape[0], t.shape[1] + pad), 0x55, dtype=torch.uint8, device=DEV).view(t.dtype)  # what lies between the rows
+    wide[:, :t.shape[1]] = t
+    return wide[:, :t.shape[1]]
+
+
+def _check(ops, kind, M, N, K, tile, dt, g, group=False, k0=0, row_sx=True, col_sw=True, has_bias=True, neg=False, add=False, pad=0):
+    fa, fb = FORMATS[kind]
+    a, b = _codes(g, (M, k0 + K), fa), _codes(g, (N, k0 + K), fb)
+    sx = (g.random(M if row_sx else 1) * 30 + 10).astype(np.float32)
+    sw = np.ones(1, np.float32) if group else (g.random(N if col_sw else 1) * 30 + 10).astype(np.float32)
+    av, bv = O.code_values(a, fa)[:, k0:].astype(np.float64), O.code_values(b, fb)[:, k0:].astype(np.float64)
+    gd = None
+    if group:
+        fac = np.zeros(((k0 + K) // 128, N), np.float32)
+        fac[:] = g.random(fac.shape) * 0.09 + 0.01
+        bv = bv * np.repeat(fac.astype(np.float64).T, 128, axis=1)[:, k0:]
+        gd = torch.from_numpy(fac).to(DEV)
+    den = sx.astype(np.float64)[:, None] * sw.astype(np.float64)[None, :]
+    want, mag = av @ bv.T / den, np.abs(av) @ np.abs(bv).T / den
+    bias = g.standard_normal(N).astype(np.float32) if has_bias else None
+    bias_t = None
+    if has_bias:
+        bias_t = torch.from_numpy(bias).to(DEV).to(dt)
+        bias = bias_t.float().cpu().numpy()
+        want, mag = want + bias, mag + np.abs(bias)
+    addend = None
+    if add:
+        addend = torch.randn(M, N, device=DEV).to(dt)
+        want, mag = want + addend.double().cpu().numpy(), mag + addend.double().abs().cpu().numpy()
+    ad, bd = _dev(a, fa, pad), _dev(b, fb, pad)
+    esz = 2 if fb == O.FMT_INT4 else 1
+    rg = [ops.Range(k0, K, torch.from_numpy(sx).to(DEV), torch.from_numpy(sw).to(DEV), 1 if neg else 0, int(row_sx), int(col_sw and not group))]
+    gdesc = ops.gemm_desc(torch.zeros_like(ad) if neg else ad, bd, rg, m=M, n=N, a_fmt=fa, b_fmt=fb, out_dtype=dt, lda=k0 + K + pad,
+                          ldb=(k0 + K) // esz + pad, bias=bias_t, a_neg=ad if neg else None, tile=tile, group_dequant=gd, addend=addend)
+    ws = torch.empty(ops.gemm_workspace_bytes(gdesc), dtype=torch.uint8, device=DEV) if group else None
+    assert tile == 0 or ops.gemm_plan(gdesc, ws)["tile"] == tile
+    got = ops.gemm_launch(gdesc, ws).double().cpu().numpy()
+    # fp32 arithmetic of the scaling (and of the group sums: one rounding per group and per share), the matrix cores' e4m3
+    # sums, and the output's one rounding
+    tol = (4e-6 + (2.0 ** -23 * ((k0 + K) // 128 + 8) if group else 0.0)) * mag + 1e-30
+    if kind == "e4m3":
+        tol = tol + 3e-4 * mag
+    tol = tol + {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dt] * np.abs(want) + (2.0 ** -24 if dt == torch.float16 else 0.0)
+    err = np.abs(got - want)
+    assert np.isfinite(got).all() and (err <= tol).all(), (kind, M, N, K, tile, dt, float((err - tol).max()))
+
+
+@pytest.mark.parametrize("kind,group", [("int8", False), ("e4m3", False), ("int4", False), ("int4", True)])
+@pytest.mark.parametrize("tile", [22, 23, 24, 25])
+def test_edges_of_tiles_and_of_k(ops, kind, group, tile):
+    g = np.random.default_rng(100 * tile + len(kind) + group)
+    step = 128 if group else 32 if kind == "int4" else 16
+    for K in (step, 128, 1024 - step, 1024, 1024 + step, 2048 + step, 3072, 4096, 4096 + step, 6144 + step):
+        K = max(step, K // step * step)
+        M, N = int(g.choice([1, 2, 15, 16, 17, 31, 33, 50])), int(g.choice([4, 16, 36, 64, 100])) + (0 if group else int(g.integers(0, 3)))
+        _check(ops, kind, M, N, K, tile, [torch.float32, torch.bfloat16, torch.float16][int(g.integers(0, 3))], g, group=group)
+
+
+@pytest.mark.parametrize("kind,group", [("int8", False), ("e4m3", False), ("int4", False), ("int4", True)])
+def test_forms_of_the_call(ops, kind, group):
+    g = np.random.default_rng(7)
+    for i, opt in enumerate([dict(), dict(row_sx=False, col_sw=False), dict(has_bias=False), dict(neg=True), dict(add=True), dict(pad=16),
+                             dict(k0=128), dict(k0=256, pad=32, add=True)]):
+        _check(ops, kind, 37, 104, 640, (22, 23, 24, 25, 0)[i % 5], (torch.bfloat16, torch.float32)[i & 1], g, group=group, **opt)
+
+
+@pytest.mark.parametrize("kind", ["int8", "e4m3", "int4"])
+def test_raw_accumulators_and_batches(ops, kind):
+    fa, fb = FORMATS[kind]
+    g = np.random.default_rng(3)
+    M, N, K = 21, 70, 1184
+    a, b = _codes(g, (2 * M, K), fa), _codes(g, (2 * N, K), fb)
+    av, bv = O.code_values(a, fa).astype(np.float64), O.code_values(b, fb).astype(np.float64)
+    kb = K // 2 if kind == "int4" else K
+    for tile in (22, 23, 24, 25):
+        out = ops.gemm(_dev(a, fa), _dev(b, fb), [ops.Range(0, K, None, None)], m=M, n=N, a_fmt=fa, b_fmt=fb, out_dtype="acc", lda=K, ldb=kb,
+                       tile=tile, batch=2, batch_stride_a=M * K, batch_stride_b=N * kb)
+        got = out.double().cpu().numpy().reshape(2, M, N)
+        for z in range(2):
+            x, y = av[z * M:(z + 1) * M], bv[z * N:(z + 1) * N]
+            if kind == "e4m3":
+                assert (np.abs(got[z] - x @ y.T) <= 3e-4 * (np.abs(x) @ np.abs(y).T)).all()
+            else:
+                assert (got[z] == x @ y.T).all()
+
+
+def test_what_the_tiles_do_not_serve_is_refused(ops):
+    g = np.random.default_rng(1)
+    a, b = _dev(_codes(g, (40, 256), O.FMT_INT8), O.FMT_INT8), _dev(_codes(g, (64, 256), O.FMT_INT8), O.FMT_INT8)
+    one = torch.ones(1, device=DEV)
+    kw = dict(m=40, n=64, a_fmt=O.FMT_INT8, b_fmt=O.FMT_INT8, out_dtype=torch.float32, lda=256, ldb=256, tile=24)
+    for ranges in ([ops.Range(0, 256, one, one, 2)], [ops.Range(0, 128, one, one), ops.Range(128, 128, one, one)]):
+        with pytest.raises(RuntimeError, match="tiles 22 to 25"):
+            ops.gemm(a, b, ranges, **kw)
+    with pytest.raises(RuntimeError, match="is not in 0..25"):
+        ops.gemm(a, b, [ops.Range(0, 256, one, one)], **{**kw, "tile": 26})
