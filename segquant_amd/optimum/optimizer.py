@@ -329,6 +329,7 @@ class DefaultOptimizer(BaseOptimizer):
         if plain:
             hit = plan.setdefault("launches", {}).get((x2.shape[0], x.dtype, None if bias is None else bias.data_ptr()))
             if hit is not None:
+                ops._need_cuda(x2)  # (the first call of a token count has its tensors checked one by one; this one takes an address)
                 return self._relaunch(hit, x2, fresh)
         if gate is not None:
             gate = _readable_rows(gate.reshape(-1, K))
