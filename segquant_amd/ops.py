@@ -337,6 +337,13 @@ def linear(q, g, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     return out
 
 
+def linear_again(qd, gd, stream: int) -> None:
+    """``segq_linear`` on two descriptors that are complete, the workspace of an earlier :func:`linear` included."""
+    rc = L.lib().segq_linear(C.byref(qd), C.byref(gd), stream)
+    if rc:
+        L.check(rc)
+
+
 def gemm_desc(a: torch.Tensor, b: torch.Tensor, ranges: Sequence[Range], *, m: int, n: int, a_fmt: str, b_fmt: str,
          out_dtype, lda: int, ldb: int, a_neg: Optional[torch.Tensor] = None,
          bias: Optional[torch.Tensor] = None, batch: int = 1, batch_stride_a: int = 0, batch_stride_b: int = 0,

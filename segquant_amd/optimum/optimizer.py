@@ -277,6 +277,10 @@ class DefaultOptimizer(BaseOptimizer):
         """Final (..., out) result in ``x.dtype``: the two launches of :meth:`fused_launches`
         through one call of the library (``segq_linear``), or through two when a
         ``record_launches`` block is timing the kernels apart."""
+        if pre_op is None and gate is None and col_div is None and addend is None:
+            out = self._again(x, bias)
+            if out is not None:
+                return out
         q, g, ws = self.fused_launches(x, bias, pre_op=pre_op, gate=gate, col_div=col_div, addend=addend)
         if ops.recording_launches():
             ops.quantize_launch(q)
@@ -560,6 +564,36 @@ class DefaultOptimizer(BaseOptimizer):
                 ws = ops.int4_workspace(dev, need)
         out = ops.gemm_launch(g, ws)
         return out.view(*parts[0].shape[:-1], N)
+
+    def _again(self, x, bias):
+        """A plain forward whose descriptors and buffers the previous call on this stream has left: new input and
+        output addresses and the library call, or None if there is no such call behind it.  What a small layer
+        costs is the host: through ``fused_launches`` a (2, 256) x 1024 layer takes 12.7 us a pass, 5.8 of them
+        in the library and its two launches, like this 9.9."""
+        plan = self._plan
+        if plan is None or ops.recording_launches() or not (x.is_cuda and x.is_contiguous()):
+            return None
+        cache = plan.get("launches")
+        shape = x.shape
+        if cache is None or shape[-1] != plan["K"]:
+            return None
+        dtype = x.dtype
+        hit = cache.get((x.numel() // plan["K"], dtype, None if bias is None else bias.data_ptr()))
+        bufs = None if hit is None else hit.get("buffers")
+        if bufs is None:
+            return None
+        dev = x.device
+        stream = ops._stream(dev)
+        reuse = bufs.get(stream)
+        if reuse is None or (hit["need"] and not reuse[1].workspace):
+            return None
+        out = torch.empty((*shape[:-1], hit["N"]), dtype=dtype, device=dev)
+        qd, gd = reuse[0], reuse[1]
+        qd.x = x.data_ptr()
+        qd.ldx = plan["K"]
+        gd.out = out.data_ptr()
+        ops.linear_again(qd, gd, stream)
+        return out
 
     def _relaunch(self, hit, x2, fresh=False):
         """The launches of :meth:`fused_launches` for another input of a token count seen before:

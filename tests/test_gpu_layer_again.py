@@ -1,4 +1,4 @@
-"""Repeated forwards of one layer."""
+"""Repeated forwards of one layer take the short way; each must be bit-equal to a fresh layer's first forward."""
 import pytest
 import torch
 
@@ -18,6 +18,37 @@ def _layer(seed, dynamic, dt, m=40):
     layer.calibrate(x)
     layer.finish_calibrate()
     return layer
+
+
+@pytest.mark.parametrize("dynamic", [False, True])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_repeated_forwards(dynamic, dt):
+    layer = _layer(5, dynamic, dt)
+    kept, want = [], []
+    side = torch.cuda.Stream()
+    for i in range(12):
+        x = torch.randn(40, 1168, device=DEV).to(dt)
+        form = i % 6
+        if form == 1:
+            x = x.view(2, 20, 1168)
+        elif form == 2:  # rows of a wider tensor
+            x = torch.cat([x, x], dim=1)[:, :1168]
+        elif form == 3:  # another token count
+            x = x[:24]
+        if form == 4:
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                y = layer(x)
+            torch.cuda.current_stream().wait_stream(side)
+            x.record_stream(side)
+            y.record_stream(torch.cuda.current_stream())
+        else:
+            y = layer(x)
+        assert y.shape == (*x.shape[:-1], 1000) and y.dtype == dt
+        kept.append(y)
+        want.append(_layer(5, dynamic, dt)(x))
+    for y, w in zip(kept, want):  # earlier outputs are not overwritten by later calls
+        assert torch.equal(y, w)
 
 
 def test_what_a_repeated_call_refuses():
