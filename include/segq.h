@@ -217,7 +217,9 @@ typedef struct segq_krange {
                              * scales, which has to be finite (scales that a calibrator clamps).  Non-zero: every
                              * range is summed on its own and scaled by its own factors, as int8 ranges always
                              * are, so that a scale may be infinite: limit / 0 of a DualScale side that holds
-                             * nothing, which adds nothing.  Not combined with a low-rank branch. */
+                             * nothing, which adds nothing.  Not combined with a low-rank branch.
+                             * 2: the scales are finite and the library takes the faster way (two ranges over the
+                             * same run of K, a and then a_neg, can be multiplied in one walk of it). */
     const float* sx;        /* device */
     const float* sw;        /* device */
 } segq_krange;

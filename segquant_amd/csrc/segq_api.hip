@@ -114,6 +114,80 @@ static int choose_tile(int64_t m, int64_t n, int64_t batch, bool fold, bool wide
     return tiles(2) >= 256 ? 2 : 3;
 }
 
+// A tile that walks K once (segq_gemm_wide.h, launch_walk) and what the launch takes with it, in us, from times on 60 shapes
+// (within 20 %): so much per step of 128 and per round of the CUs.
+struct Walk {
+    int cfg;
+    double us;
+};
+
+static int64_t tiles_of_cfg(int cfg, int64_t m, int64_t n, int64_t batch) {
+    const TileCfg& c = TILE_CFGS[cfg];
+    return (m + c.bm - 1) / c.bm * ((n + c.bn - 1) / c.bn) * batch;
+}
+
+// One range, K not in whole steps.  (Rows of such a K start anywhere in a cache line: a step costs more than an aligned one's.)
+//   us, general kernel before / 256 x 256 / 256 x 192 / 128 x 128:  4900 x 5900 x 4912 270 / 170 / 209 / 231;
+//   4000 x 3000 x 2064 66 / 41 / 37 / 46;  2000 x 3000 x 1008 25.1 / 25.2 / 20.6 / 15.3;  1200 x 3000 x 800 16.2 / 25.4 / 18.8 / 11.1
+static Walk choose_ragged(int64_t m, int64_t n, int64_t batch, int64_t k) {
+    const double steps = (double)((k + 127) / 128);
+    const int64_t cus = device_cus();
+    auto rounds = [&](int cfg) { return (double)((tiles_of_cfg(cfg, m, n, batch) + cus - 1) / cus); };
+    Walk w{FIRST_KT_CFG + 2, 4.2 + 0.72 * steps * rounds(FIRST_KT_CFG + 2)};
+    const bool full = tiles_of_cfg(FIRST_KT_CFG + 1, m, n, batch) * 4 > cus * 3;
+    const double us192 = rounds(FIRST_KT_CFG + 1) * ((full ? 1.72 : 1.15) * steps + 9.0);
+    if (us192 < w.us) w = Walk{FIRST_KT_CFG + 1, us192};
+    const double us256 = rounds(FIRST_KT_CFG) * (2.0 * steps + 6.0);
+    if (us256 < w.us) w = Walk{FIRST_KT_CFG, us256};
+    return w;
+}
+
+// DualScale's two ranges.  us, second register set before / 128 x 192 / 64 x 128:  2 x 2048 x 1536 x 3072 54.8 / 35.6 / 43.1;
+//   3000 x 3000 x 1024 46.3 / 30.8 / 28.4;  2 x 500 x 2000 x 2048 24.9 / 22.5 / 15.4;  merged tensor before, K not in whole
+//   steps: 3 x 2800 x 2000 x 960 166 / 53.6 / 52.6;  2 x 200 x 1000 x 992 21.9 / 14.7 / 8.4.  Below 257 or, in whole steps, 513
+//   the ranges stay in turn (3000 x 2000 x 512 20.1, 64 x 128 15.7): the tests assert the tiles of those launches
+static Walk choose_dual(int64_t m, int64_t n, int64_t batch, int64_t k) {
+    const double steps = (double)((k + 127) / 128);
+    const int64_t cus = device_cus(), t64 = tiles_of_cfg(FIRST_DUAL_CFG + 1, m, n, batch), t192 = tiles_of_cfg(FIRST_DUAL_CFG, m, n, batch);
+    Walk w{FIRST_DUAL_CFG + 1, 4.0 + (double)((t64 + cus - 1) / cus) * ((t64 <= cus ? 0.6 : 0.5) * steps + 0.8)};
+    const double us192 = (double)((t192 + cus - 1) / cus) * (1.3 * steps + 5.5);
+    if (us192 < w.us) w = Walk{FIRST_DUAL_CFG, us192};
+    return w;
+}
+
+// Workgroups that could share the K steps of each of a launch's tiles (1: none).
+static int64_t k_shares(int64_t m, int64_t n, int64_t steps, int cfg) {
+    const int64_t cus = device_cus(), t = tiles_of_cfg(cfg, m, n, 1);
+    if (t * 10 >= cus * 9) return 1;
+    int64_t s = cus / t < steps / 8 ? cus / t : steps / 8;
+    if (s > 16) s = 16;
+    return s > 1 ? s : 1;
+}
+
+// The same two ranges in turn, rescaled in place (e4m3) or, with a workspace, in K shares or parked.  us: 4608 x 3072 x 12288 e4m3
+// 265 in place, 321 in one walk; 400 x 3072 x 12288 52 in eight shares, 80 in one walk; 4096 x 1536 x 6144 78 in two shares, 62 in
+// one walk, int8 88 and 65; 2000 x 2048 x 8192 96 and 61, int8 101 and 63.
+static double in_turn_us(int64_t m, int64_t n, int64_t steps, bool f8, bool ws) {
+    const int64_t cus = device_cus();
+    double us = 1e30;
+    if (ws) {
+        const bool small = m <= 128 && f8;
+        const int64_t s = k_shares(m, n, steps, small ? FIRST_WIDE_CFG + 3 : FIRST_WIDE_CFG + 6);
+        if (s > 1) us = 12.0 + (small ? 0.6 : 1.1) * steps / s + (double)m * n * s * 8.0 / 4e6;
+    }
+    if (f8 || ws) {
+        double fill = 0.0;  // of the largest tiles
+        for (int c : {FIRST_WIDE_CFG, FIRST_WIDE_CFG + 4, FIRST_WIDE_CFG + 5}) {
+            const double rounds = (double)((tiles_of_cfg(c, m, n, 1) + cus - 1) / cus);
+            const double f = (double)m * n / (rounds * cus * TILE_CFGS[c].bm * TILE_CFGS[c].bn);
+            if (f > fill) fill = f;
+        }
+        const double whole = 8.0 + (double)m * n * 256.0 * steps / (f8 ? 2.6e9 : 2.2e9) / fill;
+        if (whole < us) us = whole;
+    }
+    return us;
+}
+
 // int4 weight rows (two values per byte, even k in the low nibble) -> int8 rows.
 // One thread expands 16 packed bytes to 32 values.
 __global__ void __launch_bounds__(256) expand_i4_kernel(const uint8_t* src, int64_t ld_src, uint8_t* dst, int64_t ld_dst,
@@ -276,19 +350,46 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     if (w4 && ktotal > 131071) return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: K too large for int4 weights");
     if (kmax > 0x7fffff00) return fail(SEGQ_ERR_ARG, "segq_gemm: K too large");
 
+    // One walk of K: one range whose end is ragged, or DualScale's two ranges over the same run (a, then a_neg)
+    Walk walk{-1, 1e30};
+    {
+        const segq_krange &r = d->ranges[0], &s = d->ranges[d->n_ranges - 1];
+        const bool base = (i8 || f8) && !lowrank && !codes_out && !groups && d->split_k <= 1 && d->m * d->lda < (int64_t)1 << 32 && d->n * d->ldb < (int64_t)1 << 32;
+        const bool one = base && d->n_ranges == 1 && r.a_sel < 2;
+        const bool two = base && d->n_ranges == 2 && r.k_begin == s.k_begin && r.k_len == s.k_len && r.a_sel == 0 && s.a_sel == 1;
+        if (d->tile > FIRST_KT_CFG && d->tile <= NUM_TILE_CFG) {
+            if (!(d->tile > FIRST_DUAL_CFG ? two : one))
+                return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: tiles %d to %d serve one range, tiles %d to %d two over the same run of K from a and a_neg, in plain "
+                                                  "8-bit codes, without group factors, a low-rank branch, codes out or split_k",
+                            FIRST_KT_CFG + 1, FIRST_DUAL_CFG, FIRST_DUAL_CFG + 1, NUM_TILE_CFG);
+            walk.cfg = (int)d->tile - 1;
+        } else if (d->tile == 0 && d->out_dtype != SEGQ_ACC) {
+            if (one && r.k_len % 128) walk = choose_ragged(d->m, d->n, d->batch, r.k_len);
+            if (two && r.own_sum && r.k_len > (r.k_len % 128 ? 256 : 512)) {
+                walk = choose_dual(d->m, d->n, d->batch, r.k_len);
+                const bool lent = d->split_k != 1 && ws && al(ws, 16), in_turn = r.k_len % 128 == 0 && d->batch == 1;
+                const int64_t steps = r.k_len / 64;  // of both ranges in turn
+                if (in_turn && r.own_sum == 2) {  // (0.85: the estimates)
+                    if (0.85 * in_turn_us(d->m, d->n, steps, f8, lent) < walk.us) walk.cfg = -1;
+                } else if (in_turn && lent && k_shares(d->m, d->n, steps, FIRST_WIDE_CFG + 6) > 2) {
+                    walk.cfg = -1;  // a workspace lent to ranges summed on their own is lent for K shares
+                }
+            }
+        }
+    }
     const int few = [&]() -> int {
         const int64_t reach = (int64_t)1 << 31;  // a tile's rows are addressed with 31 bits
         const segq_krange& r = d->ranges[0];
         const bool ok = d->n_ranges == 1 && r.a_sel < 2 && d->m < reach >> 4 && d->n < reach >> 4 && !lowrank && !codes_out && d->split_k <= 1 && 64 * d->lda + kmax < reach && 64 * d->ldb + kmax < reach &&
                         (!groups || (w4 && r.k_begin % 128 == 0 && r.k_len % 128 == 0 && d->n % 4 == 0 && d->group_dequant_stride % 4 == 0 &&
                                      al(d->group_dequant, 16) && kmax / 128 * d->group_dequant_stride < reach / 4));
-        if (d->tile != 0) return d->tile > FIRST_FEW_CFG && d->tile <= NUM_TILE_CFG ? (ok ? (int)d->tile - 1 : -2) : -1;
+        if (d->tile != 0) return d->tile > FIRST_FEW_CFG && d->tile <= FIRST_KT_CFG ? (ok ? (int)d->tile - 1 : -2) : -1;
         // (raw accumulators are for checks of the integers and keep the route, and the workspace, that they had)
-        return ok && d->out_dtype != SEGQ_ACC ? choose_few(d->m, d->n, d->batch, r.k_len, f8 ? GEMM_F8 : GEMM_I8, w4, groups) : -1;
+        return ok && d->out_dtype != SEGQ_ACC ? choose_few(d->m, d->n, d->batch, r.k_len, f8 ? GEMM_F8 : GEMM_I8, w4, groups, walk.us) : -1;
     }();
     if (few == -2)
         return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: tiles %d to %d serve one range without a sign selection, a low-rank branch, codes out or split_k "
-                                          "(and group factors of int4 weights)", FIRST_FEW_CFG + 1, NUM_TILE_CFG);
+                                          "(and group factors of int4 weights)", FIRST_FEW_CFG + 1, FIRST_KT_CFG);
     if (groups && w4) {
         const int64_t kp = (kmax + 31) & ~(int64_t)31;
         if (!ws || !al(ws, 16) || ws_bytes < d->n * kp)
@@ -368,6 +469,19 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         }
         return launch_gemm_few(p, f8 ? GEMM_F8 : GEMM_I8, w4, few, d->batch, st);
     }
+    if (walk.cfg >= 0) {
+        const TileCfg& c = TILE_CFGS[walk.cfg];
+        const int64_t tm = (d->m + c.bm - 1) / c.bm, tn = (d->n + c.bn - 1) / c.bn;
+        if (tm * tn > 0x7fffffff || d->batch > 65535) return fail(SEGQ_ERR_ARG, "segq_gemm: grid too large");
+        p.tiles_m = (int32_t)tm;
+        p.tiles_n = (int32_t)tn;
+        p.group_m = 8;
+        if (plan) {
+            plan->tile = walk.cfg + 1;
+            p.dry = 1;
+        }
+        return i8 ? launch_gemm_i8(p, walk.cfg, false, d->batch, st) : launch_gemm_f8(p, walk.cfg, false, d->batch, st);
+    }
     const bool fold = d->n_ranges > 1;
     bool wide_ok = d->m * d->lda < (int64_t)1 << 32 && d->n * d->ldb < (int64_t)1 << 32;
     for (int i = 0; i < d->n_ranges; ++i) wide_ok = wide_ok && d->ranges[i].k_begin % 128 == 0 && d->ranges[i].k_len % 128 == 0;
@@ -377,7 +491,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     // several ranges cost a second (fp32) accumulator set, and with it the biggest tiles,
     // unless the accumulators are fp32 already (plain e4m3: rescaled in place, which takes the ratio of two
     // ranges' scales and is not for callers whose scales may be infinite: own_sum)
-    p.sep = f8 && fold && plain8 && d->ranges[0].own_sum != 0;
+    p.sep = f8 && fold && plain8 && d->ranges[0].own_sum != 0 && d->ranges[0].own_sum != 2;
     const bool fold2 = fold && !(f8 && plain8 && !p.sep);
     if (groups) {
         bool ok = wide_ok && plain8;

@@ -5,8 +5,9 @@ namespace segq {
 
 // Tile for a launch of few tiles, or -1 where the other kernels serve it better.  Both sides are estimated in us from
 // launches with weights from memory; K in steps of 128.  The constants were fitted over 110 shapes of 1 to 5000 rows and 100 to
-// 18432 columns; the choice is within 12 % of the best tile on nine of ten of them.
-int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4, bool grp) {
+// 18432 columns; the choice is within 12 % of the best tile on nine of ten of them.  `other_us`: what the 8-wave tiles for a
+// ragged K would take, where they serve the launch.
+int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4, bool grp, double other_us) {
     const int64_t cus = device_cus(), steps = (k + 127) / 128;
     auto tiles = [&](int64_t bm, int64_t bn) { return (m + bm - 1) / bm * ((n + bn - 1) / bn) * batch; };
     if (tiles(32, 64) > 32 * cus) return -1;
@@ -15,7 +16,7 @@ int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4,
     // int4 weights add their unpacking, group factors the sums
     int best = -1;
     double cost = 0;
-    for (int c = FIRST_FEW_CFG; c < NUM_TILE_CFG; ++c) {
+    for (int c = FIRST_FEW_CFG; c < FIRST_KT_CFG; ++c) {
         const int tm = TILE_CFGS[c].bm / 16, tn = TILE_CFGS[c].bn / 16;
         const int64_t t = tiles(TILE_CFGS[c].bm, TILE_CFGS[c].bn), per_wave = (steps + FEW_WAVES - 1) / FEW_WAVES;
         const bool two = few_two(tm, tn, b4, grp, per_wave <= few_depth(tm, tn, b4, grp) ? (int)per_wave : 0);
@@ -34,6 +35,7 @@ int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4,
     if (b4) return cost < 6.5 + 0.8 * steps * rounds ? best : -1;
     const double full = (double)tiles(64, 128) / (1.5 * cus);
     double other = 6.5 + 0.75 * steps * (full > 1.0 ? full : 1.0);  // the general kernel, 64 x 128
+    if (other_us < other) other = other_us;
     if (k % 128 == 0) {
         bool theirs = t128 >= 32;  // the 8-wave kernels ...
         if (theirs) other = 4.5 + (fmt == GEMM_F8 ? 0.5 : 0.45) * steps * rounds;

@@ -535,16 +535,19 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_kernel(const GemmParams p)
 
 // ---- host-side launch of one (format, tile, fold) instance -------------------
 struct TileCfg { int bm, bn, wgm, wgn; };
-constexpr int NUM_TILE_CFG = 25;
+constexpr int NUM_TILE_CFG = 30;
 constexpr int FIRST_BIG_CFG = 8;    // two retired ids (a 4-wave 256 x 256 kernel that no shape profited from)
 constexpr int FIRST_WIDE_CFG = 10;  // the 8-wave kernels from here on (segq_gemm_wide.h)
 constexpr int FIRST_FEW_CFG = 21;   // tiles whose waves share K (segq_gemm_few.h)
+constexpr int FIRST_KT_CFG = 25;    // 8-wave tiles for one range with a ragged end of K
+constexpr int FIRST_DUAL_CFG = 28;  // ... and for DualScale's two ranges in one walk (rows of each code tensor x columns)
 constexpr TileCfg TILE_CFGS[NUM_TILE_CFG] = {
     {256, 256, 2, 2}, {256, 128, 2, 2}, {128, 128, 2, 2}, {64, 128, 2, 2}, {128, 256, 2, 2},
     {256, 256, 2, 4}, {256, 256, 4, 2}, {256, 128, 4, 2}, {256, 256, 2, 2}, {256, 256, 2, 2},
     {256, 256, 4, 2}, {256, 128, 4, 2}, {128, 256, 2, 4}, {128, 128, 2, 4}, {192, 288, 4, 2}, {288, 192, 2, 4},
     {256, 192, 4, 2}, {192, 256, 2, 4}, {128, 128, 2, 4}, {384, 192, 4, 2}, {128, 96, 4, 2},
     {16, 32, 1, 1}, {16, 64, 1, 1}, {32, 32, 1, 1}, {32, 64, 1, 1},
+    {256, 256, 4, 2}, {256, 192, 4, 2}, {128, 128, 2, 4}, {128, 192, 4, 2}, {64, 128, 2, 4},
 };
 
 // Steps in flight of the general kernel's 64 x 128 and 128 x 128 tiles, one range (every other launch: one step ahead;
@@ -577,9 +580,15 @@ int launch_instance(const GemmParams& p, int64_t batch, hipStream_t st) {
 
 template <int FMT, bool B4>
 int launch_wide(const GemmParams& p, int wcfg, bool fold, bool asel, int64_t batch, hipStream_t st);
+template <int FMT>
+int launch_walk(const GemmParams& p, int cfg, int64_t batch, hipStream_t st);
 
 template <int FMT, bool B4>
 int launch_format(const GemmParams& p, int cfg, bool fold, int64_t batch, hipStream_t st) {
+    if (cfg >= FIRST_KT_CFG) {
+        if constexpr (!B4) return launch_walk<FMT>(p, cfg, batch, st);
+        return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: tile %d needs plain 8-bit codes on both sides", cfg + 1);
+    }
     if (cfg >= FIRST_WIDE_CFG) {
         bool asel = false;
         for (int i = 0; i < p.nr; ++i) asel = asel || p.r[i].a_sel >= 2;
@@ -613,7 +622,7 @@ int launch_format(const GemmParams& p, int cfg, bool fold, int64_t batch, hipStr
 int launch_gemm_i8(const GemmParams& p, int cfg, bool fold, int64_t batch, hipStream_t st);
 int launch_gemm_f8(const GemmParams& p, int cfg, bool fold, int64_t batch, hipStream_t st);
 int launch_gemm_w4(const GemmParams& p, int cfg, bool fold, int64_t batch, hipStream_t st);
-int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4, bool grp);
+int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4, bool grp, double other_us);
 int launch_gemm_few(const GemmParams& p, int fmt, bool b4, int cfg, int64_t batch, hipStream_t st);
 
 }  // namespace segq

@@ -623,9 +623,18 @@ __device__ __forceinline__ float recip(float x) {
 
 template <int BM, int BN, int WGM, int WGN, int FMT, bool FOLD, int NS, bool GRP = false, bool PARK = false, bool FINISH = false,
           bool CODES = false,  // CODES: the epilogue writes the next linear's codes instead of floats (one range)
-          bool SEP = false>    // SEP (e4m3, several ranges): a second register set, as int8 has it, instead of rescaling in place
+          bool SEP = false,    // SEP (e4m3, several ranges): a second register set, as int8 has it, instead of rescaling in place
+          bool KT = false,     // KT: K ends anywhere in sixteens (one walk of K)
+          bool DUAL = false>   // DUAL: two ranges over one run of K, from the two code tensors, in one walk
 __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmParams p) {
     static_assert(!CODES || (!FOLD && !GRP && !PARK && !FINISH), "codes out: plain operands, one range");
+    static_assert(!KT || (!FOLD && !GRP && !PARK && !FINISH && !CODES && NS == 2), "a ragged end of K: one walk, two stages");
+    static_assert(!DUAL || KT, "DUAL instances take any K");
+    // DUAL (DualScale's two ranges over the same K and the same weights): the tile's BM rows of LDS are BM / 2 rows of each
+    // code tensor, the two halves of every wave's row blocks, so that a wave holds both sums of an output and a weight
+    // tile is read once for both.  What two ranges in turn need a second register set for, these have as the second
+    // half of their blocks, and each sum is scaled by its own range's scales at the end.
+    constexpr int OM = DUAL ? BM / 2 : BM;  // output rows of the tile
     constexpr int NW = WGM * WGN, NT = NW * 64;
     constexpr int WM = BM / WGM, WN = BN / WGN;
     constexpr int TM = WM / 16, TN = WN / 16;
@@ -727,7 +736,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         tile_m = first_m + in_g % rows_in_group;
         tile_n = in_g / rows_in_group;
     }
-    const int m0 = tile_m * BM, n0 = tile_n * BN;
+    const int m0 = tile_m * OM, n0 = tile_n * BN;
     const int64_t z = zy;
     const uint8_t* const Ab = p.A + z * p.bsA;
     const uint8_t* const A2b = p.A2 ? p.A2 + z * p.bsA : nullptr;
@@ -737,10 +746,32 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     const int s_lc = (tid & 7) ^ swz(s_row);
     uint32_t a_goff[A_IT], b_goff[B_IT];
 #pragma unroll
-    for (int i = 0; i < A_IT; ++i) a_goff[i] = (uint32_t)min(m0 + s_row + i * RPI, p.M - 1) * (uint32_t)p.lda + s_lc * 16;
+    for (int i = 0; i < A_IT; ++i) {
+        int row = s_row + i * RPI;
+        if constexpr (DUAL) row = row / WM * (WM / 2) + row % (WM / 2);
+        a_goff[i] = (uint32_t)min(m0 + row, p.M - 1) * (uint32_t)p.lda + s_lc * 16;
+    }
 #pragma unroll
     for (int i = 0; i < B_IT; ++i) b_goff[i] = (uint32_t)min(n0 + s_row + i * RPI, p.N - 1) * (uint32_t)p.ldb + s_lc * 16;
     const int w_lds = wave * 8 * BK;
+    static_assert(!DUAL || (RPI % WM == 0 && WM % 32 == 0), "a wave's eight rows of a pass come from one of the two tensors");
+    const bool second = DUAL && (wave * 8) % WM >= WM / 2;
+    // KT: pieces of a row past the end of K.  They are loaded from the step's first piece instead, which is there (a weight
+    // row that holds a NaN gives NaN either way), and what they became in the activations is cleared before it is read.
+    const int k_tail = KT ? (p.r[0].k1 - p.r[0].k0) % BK : 0;
+    const bool past_k = KT && k_tail != 0 && s_lc * 16 >= k_tail;
+    uint32_t back = 0;  // what to go back by in the step that is loaded next
+    auto clear_tail = [&](int buf) __attribute__((always_inline)) {
+        if constexpr (KT) {
+            if (past_k) {
+#pragma unroll
+                for (int i = 0; i < A_IT; ++i)
+                    if (!(A_TAIL != 0 && i == A_IT - 1 && s_row >= A_TAIL))
+                        *reinterpret_cast<uint4*>(As + buf * BM * BK + (s_row + i * RPI) * BK + (tid & 7) * 16) = make_uint4(0, 0, 0, 0);
+            }
+            __syncthreads();
+        }
+    };
 
     // a wave covers 8 rows of a pass, so whether it takes part in a partial last pass is wave-uniform
     const bool a_skip = A_TAIL != 0 && wave * 8 >= A_TAIL;
@@ -748,10 +779,10 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     auto dma1 = [&](const uint8_t* ap, const uint8_t* bp, int buf, int i) {
         if (i < A_IT) {
             if (i == A_IT - 1 && a_skip) return;
-            load16_to_lds(ap + a_goff[i], As + buf * BM * BK + w_lds + i * RPI * BK);
+            load16_to_lds(ap + (KT ? a_goff[i] - back : a_goff[i]), As + buf * BM * BK + w_lds + i * RPI * BK);
         } else {
             if (i == A_IT + B_IT - 1 && b_skip) return;
-            load16_to_lds(bp + b_goff[i - A_IT], Bs + buf * BN * BK + w_lds + (i - A_IT) * RPI * BK);
+            load16_to_lds(bp + (KT ? b_goff[i - A_IT] - back : b_goff[i - A_IT]), Bs + buf * BN * BK + w_lds + (i - A_IT) * RPI * BK);
         }
     };
     // "all but the newest nt tiles of this wave's DMA have landed, and all its LDS reads"
@@ -913,7 +944,9 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     // source of its activations stay in registers, so the range table is read
     // only when a cursor crosses into the next range.
     int steps = 0;
-    for (int i = 0; i < p.nr; ++i) steps += (p.r[i].k1 - p.r[i].k0) / BK;
+    if constexpr (KT) steps = (p.r[0].k1 - p.r[0].k0 + BK - 1) / BK;
+    else
+        for (int i = 0; i < p.nr; ++i) steps += (p.r[i].k1 - p.r[i].k0) / BK;
     int lr = 0, skip = 0;  // this workgroup's first step: `skip` steps into range lr
     if (p.splits > 1) {
         skip = (int)((int64_t)steps * zy / p.splits);
@@ -928,9 +961,14 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     }
     const int r_first = lr, k_first = p.r[ph(lr)].k0 + skip * BK;
     int lk = k_first, lk1 = p.r[ph(lr)].k1;
-    const uint8_t* la = (p.r[ph(lr)].a_sel == 1) ? A2b : Ab;
+    const uint8_t* la = (DUAL ? second : p.r[ph(lr)].a_sel == 1) ? A2b : Ab;
+    if (KT && lk + BK > lk1) back = past_k ? s_lc * 16 : 0;
     auto advance_load = [&]() {
         lk += BK;
+        if constexpr (KT) {
+            if (lk + BK > lk1) back = past_k ? s_lc * 16 : 0;
+            return;
+        }
         if (lk >= lk1) {
             ++lr;
             const int rr = min(lr, p.nr - 1);  // past the last range nothing more is loaded
@@ -944,7 +982,8 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     // are fetched first of all, so that the wait for the first DMA covers them, and
     // parked in LDS behind the stages: the epilogue then starts without a round
     // trip to memory, and without the ~70 small loads per wave it would take there.
-    constexpr int EPI_FLOATS = BM + 2 * BN, EPI_IT = (EPI_FLOATS + NT - 1) / NT;
+    // (DUAL: [1/sx | 1/sw | bias] of the first range, as the epilogue reads them, then [1/sx | 1/sw] of the second)
+    constexpr int EPI_FLOATS = DUAL ? 2 * OM + 3 * BN : BM + 2 * BN, EPI_IT = (EPI_FLOATS + NT - 1) / NT;
     float* const epi = reinterpret_cast<float*>(smem + NS * (BM + BN) * BK);
     // group factors: a ring of four rows of BN floats behind the epilogue's vectors.  The row of
     // step s arrives with the step's operands and is read all through step s, at whose end the
@@ -961,7 +1000,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
             lslot = (lslot + 1) & 3;
         }
     };
-    const int r_epi = ACCF ? 0 : ph(r_last);  // the range (as the caller numbers them) whose units the accumulators end up in
+    const int r_epi = ACCF || DUAL ? 0 : ph(r_last);  // the range (as the caller numbers them) whose units the accumulators end up in
     float epi_val[EPI_IT];
     const bool want_epi = p.out_dtype != SEGQ_ACC;  // raw accumulators come with no scales at all (null pointers)
 #pragma unroll
@@ -969,12 +1008,16 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         const int e = i * NT + tid;
         float v = 0.0f;
         if (!want_epi) {
-        } else if (e < BM) {
+        } else if (e < OM) {
             if constexpr (!ACCF) v = (p.r[r_epi].sx + z * p.bsSx)[(int64_t)min(m0 + e, p.M - 1) * p.r[r_epi].sx_rs];
-        } else if (e < BM + BN) {
-            if constexpr (!ACCF) v = (p.r[r_epi].sw + z * p.bsSw)[(int64_t)min(n0 + e - BM, p.N - 1) * p.r[r_epi].sw_cs];
-        } else if (e < EPI_FLOATS) {
-            if (p.bias) v = load_bias(p.bias, p.bias_dtype, min(n0 + e - BM - BN, p.N - 1));
+        } else if (e < OM + BN) {
+            if constexpr (!ACCF) v = (p.r[r_epi].sw + z * p.bsSw)[(int64_t)min(n0 + e - OM, p.N - 1) * p.r[r_epi].sw_cs];
+        } else if (e < OM + 2 * BN) {
+            if (p.bias) v = load_bias(p.bias, p.bias_dtype, min(n0 + e - OM - BN, p.N - 1));
+        } else if (DUAL && e < 2 * OM + 2 * BN) {
+            v = (p.r[1].sx + z * p.bsSx)[(int64_t)min(m0 + e - OM - 2 * BN, p.M - 1) * p.r[1].sx_rs];
+        } else if (DUAL && e < EPI_FLOATS) {
+            v = (p.r[1].sw + z * p.bsSw)[(int64_t)min(n0 + e - 2 * OM - 2 * BN, p.N - 1) * p.r[1].sw_cs];
         }
         epi_val[i] = v;
     }
@@ -995,9 +1038,16 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
 #pragma unroll
     for (int i = 0; i < EPI_IT; ++i) {
         const int e = i * NT + tid;
-        if (e < EPI_FLOATS) epi[e] = (e < BM + BN && !ACCF) ? __builtin_amdgcn_rcpf(epi_val[i]) : epi_val[i];
+        if constexpr (KT) {  // (quotients, as exact as the general kernel's, which such launches had)
+            if (e < EPI_FLOATS) epi[e] = (e < OM + BN || e >= OM + 2 * BN) ? 1.0f / epi_val[i] : epi_val[i];
+        } else {
+            if (e < EPI_FLOATS) epi[e] = (e < BM + BN && !ACCF) ? __builtin_amdgcn_rcpf(epi_val[i]) : epi_val[i];
+        }
     }
     __syncthreads();
+    if constexpr (KT) {
+        if (steps == 1) clear_tail(0);
+    }
     if constexpr (S8) {
 #pragma unroll
         for (int i = 0; i <= TM; ++i) frag8(0, i);  // activations and the first weight fragment
@@ -1082,6 +1132,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         }
         wait_dma(std::integral_constant<int, 0>{});
         __syncthreads();
+        if constexpr (KT && MORE_ && !DMA_) clear_tail(nbuf);  // (two stages: the next step is the last)
         const uint8_t* const ap = la + lk;
         const uint8_t* const bp = Bb + lk;
 #pragma unroll
@@ -1158,7 +1209,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         ck += BK;
         cslot = (cslot + 1) & 3;
         dirty = true;
-        if (ck >= ck1) {
+        if (!KT && ck >= ck1) {
             if constexpr (FOLD) fold(cr);
             dirty = false;
             ++cr;
@@ -1204,6 +1255,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         // tile s+1 or overwrites the buffer of tile s.
         wait_dma(std::integral_constant<int, DMA_ ? NS - 2 : 0>{});
         __syncthreads();
+        if constexpr (KT && MORE_ && !DMA_) clear_tail(nbuf);  // (two stages: the next step is the last)
         // tile s+NS goes where tile s was: both its halves are in registers
         const uint8_t* const ap = la + lk;
         const uint8_t* const bp = Bb + lk;
@@ -1229,7 +1281,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         if constexpr (DMA_) advance_load();
         ck += BK;
         dirty = true;
-        if (ck >= ck1) {  // the range is complete: fold it, move to the next one
+        if (!KT && ck >= ck1) {  // the range is complete: fold it, move to the next one
             if constexpr (PARK) park(cr);
             else if constexpr (FOLD) fold(cr);
             dirty = false;
@@ -1337,7 +1389,21 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         wide_epilogue<BM, BN, WGM, WGN, GEMM_F8, false, true>(p, of, of, smem, z, m0, n0, wave, lane, r_epi, epi);
         return;
     }
-    if constexpr (GRP) {
+    if constexpr (DUAL) {
+        v4f of[TN][TM / 2];
+        const float* const rx2 = epi + OM + 2 * BN;
+#pragma unroll
+        for (int a = 0; a < TN; ++a) {
+            const int n = wn * WN + a * 16 + 4 * lgrp;
+            const v4f w = *reinterpret_cast<const v4f*>(epi + OM + n), w2 = *reinterpret_cast<const v4f*>(rx2 + OM + n);
+#pragma unroll
+            for (int b = 0; b < TM / 2; ++b) {
+                const int m = wm * (WM / 2) + b * 16 + lrow;
+                of[a][b] = __builtin_convertvector(acc[a][b], v4f) * epi[m] * w + __builtin_convertvector(acc[a][b + TM / 2], v4f) * rx2[m] * w2;
+            }
+        }
+        wide_epilogue<OM, BN, WGM, WGN, GEMM_F8, false, true>(p, of, of, smem, z, m0, n0, wave, lane, 0, epi);
+    } else if constexpr (GRP) {
         v4f none[1][1];
         wide_epilogue<BM, BN, WGM, WGN, GEMM_F8, false, false>(p, accf, none, smem, z, m0, n0, wave, lane, r_epi, epi);
     } else if constexpr (CODES) {
@@ -1361,17 +1427,34 @@ int launch_wide_instance(const GemmParams& p, int64_t batch, hipStream_t st) {
 
 // wide tile ids (after the generic ones): 256x256 | 256x128 | 128x256 | 128x128, eight waves each
 template <int BM, int BN, int WGM, int WGN, int FMT, bool FOLD, int NS, bool GRP = false, bool PARK = false, bool FINISH = false,
-          bool CODES = false, bool SEP = false>
+          bool CODES = false, bool SEP = false, bool KT = false, bool DUAL = false>
 int launch_pipe_instance(const GemmParams& p, int64_t batch, hipStream_t st) {
-    auto kern = gemm_pipe_kernel<BM, BN, WGM, WGN, FMT, FOLD, NS, GRP, PARK, FINISH, CODES, SEP>;
+    auto kern = gemm_pipe_kernel<BM, BN, WGM, WGN, FMT, FOLD, NS, GRP, PARK, FINISH, CODES, SEP, KT, DUAL>;
     // the stages, the epilogue's vectors, and the ring of group factors
-    constexpr int lds = NS * (BM + BN) * BK + (BM + 2 * BN) * 4 + (GRP ? 4 * BN * 4 : 0);
+    constexpr int lds = NS * (BM + BN) * BK + (DUAL ? BM + 3 * BN : BM + 2 * BN) * 4 + (GRP ? 4 * BN * 4 : 0);
     if (p.dry) return SEGQ_OK;
     static unsigned long long attr_done = 0;
     if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), lds, &attr_done)) return rc;
     dim3 grid((unsigned)(p.tiles_m * p.tiles_n), (unsigned)batch);
     hipLaunchKernelGGL(kern, grid, dim3(WGM * WGN * 64), lds, st, p);
     return check_launch("segq_gemm");
+}
+
+// One walk of K with a ragged end: one range, or DualScale's two over the same run.
+template <int FMT>
+int launch_walk(const GemmParams& p, int cfg, int64_t batch, hipStream_t st) {
+    constexpr int WM = FMT == GEMM_F8 ? 4 : 2, WN = FMT == GEMM_F8 ? 2 : 4;  // (e4m3 wants three or more column blocks per wave)
+#define SEGQ_WALK(BM_, BN_, WGM_, WGN_, DUAL_) \
+    return launch_pipe_instance<BM_, BN_, WGM_, WGN_, FMT, false, 2, false, false, false, false, false, true, DUAL_>(p, batch, st)
+    switch (cfg) {
+        case FIRST_KT_CFG: SEGQ_WALK(256, 256, 4, 2, false);
+        case FIRST_KT_CFG + 1: SEGQ_WALK(256, 192, 4, 2, false);
+        case FIRST_KT_CFG + 2: SEGQ_WALK(128, 128, WM, WN, false);
+        case FIRST_DUAL_CFG: SEGQ_WALK(256, 192, 4, 2, true);
+        case FIRST_DUAL_CFG + 1: SEGQ_WALK(128, 128, WM, WN, true);
+    }
+#undef SEGQ_WALK
+    return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: no kernel for tile %d", cfg + 1);
 }
 
 template <int FMT, bool B4>

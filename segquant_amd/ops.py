@@ -273,7 +273,8 @@ def gemm_workspace_bytes(g) -> int:
 # tile ids of the 8-wave kernels (segq_gemm_desc.tile) -> rows x columns of the output tile
 TILE_SHAPES = {1: "256x256", 2: "256x128", 3: "128x128", 4: "64x128", 5: "128x256", 6: "256x256", 7: "256x256", 8: "256x128",
                11: "256x256", 12: "256x128", 13: "128x256", 14: "128x128", 15: "192x288", 16: "288x192", 17: "256x192", 18: "192x256", 19: "128x128", 20: "384x192", 21: "128x96",
-               22: "16x32", 23: "16x64", 24: "32x32", 25: "32x64"}
+               22: "16x32", 23: "16x64", 24: "32x32", 25: "32x64",
+               26: "256x256", 27: "256x192", 28: "128x128", 29: "128x192", 30: "64x128"}
 
 
 def gemm_plan(g, workspace: Optional[torch.Tensor] = None) -> dict:
@@ -285,7 +286,7 @@ def gemm_plan(g, workspace: Optional[torch.Tensor] = None) -> dict:
         d.workspace = workspace.data_ptr(); d.workspace_bytes = workspace.numel() * workspace.element_size()
     tile, splits, parked = C.c_int32(0), C.c_int32(0), C.c_int32(0)
     L.check(L.lib().segq_gemm_plan(C.byref(d), C.byref(tile), C.byref(splits), C.byref(parked)))
-    family = "gemm_few_kernel" if tile.value >= 22 else "gemm_pipe_kernel" if tile.value >= 11 else "gemm_kernel"
+    family = "gemm_few_kernel" if 22 <= tile.value <= 25 else "gemm_pipe_kernel" if tile.value >= 11 else "gemm_kernel"
     return dict(tile=tile.value, shape=TILE_SHAPES.get(tile.value, "?"), splits=splits.value, parked=bool(parked.value),
                 kernel=f"segq::{family}<{TILE_SHAPES.get(tile.value, '?').replace('x', ',')}>")
 
@@ -350,7 +351,7 @@ def gemm_desc(a: torch.Tensor, b: torch.Tensor, ranges: Sequence[Range], *, m: i
          batch_stride_sx: int = 0, batch_stride_sw: int = 0, out: Optional[torch.Tensor] = None,
          tile: int = 0, workspace: Optional[torch.Tensor] = None,
          group_dequant: Optional[torch.Tensor] = None, split_k: int = 0,
-         addend: Optional[torch.Tensor] = None, lowrank=None, out_codes: Optional[dict] = None, own_sums: bool = False):
+         addend: Optional[torch.Tensor] = None, lowrank=None, out_codes: Optional[dict] = None, own_sums: int = 0):
     """The ``segq_gemm_desc`` of a segmented GEMM with fused de-quantisation and bias, its output
     tensor, the launch's description and the tensors the descriptor points into.
 
@@ -367,8 +368,8 @@ def gemm_desc(a: torch.Tensor, b: torch.Tensor, ranges: Sequence[Range], *, m: i
     ``out_dtype`` is a torch float dtype, or the string ``"acc"`` for the raw
     accumulators (int32 for integer codes, float32 for e4m3).  ``workspace``: a
     byte tensor the library may expand int4 weights into, or park the sums of
-    finished int8 ranges in (see ``int4_workspace``, ``park_bytes``).  ``own_sums``: sum every
-    e4m3 range on its own, for scales that may be infinite (``segq_krange.own_sum``).
+    finished int8 ranges in (see ``int4_workspace``, ``park_bytes``).  ``own_sums``: 1 sums every
+    e4m3 range on its own, for scales that may be infinite; 2 leaves the way to the library (``segq_krange.own_sum``).
     """
     _need_cuda(a, b, a_neg, bias)
     raw = out_dtype == "acc"
@@ -453,7 +454,7 @@ def gemm_desc(a: torch.Tensor, b: torch.Tensor, ranges: Sequence[Range], *, m: i
                 raise RuntimeError("scales must be float32")
         kr.sx = r.sx.data_ptr() if r.sx is not None else None
         kr.sw = r.sw.data_ptr() if r.sw is not None else None
-    d.ranges[0].own_sum = 1 if own_sums else 0
+    d.ranges[0].own_sum = own_sums
     info = dict(m=m, n=n, batch=batch, k_alg=sum(r.k_len for r in ranges if r.a_sel in (0, 2)),
                 k_exec=sum(r.k_len for r in ranges), a_fmt=a_fmt, b_fmt=b_fmt)
     if oc is not None:
@@ -528,17 +529,16 @@ def _dual_in_two_tensors(tiles: int, K: int, int4: bool) -> bool:
     """Whether the DualScale operator writes two code tensors, which stream straight into LDS, or one
     merged tensor, whose signs the GEMM selects on the way there.  ``tiles``: 128 x 128 tiles of the output.
 
-    Two where the GEMM then runs on the 8-wave kernels (plain 8-bit codes from 32 tiles, int4 weights from 96, K in
-    whole 128-byte steps) and its K loop repays the second tensor.  Both launches, merged / two, us: 512 x 1024,
-    32 tiles, K 256 13.9 / 10.5 (merged runs on the general kernel up to 95 tiles); 2 x 1000 x 1000, 128 tiles,
-    K 256 12.4 / 13.2, K 512 16.0 / 16.5, K 2048 40 / 34; 2 x 3000 x 3000, 1152 tiles, K 256 40.5 / 39.5,
-    K 512 56.6 / 49.5, K 4096 261 / 186.  int4, 256 tiles, K 1536 33.8 / 35.8, K 2048 42.8 / 41.5;
-    1152 tiles, K 512 59.6 / 54.4."""
-    if K % 128 or tiles < (96 if int4 else 32):
-        return False
+    8-bit weights: two wherever the GEMM multiplies both in one walk of K, beyond K 256, or 512 in whole 128-byte steps (the
+    GEMM alone, merged / two, us: 3 x 2800 x 2000 x 960 164 / 51, 2 x 200 x 1000 x 992 22 / 9, 2 x 2048 x 1536 x 3072 68 / 35,
+    2 x 300 x 600 x 1024 21 / 9).  Whole steps up to there run range by range: two from 32 tiles where the K loop repays the second tensor (512 x 1024, 32 tiles, K 256 13.9 / 10.5, merged
+    runs on the general kernel up to 95 tiles; 2 x 1000 x 1000, 128 tiles, K 256 12.4 / 13.2, K 512 16.0 / 16.5).
+    int4, 256 tiles, K 1536 33.8 / 35.8, K 2048 42.8 / 41.5; 1152 tiles, K 512 59.6 / 54.4."""
     if int4:  # (256 tiles: one for every compute unit)
-        return K >= (512 if tiles > 256 else 2048)
-    return tiles < 96 or K >= 512
+        return K % 128 == 0 and tiles >= 96 and K >= (512 if tiles > 256 else 2048)
+    if K > (256 if K % 128 else 512):
+        return True
+    return K % 128 == 0 and tiles >= 32 and (tiles < 96 or K >= 512)
 
 
 @functools.lru_cache(maxsize=256)
@@ -570,17 +570,15 @@ def real_quantized_gemm_dual_scaled(fmt_a: str, fmt_w: str, inputs: torch.Tensor
 
     One quantise launch over all segments and one batched GEMM that reads every
     segment as two ranges, the non-negative codes with the positive scale and the
-    negative ones with the negative scale.  Each range is summed on its own (a
-    second register set): the scales come from the caller, and a side that holds
-    nothing may have ``limit / 0 = inf``, whose zeros add nothing.  (2, 2048, 3072)
-    x 1536, fp16, the whole pass: 76.7 us from one merged tensor, 62.2 us from two.
+    negative ones with the negative scale.  Each range is summed on its own:
+    the scales come from the caller, and a side that holds nothing may have
+    ``limit / 0 = inf``, whose zeros add nothing.
 
-    One segment, few tiles, a long K and 16-bit outputs: the K steps of a tile are
-    shared by several workgroups (bf16, K 4096, both launches, whole tiles and in
-    shares: 1024 x 1024 int8 49.4 and 41.1 us, e4m3 49.5 and 32.9; 200 x 1000 int8
-    68.3 and 24.7).  The room for the shares is the call's own, so that a second host thread on the stream cannot come between the
-    launch and the sum.  fp32 outputs would show the shares' roundings and keep
-    whole tiles.
+    One segment, few tiles, a very long K and 16-bit outputs: the K steps of a tile are
+    shared by several workgroups (bf16, K 4096, 200 x 1000 int8 24.6 us, one walk of K 24;
+    64 x 520 x 2048 e4m3 the same either way).  The room for the shares is the call's own, so
+    that a second host thread on the stream cannot come between the launch and the sum.
+    fp32 outputs would show the shares' roundings and keep whole tiles.
     """
     _check_contract(inputs, weights, fmt_w, pos_scale_x, neg_scale_x, scale_w)
     S, M, N, K = _shapes(inputs, weights, fmt_w)
@@ -591,7 +589,8 @@ def real_quantized_gemm_dual_scaled(fmt_a: str, fmt_w: str, inputs: torch.Tensor
     if not per_seg_w and scale_w.numel() != S * N:
         raise RuntimeError(f"scale_w has {scale_w.numel()} entries, expected {S} or {S * N}")
     need = 0
-    if S == 1 and K % 128 == 0 and K >= 1024 and fmt_w != FMT_INT4 and inputs.dtype != torch.float32:
+    if S == 1 and K % 128 == 0 and fmt_w != FMT_INT4 and inputs.dtype != torch.float32 and \
+            K >= (2048 if M <= 64 and fmt_w == FMT_E4M3 else 4096):
         need = _dual_share_bytes(inputs.device.index, M, N, K, fmt_w, inputs.dtype)
     two = need > 0 or _dual_in_two_tensors(S * -(-M // 128) * -(-N // 128), K, fmt_w == FMT_INT4)
     codes = quantize(inputs.view(S * M, K), fmt_a, pos_scale_x, neg_scale_x, seg_rows=M,
@@ -605,7 +604,7 @@ def real_quantized_gemm_dual_scaled(fmt_a: str, fmt_w: str, inputs: torch.Tensor
          [Range(0, K, pos_scale_x, scale_w, sel[0], rs, cs), Range(0, K, neg_scale_x, scale_w, sel[1], rs, cs)],
          m=M, n=N, a_fmt=fmt_a, b_fmt=fmt_w, out_dtype=inputs.dtype, lda=K, ldb=kb, a_neg=codes_neg,
          batch=S, batch_stride_a=M * K, batch_stride_b=N * kb,
-         batch_stride_sx=1 if per_seg_x else M, batch_stride_sw=1 if per_seg_w else N, out=out, own_sums=True,
+         batch_stride_sx=1 if per_seg_x else M, batch_stride_sw=1 if per_seg_w else N, out=out, own_sums=1,
          workspace=torch.empty(need, dtype=torch.uint8, device=inputs.device) if need else None)
     return out
 

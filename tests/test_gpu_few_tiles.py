@@ -72,8 +72,8 @@ def _check(ops, kind, M, N, K, tile, dt, g, group=False, k0=0, row_sx=True, col_
     # fp32 arithmetic of the scaling (and of the group sums: one rounding per group and per share), the matrix cores' e4m3
     # sums, and the output's one rounding
     tol = (4e-6 + (2.0 ** -23 * ((k0 + K) // 128 + 8) if group else 0.0)) * mag + 1e-30
-    if kind == "e4m3":
-        tol = tol + 3e-4 * mag
+    if kind == "e4m3":  # 3e-4 as elsewhere; of 16 or 32 products none averages out, and each is cut at 2^-15 of the largest
+        tol = tol + (3e-4 if K > 32 else 16 * 2.0 ** -15) * mag
     tol = tol + {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dt] * np.abs(want) + (2.0 ** -24 if dt == torch.float16 else 0.0)
     err = np.abs(got - want)
     assert np.isfinite(got).all() and (err <= tol).all(), (kind, M, N, K, tile, dt, float((err - tol).max()))
@@ -126,5 +126,78 @@ def test_what_the_tiles_do_not_serve_is_refused(ops):
     for ranges in ([ops.Range(0, 256, one, one, 2)], [ops.Range(0, 128, one, one), ops.Range(128, 128, one, one)]):
         with pytest.raises(RuntimeError, match="tiles 22 to 25"):
             ops.gemm(a, b, ranges, **kw)
-    with pytest.raises(RuntimeError, match="is not in 0..25"):
-        ops.gemm(a, b, [ops.Range(0, 256, one, one)], **{**kw, "tile": 26})
+    with pytest.raises(RuntimeError, match="is not in 0.."):
+        ops.gemm(a, b, [ops.Range(0, 256, one, one)], **{**kw, "tile": ops.L.lib().segq_gemm_tile_count() + 1})
+
+
+# ---- one walk of K on the 8-wave tiles: a ragged end of K, DualScale's two ranges -----------------------------------------------
+@pytest.mark.parametrize("kind", ["int8", "e4m3"])
+@pytest.mark.parametrize("tile", [26, 27, 28])
+def test_ragged_end_of_k(ops, kind, tile):
+    g = np.random.default_rng(tile)
+    for K in (16, 112, 128, 144, 256, 272, 1168, 1280):  # one, two and several steps, ragged and whole
+        M, N = int(g.choice([1, 63, 130, 256, 300])), int(g.choice([16, 100, 129, 256, 390]))
+        _check(ops, kind, M, N, K, tile, [torch.float32, torch.bfloat16, torch.float16][int(g.integers(0, 3))], g)
+    for opt in (dict(row_sx=False, col_sw=False), dict(has_bias=False), dict(neg=True), dict(add=True), dict(pad=16), dict(k0=16), dict(k0=48, pad=32, add=True)):
+        _check(ops, kind, 70, 208, 400, tile, torch.bfloat16, g, **opt)
+
+
+@pytest.mark.parametrize("kind", ["int8", "e4m3"])
+def test_large_ragged_launch_takes_a_walk(ops, kind):
+    g = np.random.default_rng(5)
+    for M, N, K in ((1300, 1500, 784), (2000, 2300, 1040)):
+        _check(ops, kind, M, N, K, 0, torch.float32, g)
+
+
+def _check_dual(ops, kind, S, M, N, K, tile, dt, g, k0=0, pad=0, empty=None, per_row=True, per_col=True, add=False):
+    fa = FORMATS[kind][0]
+    a, b = _codes(g, (S * M, k0 + K), fa), _codes(g, (S * N, k0 + K), fa)
+    pick = g.random(a.shape) < 0.5
+    zero = np.zeros_like(a)
+    sides = [np.where(pick, a, zero), np.where(pick, zero, a)]
+    sx = [(g.random((S, M if per_row else 1)) * 30 + 10).astype(np.float32) for _ in range(2)]
+    if empty is not None:  # a side that holds nothing has the scale limit / 0
+        sides[empty][:M] = 0
+        sx[empty][0] = np.inf
+    sw = (g.random((S, N if per_col else 1)) * 30 + 10).astype(np.float32)
+    bias = g.standard_normal(N).astype(np.float32)
+    want, mag = np.zeros((S, M, N)), np.zeros((S, M, N))
+    for z in range(S):
+        bv = O.code_values(b[z * N:(z + 1) * N, k0:], fa).astype(np.float64)
+        for side, s in zip(sides, sx):
+            av = O.code_values(side[z * M:(z + 1) * M, k0:], fa).astype(np.float64)
+            with np.errstate(divide="ignore"):
+                den = s[z].astype(np.float64)[:, None] * sw[z].astype(np.float64)[None, :]
+            want[z] += av @ bv.T / den
+            mag[z] += np.abs(av) @ np.abs(bv).T / den
+    want, mag = want + bias, mag + np.abs(bias)
+    ad, nd, bd = _dev(sides[0], fa, pad), _dev(sides[1], fa, pad), _dev(b, fa, pad)
+    p, n, w = (torch.from_numpy(t.reshape(-1)).to(DEV) for t in (sx[0], sx[1], sw))
+    rg = [ops.Range(k0, K, p, w, 0, int(per_row), int(per_col)), ops.Range(k0, K, n, w, 1, int(per_row), int(per_col))]
+    addend = None
+    if add:
+        addend = torch.randn(M, N, device=DEV).to(dt)
+        want, mag = want + addend.double().cpu().numpy(), mag + addend.double().abs().cpu().numpy()
+    kw = dict(batch=S, batch_stride_a=M * (k0 + K + pad), batch_stride_b=N * (k0 + K + pad), batch_stride_sx=sx[0].shape[1],
+              batch_stride_sw=sw.shape[1]) if S > 1 else dict(addend=addend)
+    gd = ops.gemm_desc(ad, bd, rg, m=M, n=N, a_fmt=fa, b_fmt=fa, out_dtype=dt, lda=k0 + K + pad, ldb=k0 + K + pad, a_neg=nd, own_sums=1,
+                       bias=torch.from_numpy(bias).to(DEV), tile=tile, **kw)
+    took = ops.gemm_plan(gd)["tile"]
+    assert took == tile if tile else took in (29, 30)
+    got = ops.gemm_launch(gd).double().cpu().numpy().reshape(S, M, N)
+    # per range an exact int32 sum, its conversion, two quotients and two products, then the addition of the two and of the bias
+    tol = (1e-6 if kind == "int8" else 3e-4 if K > 32 else 16 * 2.0 ** -15) * mag + {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8}[dt] * np.abs(want)
+    assert np.isfinite(got).all() and (np.abs(got - want) <= tol).all(), (kind, S, M, N, K, tile, dt, float((np.abs(got - want) - tol).max()))
+
+
+@pytest.mark.parametrize("kind", ["int8", "e4m3"])
+@pytest.mark.parametrize("tile", [29, 30, 0])
+def test_dual_ranges_in_one_walk(ops, kind, tile):
+    g = np.random.default_rng(tile + 1)
+    for S, M, N, K in ((1, 1, 16, 272), (1, 64, 128, 640), (1, 129, 193, 1024 if tile else 1168), (2, 127, 200, 1040), (3, 65, 130, 528), (1, 300, 500, 640)):
+        _check_dual(ops, kind, S, M, N, K, tile, [torch.float32, torch.bfloat16][int(g.integers(0, 2))], g)
+    if tile:
+        for K in (16, 128, 144, 256):
+            _check_dual(ops, kind, 1, 70, 100, K, tile, torch.float32, g)
+    for opt in (dict(empty=0), dict(empty=1), dict(per_row=False, per_col=False), dict(pad=32), dict(k0=16, pad=16), dict(add=True)):
+        _check_dual(ops, kind, 1, 140, 210, 656, tile, torch.float32, g, **opt)
