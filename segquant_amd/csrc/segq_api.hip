@@ -46,6 +46,7 @@ int reserve_lds(const void* kern, int bytes, unsigned long long* done) {
 }
 
 int quantize_impl(const segq_quant_desc* d, hipStream_t st, const float* scale_by_value);
+int quantize_check(const segq_quant_desc* d);
 int quantize_many_impl(const segq_quant_desc* descs, int32_t n, hipStream_t st);
 int fake_e4m3_impl(const void* x, void* out, int32_t dtype, int64_t numel, hipStream_t st);
 int quantize_groups_impl(const void* w, int32_t w_dtype, int64_t n, int64_t k, void* codes, int32_t fmt, const float* scales,
@@ -268,7 +269,9 @@ struct GemmPlan {
 
 // plan != nullptr: nothing is launched; *plan says what the launch would do if the caller lent
 // as much workspace as the library can make use of (probe) or with d's own workspace (!probe).
-static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = nullptr, bool probe = true) {
+// q: a quantise step that the launch may do by itself; *fused says whether it did.  If it does not, nothing is launched.
+static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = nullptr, bool probe = true, const segq_quant_desc* q = nullptr,
+                     bool* fused = nullptr) {
     const bool need = plan != nullptr && probe;
     if (plan) *plan = GemmPlan{0, 0, 1, 0};
     if (!d) return fail(SEGQ_ERR_ARG, "segq_gemm: null descriptor");
@@ -387,6 +390,10 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         // (raw accumulators are for checks of the integers and keep the route, and the workspace, that they had)
         return ok && d->out_dtype != SEGQ_ACC ? choose_few(d->m, d->n, d->batch, r.k_len, f8 ? GEMM_F8 : GEMM_I8, w4, groups, walk.us) : -1;
     }();
+    if (q) {
+        *fused = few >= FIRST_FEW_CFG && TILE_CFGS[few].bm == 16 && d->m <= 16 && d->ranges[0].k_len <= 128 * 8 * (TILE_CFGS[few].bn == 32 ? 4 : 3);
+        if (!*fused) return SEGQ_OK;
+    }
     if (few == -2)
         return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: tiles %d to %d serve one range without a sign selection, a low-rank branch, codes out or split_k "
                                           "(and group factors of int4 weights)", FIRST_FEW_CFG + 1, FIRST_KT_CFG);
@@ -467,7 +474,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
             if (groups) plan->bytes = d->n * ((kmax + 31) & ~(int64_t)31);  // asked for above, whatever the tile
             p.dry = 1;
         }
-        return launch_gemm_few(p, f8 ? GEMM_F8 : GEMM_I8, w4, few, d->batch, st);
+        return launch_gemm_few(p, f8 ? GEMM_F8 : GEMM_I8, w4, few, d->batch, st, q);
     }
     if (walk.cfg >= 0) {
         const TileCfg& c = TILE_CFGS[walk.cfg];
@@ -730,6 +737,16 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     return launch_gemm_w4(p, cfg, fold, d->batch, st);
 }
 
+// Whether the GEMM may do the quantise step of a linear by itself: up to 16 rows with one scale or one per row, no producer
+// fused in front, and, dynamic, the scales it divides by are the ones it makes.
+static bool one_launch(const segq_quant_desc* q, const segq_gemm_desc* g) {
+    const segq_krange& r = g->ranges[0];
+    return q->rows > 0 && q->rows <= 16 && g->n_ranges == 1 && g->batch == 1 && r.a_sel == 0 && r.k_begin == 0 && r.k_len == q->cols && !q->dual && q->n_kseg == 1 &&
+           q->pre_op == SEGQ_PRE_NONE && !q->gate && !q->col_div && (q->seg_rows <= 0 || q->seg_rows >= q->rows) && (q->row_stride | 1) == 1 &&
+           (q->code_fmt == SEGQ_CODE_I8 || q->code_fmt == SEGQ_CODE_E4M3) && g->tile == 0 && g->out_dtype != SEGQ_ACC && q->ldx < (int64_t)1 << 24 &&
+           (!q->dynamic || (r.sx == q->scale && (q->rows == 1 || (q->row_stride == 1 && r.sx_row_stride == 1))));
+}
+
 // ---- the library's own scratch memory, for segq_gemm_noalloc -------------------------------
 // One array per GPU the library runs on, held until the process ends.  In host code the name
 // `scratch` is only a handle for hipGetSymbolAddress: the device address it resolves to (one per
@@ -900,6 +917,13 @@ int segq_linear(const segq_quant_desc* q, const segq_gemm_desc* g, segq_stream_t
             if (!in_pos && !in_neg)
                 return fail(SEGQ_ERR_ARG, "segq_linear: range %d divides by scales the dynamic quantise step does not write", i);
         }
+    }
+    if (one_launch(q, g)) {
+        const int rc = quantize_check(q);
+        if (rc != SEGQ_OK) return rc;
+        bool fused = false;
+        const int rc2 = gemm_impl(g, static_cast<hipStream_t>(stream), nullptr, true, q, &fused);
+        if (rc2 != SEGQ_OK || fused) return rc2;
     }
     const int rc = quantize_impl(q, static_cast<hipStream_t>(stream), nullptr);
     if (rc != SEGQ_OK) return rc;

@@ -18,6 +18,7 @@
 // traffic, so that no load hangs on a branch and each unit is waited for alone.
 #pragma once
 #include "segq_gemm_kernel.h"
+#include "segq_encode.h"
 
 namespace segq {
 
@@ -43,6 +44,12 @@ struct FewParams {
     int32_t tiles_m, tiles_n;
     int32_t out_dtype, bias_dtype;
     int32_t vec_store, vec_add;
+    // the quantise step in front of up to 16 rows (QE instances; A is not read): x, its codes and, dynamic, its scales
+    const void* X;
+    float* q_scale;
+    uint8_t* codes;
+    int64_t ldx, ld_codes;
+    int32_t x_dtype, q_rs, dynamic, pad_;
 };
 
 // Registers of a unit of operands, and units of K in flight per wave: of a short K all of them (at most four, and no more
@@ -64,8 +71,13 @@ template <int TM, int TN, bool B4> constexpr int few_patch() {
 }
 
 // ITER: units per wave of a short K, all asked for at once (no loop, and registers for no more than these); 0: any number.
-template <int TM, int TN, int FMT, bool B4, bool GRP, int ITER>
-__global__ void __launch_bounds__(FEW_WAVES * 64, few_two(TM, TN, B4, GRP, ITER) ? 4 : 2) gemm_few_kernel(const FewParams p) {
+// QE: the linear's quantise step runs here as well (2, 4: bytes of an element of x): a wave loads the floats of its units and
+// encodes each on its way to the patch, so that the linear is one launch and the codes need no trip through memory.  Every
+// workgroup encodes all of its 16 rows, which is why it serves no more; the first column of tiles also leaves the codes
+// and the dynamic scales where the quantise launch would have.  2 x 1536 -> 9216 fp16: both launches 9.4 us
+// and the gap between them, this 7.6; dynamic 8 x 3072 -> 6144 10.0 and 8.4; 16 x 3072 -> 18432 20.0 and 20.3.
+template <int TM, int TN, int FMT, bool B4, bool GRP, int ITER, int QE = 0>
+__global__ void __launch_bounds__(FEW_WAVES * 64, QE == 0 && few_two(TM, TN, B4, GRP, ITER) ? 4 : 2) gemm_few_kernel(const FewParams p) {
     constexpr int NW = FEW_WAVES, BM = TM * 16, BN = TN * 16, NB = TM * TN;
     constexpr bool F8 = FMT == GEMM_F8;
     constexpr int UNIT = 128;               // K of one unit
@@ -74,6 +86,8 @@ __global__ void __launch_bounds__(FEW_WAVES * 64, few_two(TM, TN, B4, GRP, ITER)
     constexpr int PATCH = few_patch<TM, TN, B4>();
     constexpr int OWN = (NB + NW - 1) / NW;  // 16 x 16 blocks a wave finishes
     static_assert(!B4 || !F8, "int4 weights pair with int8 activations");
+    static_assert(QE == 0 || (TM == 1 && ITER > 0), "quantising: 16 rows, all of K in registers");
+    constexpr int XL = QE == 0 ? 1 : QE;  // 16-byte loads for 16 elements
     typedef typename AccT<FMT>::type acc_t;
     typedef typename std::conditional<GRP, v4f, acc_t>::type sum_t;
 
@@ -99,7 +113,7 @@ __global__ void __launch_bounds__(FEW_WAVES * 64, few_two(TM, TN, B4, GRP, ITER)
     // Resources that start at the tile's first row and end with its last row's last code (the host has checked
     // that a tile's rows span less than 2^31 bytes).
     constexpr uint32_t NOWHERE = 0x80000000u;  // past the end of any of them
-    const uint8_t* const Ab = p.A + z * p.bsA + (int64_t)m0 * p.lda;
+    const uint8_t* const Ab = QE ? nullptr : p.A + z * p.bsA + (int64_t)m0 * p.lda;
     const uint8_t* const Bb = p.B + z * p.bsB + (int64_t)n0 * p.ldb;
     const int rows_a = min(BM, p.M - m0), rows_b = min(BN, p.N - n0);
     const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc(
@@ -117,15 +131,30 @@ __global__ void __launch_bounds__(FEW_WAVES * 64, few_two(TM, TN, B4, GRP, ITER)
 #pragma unroll
     for (int i = 0; i < TN * LB; ++i) b_off[i] = (uint32_t)min(i * (16 / LB) + b_row, rows_b - 1) * (uint32_t)p.ldb + b_pc * 16;
 
+    // QE: 16 elements of a row per lane instead of their 16 codes; rows past M read as zeros
+    const __amdgpu_buffer_rsrc_t rsx = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<void*>(p.X), 0, QE ? (int)(((rows_a - 1) * (uint32_t)p.ldx + (uint32_t)k1) * QE) : 0, 0x00020000);
+    uint32_t x_off[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) x_off[i] = i * 8 + a_row < rows_a ? ((uint32_t)(i * 8 + a_row) * (uint32_t)p.ldx + a_pc * 16) * QE : NOWHERE;
+
     // Unit u in registers.
     const int units = (k1 - k0 + UNIT - 1) / UNIT;
-    v4u qa[DEPTH][TM * LA], qb[DEPTH][TN * LB];
+    v4u qx[QE ? DEPTH : 1][2][XL];
+    v4u qa[QE ? 1 : DEPTH][TM * LA], qb[DEPTH][TN * LB];
     v4f qg[GRP ? DEPTH : 1][GRP ? TN : 1];
-    auto load_unit = [&](int u, v4u (&a)[TM * LA], v4u (&b)[TN * LB], v4f (&g)[GRP ? TN : 1]) __attribute__((always_inline)) {
+    auto load_unit = [&](int u, v4u (&a)[TM * LA], v4u (&b)[TN * LB], v4f (&g)[GRP ? TN : 1], v4u (&x)[2][XL]) __attribute__((always_inline)) {
         const int k = min(k0 + min(u, units) * UNIT, k1);  // (uniform: the scalar offset of the loads)
         const bool a_in = k + a_pc * 16 < k1, b_in = k + b_pc * (B4 ? 32 : 16) < k1;
 #pragma unroll
-        for (int i = 0; i < TM * LA; ++i) a[i] = __builtin_amdgcn_raw_buffer_load_b128(rsa, a_in ? a_off[i] : NOWHERE, k, 0);
+        for (int i = 0; i < TM * LA; ++i) {
+            if constexpr (QE) {
+#pragma unroll
+                for (int j = 0; j < XL; ++j) x[i][j] = __builtin_amdgcn_raw_buffer_load_b128(rsx, a_in && x_off[i] != NOWHERE ? x_off[i] + j * 16 : NOWHERE, k * QE, 0);
+            } else {
+                a[i] = __builtin_amdgcn_raw_buffer_load_b128(rsa, a_in ? a_off[i] : NOWHERE, k, 0);
+            }
+        }
 #pragma unroll
         for (int i = 0; i < TN * LB; ++i) b[i] = __builtin_amdgcn_raw_buffer_load_b128(rsb, b_in ? b_off[i] : NOWHERE, B4 ? k >> 1 : k, 0);
         if constexpr (GRP) {  // four factors at a time (the host has checked that columns and rows come in fours)
@@ -156,6 +185,7 @@ __global__ void __launch_bounds__(FEW_WAVES * 64, few_two(TM, TN, B4, GRP, ITER)
 #pragma unroll
         for (int i = 0; i < TM * LA; ++i)  // (rows 8 apart: the swizzle's top bit flips)
             *reinterpret_cast<v4u*>(patch + i * 1024 + ((i & 1) ? a_st ^ 64 : a_st)) = qa_[i];
+        __builtin_amdgcn_wave_barrier();  // what a lane reads, others have written: no reordering across here
         v4i a0[TM], a1[TM];
 #pragma unroll
         for (int s = 0; s < TM; ++s) {
@@ -167,6 +197,7 @@ __global__ void __launch_bounds__(FEW_WAVES * 64, few_two(TM, TN, B4, GRP, ITER)
             // (one block of weights after the other through the same place: a smaller patch, and a second workgroup on the CU)
 #pragma unroll
             for (int i = 0; i < LB; ++i) *reinterpret_cast<v4u*>(pb + i * 1024 + ((!B4 && i == 1) ? b_st ^ 64 : b_st)) = qb_[t * LB + i];
+            __builtin_amdgcn_wave_barrier();
             v4i b0, b1;
             if constexpr (B4) {
                 const v4u w4 = *reinterpret_cast<const v4u*>(pb + f4);
@@ -203,7 +234,7 @@ __global__ void __launch_bounds__(FEW_WAVES * 64, few_two(TM, TN, B4, GRP, ITER)
 
     // ---- this wave's units: wave, wave + NW, ...
 #pragma unroll
-    for (int d = 0; d < DEPTH; ++d) load_unit(wave + d * NW, qa[d], qb[d], qg[GRP ? d : 0]);
+    for (int d = 0; d < DEPTH; ++d) load_unit(wave + d * NW, qa[QE ? 0 : d], qb[d], qg[GRP ? d : 0], qx[QE ? d : 0]);
 
     // What this wave finishes: block i of the tile is column block i / TM, row block i % TM.  Its scales and
     // bias are asked for behind the first operands, so that the end of the launch waits for no memory; loads that
@@ -229,7 +260,91 @@ __global__ void __launch_bounds__(FEW_WAVES * 64, few_two(TM, TN, B4, GRP, ITER)
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (ITER > 0) {
+    [[maybe_unused]] float own_scale = 0.0f;  // dynamic: of row lrow
+    if constexpr (QE != 0) {
+        auto floats = [&](const v4u (&x)[XL], float (&v)[16]) __attribute__((always_inline)) {
+            if constexpr (QE == 4) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[i] = __uint_as_float(x[i / 4][i % 4]);
+            } else if (p.x_dtype == SEGQ_BF16) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[i] = __uint_as_float((i & 1) ? x[i / 8][i / 2 % 4] & 0xffff0000u : x[i / 8][i / 2 % 4] << 16);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[i] = f16_bits_to_f32((i & 1) ? x[i / 8][i / 2 % 4] >> 16 : x[i / 8][i / 2 % 4] & 0xffffu);
+            }
+        };
+        const int halves = rows_a > 8 ? 2 : 1;  // of the 16 rows; what is not there is zeros already
+        float s[2];
+        if (p.dynamic) {
+            // the quantise kernels' maximum and scale: non-negative floats are ordered like their bits, and a NaN wins
+            uint32_t amax[2] = {0, 0};
+#pragma unroll
+            for (int d = 0; d < DEPTH; ++d)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    if (i >= halves) continue;
+                    float v[16];
+                    floats(qx[d][i], v);
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) amax[i] = max(amax[i], __float_as_uint(fabsf(v[j])));
+                }
+            uint32_t* const red = reinterpret_cast<uint32_t*>(smem);  // [NW][16]
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+#pragma unroll
+                for (int o = 4; o > 0; o >>= 1) amax[i] = max(amax[i], (uint32_t)__shfl_xor((int)amax[i], o, 64));
+                if (a_pc == 0) red[wave * 16 + i * 8 + a_row] = amax[i];
+            }
+            __syncthreads();
+            auto scale_of = [&](int row) {
+                uint32_t t = 0;
+#pragma unroll
+                for (int w = 0; w < NW; ++w) t = max(t, red[w * 16 + row]);
+                return (F8 ? 448.0f : 127.0f) / __uint_as_float(max(t, 0x33800000u));  // 2^-24
+            };
+            s[0] = scale_of(a_row);
+            s[1] = scale_of(8 + a_row);
+            own_scale = scale_of(lrow);
+            __syncthreads();  // (the patches lie over the maxima)
+            if (tile_n == 0 && wave == 0 && a_pc == 0) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    if (i * 8 + a_row < rows_a) p.q_scale[(int64_t)(i * 8 + a_row) * p.q_rs] = s[i];
+            }
+        } else {
+            s[0] = p.q_scale[(int64_t)min(a_row, rows_a - 1) * p.q_rs];
+            s[1] = p.q_scale[(int64_t)min(8 + a_row, rows_a - 1) * p.q_rs];
+        }
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            // (unpacked again: kept from the maximum on, the floats would take twice the registers)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < XL; ++j) asm volatile("" : "+v"(qx[d][i][j]));
+            v4u c[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                if (i >= halves) continue;
+                float v[16];
+                floats(qx[d][i], v);
+#pragma unroll
+                for (int j = 0; j < 16; ++j) v[j] *= s[i];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    c[i][j] = F8 ? pack4_e4m3(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]) : pack4_i8(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
+            }
+            const int k = k0 + (wave + d * NW) * UNIT + a_pc * 16;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                if (k >= k1 || i * 8 + a_row >= rows_a) c[i] = v4u{0, 0, 0, 0};  // (0 times an infinite scale is a NaN)
+                else if (tile_n == 0) *reinterpret_cast<v4u*>(p.codes + (int64_t)(i * 8 + a_row) * p.ld_codes + k) = c[i];
+            }
+            if (!GRP || wave + d * NW < units) multiply(c, qb[d], qg[GRP ? d : 0]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    } else if constexpr (ITER > 0) {
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
             if (!GRP || wave + d * NW < units) multiply(qa[d], qb[d], qg[GRP ? d : 0]);
@@ -243,7 +358,7 @@ __global__ void __launch_bounds__(FEW_WAVES * 64, few_two(TM, TN, B4, GRP, ITER)
                 if (!GRP || u < units) multiply(qa[d], qb[d], qg[GRP ? d : 0]);  // (a group factor may be infinite)
                 if (--left <= 0) break;
                 __builtin_amdgcn_sched_barrier(0);
-                load_unit(u + DEPTH * NW, qa[d], qb[d], qg[GRP ? d : 0]);
+                load_unit(u + DEPTH * NW, qa[d], qb[d], qg[GRP ? d : 0], qx[0]);
                 __builtin_amdgcn_sched_barrier(0);
                 u += NW;
             }
@@ -283,7 +398,7 @@ __global__ void __launch_bounds__(FEW_WAVES * 64, few_two(TM, TN, B4, GRP, ITER)
             }
             continue;
         }
-        const float rx = 1.0f / __uint_as_float(sx_raw[i]);
+        const float rx = 1.0f / (QE && p.dynamic ? own_scale : __uint_as_float(sx_raw[i]));
         float o[4];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
@@ -316,9 +431,9 @@ __global__ void __launch_bounds__(FEW_WAVES * 64, few_two(TM, TN, B4, GRP, ITER)
     }
 }
 
-template <int TM, int TN, int FMT, bool B4, bool GRP, int ITER>
+template <int TM, int TN, int FMT, bool B4, bool GRP, int ITER, int QE = 0>
 int launch_few_instance(const FewParams& p, int64_t batch, hipStream_t st) {
-    auto kern = gemm_few_kernel<TM, TN, FMT, B4, GRP, ITER>;
+    auto kern = gemm_few_kernel<TM, TN, FMT, B4, GRP, ITER, QE>;
     constexpr int lds = FEW_WAVES * few_patch<TM, TN, B4>();
     static unsigned long long attr_done = 0;
     if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), lds, &attr_done)) return rc;
@@ -330,6 +445,18 @@ template <int TM, int TN, int FMT, bool B4, bool GRP>
 int launch_few_tile(const FewParams& p, int64_t batch, hipStream_t st) {
     constexpr int DEPTH = few_depth(TM, TN, B4, GRP);
     const int per_wave = ((p.k1 - p.k0 + 127) / 128 + FEW_WAVES - 1) / FEW_WAVES;
+    if constexpr (TM == 1) {
+        if (p.X) {  // (the host has checked: four units per wave at most)
+            const bool f32 = p.x_dtype == SEGQ_F32;
+#define SEGQ_QE(ITER_) return f32 ? launch_few_instance<TM, TN, FMT, B4, GRP, ITER_, 4>(p, batch, st) : launch_few_instance<TM, TN, FMT, B4, GRP, ITER_, 2>(p, batch, st)
+            if (per_wave == 1) SEGQ_QE(1);
+            if (per_wave == 2) SEGQ_QE(2);
+            if (per_wave == 3) SEGQ_QE(3);
+            if constexpr (TN == 2) SEGQ_QE(4);
+            return fail(SEGQ_ERR_UNSUPPORTED, "segq_linear: K too long for a quantise step in the GEMM");  // (not reached)
+#undef SEGQ_QE
+        }
+    }
     if (per_wave > DEPTH) return launch_few_instance<TM, TN, FMT, B4, GRP, 0>(p, batch, st);
     if (per_wave == 1) return launch_few_instance<TM, TN, FMT, B4, GRP, 1>(p, batch, st);
     if (per_wave == 2) return launch_few_instance<TM, TN, FMT, B4, GRP, 2>(p, batch, st);

@@ -55,12 +55,23 @@ int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4,
     return cost < other ? best : -1;
 }
 
-int launch_gemm_few(const GemmParams& g, int fmt, bool b4, int cfg, int64_t batch, hipStream_t st) {
+int launch_gemm_few(const GemmParams& g, int fmt, bool b4, int cfg, int64_t batch, hipStream_t st, const segq_quant_desc* q) {
     if (g.dry) return SEGQ_OK;
     const KRange& r = g.r[0];
-    const FewParams p = {r.a_sel == 1 ? g.A2 : g.A, g.B, g.C, r.sx, r.sw, g.bias, g.addend, g.grw,
+    FewParams p = {r.a_sel == 1 ? g.A2 : g.A, g.B, g.C, r.sx, r.sw, g.bias, g.addend, g.grw,
                          g.lda, g.ldb, g.ldc, g.ldadd, g.grw_gs, g.bsA, g.bsB, g.bsC, g.bsSx, g.bsSw,
-                         g.M, g.N, r.k0, r.k1, r.sx_rs, r.sw_cs, g.tiles_m, g.tiles_n, g.out_dtype, g.bias_dtype, g.vec_store, g.vec_add};
+                         g.M, g.N, r.k0, r.k1, r.sx_rs, r.sw_cs, g.tiles_m, g.tiles_n, g.out_dtype, g.bias_dtype, g.vec_store, g.vec_add,
+                   nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, 0};
+    if (q) {
+        p.X = q->x;
+        p.q_scale = q->scale;
+        p.codes = static_cast<uint8_t*>(q->codes);
+        p.ldx = q->ldx;
+        p.ld_codes = q->ld_codes;
+        p.x_dtype = q->x_dtype;
+        p.q_rs = (int32_t)q->row_stride;
+        p.dynamic = q->dynamic;
+    }
     const int f = cfg - FIRST_FEW_CFG;
     if (fmt == GEMM_F8) return launch_few_format<GEMM_F8, false, false>(p, f, batch, st);
     if (!b4) return launch_few_format<GEMM_I8, false, false>(p, f, batch, st);

@@ -718,6 +718,13 @@ static int launch_params(const QuantParams& p, hipStream_t st) {
     }
 }
 
+// The checks of a quantise launch without the launch.
+int quantize_check(const segq_quant_desc* d) {
+    QuantParams p;
+    bool empty;
+    return quant_params(d, nullptr, p, &empty);
+}
+
 int quantize_impl(const segq_quant_desc* d, hipStream_t st, const float* scale_by_value) {
     QuantParams p;
     bool empty;

@@ -201,3 +201,45 @@ def test_dual_ranges_in_one_walk(ops, kind, tile):
             _check_dual(ops, kind, 1, 70, 100, K, tile, torch.float32, g)
     for opt in (dict(empty=0), dict(empty=1), dict(per_row=False, per_col=False), dict(pad=32), dict(k0=16, pad=16), dict(add=True)):
         _check_dual(ops, kind, 1, 140, 210, 656, tile, torch.float32, g, **opt)
+
+
+# ---- a linear of up to 16 rows in one launch ---------------------------------------------------------------------------------
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind,group", [("int8", False), ("e4m3", False), ("int4", False), ("int4", True)])
+@pytest.mark.parametrize("dynamic", [False, True])
+def test_linear_in_one_launch(ops, kind, group, dynamic, dt):
+    """``segq_linear`` on 1 to 17 rows against its two launches apart: codes, scales and outputs bit for bit, rows that hold
+    zeros, NaN, infinities and the largest value, inputs that are column slices, K of one to four units per wave and beyond."""
+    fa, fb = FORMATS[kind]
+    g = np.random.default_rng(11)
+    for M, N, K in ((1, 64, 256), (16, 100, 1024), (5, 36, 1152), (9, 260, 2048), (16, 132, 3072), (3, 96, 4096), (2, 64, 4224), (17, 64, 512)):
+        K = K if group or kind == "int4" else K - 16
+        w = _dev(_codes(g, (N, K), fb), fb)
+        wide = torch.randn(M, K + 32, device=DEV)
+        wide[:, 7] *= 20
+        if dynamic and M > 4:
+            wide[0, 3] = float("nan")
+            wide[1, 5] = float("inf")
+            wide[2] = 0
+            wide[3, K - 1] = torch.finfo(dt).max
+        x = wide.to(dt)[:, 16:16 + K]
+        sw = torch.rand(N, device=DEV) + 0.5
+        gd = torch.rand(K // 128, N, device=DEV) if group else None
+        bias = torch.randn(N, device=DEV).to(dt)
+
+        def descs():
+            scale = torch.full((M,), 7.0, device=DEV) if dynamic else torch.rand(M, device=DEV, generator=torch.Generator(device=DEV).manual_seed(M)) * 20 + 1
+            q = ops.quantize_desc(x, fa, scale, row_stride=1, dynamic=dynamic)
+            d = ops.gemm_desc(q[1], w, [ops.Range(0, K, scale, sw, 0, 1, 1)], m=M, n=N, a_fmt=fa, b_fmt=fb, out_dtype=dt, lda=K,
+                              ldb=K // 2 if kind == "int4" else K, bias=bias, group_dequant=gd)
+            nb = ops.gemm_workspace_bytes(d)
+            return q, d, torch.empty(nb, dtype=torch.uint8, device=DEV) if nb else None, scale
+        q, d, ws, scale = descs()
+        out = ops.linear(q, d, ws)
+        q2, d2, ws2, scale2 = descs()
+        ops.quantize_launch(q2)
+        want = ops.gemm_launch(d2, ws2)
+        what = (kind, group, dynamic, dt, M, N, K)
+        assert torch.equal(q[1].view(torch.uint8), q2[1].view(torch.uint8)), what
+        assert torch.equal(scale.view(torch.int32), scale2.view(torch.int32)), what
+        assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.nan_to_num(), want.nan_to_num()), what
