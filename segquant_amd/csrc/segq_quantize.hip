@@ -280,14 +280,13 @@ __device__ __forceinline__ float wave_max(float v) {  // of non-negative values 
     return v;
 }
 
-// One workgroup per row, for rows longer than a wave can hold.  All loads of
-// the row are issued before anything is computed; up to CACHE runs per thread
-// stay in registers in packed form between the reduction and the encode, longer
-// rows are read again (they hit in L2).
-template <int DT, int FMT, bool DUAL, bool PRE>
-__global__ void __launch_bounds__(256) quant_dynamic_kernel(const QuantParams p) {
-    constexpr int CACHE = 4;
-    __shared__ float red[2][4];
+// One workgroup per row.  All loads of the row are issued before anything is computed; up to
+// CACHE runs per thread stay in registers in packed form between the reduction and the encode,
+// longer rows are read again (they hit in L2).  CACHE 1: a run per thread (up to eight waves).
+template <int DT, int FMT, int CACHE, bool DUAL, bool PRE>
+__global__ void __launch_bounds__(CACHE == 4 ? 256 : 512) quant_dynamic_kernel(const QuantParams p) {
+    __shared__ float red[2][8];
+    const int nt = blockDim.x, nw = nt >> 6;
     const int64_t row = blockIdx.x;
     const size_t esz = (DT == SEGQ_F32) ? 4 : 2;
     const uint8_t* xrow = static_cast<const uint8_t*>(p.x) + row * p.ldx * esz;
@@ -299,20 +298,20 @@ __global__ void __launch_bounds__(256) quant_dynamic_kernel(const QuantParams p)
         RawRun<DT> raw[CACHE];
 #pragma unroll
         for (int i = 0; i < CACHE; ++i) {
-            const int c = c0 + threadIdx.x + i * 256;
+            const int c = c0 + threadIdx.x + i * nt;
             if (c < c1) load_run<DT, PRE>(p, xrow, row, c, raw[i]);
         }
         float amax_p = 0.0f, amax_n = 0.0f;
 #pragma unroll
         for (int i = 0; i < CACHE; ++i) {
-            const int c = c0 + threadIdx.x + i * 256;
+            const int c = c0 + threadIdx.x + i * nt;
             if (c < c1) {
                 float v[16];
                 raw_to_f32<DT>(raw[i], v);
                 track_amax<DUAL>(v, amax_p, amax_n, dual);
             }
         }
-        for (int c = c0 + threadIdx.x + CACHE * 256; c < c1; c += 256) {
+        for (int c = c0 + threadIdx.x + CACHE * nt; c < c1; c += nt) {
             RawRun<DT> t;
             float v[16];
             load_run<DT, PRE>(p, xrow, row, c, t);
@@ -327,8 +326,10 @@ __global__ void __launch_bounds__(256) quant_dynamic_kernel(const QuantParams p)
             red[1][threadIdx.x >> 6] = amax_n;
         }
         __syncthreads();
-        amax_p = max_nn(max_nn(red[0][0], red[0][1]), max_nn(red[0][2], red[0][3]));
-        amax_n = max_nn(max_nn(red[1][0], red[1][1]), max_nn(red[1][2], red[1][3]));
+        for (int w = 0; w < nw; ++w) {  // (this thread's own maxima among them)
+            amax_p = max_nn(amax_p, red[0][w]);
+            amax_n = max_nn(amax_n, red[1][w]);
+        }
         float s_pos, s_neg;
         if (dual) {
             s_pos = qmax_pos<FMT>() / fmaxf(amax_p, eps);
@@ -343,14 +344,14 @@ __global__ void __launch_bounds__(256) quant_dynamic_kernel(const QuantParams p)
         }
 #pragma unroll
         for (int i = 0; i < CACHE; ++i) {
-            const int c = c0 + threadIdx.x + i * 256;
+            const int c = c0 + threadIdx.x + i * nt;
             if (c < c1) {
                 float v[16];
                 raw_to_f32<DT>(raw[i], v);
                 encode16<FMT>(p, row, (int64_t)c << 4, v, s_pos, s_neg, two);
             }
         }
-        for (int c = c0 + threadIdx.x + CACHE * 256; c < c1; c += 256) {
+        for (int c = c0 + threadIdx.x + CACHE * nt; c < c1; c += nt) {
             RawRun<DT> t;
             float v[16];
             load_run<DT, PRE>(p, xrow, row, c, t);
@@ -364,7 +365,7 @@ __global__ void __launch_bounds__(256) quant_dynamic_kernel(const QuantParams p)
 // For rows of up to 64 * CPL runs: the whole row is in flight at once, the
 // maximum is reduced with cross-lane shuffles only, and four rows share a
 // workgroup without ever synchronising.
-template <int DT, int FMT, int CPL, bool DUAL, bool PRE, bool KEEP = (CPL <= 4)>
+template <int DT, int FMT, int CPL, bool DUAL, bool PRE>
 __global__ void __launch_bounds__(256) quant_dynamic_wave_kernel(const QuantParams p) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -382,22 +383,14 @@ __global__ void __launch_bounds__(256) quant_dynamic_wave_kernel(const QuantPara
             const int c = c0 + lane + i * 64;
             if (c < c1) load_run<DT, PRE>(p, xrow, row, c, raw[i]);
         }
-        // short rows: unpack once and keep the floats (64 registers) instead of unpacking
-        // again for the encode; longer rows stay packed
-        float vf[KEEP ? CPL : 1][16];
         float amax_p = 0.0f, amax_n = 0.0f;
 #pragma unroll
         for (int i = 0; i < CPL; ++i) {
             const int c = c0 + lane + i * 64;
             if (c < c1) {
-                if constexpr (KEEP) {
-                    raw_to_f32<DT>(raw[i], vf[i]);
-                    track_amax<DUAL>(vf[i], amax_p, amax_n, dual);
-                } else {
-                    float v[16];
-                    raw_to_f32<DT>(raw[i], v);
-                    track_amax<DUAL>(v, amax_p, amax_n, dual);
-                }
+                float v[16];
+                raw_to_f32<DT>(raw[i], v);
+                track_amax<DUAL>(v, amax_p, amax_n, dual);
             }
         }
         amax_p = wave_max(amax_p);
@@ -418,13 +411,9 @@ __global__ void __launch_bounds__(256) quant_dynamic_wave_kernel(const QuantPara
         for (int i = 0; i < CPL; ++i) {
             const int c = c0 + lane + i * 64;
             if (c < c1) {
-                if constexpr (KEEP) {
-                    encode16<FMT>(p, row, (int64_t)c << 4, vf[i], s_pos, s_neg, two);
-                } else {
-                    float v[16];
-                    raw_to_f32<DT>(raw[i], v);
-                    encode16<FMT>(p, row, (int64_t)c << 4, v, s_pos, s_neg, two);
-                }
+                float v[16];
+                raw_to_f32<DT>(raw[i], v);
+                encode16<FMT>(p, row, (int64_t)c << 4, v, s_pos, s_neg, two);
             }
         }
     }
@@ -618,17 +607,23 @@ static int launch_quant(const QuantParams& p, hipStream_t st) {
                 return check_launch("segq_quantize");
             }
         }
-        if (longest <= 64 * 4) {
-            if (p.dual) hipLaunchKernelGGL((quant_dynamic_wave_kernel<DT, FMT, 4, true, PRE>), wgrid, dim3(256), 0, st, p);
-            else hipLaunchKernelGGL((quant_dynamic_wave_kernel<DT, FMT, 4, false, PRE>), wgrid, dim3(256), 0, st, p);
+        // A run per thread wherever that many waves of many rows fit the chip at a time: rows of up to 4096 elements, longer
+        // ones while there are at most three workgroups per CU.  One wave per row does its runs one after the other, with
+        // the activation function in front of each (bf16, x gelu(gate), us, wave per row / this: 400 x 5120 17.7 / 7.2, 1000 x
+        // 1280 9.0 / 6.7, 8192 x 2560 37.4 / 35.7; 8192 x 5120 61.7 / 94.8, where a workgroup's waves wait for each other
+        // with too few workgroups on the CU)
+        if (longest <= 64 * 4 || (longest <= 64 * 8 && p.rows <= 3 * (int64_t)device_cus())) {
+            const dim3 runs((unsigned)((longest + 63) / 64 * 64));
+            if (p.dual) hipLaunchKernelGGL((quant_dynamic_kernel<DT, FMT, 1, true, PRE>), bgrid, runs, 0, st, p);
+            else hipLaunchKernelGGL((quant_dynamic_kernel<DT, FMT, 1, false, PRE>), bgrid, runs, 0, st, p);
         } else if (longest <= 64 * 8 && longest % 256 != 0) {
             // rows a workgroup's 256 threads would share unevenly (320 runs: a quarter of the threads
             // with two, the rest with one) stay with one wave per row
             if (p.dual) hipLaunchKernelGGL((quant_dynamic_wave_kernel<DT, FMT, 8, true, PRE>), wgrid, dim3(256), 0, st, p);
             else hipLaunchKernelGGL((quant_dynamic_wave_kernel<DT, FMT, 8, false, PRE>), wgrid, dim3(256), 0, st, p);
         } else {
-            if (p.dual) hipLaunchKernelGGL((quant_dynamic_kernel<DT, FMT, true, PRE>), bgrid, dim3(256), 0, st, p);
-            else hipLaunchKernelGGL((quant_dynamic_kernel<DT, FMT, false, PRE>), bgrid, dim3(256), 0, st, p);
+            if (p.dual) hipLaunchKernelGGL((quant_dynamic_kernel<DT, FMT, 4, true, PRE>), bgrid, dim3(256), 0, st, p);
+            else hipLaunchKernelGGL((quant_dynamic_kernel<DT, FMT, 4, false, PRE>), bgrid, dim3(256), 0, st, p);
         }
     } else {
         const int64_t runs = p.rows * (p.cols >> 4);
