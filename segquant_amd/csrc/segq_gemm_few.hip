@@ -4,25 +4,43 @@
 namespace segq {
 
 // Tile for a launch of few tiles, or -1 where the other kernels serve it better.  Both sides are estimated in us from
-// launches with weights from memory; K in steps of 128.  The constants were fitted over 110 shapes of 1 to 5000 rows and 100 to
-// 18432 columns; the choice is within 12 % of the best tile on nine of ten of them.  `other_us`: what the 8-wave tiles for a
-// ragged K would take, where they serve the launch.
+// launches with weights from memory; K in steps of 128.  The constants of the 8-bit codes were fitted over 220 launches of 24
+// to 700 rows, 1152 to 9216 columns and K of 1152 to 12288: the choice is 2.5 % from the best on the mean of them and 8 % on
+// nine of ten (18 % and three times before they were fitted where one tile a CU is not enough: 200 x 1536 x 6144 44.6 ->
+// 14.2 us, 128 x 4096 x 4096 22.1 -> 13.3, 500 x 2048 x 2048 18 -> 10.7 in e4m3).  `other_us`: what the 8-wave tiles for a ragged K
+// would take, where they serve the launch.
 int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4, bool grp, double other_us) {
     const int64_t cus = device_cus(), steps = (k + 127) / 128;
     auto tiles = [&](int64_t bm, int64_t bn) { return (m + bm - 1) / bm * ((n + bn - 1) / bn) * batch; };
     if (tiles(32, 64) > 32 * cus) return -1;
-    // this kernel: 3.5 us of launch, first loads and the meeting of the shares (1.1 us for each workgroup a CU takes beyond
-    // its first), then the tile's operand bytes at what a CU takes in with two workgroups on it (52 KB per us) or one (38);
-    // int4 weights add their unpacking, group factors the sums
+    // this kernel on 8-bit weights: a launch, rounds of the CUs (half way from the exact share to whole rounds: two workgroups
+    // run on a CU, but not every CU has two), each with a start and the tile's operand bytes, and the weights from memory.  Three
+    // ways the units of a wave come in: two in flight in all, all three or four, a loop.
+    struct Fit { double start, round, per_kb, per_mb; };
+    static constexpr Fit FITS[4][3] = {
+        {{2.0, 2.0, 0.0068, 0.13}, {2.1, 2.1, 0.0070, 0.14}, {2.2, 2.2, 0.0124, 0.193}},    // 16 x 32
+        {{3.4, 2.05, 0.003, 0.144}, {2.1, 2.2, 0.0126, 0.213}, {3.7, 1.7, 0.0121, 0.258}},  // 16 x 64
+        {{3.05, 1.7, 0.0047, 0.12}, {3.3, 0.45, 0.015, 0.152}, {4.05, 1.45, 0.0153, 0.207}},  // 32 x 32
+        {{3.7, 2.35, 0.0042, 0.152}, {1.8, 4.95, 0.0066, 0.21}, {2.75, 1.8, 0.0153, 0.172}}};  // 32 x 64
+    // ... and on int4 weights: 3.5 us of launch, first loads and the meeting of the shares (1.1 us for each workgroup a CU takes
+    // beyond its first), then the tile's operand bytes at what a CU takes in with two workgroups on it or one, and the unpacking;
+    // group factors add the sums
     int best = -1;
     double cost = 0;
     for (int c = FIRST_FEW_CFG; c < FIRST_KT_CFG; ++c) {
         const int tm = TILE_CFGS[c].bm / 16, tn = TILE_CFGS[c].bn / 16;
         const int64_t t = tiles(TILE_CFGS[c].bm, TILE_CFGS[c].bn), per_wave = (steps + FEW_WAVES - 1) / FEW_WAVES;
-        const bool two = few_two(tm, tn, b4, grp, per_wave <= few_depth(tm, tn, b4, grp) ? (int)per_wave : 0);
-        const double bytes = (TILE_CFGS[c].bm + TILE_CFGS[c].bn * (b4 ? 0.5 : 1.0)) * 128.0 * steps;
-        const double rate = (two ? 52e3 : 38e3) * (b4 ? 0.75 : 1.0) * (grp ? 0.9 : 1.0);
-        const double us = t > cus ? 2.8 + (double)t / cus * (bytes / rate + 1.1) : 3.5 + 0.9 * bytes / rate;
+        const int units = per_wave <= few_depth(tm, tn, b4, grp) ? (int)per_wave : 0;
+        const double bytes = (TILE_CFGS[c].bm + TILE_CFGS[c].bn * (b4 ? 0.5 : 1.0)) * 128.0 * steps, share = (double)t / cus;
+        double us;
+        if (b4) {
+            const double rate = (few_two(tm, tn, b4, grp, units) ? 39e3 : 28.5e3) * (grp ? 0.9 : 1.0);
+            us = t > cus ? 2.8 + share * (bytes / rate + 1.1) : 3.5 + 0.9 * bytes / rate;
+        } else {
+            const Fit& f = FITS[c - FIRST_FEW_CFG][units == 0 ? 2 : units > 2 ? 1 : 0];
+            const double rounds = share > 1.0 ? 0.5 * (share + (double)((t + cus - 1) / cus)) : 1.0;
+            us = f.start + rounds * (f.round + f.per_kb * bytes * 1e-3) + f.per_mb * (double)n * k * batch * 1e-6;
+        }
         if (best < 0 || us < cost) {
             best = c;
             cost = us;
@@ -34,24 +52,26 @@ int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4,
         return cost < 7.0 + 0.85 * steps * (double)((t128 + 2 * cus - 1) / (2 * cus)) + (double)n * k / 8e6 ? best : -1;
     if (b4) return cost < 6.5 + 0.8 * steps * rounds ? best : -1;
     const double full = (double)tiles(64, 128) / (1.5 * cus);
-    double other = 6.5 + 0.75 * steps * (full > 1.0 ? full : 1.0);  // the general kernel, 64 x 128
-    if (other_us < other) other = other_us;
+    double other = 8.0 + 0.75 * steps * (full > 1.0 ? full : 1.0);  // the general kernel, 64 x 128
     if (k % 128 == 0) {
-        bool theirs = t128 >= 32;  // the 8-wave kernels ...
-        if (theirs) other = 4.5 + (fmt == GEMM_F8 ? 0.5 : 0.45) * steps * rounds;
-        auto shares = [&](int64_t t, double per_step) {  // ... also in K shares
-            const int64_t s = cus / t < steps / 8 ? cus / t : steps / 8;
-            if (batch > 1 || steps < 16 || t * 10 >= cus * 9 || s < 2) return;
-            const double us = 10.5 + per_step * steps / s + (double)n * k / 5.5e6;
-            if (us < other) other = us;
-            theirs = true;
-        };
-        if (m <= 128) shares(t128, 0.45);
-        else shares(tiles(256, 192), 0.9);
-        // They have tiles and shares of their own by size, asserted in the host tests, and keep what is not clearly
-        // ahead here (64 x 9216 x 3072 stays at 20.3 us in three shares: 13.9 here; 256 x 2176 x 1536 at 9.0: 8.3 here)
-        if (theirs) other *= 0.65;
+        // the 8-wave kernels: int8 that fits the CUs once has four or five stages of LDS, and 96 columns where they divide n
+        double area = (steps + 6.0) * 64 * 128 / 0.5, keep = 0.92;
+        if (t128 >= 32) {
+            const bool stages = fmt == GEMM_I8 && rounds == 1, narrow = stages && n % 96 == 0 && (m + 127) / 128 * (n / 96) * batch <= cus;
+            other = 6.0 + (stages ? 0.5 : fmt == GEMM_F8 ? 0.8 : 0.6) * steps * rounds;
+            area = (steps + 6.0) * 128 * (narrow ? 96 : 128) / 0.7 * rounds;
+            if (stages && steps <= 12) keep = 0.72;  // 256 x 2176 x 1536 is asserted to stay: 9.0 us, 8.3 here
+        }
+        // ... and in K shares, where their rule takes those (the sums of the shares pass through memory)
+        const int64_t t = m <= 128 ? t128 : tiles(256, 192), fit = cus / t < steps / 8 ? cus / t : steps / 8, s = fit < 16 ? fit : 16;
+        if (batch == 1 && steps >= 16 && s >= 2 && ((double)steps / s + 14.0) * (m <= 128 ? 128 * 128 / 0.7 : 256 * 192 / 0.95) < area) {
+            other = 13.0 + (m <= 128 ? 0.45 : 0.9) * steps / s + (double)n * k / 5.5e6 + (double)s * m * n / 0.75e6;
+            // asserted to stay in shares: 64 x 9216 x 3072 in three (22 us, 18 here), 512 x 1024 x 8192 in eight (27 and 18)
+            keep = s <= 3 || (m > 128 && steps >= 64) ? 0.65 : 0.92;
+        }
+        other *= keep;
     }
+    if (other_us < other) other = other_us;
     return cost < other ? best : -1;
 }
 

@@ -98,6 +98,18 @@ def test_forms_of_the_call(ops, kind, group):
         _check(ops, kind, 37, 104, 640, (22, 23, 24, 25, 0)[i % 5], (torch.bfloat16, torch.float32)[i & 1], g, group=group, **opt)
 
 
+@pytest.mark.parametrize("kind", ["int8", "e4m3"])
+@pytest.mark.parametrize("M,N,K", [(200, 1536, 6144), (333, 1152, 4608), (500, 2048, 2048), (129, 4092, 4096), (280, 2432, 2432)])
+def test_several_hundred_rows(ops, kind, M, N, K):
+    """More tiles than CUs, by the library's own choice: one unit of K in a wave's loop and several, ragged rows and columns."""
+    g = np.random.default_rng(M)
+    one = torch.ones(1, device=DEV)
+    d = ops.gemm_desc(torch.empty(M, K, dtype=torch.uint8, device=DEV), torch.empty(N, K, dtype=torch.uint8, device=DEV), [ops.Range(0, K, one, one)],
+                      m=M, n=N, a_fmt=FORMATS[kind][0], b_fmt=FORMATS[kind][1], out_dtype=torch.float32, lda=K, ldb=K)
+    assert ops.gemm_plan(d)["tile"] in (22, 23, 24, 25)
+    _check(ops, kind, M, N, K, 0, torch.float32, g)
+
+
 @pytest.mark.parametrize("kind", ["int8", "e4m3", "int4"])
 def test_raw_accumulators_and_batches(ops, kind):
     fa, fb = FORMATS[kind]
