@@ -68,7 +68,7 @@ int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4,
         if (batch == 1 && steps >= 16 && s >= 2 && ((double)steps / s + 14.0) * (m <= 128 ? 128 * 128 / 0.7 : 256 * 192 / 0.95) < area) {
             other = 13.0 + (m <= 128 ? 0.45 : 0.9) * steps / s + (double)n * k / 5.5e6 + (double)s * m * n / 0.75e6;
             // asserted to stay in shares: 64 x 9216 x 3072 in three (22 us, 18 here), 512 x 1024 x 8192 in eight (27 and 18)
-            keep = s <= 3 || (m > 128 && steps >= 64) ? 0.65 : 0.92;
+            keep = s <= 3 || (m > 256 && steps >= 64) ? 0.65 : 0.92;
         }
         other *= keep;
     }
