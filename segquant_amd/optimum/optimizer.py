@@ -585,7 +585,7 @@ class DefaultOptimizer(BaseOptimizer):
         dev = x.device
         stream = ops._stream(dev)
         reuse = bufs.get(stream)
-        if reuse is None or (hit["need"] and not reuse[1].workspace):
+        if reuse is None:
             return None
         out = torch.empty((*shape[:-1], hit["N"]), dtype=dtype, device=dev)
         qd, gd = reuse[0], reuse[1]
@@ -625,6 +625,8 @@ class DefaultOptimizer(BaseOptimizer):
         qd.ldx = ops.row_stride(x2)
         qd.codes = gd.a = codes.data_ptr()
         gd.out = out.data_ptr()
+        if ws is not None:  # (the copied descriptor names the workspace of the stream that the first call ran on)
+            gd.workspace, gd.workspace_bytes = ws.data_ptr(), ws.numel()
         held = [codes, hit["static"]]
         result = codes
         if hit["dual"]:
