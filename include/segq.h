@@ -385,7 +385,8 @@ int segq_device_info(int32_t* compute_units, int32_t* max_engine_clock_khz);
  * workspace that g reads as its a (and a_neg).  Replaces the body of
  * real_quantized_gemm_scaled / real_quantized_gemm_dual_scaled
  * (segquant/src/real_quant/real_gemm.cu:643-894) without their temporaries,
- * host synchronisation or per-call device allocation. */
+ * host synchronisation or per-call device allocation.  One launch for up to 16 rows where that is
+ * the faster way, two otherwise; the output may lie over q's x, which then takes the two. */
 int segq_linear(const segq_quant_desc* q, const segq_gemm_desc* g, segq_stream_t stream);
 
 /* out[i] = float(e4m3(x[i])) in the dtype of x.  Replaces fake_e4m3fy

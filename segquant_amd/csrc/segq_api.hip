@@ -737,10 +737,20 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     return launch_gemm_w4(p, cfg, fold, d->batch, st);
 }
 
+static bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+    const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+    return pa < pb + (uintptr_t)b_bytes && pb < pa + (uintptr_t)a_bytes;
+}
+
 // Whether the GEMM may do the quantise step of a linear by itself: up to 16 rows with one scale or one per row, no producer
-// fused in front, and, dynamic, the scales it divides by are the ones it makes.
+// fused in front, and, dynamic, the scales it divides by are the ones it makes.  Every workgroup of that launch reads all of x
+// while others store already, so nothing it writes may lie over x; the two launches have read all of x before the first store.
 static bool one_launch(const segq_quant_desc* q, const segq_gemm_desc* g) {
     const segq_krange& r = g->ranges[0];
+    const int64_t xsz = q->x_dtype == SEGQ_F32 ? 4 : 2, osz = g->out_dtype == SEGQ_F32 ? 4 : 2;
+    const int64_t x_bytes = ((q->rows - 1) * q->ldx + q->cols) * xsz;
+    if (overlap(q->x, x_bytes, g->out, ((g->m - 1) * g->ldo + g->n) * osz) || overlap(q->x, x_bytes, q->codes, (q->rows - 1) * q->ld_codes + q->cols))
+        return false;
     return q->rows > 0 && q->rows <= 16 && g->n_ranges == 1 && g->batch == 1 && r.a_sel == 0 && r.k_begin == 0 && r.k_len == q->cols && !q->dual && q->n_kseg == 1 &&
            q->pre_op == SEGQ_PRE_NONE && !q->gate && !q->col_div && (q->seg_rows <= 0 || q->seg_rows >= q->rows) && (q->row_stride | 1) == 1 &&
            (q->code_fmt == SEGQ_CODE_I8 || q->code_fmt == SEGQ_CODE_E4M3) && g->tile == 0 && g->out_dtype != SEGQ_ACC && q->ldx < (int64_t)1 << 24 &&

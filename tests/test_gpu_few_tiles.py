@@ -255,3 +255,30 @@ def test_linear_in_one_launch(ops, kind, group, dynamic, dt):
         assert torch.equal(q[1].view(torch.uint8), q2[1].view(torch.uint8)), what
         assert torch.equal(scale.view(torch.int32), scale2.view(torch.int32)), what
         assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.nan_to_num(), want.nan_to_num()), what
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dynamic", [False, True])
+def test_linear_over_its_own_input(ops, dynamic, dt):
+    """A square linear whose output takes the place of its input, whole and shifted by some rows: the codes are those of the
+    input, and the result is that of the call with an output of its own, however the workgroups follow each other."""
+    g = np.random.default_rng(12)
+    K = 2048
+    w = _dev(_codes(g, (K, K), O.FMT_INT8), O.FMT_INT8)
+    one = torch.ones(1, device=DEV)
+    for M in (1, 16):
+        for shift in (0, 1, M - 1, M):
+            x = torch.randn(M, K, device=DEV).to(dt)
+
+            def run(buf, out):
+                buf[:M] = x
+                scale = torch.full((M,), 20.0, device=DEV)
+                q = ops.quantize_desc(buf[:M], O.FMT_INT8, scale, row_stride=1, dynamic=dynamic)
+                d = ops.gemm_desc(q[1], w, [ops.Range(0, K, scale, one, 0, 1, 0)], m=M, n=K, a_fmt=O.FMT_INT8, b_fmt=O.FMT_INT8, out_dtype=dt,
+                                  lda=K, ldb=K, out=out)
+                return ops.linear(q, d), q[1], scale
+            buf = torch.empty(2 * M, K, device=DEV, dtype=dt)
+            want, codes, scale = run(buf, torch.empty(M, K, device=DEV, dtype=dt))
+            for _ in range(10):
+                got, c2, s2 = run(buf, buf[shift:shift + M])
+                assert torch.equal(c2, codes) and torch.equal(s2, scale) and torch.equal(got, want), (dynamic, dt, M, shift)
