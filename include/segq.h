@@ -217,9 +217,7 @@ typedef struct segq_krange {
                              * scales, which has to be finite (scales that a calibrator clamps).  Non-zero: every
                              * range is summed on its own and scaled by its own factors, as int8 ranges always
                              * are, so that a scale may be infinite: limit / 0 of a DualScale side that holds
-                             * nothing, which adds nothing.  Not combined with a low-rank branch.
-                             * 2: the scales are finite and the library takes the faster way (two ranges over the
-                             * same run of K, a and then a_neg, can be multiplied in one walk of it). */
+                             * nothing, which adds nothing.  Not combined with a low-rank branch. */
     const float* sx;        /* device */
     const float* sw;        /* device */
 } segq_krange;
@@ -320,7 +318,9 @@ typedef struct segq_gemm_desc {
     const float* out_scale; /* device: one float */
     const float* out_scale_neg; /* device or NULL */
     int32_t out_code_fmt;   /* SEGQ_CODE_I8 | SEGQ_CODE_E4M3 */
-    int32_t reserved2;
+    int32_t finite_scales;  /* 0, or non-zero: the scales of all ranges are finite, and without own_sum the library
+                         * takes the faster way to sum them (two ranges over the same run of K, a and then a_neg,
+                         * can be multiplied in one walk of it, each with its own sums) */
     segq_krange ranges[SEGQ_MAX_RANGES];
 } segq_gemm_desc;
 

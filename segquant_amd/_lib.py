@@ -60,7 +60,7 @@ class GemmDesc(C.Structure):
         ("lowrank_t", C.c_void_p), ("ld_lowrank_t", C.c_int64), ("lowrank_l2t", C.c_void_p), ("ld_lowrank_l2t", C.c_int64),
         ("lowrank_rank", C.c_int32), ("out_pre_op", C.c_int32),
         ("out_codes", C.c_void_p), ("out_codes_neg", C.c_void_p), ("ld_out_codes", C.c_int64),
-        ("out_scale", C.c_void_p), ("out_scale_neg", C.c_void_p), ("out_code_fmt", C.c_int32), ("reserved2", C.c_int32),
+        ("out_scale", C.c_void_p), ("out_scale_neg", C.c_void_p), ("out_code_fmt", C.c_int32), ("finite_scales", C.c_int32),
         ("ranges", KRange * SEGQ_MAX_RANGES),
     ]
 

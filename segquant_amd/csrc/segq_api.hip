@@ -368,11 +368,11 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
             walk.cfg = (int)d->tile - 1;
         } else if (d->tile == 0 && d->out_dtype != SEGQ_ACC) {
             if (one && r.k_len % 128) walk = choose_ragged(d->m, d->n, d->batch, r.k_len);
-            if (two && r.own_sum && r.k_len > (r.k_len % 128 ? 256 : 512)) {
+            if (two && (r.own_sum || d->finite_scales) && r.k_len > (r.k_len % 128 ? 256 : 512)) {
                 walk = choose_dual(d->m, d->n, d->batch, r.k_len);
                 const bool lent = d->split_k != 1 && ws && al(ws, 16), in_turn = r.k_len % 128 == 0 && d->batch == 1;
                 const int64_t steps = r.k_len / 64;  // of both ranges in turn
-                if (in_turn && r.own_sum == 2) {  // (0.85: the estimates)
+                if (in_turn && !r.own_sum) {  // (0.85: the estimates)
                     if (0.85 * in_turn_us(d->m, d->n, steps, f8, lent) < walk.us) walk.cfg = -1;
                 } else if (in_turn && lent && k_shares(d->m, d->n, steps, FIRST_WIDE_CFG + 6) > 2) {
                     walk.cfg = -1;  // a workspace lent to ranges summed on their own is lent for K shares
@@ -498,7 +498,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     // several ranges cost a second (fp32) accumulator set, and with it the biggest tiles,
     // unless the accumulators are fp32 already (plain e4m3: rescaled in place, which takes the ratio of two
     // ranges' scales and is not for callers whose scales may be infinite: own_sum)
-    p.sep = f8 && fold && plain8 && d->ranges[0].own_sum != 0 && d->ranges[0].own_sum != 2;
+    p.sep = f8 && fold && plain8 && d->ranges[0].own_sum != 0;
     const bool fold2 = fold && !(f8 && plain8 && !p.sep);
     if (groups) {
         bool ok = wide_ok && plain8;

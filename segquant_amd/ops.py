@@ -351,7 +351,8 @@ def gemm_desc(a: torch.Tensor, b: torch.Tensor, ranges: Sequence[Range], *, m: i
          batch_stride_sx: int = 0, batch_stride_sw: int = 0, out: Optional[torch.Tensor] = None,
          tile: int = 0, workspace: Optional[torch.Tensor] = None,
          group_dequant: Optional[torch.Tensor] = None, split_k: int = 0,
-         addend: Optional[torch.Tensor] = None, lowrank=None, out_codes: Optional[dict] = None, own_sums: int = 0):
+         addend: Optional[torch.Tensor] = None, lowrank=None, out_codes: Optional[dict] = None, own_sums: bool = False,
+         finite_scales: bool = False):
     """The ``segq_gemm_desc`` of a segmented GEMM with fused de-quantisation and bias, its output
     tensor, the launch's description and the tensors the descriptor points into.
 
@@ -368,8 +369,9 @@ def gemm_desc(a: torch.Tensor, b: torch.Tensor, ranges: Sequence[Range], *, m: i
     ``out_dtype`` is a torch float dtype, or the string ``"acc"`` for the raw
     accumulators (int32 for integer codes, float32 for e4m3).  ``workspace``: a
     byte tensor the library may expand int4 weights into, or park the sums of
-    finished int8 ranges in (see ``int4_workspace``, ``park_bytes``).  ``own_sums``: 1 sums every
-    e4m3 range on its own, for scales that may be infinite; 2 leaves the way to the library (``segq_krange.own_sum``).
+    finished int8 ranges in (see ``int4_workspace``, ``park_bytes``).  ``own_sums`` sums every
+    e4m3 range on its own, for scales that may be infinite; ``finite_scales``, of scales that are not, leaves the way to
+    the library (``segq_krange.own_sum``, ``segq_gemm_desc.finite_scales``).
     """
     _need_cuda(a, b, a_neg, bias)
     raw = out_dtype == "acc"
@@ -454,7 +456,8 @@ def gemm_desc(a: torch.Tensor, b: torch.Tensor, ranges: Sequence[Range], *, m: i
                 raise RuntimeError("scales must be float32")
         kr.sx = r.sx.data_ptr() if r.sx is not None else None
         kr.sw = r.sw.data_ptr() if r.sw is not None else None
-    d.ranges[0].own_sum = own_sums
+    d.ranges[0].own_sum = 1 if own_sums else 0
+    d.finite_scales = 1 if finite_scales else 0
     info = dict(m=m, n=n, batch=batch, k_alg=sum(r.k_len for r in ranges if r.a_sel in (0, 2)),
                 k_exec=sum(r.k_len for r in ranges), a_fmt=a_fmt, b_fmt=b_fmt)
     if oc is not None:
@@ -604,7 +607,7 @@ def real_quantized_gemm_dual_scaled(fmt_a: str, fmt_w: str, inputs: torch.Tensor
          [Range(0, K, pos_scale_x, scale_w, sel[0], rs, cs), Range(0, K, neg_scale_x, scale_w, sel[1], rs, cs)],
          m=M, n=N, a_fmt=fmt_a, b_fmt=fmt_w, out_dtype=inputs.dtype, lda=K, ldb=kb, a_neg=codes_neg,
          batch=S, batch_stride_a=M * K, batch_stride_b=N * kb,
-         batch_stride_sx=1 if per_seg_x else M, batch_stride_sw=1 if per_seg_w else N, out=out, own_sums=1,
+         batch_stride_sx=1 if per_seg_x else M, batch_stride_sw=1 if per_seg_w else N, out=out, own_sums=True,
          workspace=torch.empty(need, dtype=torch.uint8, device=inputs.device) if need else None)
     return out
 

@@ -377,7 +377,7 @@ class DefaultOptimizer(BaseOptimizer):
         gdq = plan.get("group_dequant")
         add2 = None if addend is None else addend.reshape(M, N).contiguous()
         kw = dict(m=M, n=N, a_fmt=plan["fa"], b_fmt=plan["fw"], out_dtype=x.dtype, lda=K, ldb=ldb, bias=bias, a_neg=codes_neg,
-                  group_dequant=gdq, out_codes=out_codes, own_sums=2 if dual and S == 1 else 0)
+                  group_dequant=gdq, out_codes=out_codes, finite_scales=dual and S == 1)
         g = None
         if "l2t" in plan:
             # the SVD optimiser's low-rank branch: inside the GEMM's epilogue where the library has a
@@ -478,7 +478,7 @@ class DefaultOptimizer(BaseOptimizer):
             ranges.append(ops.Range(0, K, neg[0], plan["sw"], 1, 0, plan["sw_cs"]))
         g = ops.gemm_desc(codes, plan["w"], ranges, m=M, n=N, a_fmt=plan["fa"], b_fmt=plan["fw"], out_dtype=out_dtype, lda=K,
                           ldb=K // 2 if plan["fw"] == ops.FMT_INT4 else K, bias=bias, a_neg=codes_neg,
-                          group_dequant=plan.get("group_dequant"), own_sums=2 if self.dual_scale else 0)
+                          group_dequant=plan.get("group_dequant"), finite_scales=self.dual_scale)
         ws = None
         int4 = plan["fw"] == ops.FMT_INT4
         if M >= 3072 or not int4 or plan.get("group_dequant") is not None:

@@ -629,6 +629,33 @@ def test_plan_of_ranges_summed_on_their_own():
     assert plan(2000, 4000, tile=15)[0] == 2 and plan(2000, 4000, tile=15, own=0)[0] == 0
 
 
+def test_any_own_sum_is_kept_apart_and_finite_scales_leave_the_way_open():
+    """Every non-zero own_sum means ranges summed on their own (a scale may be infinite), on tiles that do not carry the sums
+    from range to range; finite_scales alone lets the library choose, and own_sum goes before it."""
+    from segquant_amd import _lib as L
+    lib = L.lib()
+
+    def plan(m, n, k, own=0, finite=0):
+        d = L.GemmDesc()
+        d.a_fmt = d.b_fmt = 1
+        d.out_dtype = d.bias_dtype = 2
+        d.m, d.n, d.lda, d.ldb, d.ldo, d.batch, d.n_ranges = m, n, k, k, n, 1, 2
+        d.a, d.a_neg, d.b, d.out = 0x10000000, 0x20000000, 0x30000000, 0x40000000
+        for i in range(2):
+            d.ranges[i].k_len, d.ranges[i].a_sel, d.ranges[i].sx, d.ranges[i].sw = k, i, 0x60000000, 0x70000000
+        d.ranges[0].own_sum, d.finite_scales = own, finite
+        t, s = ctypes.c_int32(0), ctypes.c_int32(0)
+        assert lib.segq_gemm_plan(ctypes.byref(d), ctypes.byref(t), ctypes.byref(s), None) == 0
+        return t.value, s.value
+
+    for m, n, k in ((4608, 3072, 12288), (4096, 1536, 6144), (2000, 2048, 512)):
+        apart = plan(m, n, k, own=1)
+        assert all(plan(m, n, k, own=own, finite=f) == apart for own in (2, 7, -1) for f in (0, 1)), (m, n, k)
+    # the first shape is faster with its sums carried from range to range, the second in one walk of K
+    assert plan(4608, 3072, 12288, finite=1) == plan(4608, 3072, 12288) != plan(4608, 3072, 12288, own=1)
+    assert plan(4096, 1536, 6144, finite=1) == plan(4096, 1536, 6144, own=1) != plan(4096, 1536, 6144)
+
+
 def _kernel_registers():
     """Mangled kernel name -> vector registers per lane, from the metadata the compiler leaves in the library built here."""
     import struct
