@@ -60,6 +60,12 @@ def _stream(device=None) -> int:
     return torch.cuda.current_stream(idx).cuda_stream
 
 
+def capturing() -> bool:
+    """Whether the current stream records a graph.  The buffers that calls share are not for it: the graph holds their
+    addresses and may be replayed on any stream, next to another graph and to eager calls, long after they were given back."""
+    return torch.cuda.is_current_stream_capturing()
+
+
 # When set to a list, every quantise / GEMM launch is bracketed by events on the
 # launching stream and (kind, start, end, info) is appended; see record_launches.
 _launch_log = None
@@ -239,7 +245,7 @@ class Range:
 
 
 _int4_ws = {}
-_retired_ws = []  # outgrown buffers stay allocated: a captured HIP graph may still hold their address
+_retired_ws = []  # outgrown buffers stay allocated: descriptors that layers keep may still name them
 
 
 def int4_workspace(device, nbytes: int) -> torch.Tensor:
@@ -247,7 +253,10 @@ def int4_workspace(device, nbytes: int) -> torch.Tensor:
     weights, parked partial sums of int8 ranges, split-K partial results), one per device
     and stream: launches on one stream run in order and the contents only live for the
     duration of one GEMM launch, so every layer on that stream can share it.  Grown on
-    demand; a buffer that was handed out is never freed."""
+    demand; a buffer that was handed out is never freed.  A stream that records a graph gets
+    memory of its own, which is the graph's."""
+    if capturing():
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
     dev = torch.device(device)
     if dev.index is None:
         dev = torch.device(dev.type, torch.cuda.current_device())

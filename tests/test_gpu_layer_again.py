@@ -63,3 +63,36 @@ def test_what_a_repeated_call_refuses():
     wide = torch.randn(40 * 1168 + 1, device=DEV).to(torch.bfloat16)
     with pytest.raises(RuntimeError, match="aligned"):
         layer(wide[1:].view(40, 1168))
+
+
+@pytest.mark.parametrize("m", [8, 40])
+@pytest.mark.parametrize("dynamic", [False, True])
+def test_a_captured_forward_outlives_the_layers_buffers(dynamic, m):
+    """Recorded on the stream that the layer was warmed up on, and replayed after that stream's buffers were given back (other
+    token counts have taken the layer's few places): one launch for 8 rows, two for 40, each replay as a fresh layer's forward."""
+    dt = torch.bfloat16
+    layer, fresh = _layer(5, dynamic, dt), _layer(5, dynamic, dt)
+    xs = [torch.randn(m, 1168, device=DEV).to(dt) for _ in range(3)]
+    want = [fresh(x).clone() for x in xs]
+    held = xs[0].clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            layer(held)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = layer(held)
+    with torch.cuda.stream(side):
+        for other in range(50, 62):
+            for _ in range(2):
+                layer(torch.randn(other, 1168, device=DEV).to(dt))
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    for i in (0, 1, 2, 1):
+        junk = [torch.full((1 << 12,), 0x7FC0, dtype=torch.int16, device=DEV) for _ in range(200)]
+        held.copy_(xs[i])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[i]) and all(int((t != 0x7FC0).sum()) == 0 for t in junk), (dynamic, m, i)

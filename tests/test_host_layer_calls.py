@@ -20,11 +20,11 @@ def _hit(need=0, workspace=None):
 def layer(monkeypatch):
     """An optimiser without weights, and the current stream under the test's control."""
     opt = object.__new__(opt_mod.DefaultOptimizer)
-    opt.stream = "A"
-    rooms = {}
+    opt.stream, opt.capture = "A", False
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: opt.capture)
     monkeypatch.setattr(ops, "_stream", lambda device=None: opt.stream)
-    monkeypatch.setattr(ops, "int4_workspace", lambda device, n: rooms.setdefault(opt.stream, torch.empty(n, dtype=torch.uint8)))
-    opt.rooms = rooms
+    monkeypatch.setattr(ops, "_int4_ws", {})
     return opt
 
 
@@ -37,4 +37,20 @@ def test_descriptors_of_another_stream_get_that_streams_workspace(layer):
         layer.stream = stream
         layer._relaunch(hit, x)
         kept = hit["buffers"][stream][1]
-        assert kept.workspace == layer.rooms[stream].data_ptr() and kept.workspace_bytes == 64
+        assert kept.workspace == ops.int4_workspace("cpu", 64).data_ptr() and kept.workspace_bytes == 64
+
+
+def test_a_capture_takes_buffers_of_its_own(layer):
+    """What a graph replays must not lie where eager calls, or another graph captured on the same stream, put theirs, nor where
+    a layer fed with many token counts gives its buffers back."""
+    room = ops.int4_workspace("cpu", 64)
+    hit, x = _hit(64, room.data_ptr()), torch.empty(M, K)
+    eager = layer._relaunch(hit, x)
+    layer.capture = True
+    first, second = layer._relaunch(hit, x), layer._relaunch(hit, x)
+    layer.capture = False
+    after = layer._relaunch(hit, x)
+    assert after[0][0].codes == eager[0][0].codes and after[1][0].workspace == room.data_ptr()  # eager calls reuse theirs
+    for at in (lambda r: r[0][0].codes, lambda r: r[1][0].workspace, lambda r: r[2].data_ptr()):
+        assert len({at(r) for r in (eager, first, second)}) == 3
+    assert list(hit["buffers"]) == ["A"] and ops.int4_workspace("cpu", 64) is room
