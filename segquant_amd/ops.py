@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import ctypes as C
 import functools
+import threading
 from dataclasses import dataclass
 from typing import Optional, Sequence
 
@@ -64,6 +65,16 @@ def capturing() -> bool:
     """Whether the current stream records a graph.  The buffers that calls share are not for it: the graph holds their
     addresses and may be replayed on any stream, next to another graph and to eager calls, long after they were given back."""
     return torch.cuda.is_current_stream_capturing()
+
+
+_locks = {}
+
+
+def stream_lock(stream: int):
+    """Held from the first to the last launch of a call whose buffers other calls on the stream share: the launches of a
+    stream run in the order in which they were enqueued, and two host threads may be enqueueing on it."""
+    lock = _locks.get(stream)
+    return lock if lock is not None else _locks.setdefault(stream, threading.RLock())
 
 
 # When set to a list, every quantise / GEMM launch is bracketed by events on the
@@ -252,7 +263,7 @@ def int4_workspace(device, nbytes: int) -> torch.Tensor:
     """A scratch tensor of at least ``nbytes`` for ``gemm``'s ``workspace`` (expanded int4
     weights, parked partial sums of int8 ranges, split-K partial results), one per device
     and stream: launches on one stream run in order and the contents only live for the
-    duration of one GEMM launch, so every layer on that stream can share it.  Grown on
+    duration of one GEMM call (see ``stream_lock``), so every layer on that stream can share it.  Grown on
     demand; a buffer that was handed out is never freed.  A stream that records a graph gets
     memory of its own, which is the graph's."""
     if capturing():
@@ -303,10 +314,12 @@ def gemm_plan(g, workspace: Optional[torch.Tensor] = None) -> dict:
 def gemm_launch(g, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Enqueue the GEMM described by ``g``, lending it ``workspace`` (a byte tensor) if given."""
     d, out, info, _keep = g
-    if workspace is not None:
-        _need_cuda(workspace)
-        d.workspace = workspace.data_ptr(); d.workspace_bytes = workspace.numel() * workspace.element_size()
-    L.check(_launch("gemm", info, lambda: L.lib().segq_gemm(C.byref(d), _stream())))
+    stream = _stream()
+    with stream_lock(stream):
+        if workspace is not None:
+            _need_cuda(workspace)
+            d.workspace = workspace.data_ptr(); d.workspace_bytes = workspace.numel() * workspace.element_size()
+        L.check(_launch("gemm", info, lambda: L.lib().segq_gemm(C.byref(d), stream)))
     return out
 
 
@@ -340,15 +353,17 @@ def linear(q, g, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     writes, and with dynamic scales the scale tensors it fills."""
     qd, _codes, qinfo, _k1 = q
     gd, out, ginfo, _k2 = g
-    if workspace is not None:
-        _need_cuda(workspace)
-        gd.workspace = workspace.data_ptr(); gd.workspace_bytes = workspace.numel() * workspace.element_size()
-    L.check(_launch("linear", dict(q=qinfo, g=ginfo), lambda: L.lib().segq_linear(C.byref(qd), C.byref(gd), _stream())))
+    stream = _stream()
+    with stream_lock(stream):
+        if workspace is not None:
+            _need_cuda(workspace)
+            gd.workspace = workspace.data_ptr(); gd.workspace_bytes = workspace.numel() * workspace.element_size()
+        L.check(_launch("linear", dict(q=qinfo, g=ginfo), lambda: L.lib().segq_linear(C.byref(qd), C.byref(gd), stream)))
     return out
 
 
 def linear_again(qd, gd, stream: int) -> None:
-    """``segq_linear`` on two descriptors that are complete, the workspace of an earlier :func:`linear` included."""
+    """``segq_linear`` on two descriptors that are complete, their workspace included; under the stream's lock."""
     rc = L.lib().segq_linear(C.byref(qd), C.byref(gd), stream)
     if rc:
         L.check(rc)

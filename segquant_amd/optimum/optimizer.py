@@ -281,12 +281,13 @@ class DefaultOptimizer(BaseOptimizer):
             out = self._again(x, bias)
             if out is not None:
                 return out
-        q, g, ws = self.fused_launches(x, bias, pre_op=pre_op, gate=gate, col_div=col_div, addend=addend)
-        if ops.recording_launches():
-            ops.quantize_launch(q)
-            out = ops.gemm_launch(g, ws)
-        else:
-            out = ops.linear(q, g, ws)
+        with ops.stream_lock(ops._stream(x.device)):
+            q, g, ws = self.fused_launches(x, bias, pre_op=pre_op, gate=gate, col_div=col_div, addend=addend)
+            if ops.recording_launches():
+                ops.quantize_launch(q)
+                out = ops.gemm_launch(g, ws)
+            else:
+                out = ops.linear(q, g, ws)
         return out.view(*x.shape[:-1], out.shape[-1])
 
     def fused_launches(self, x: torch.Tensor, bias=None, pre_op=None, gate=None, col_div=None, addend=None, fresh=False,
@@ -300,6 +301,7 @@ class DefaultOptimizer(BaseOptimizer):
         stream (launches on one stream run in order, and the codes only live from the quantise
         launch to the GEMM that follows it); ``fresh=True`` allocates new ones, for callers that
         hold several launches of one layer at once, and so does a call whose stream records a graph.
+        Threads that share a stream hold ``ops.stream_lock`` from here to the last of the launches.
 
         Quantise + segmented GEMM with
         de-quantisation and bias fused.  Equivalent to ``forward`` followed by
@@ -587,11 +589,12 @@ class DefaultOptimizer(BaseOptimizer):
         if reuse is None or (stream and ops.capturing()):  # (the default stream records no graph: 0.3 us saved)
             return None
         out = torch.empty((*shape[:-1], hit["N"]), dtype=dtype, device=dev)
-        qd, gd = reuse[0], reuse[1]
-        qd.x = x.data_ptr()
-        qd.ldx = plan["K"]
-        gd.out = out.data_ptr()
-        ops.linear_again(qd, gd, stream)
+        qd, gd, lock = reuse[0], reuse[1], reuse[4]
+        with lock:
+            qd.x = x.data_ptr()
+            qd.ldx = plan["K"]
+            gd.out = out.data_ptr()
+            ops.linear_again(qd, gd, stream)
         return out
 
     def _relaunch(self, hit, x2, fresh=False):
@@ -610,7 +613,7 @@ class DefaultOptimizer(BaseOptimizer):
                 bufs.pop(next(iter(bufs)))  # streams come and go: keep the buffers of the last few
             reuse = bufs.get(stream)
             if reuse is not None:  # descriptors, codes and scales of the previous call on this stream
-                qd, gd, result, held = reuse
+                qd, gd, result, held, _ = reuse
                 qd.x = x2.data_ptr()
                 qd.ldx = ops.row_stride(x2)
                 gd.out = out.data_ptr()
@@ -646,6 +649,6 @@ class DefaultOptimizer(BaseOptimizer):
             for i, (which, s_) in enumerate(hit["sx_src"]):
                 gd.ranges[i].sx = base[which] + 4 * M * s_
         if stream is not None:
-            hit["buffers"][stream] = (qd, gd, result, held)
+            hit["buffers"][stream] = (qd, gd, result, held, ops.stream_lock(stream))
         keep = (x2, out, held)
         return (qd, result, hit["q"][1], keep), (gd, out, hit["g"][1], keep), ws

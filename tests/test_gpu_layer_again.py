@@ -96,3 +96,24 @@ def test_a_captured_forward_outlives_the_layers_buffers(dynamic, m):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want[i]) and all(int((t != 0x7FC0).sum()) == 0 for t in junk), (dynamic, m, i)
+
+
+@pytest.mark.parametrize("dynamic", [False, True])
+def test_two_threads_on_one_stream(dynamic):
+    """The code buffer and the descriptors of a layer are one set per stream, whichever thread calls."""
+    import threading
+    layer, fresh = _layer(5, dynamic, torch.bfloat16), _layer(5, dynamic, torch.bfloat16)
+    xs = [torch.randn(40, 1168, device=DEV).to(torch.bfloat16) for _ in range(3)]
+    want = [fresh(x).clone() for x in xs]
+    for _ in range(2):
+        layer(xs[0])
+    torch.cuda.synchronize()
+    got = [[] for _ in xs]
+    threads = [threading.Thread(target=lambda i=i: got[i].extend(layer(xs[i]) for _ in range(100))) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for i, outs in enumerate(got):
+        assert len(outs) == 100 and all(torch.equal(o, want[i]) for o in outs), (dynamic, i)

@@ -1,4 +1,7 @@
 """What a layer keeps between calls, on the host: descriptors filled for CPU buffers, nothing launched."""
+import threading
+import time
+
 import pytest
 import torch
 
@@ -54,3 +57,49 @@ def test_a_capture_takes_buffers_of_its_own(layer):
     for at in (lambda r: r[0][0].codes, lambda r: r[1][0].workspace, lambda r: r[2].data_ptr()):
         assert len({at(r) for r in (eager, first, second)}) == 3
     assert list(hit["buffers"]) == ["A"] and ops.int4_workspace("cpu", 64) is room
+
+
+class _OnTheGpu:
+    """Enough of a tensor for a repeated call, wherever its memory is."""
+    is_cuda = True
+    device = torch.device("cpu")
+
+    def __init__(self):
+        self.t = torch.empty(M, K)
+        self.shape, self.dtype = self.t.shape, self.t.dtype
+        self.is_contiguous, self.numel, self.data_ptr = self.t.is_contiguous, self.t.numel, self.t.data_ptr
+
+
+def test_repeated_calls_of_two_threads_keep_their_tensors_together(layer, monkeypatch):
+    """Two threads on one stream share the descriptors and buffers of a layer: between one call's addresses and the end of its
+    launches no other call may write its own (the library is entered without the interpreter's lock)."""
+    inside, seen = [0], []
+
+    class Library:
+        def segq_linear(self, qd, gd, stream):
+            q, g = qd._obj, gd._obj
+            inside[0] += 1
+            first = (q.x, g.out, inside[0])
+            time.sleep(1e-3)
+            seen.append((first, (q.x, g.out, inside[0])))
+            inside[0] -= 1
+            return 0
+
+    monkeypatch.setattr(ops.L, "lib", lambda: Library())
+    hit = _hit()
+    layer._relaunch(hit, torch.empty(M, K))
+    layer._plan = {"K": K, "launches": {(M, torch.float32, None): hit}}
+    outs = {}
+
+    def calls(x):
+        outs[x] = [layer._again(x, None) for _ in range(25)]
+
+    xs = [_OnTheGpu() for _ in range(3)]
+    threads = [threading.Thread(target=calls, args=(x,)) for x in xs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(a == b and a[2] == 1 for a, b in seen) and len(seen) == 75
+    owner = {o.data_ptr(): x.data_ptr() for x in xs for o in outs[x]}
+    assert all(owner[out] == x for (x, out, _), _ in seen)
