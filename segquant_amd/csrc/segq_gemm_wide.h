@@ -205,7 +205,7 @@ __device__ __forceinline__ void wide_epilogue(const GemmParams& p, typename AccT
     float rx[TM];
     // epi: the tile's vectors parked in LDS by the caller, [1/sx BM | 1/sw BN | bias BN]
     if constexpr (!FOLD) {
-        if (via_lds && epi) {
+        if (epi) {
 #pragma unroll
             for (int b = 0; b < TM; ++b) rx[b] = epi[wm * WM + b * 16 + lrow];
         } else {
@@ -277,11 +277,21 @@ __device__ __forceinline__ void wide_epilogue(const GemmParams& p, typename AccT
 #pragma unroll
     for (int a = 0; a < TN; ++a) {
         float rw[4];
-        if constexpr (!FOLD) range_rw(r_epi, a, rw);
         float bv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (p.bias) {
+        if (epi) {  // (fp32 outputs and ragged columns too: the same factors as above, and no loads behind the K loop)
+            const v4f w = *reinterpret_cast<const v4f*>(epi + BM + wn * WN + a * 16 + 4 * lgrp);
+            const v4f bb = *reinterpret_cast<const v4f*>(epi + BM + BN + wn * WN + a * 16 + 4 * lgrp);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) bv[v] = load_bias(p.bias, p.bias_dtype, min(n_base + a * 16 + v, p.N - 1));
+            for (int v = 0; v < 4; ++v) {
+                rw[v] = w[v];
+                bv[v] = bb[v];
+            }
+        } else {
+            if constexpr (!FOLD) range_rw(r_epi, a, rw);
+            if (p.bias) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) bv[v] = load_bias(p.bias, p.bias_dtype, min(n_base + a * 16 + v, p.N - 1));
+            }
         }
 #pragma unroll
         for (int b = 0; b < TM; ++b) {

@@ -154,6 +154,18 @@ def test_ragged_end_of_k(ops, kind, tile):
         _check(ops, kind, 70, 208, 400, tile, torch.bfloat16, g, **opt)
 
 
+@pytest.mark.parametrize("tile", [26, 27, 28])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_ragged_end_of_k_scales_as_the_general_kernel(ops, tile, dt):
+    """int8 sums are exact and both kernels multiply them by quotients: the same bits, with aligned rows of the output and others."""
+    g = np.random.default_rng(tile)
+    for M, N, K in ((200, 300, 208), (65, 257, 1040), (256, 384, 144)):
+        a, b = (_dev(_codes(g, (r, K), O.FMT_INT8), O.FMT_INT8) for r in (M, N))
+        rg = [ops.Range(0, K, *(torch.from_numpy((g.random(r) * 30 + 10).astype(np.float32)).to(DEV) for r in (M, N)), 0, 1, 1)]
+        out = [ops.gemm(a, b, rg, m=M, n=N, a_fmt=O.FMT_INT8, b_fmt=O.FMT_INT8, out_dtype=dt, lda=K, ldb=K, tile=t) for t in (tile, 4)]
+        assert torch.equal(*out), (M, N, K, float((out[0] - out[1]).abs().max()))
+
+
 @pytest.mark.parametrize("kind", ["int8", "e4m3"])
 def test_large_ragged_launch_takes_a_walk(ops, kind):
     g = np.random.default_rng(5)
