@@ -130,7 +130,11 @@ static int64_t tiles_of_cfg(int cfg, int64_t m, int64_t n, int64_t batch) {
 // One range, K not in whole steps.  (Rows of such a K start anywhere in a cache line: a step costs more than an aligned one's.)
 //   us, general kernel before / 256 x 256 / 256 x 192 / 128 x 128:  4900 x 5900 x 4912 270 / 170 / 209 / 231;
 //   4000 x 3000 x 2064 66 / 41 / 37 / 46;  2000 x 3000 x 1008 25.1 / 25.2 / 20.6 / 15.3;  1200 x 3000 x 800 16.2 / 25.4 / 18.8 / 11.1
-static Walk choose_ragged(int64_t m, int64_t n, int64_t batch, int64_t k) {
+// `scattered`: fp32 outputs whose rows do not start on the boundaries of whole stores are written value by value, which costs a
+// 128 x 128 tile of these kernels more than one of the general kernel (64 x 128): a short K stays with that (cfg -1) while its tiles
+// fit the CUs once.  us, 128 x 128 / general: 748 x 383 x 208 9.0 / 7.6; 869 x 479 x 160 9.2 / 7.9; 762 x 2595 x 1264 18.5 / 20.6.
+// Of 971 such launches 2.8 % are slower than on the general kernel by 3 % or more, 42 % without this line (16-bit outputs: 0.4 %).
+static Walk choose_ragged(int64_t m, int64_t n, int64_t batch, int64_t k, bool scattered) {
     const double steps = (double)((k + 127) / 128);
     const int64_t cus = device_cus();
     auto rounds = [&](int cfg) { return (double)((tiles_of_cfg(cfg, m, n, batch) + cus - 1) / cus); };
@@ -140,6 +144,10 @@ static Walk choose_ragged(int64_t m, int64_t n, int64_t batch, int64_t k) {
     if (us192 < w.us) w = Walk{FIRST_KT_CFG + 1, us192};
     const double us256 = rounds(FIRST_KT_CFG) * (2.0 * steps + 6.0);
     if (us256 < w.us) w = Walk{FIRST_KT_CFG, us256};
+    if (scattered && w.cfg == FIRST_KT_CFG + 2 && tiles_of_cfg(3, m, n, batch) <= cus) {
+        auto rows = [&](int cfg) { return m < TILE_CFGS[cfg].bm ? (double)m / TILE_CFGS[cfg].bm : 1.0; };  // of a tile, that are stored
+        if (1.03 * (6.2 + 1.04 * steps + rows(3)) < 4.8 + 0.83 * steps + 3.7 * rows(w.cfg)) w.cfg = -1;
+    }
     return w;
 }
 
@@ -353,6 +361,9 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     if (w4 && ktotal > 131071) return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: K too large for int4 weights");
     if (kmax > 0x7fffff00) return fail(SEGQ_ERR_ARG, "segq_gemm: K too large");
 
+    const int64_t osz = (d->out_dtype == SEGQ_F32 || d->out_dtype == SEGQ_ACC) ? 4 : 2;
+    const bool vec_store = ((d->ldo * osz) % (4 * osz) == 0) && ((d->batch_stride_out * osz) % (4 * osz) == 0) && al(d->out, 4 * osz);
+
     // One walk of K: one range whose end is ragged, or DualScale's two ranges over the same run (a, then a_neg)
     Walk walk{-1, 1e30};
     {
@@ -367,7 +378,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
                             FIRST_KT_CFG + 1, FIRST_DUAL_CFG, FIRST_DUAL_CFG + 1, NUM_TILE_CFG);
             walk.cfg = (int)d->tile - 1;
         } else if (d->tile == 0 && d->out_dtype != SEGQ_ACC) {
-            if (one && r.k_len % 128) walk = choose_ragged(d->m, d->n, d->batch, r.k_len);
+            if (one && r.k_len % 128) walk = choose_ragged(d->m, d->n, d->batch, r.k_len, osz == 4 && !vec_store);
             if (two && (r.own_sum || d->finite_scales) && r.k_len > (r.k_len % 128 ? 256 : 512)) {
                 walk = choose_dual(d->m, d->n, d->batch, r.k_len);
                 const bool lent = d->split_k != 1 && ws && al(ws, 16), in_turn = r.k_len % 128 == 0 && d->batch == 1;
@@ -457,8 +468,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         p.ldadd = d->ld_addend;
         p.vec_add = d->addend && (d->ld_addend * asz) % (4 * asz) == 0 && (d->batch_stride_out * asz) % (4 * asz) == 0 && al(d->addend, 4 * asz);
     }
-    const int64_t osz = (d->out_dtype == SEGQ_F32 || d->out_dtype == SEGQ_ACC) ? 4 : 2;
-    p.vec_store = ((d->ldo * osz) % (4 * osz) == 0) && ((d->batch_stride_out * osz) % (4 * osz) == 0) && al(d->out, 4 * osz);
+    p.vec_store = vec_store;
     p.vec_store16 = osz == 2 && d->ldo % 8 == 0 && d->batch_stride_out % 8 == 0 && al(d->out, 16);
     p.nr = d->n_ranges;
     if (few >= 0) {

@@ -167,10 +167,16 @@ def test_ragged_end_of_k_scales_as_the_general_kernel(ops, tile, dt):
 
 
 @pytest.mark.parametrize("kind", ["int8", "e4m3"])
-def test_large_ragged_launch_takes_a_walk(ops, kind):
+@pytest.mark.parametrize("M,N,K,tiles", [(1300, 1500, 784, (26, 27, 28)), (2000, 2300, 1040, (26, 27, 28)), (748, 384, 208, (26, 27, 28)),
+                                         (748, 383, 208, (4,)), (869, 479, 160, (4,)), (2000, 2301, 1040, (26, 27, 28))])
+def test_ragged_launch_takes_a_walk(ops, kind, M, N, K, tiles):
+    """... unless K is short and the rows of the output start off the boundaries of whole stores."""
     g = np.random.default_rng(5)
-    for M, N, K in ((1300, 1500, 784), (2000, 2300, 1040)):
-        _check(ops, kind, M, N, K, 0, torch.float32, g)
+    one = torch.ones(1, device=DEV)
+    d = ops.gemm_desc(torch.empty(M, K, dtype=torch.uint8, device=DEV), torch.empty(N, K, dtype=torch.uint8, device=DEV), [ops.Range(0, K, one, one)],
+                      m=M, n=N, a_fmt=FORMATS[kind][0], b_fmt=FORMATS[kind][1], out_dtype=torch.float32, lda=K, ldb=K)
+    assert ops.gemm_plan(d)["tile"] in tiles
+    _check(ops, kind, M, N, K, 0, torch.float32, g)
 
 
 def _check_dual(ops, kind, S, M, N, K, tile, dt, g, k0=0, pad=0, empty=None, per_row=True, per_col=True, add=False):
