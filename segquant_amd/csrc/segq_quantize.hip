@@ -286,7 +286,7 @@ __device__ __forceinline__ float wave_max(float v) {  // of non-negative values 
 template <int DT, int FMT, int CACHE, bool DUAL, bool PRE>
 __global__ void __launch_bounds__(CACHE == 4 ? 256 : 512) quant_dynamic_kernel(const QuantParams p) {
     __shared__ float red[2][8];
-    const int nt = blockDim.x, nw = nt >> 6;
+    const int nt = CACHE == 4 ? 256 : blockDim.x, nw = nt >> 6;
     const int64_t row = blockIdx.x;
     const size_t esz = (DT == SEGQ_F32) ? 4 : 2;
     const uint8_t* xrow = static_cast<const uint8_t*>(p.x) + row * p.ldx * esz;
@@ -326,9 +326,14 @@ __global__ void __launch_bounds__(CACHE == 4 ? 256 : 512) quant_dynamic_kernel(c
             red[1][threadIdx.x >> 6] = amax_n;
         }
         __syncthreads();
-        for (int w = 0; w < nw; ++w) {  // (this thread's own maxima among them)
-            amax_p = max_nn(amax_p, red[0][w]);
-            amax_n = max_nn(amax_n, red[1][w]);
+        if constexpr (CACHE == 4) {
+            amax_p = max_nn(max_nn(red[0][0], red[0][1]), max_nn(red[0][2], red[0][3]));
+            amax_n = max_nn(max_nn(red[1][0], red[1][1]), max_nn(red[1][2], red[1][3]));
+        } else {
+            for (int w = 0; w < nw; ++w) {  // (this thread's own maxima among them)
+                amax_p = max_nn(amax_p, red[0][w]);
+                amax_n = max_nn(amax_n, red[1][w]);
+            }
         }
         float s_pos, s_neg;
         if (dual) {
@@ -384,6 +389,7 @@ __global__ void __launch_bounds__(256) quant_dynamic_wave_kernel(const QuantPara
             if (c < c1) load_run<DT, PRE>(p, xrow, row, c, raw[i]);
         }
         float amax_p = 0.0f, amax_n = 0.0f;
+        [[maybe_unused]] float kept[16];  // a single run is unpacked once
 #pragma unroll
         for (int i = 0; i < CPL; ++i) {
             const int c = c0 + lane + i * 64;
@@ -391,6 +397,9 @@ __global__ void __launch_bounds__(256) quant_dynamic_wave_kernel(const QuantPara
                 float v[16];
                 raw_to_f32<DT>(raw[i], v);
                 track_amax<DUAL>(v, amax_p, amax_n, dual);
+                if constexpr (CPL == 1)
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) kept[j] = v[j];
             }
         }
         amax_p = wave_max(amax_p);
@@ -411,9 +420,13 @@ __global__ void __launch_bounds__(256) quant_dynamic_wave_kernel(const QuantPara
         for (int i = 0; i < CPL; ++i) {
             const int c = c0 + lane + i * 64;
             if (c < c1) {
-                float v[16];
-                raw_to_f32<DT>(raw[i], v);
-                encode16<FMT>(p, row, (int64_t)c << 4, v, s_pos, s_neg, two);
+                if constexpr (CPL == 1) {
+                    encode16<FMT>(p, row, (int64_t)c << 4, kept, s_pos, s_neg, two);
+                } else {
+                    float v[16];
+                    raw_to_f32<DT>(raw[i], v);
+                    encode16<FMT>(p, row, (int64_t)c << 4, v, s_pos, s_neg, two);
+                }
             }
         }
     }
@@ -611,8 +624,22 @@ static int launch_quant(const QuantParams& p, hipStream_t st) {
         // ones while there are at most three workgroups per CU.  One wave per row does its runs one after the other, with
         // the activation function in front of each (bf16, x gelu(gate), us, wave per row / this: 400 x 5120 17.7 / 7.2, 1000 x
         // 1280 9.0 / 6.7, 8192 x 2560 37.4 / 35.7; 8192 x 5120 61.7 / 94.8, where a workgroup's waves wait for each other
-        // with too few workgroups on the CU)
-        if (longest <= 64 * 4 || (longest <= 64 * 8 && p.rows <= 3 * (int64_t)device_cus())) {
+        // with too few workgroups on the CU).  Rows of 8192 have all four runs of 256 threads (600 rows 9.0, this 9.9).
+        // A wave per row is level with this or ahead of it where
+        //  - the rows of the launch are resident at once that way, and the producer is short: 2048 x 3072 bf16 with column
+        //    factors 9.6, this 10.3 (DualScale 11.9 and 13.3, 8192 rows 31.7 and 34.1); with an activation from ten rows per CU on;
+        //  - several segments are a wave each at most: 2048 x 4096 fp32 in four 10.5, this 12.8; 2048 x 2048 bf16 in four 6.7, this
+        //    7.4 (up to 14 rows per CU; beyond, 8192 rows 13.7, 16-bit rows go as they did).
+        const int64_t cus = device_cus();
+        const bool short_segs = longest <= 64 && p.n_kseg > 1 && (DT == SEGQ_F32 || p.rows <= 14 * cus);
+        if (short_segs) {
+            if (p.dual) hipLaunchKernelGGL((quant_dynamic_wave_kernel<DT, FMT, 1, true, PRE>), wgrid, dim3(256), 0, st, p);
+            else hipLaunchKernelGGL((quant_dynamic_wave_kernel<DT, FMT, 1, false, PRE>), wgrid, dim3(256), 0, st, p);
+        } else if (longest > 64 && longest <= 64 * 3 && p.n_kseg == 1 && p.rows > (p.pre_op ? 10 : 6) * cus &&
+                   ((p.dual && !p.pre_op) || p.rows <= (DT == SEGQ_F32 ? 10 : 14) * cus)) {
+            if (p.dual) hipLaunchKernelGGL((quant_dynamic_wave_kernel<DT, FMT, 4, true, PRE>), wgrid, dim3(256), 0, st, p);
+            else hipLaunchKernelGGL((quant_dynamic_wave_kernel<DT, FMT, 4, false, PRE>), wgrid, dim3(256), 0, st, p);
+        } else if (longest <= 64 * 4 || (longest < 64 * 8 && p.rows <= 3 * cus) || (longest == 64 * 8 && p.rows <= 2 * cus)) {
             const dim3 runs((unsigned)((longest + 63) / 64 * 64));
             if (p.dual) hipLaunchKernelGGL((quant_dynamic_kernel<DT, FMT, 1, true, PRE>), bgrid, runs, 0, st, p);
             else hipLaunchKernelGGL((quant_dynamic_kernel<DT, FMT, 1, false, PRE>), bgrid, runs, 0, st, p);

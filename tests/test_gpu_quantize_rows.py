@@ -41,3 +41,46 @@ def test_gated_rows_do_not_depend_on_the_row_count(cols):
         a, b = ops.quantize(x[:rows], "int8", pos, neg, **kw)
         out.append([t[:edge] for t in (a, b, pos, neg)])
     assert all(torch.equal(p, q) for p, q in zip(*out))
+
+
+@pytest.mark.parametrize("dual", [False, True])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("cols", [1040, 2064, 3072, 3088])
+def test_many_rows_with_divisors_equal_plain_rows(dt, cols, dual):
+    """A wave per row or a workgroup: both sides of the row counts (6 and 14 per compute unit) between which they change."""
+    from segquant_amd import ops
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for rows in (6 * cus, 6 * cus + 1, 10 * cus + 1, 14 * cus, 14 * cus + 1):
+        x = torch.randn(rows, cols, device=DEV)
+        x[0], x[1, 3], x[2, cols - 1] = 0, float("nan"), float("inf")
+        x = x.to(dt)
+        out = []
+        for div in (None, torch.ones(cols, device=DEV)):
+            pos, neg = torch.empty(rows, device=DEV), torch.empty(rows, device=DEV)
+            codes = ops.quantize(x, "int8", pos, neg if dual else None, row_stride=1, dynamic=True, col_div=div, dual=dual, two_tensors=dual)
+            out.append([t.view(torch.uint8) for t in (codes if dual else (codes,))] + [t.view(torch.int32) for t in ((pos, neg) if dual else (pos,))])
+        assert all(torch.equal(p, q) for p, q in zip(*out)), (dt, cols, dual, rows)
+
+
+@pytest.mark.parametrize("dual", [False, True])
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("widths", [(16, 1024), (16, 48, 1040), (512, 1008, 16, 528), (1024, 4096)])
+def test_segments_equal_their_own_launches(dt, widths, dual):
+    """Column segments of a wave at most, and of more, against launches of one segment each: codes and scales bit for bit."""
+    from segquant_amd import ops
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    bounds = [sum(widths[:i]) for i in range(len(widths) + 1)]
+    for rows in (1, 7, 14 * cus, 14 * cus + 1):
+        x = torch.randn(rows, bounds[-1], device=DEV)
+        x[0, bounds[1]] = float("nan")
+        x[rows - 1, :16] = 0
+        x = x.to(dt)
+        pos, neg = torch.empty(len(widths), rows, device=DEV), torch.empty(len(widths), rows, device=DEV)
+        kw = dict(row_stride=1, dynamic=True, dual=dual, two_tensors=dual)
+        got = ops.quantize(x, "int8", pos, neg if dual else None, kseg_bounds=bounds, kseg_stride=rows, **kw)
+        for s, (c0, c1) in enumerate(zip(bounds, bounds[1:])):
+            p, n = torch.empty(rows, device=DEV), torch.empty(rows, device=DEV)
+            want = ops.quantize(x[:, c0:c1].contiguous(), "int8", p, n if dual else None, **kw)
+            assert torch.equal(p.view(torch.int32), pos[s].view(torch.int32)) and (not dual or torch.equal(n.view(torch.int32), neg[s].view(torch.int32))), (dt, widths, rows, s)
+            for g, w in zip(got if dual else (got,), want if dual else (want,)):
+                assert torch.equal(g[:, c0:c1], w), (dt, widths, rows, s)
