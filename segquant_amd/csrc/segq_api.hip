@@ -197,6 +197,18 @@ static double in_turn_us(int64_t m, int64_t n, int64_t steps, bool f8, bool ws) 
     return us;
 }
 
+// What a GEMM of few tiles takes longer, in us, if each of its workgroups reads and encodes the rows of x itself: so much per
+// round of the CUs, more for more bytes and rows, and less where that passes under the wait for the weights.  Fitted over 1400
+// launches (rms 0.8).  A quantise launch takes 2 us of the GPU and 3.8 of the host, which small layers wait for: up to the sum
+// of the two the linear stays in one launch.  us, one launch / two, on the GPU alone: 8 x 9216 x 1536 int4 bf16 6.7 / 7.9 (1.9 by
+// this estimate); 16 x 9216 x 1536 fp32 dynamic 10.1 / 8.0 (5.9); 16 x 36864 x 3072 e4m3 bf16 44 / 27 (17).
+static double quantise_in_gemm_us(const segq_quant_desc* q, int64_t tiles) {
+    const int64_t cus = device_cus();
+    const double rounds = (double)((tiles + cus - 1) / cus), k = q->cols / 1024.0;
+    const bool f32 = q->x_dtype == SEGQ_F32, second = q->rows > 8;
+    return rounds * (q->dynamic ? 0.9 : 0.1) + k * (rounds * (0.83 + (second ? 0.36 : 0.0) + (f32 ? second ? 0.44 : 0.12 : 0.0)) - 0.55);
+}
+
 // int4 weight rows (two values per byte, even k in the low nibble) -> int8 rows.
 // One thread expands 16 packed bytes to 32 values.
 __global__ void __launch_bounds__(256) expand_i4_kernel(const uint8_t* src, int64_t ld_src, uint8_t* dst, int64_t ld_dst,
@@ -402,7 +414,8 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         return ok && d->out_dtype != SEGQ_ACC ? choose_few(d->m, d->n, d->batch, r.k_len, f8 ? GEMM_F8 : GEMM_I8, w4, groups, walk.us) : -1;
     }();
     if (q) {
-        *fused = few >= FIRST_FEW_CFG && TILE_CFGS[few].bm == 16 && d->m <= 16 && d->ranges[0].k_len <= 128 * 8 * (TILE_CFGS[few].bn == 32 ? 4 : 3);
+        *fused = few >= FIRST_FEW_CFG && TILE_CFGS[few].bm == 16 && d->m <= 16 && d->ranges[0].k_len <= 128 * 8 * (TILE_CFGS[few].bn == 32 ? 4 : 3) &&
+                 quantise_in_gemm_us(q, tiles_of_cfg(few, d->m, d->n, 1)) <= 5.8;
         if (!*fused) return SEGQ_OK;
     }
     if (few == -2)

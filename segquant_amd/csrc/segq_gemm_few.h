@@ -75,7 +75,7 @@ template <int TM, int TN, bool B4> constexpr int few_patch() {
 // encodes each on its way to the patch, so that the linear is one launch and the codes need no trip through memory.  Every
 // workgroup encodes all of its 16 rows, which is why it serves no more; the first column of tiles also leaves the codes
 // and the dynamic scales where the quantise launch would have.  2 x 1536 -> 9216 fp16: both launches 9.4 us
-// and the gap between them, this 7.6; dynamic 8 x 3072 -> 6144 10.0 and 8.4; 16 x 3072 -> 18432 20.0 and 20.3.
+// and the gap between them, this 7.6; dynamic 8 x 3072 -> 6144 10.0 and 8.4.  (Wide layers and long rows: quantise_in_gemm_us().)
 template <int TM, int TN, int FMT, bool B4, bool GRP, int ITER, int QE = 0>
 __global__ void __launch_bounds__(FEW_WAVES * 64, QE == 0 && few_two(TM, TN, B4, GRP, ITER) ? 4 : 2) gemm_few_kernel(const FewParams p) {
     constexpr int NW = FEW_WAVES, BM = TM * 16, BN = TN * 16, NB = TM * TN;

@@ -1,5 +1,7 @@
 """The GEMM kernel for launches of few tiles against the closed form: the edges of its tiles, of the units its waves share K
 in, of its short-K instances (one to four units per wave) and of the loop behind them."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -273,6 +275,65 @@ def test_linear_in_one_launch(ops, kind, group, dynamic, dt):
         assert torch.equal(q[1].view(torch.uint8), q2[1].view(torch.uint8)), what
         assert torch.equal(scale.view(torch.int32), scale2.view(torch.int32)), what
         assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.nan_to_num(), want.nan_to_num()), what
+
+
+def _captured(call):
+    """The graph of one call and the number of launches in it."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph(keep_graph=True)
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=stream):
+        call()
+    count = ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    graph.instantiate()
+    return graph, count.value
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kind,group", [("int8", False), ("e4m3", False), ("int4", False), ("int4", True)])
+@pytest.mark.parametrize("scales", ["tensor", "row", "dynamic"])
+def test_wide_linear_in_one_launch(ops, kind, group, scales, dt):
+    """Layers of many column tiles, on 16 x 64 too, and one scale for the tensor: codes, scales and outputs of the two launches apart
+    bit for bit, from every replay of a graph as well, and in one launch wherever the estimate says so."""
+    fa, fb = FORMATS[kind]
+    g = np.random.default_rng(13)
+    for M, N, K in ((8, 12288, 1536), (3, 12300, 1024), (8, 18432, 2048), (16, 12288, 3072), (2, 9216, 1536), (16, 36864, 3072), (17, 1024, 1024), (4, 512, 4224)):
+        w = _dev(_codes(g, (N, K), fb), fb)
+        dyn = scales == "dynamic"
+        sw = torch.rand(1 if group else N, device=DEV) + 0.5
+        gd = torch.rand(K // 128, N, device=DEV) if group else None
+        x, scale = torch.randn(M, K, device=DEV).to(dt), torch.rand(1 if scales == "tensor" else M, device=DEV) * 20 + 1
+
+        def descs(scale):
+            q = ops.quantize_desc(x, fa, scale, row_stride=int(scales != "tensor"), dynamic=dyn)
+            d = ops.gemm_desc(q[1], w, [ops.Range(0, K, scale, sw, 0, int(scales != "tensor"), int(not group))], m=M, n=N, a_fmt=fa, b_fmt=fb, out_dtype=dt,
+                              lda=K, ldb=K // 2 if kind == "int4" else K, group_dequant=gd)
+            nb = ops.gemm_workspace_bytes(d)
+            return q, d, torch.empty(nb, dtype=torch.uint8, device=DEV) if nb else None
+        what = (kind, group, scales, dt, M, N, K)
+        q, d, ws = descs(scale.clone())
+        tile = ops.gemm_plan(d, ws)["tile"]
+        graph, launches = _captured(lambda: ops.linear(q, d, ws))
+        tiles, most = -(-N // (32 if tile == 22 else 64)), 1024 * (4 if tile == 22 else 3)
+        rounds = -(-tiles // torch.cuda.get_device_properties(0).multi_processor_count)
+        f32, second = dt == torch.float32, M > 8
+        extra = rounds * (0.9 if dyn else 0.1) + K / 1024 * (rounds * (0.83 + 0.36 * second + (0.44 if second else 0.12) * f32) - 0.55)
+        if tile in (22, 23) or M > 16:  # (elsewhere the library has other launches for several rows)
+            assert launches == (1 if M <= 16 and K <= most and extra <= 5.8 else 2), (what, tile, launches)
+        for _ in range(3):
+            x.copy_(torch.randn(M, K, device=DEV))
+            q2, d2, ws2 = descs(scale.clone())
+            ops.quantize_launch(q2)
+            want = ops.gemm_launch(d2, ws2)
+            for out in (d[1], None):  # the replay's, then an eager call's
+                if out is None:
+                    out = ops.linear(q, d, ws)
+                else:
+                    out.zero_(); q[1].zero_()
+                    graph.replay()
+                assert torch.equal(q[1].view(torch.uint8), q2[1].view(torch.uint8)), what
+                assert torch.equal(q[3][1].view(torch.int32), q2[3][1].view(torch.int32)) and torch.equal(out, want), what
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
