@@ -61,20 +61,22 @@ def _stream(device=None) -> int:
     return torch.cuda.current_stream(idx).cuda_stream
 
 
-def capturing() -> bool:
-    """Whether the current stream records a graph.  The buffers that calls share are not for it: the graph holds their
-    addresses and may be replayed on any stream, next to another graph and to eager calls, long after they were given back."""
-    return torch.cuda.is_current_stream_capturing()
+def capturing(stream) -> bool:
+    """Whether ``stream``, the current one, records a graph.  The buffers that calls share are not for it: the graph holds their
+    addresses and may be replayed on any stream, next to another graph and to eager calls, long after they were given back.
+    (The default stream, 0, records none; asking costs 0.3 us.)"""
+    return stream != 0 and torch.cuda.is_current_stream_capturing()
 
 
-_locks = {}
+class _StreamLocks(dict):
+    """A lock per stream, held from the first to the last launch of a call whose buffers other calls on the stream share: the
+    launches of a stream run in the order in which they were enqueued, and two host threads may be enqueueing on it."""
+
+    def __missing__(self, stream):
+        return self.setdefault(stream, threading.RLock())
 
 
-def stream_lock(stream: int):
-    """Held from the first to the last launch of a call whose buffers other calls on the stream share: the launches of a
-    stream run in the order in which they were enqueued, and two host threads may be enqueueing on it."""
-    lock = _locks.get(stream)
-    return lock if lock is not None else _locks.setdefault(stream, threading.RLock())
+stream_lock = _StreamLocks()
 
 
 # When set to a list, every quantise / GEMM launch is bracketed by events on the
@@ -266,12 +268,13 @@ def int4_workspace(device, nbytes: int) -> torch.Tensor:
     duration of one GEMM call (see ``stream_lock``), so every layer on that stream can share it.  Grown on
     demand; a buffer that was handed out is never freed.  A stream that records a graph gets
     memory of its own, which is the graph's."""
-    if capturing():
-        return torch.empty(nbytes, dtype=torch.uint8, device=device)
     dev = torch.device(device)
     if dev.index is None:
         dev = torch.device(dev.type, torch.cuda.current_device())
-    key = (dev, _stream(dev))
+    stream = _stream(dev)
+    if capturing(stream):
+        return torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    key = (dev, stream)
     ws = _int4_ws.get(key)
     if ws is None or ws.numel() < nbytes:
         if ws is not None:
@@ -315,7 +318,7 @@ def gemm_launch(g, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Enqueue the GEMM described by ``g``, lending it ``workspace`` (a byte tensor) if given."""
     d, out, info, _keep = g
     stream = _stream()
-    with stream_lock(stream):
+    with stream_lock[stream]:
         if workspace is not None:
             _need_cuda(workspace)
             d.workspace = workspace.data_ptr(); d.workspace_bytes = workspace.numel() * workspace.element_size()
@@ -354,7 +357,7 @@ def linear(q, g, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     qd, _codes, qinfo, _k1 = q
     gd, out, ginfo, _k2 = g
     stream = _stream()
-    with stream_lock(stream):
+    with stream_lock[stream]:
         if workspace is not None:
             _need_cuda(workspace)
             gd.workspace = workspace.data_ptr(); gd.workspace_bytes = workspace.numel() * workspace.element_size()

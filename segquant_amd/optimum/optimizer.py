@@ -277,17 +277,23 @@ class DefaultOptimizer(BaseOptimizer):
         """Final (..., out) result in ``x.dtype``: the two launches of :meth:`fused_launches`
         through one call of the library (``segq_linear``), or through two when a
         ``record_launches`` block is timing the kernels apart."""
-        if pre_op is None and gate is None and col_div is None and addend is None:
-            out = self._again(x, bias)
-            if out is not None:
-                return out
-        with ops.stream_lock(ops._stream(x.device)):
-            q, g, ws = self.fused_launches(x, bias, pre_op=pre_op, gate=gate, col_div=col_div, addend=addend)
-            if ops.recording_launches():
-                ops.quantize_launch(q)
-                out = ops.gemm_launch(g, ws)
-            else:
-                out = ops.linear(q, g, ws)
+        plan = self._plan
+        # (smoothed and low-rank layers keep nothing between calls, and no call with more than an input does)
+        if plan is None or "launches" not in plan or pre_op is not None or gate is not None or col_div is not None or addend is not None:
+            return self._enqueue(x, bias, pre_op, gate, col_div, addend)
+        out = self._again(x, bias)
+        if out is None:
+            with ops.stream_lock[ops._stream(x.device)]:
+                out = self._enqueue(x, bias)
+        return out
+
+    def _enqueue(self, x, bias, pre_op=None, gate=None, col_div=None, addend=None):
+        q, g, ws = self.fused_launches(x, bias, pre_op=pre_op, gate=gate, col_div=col_div, addend=addend)
+        if ops.recording_launches():
+            ops.quantize_launch(q)
+            out = ops.gemm_launch(g, ws)
+        else:
+            out = ops.linear(q, g, ws)
         return out.view(*x.shape[:-1], out.shape[-1])
 
     def fused_launches(self, x: torch.Tensor, bias=None, pre_op=None, gate=None, col_div=None, addend=None, fresh=False,
@@ -572,8 +578,8 @@ class DefaultOptimizer(BaseOptimizer):
         costs is the host: through ``fused_launches`` a (2, 256) x 1024 layer takes 12.7 us a pass, 5.8 of them
         in the library and its two launches, like this 9.9."""
         plan = self._plan
-        cache = None if plan is None else plan.get("launches")  # (a smoothed or low-rank layer has none)
-        if cache is None or ops.recording_launches() or not (x.is_cuda and x.is_contiguous()):
+        cache = plan["launches"]
+        if ops.recording_launches() or not (x.is_cuda and x.is_contiguous()):
             return None
         shape = x.shape
         if shape[-1] != plan["K"]:
@@ -586,7 +592,7 @@ class DefaultOptimizer(BaseOptimizer):
         dev = x.device
         stream = ops._stream(dev)
         reuse = bufs.get(stream)
-        if reuse is None or (stream and ops.capturing()):  # (the default stream records no graph: 0.3 us saved)
+        if reuse is None or (stream and ops.capturing(stream)):
             return None
         out = torch.empty((*shape[:-1], hit["N"]), dtype=dtype, device=dev)
         qd, gd, lock = reuse[0], reuse[1], reuse[4]
@@ -605,9 +611,10 @@ class DefaultOptimizer(BaseOptimizer):
         dev = x2.device
         out = torch.empty((hit["M"], hit["N"]), dtype=hit["out_dtype"], device=dev)
         ws = ops.int4_workspace(dev, hit["need"]) if hit["need"] else None
-        stream = None
-        if not (fresh or ops.capturing()):
-            stream = ops._stream(dev)
+        stream = None if fresh else ops._stream(dev)
+        if stream is not None and ops.capturing(stream):
+            stream = None
+        if stream is not None:
             bufs = hit.setdefault("buffers", {})
             if stream not in bufs and len(bufs) >= 4:
                 bufs.pop(next(iter(bufs)))  # streams come and go: keep the buffers of the last few
@@ -649,6 +656,6 @@ class DefaultOptimizer(BaseOptimizer):
             for i, (which, s_) in enumerate(hit["sx_src"]):
                 gd.ranges[i].sx = base[which] + 4 * M * s_
         if stream is not None:
-            hit["buffers"][stream] = (qd, gd, result, held, ops.stream_lock(stream))
+            hit["buffers"][stream] = (qd, gd, result, held, ops.stream_lock[stream])
         keep = (x2, out, held)
         return (qd, result, hit["q"][1], keep), (gd, out, hit["g"][1], keep), ws

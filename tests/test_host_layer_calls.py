@@ -103,3 +103,31 @@ def test_repeated_calls_of_two_threads_keep_their_tensors_together(layer, monkey
     assert all(a == b and a[2] == 1 for a, b in seen) and len(seen) == 75
     owner = {o.data_ptr(): x.data_ptr() for x in xs for o in outs[x]}
     assert all(owner[out] == x for (x, out, _), _ in seen)
+
+
+def test_the_default_stream_is_not_asked_for_a_capture(monkeypatch):
+    """It records no graph, and the question costs a repeated call of a small layer some of its time."""
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: pytest.fail("asked"))
+    assert ops.capturing(0) is False
+
+
+def test_calls_that_share_no_buffers_take_no_lock(layer, monkeypatch):
+    """A layer that keeps nothing between its calls, and any call with more than an input, go straight to their launches; the
+    others hold the lock of their stream."""
+    held = []
+
+    class Lock:
+        def __enter__(self):
+            held.append(True)
+
+        def __exit__(self, *exc):
+            held.pop()
+
+    monkeypatch.setattr(ops, "stream_lock", {"A": Lock()})
+    monkeypatch.setattr(layer, "_again", lambda x, bias: None, raising=False)
+    monkeypatch.setattr(layer, "_enqueue", lambda *a: bool(held), raising=False)
+    x = torch.empty(M, K)
+    for plan, kw, locked in ((None, {}, False), ({"K": K}, {}, False), ({"K": K, "launches": {}}, {}, True),
+                             ({"K": K, "launches": {}}, {"pre_op": "gelu"}, False), ({"K": K, "launches": {}}, {"addend": x}, False)):
+        layer._plan = plan
+        assert layer.forward_fused(x, **kw) is locked
