@@ -5,10 +5,10 @@ namespace segq {
 
 // Tile for a launch of few tiles, or -1 where the other kernels serve it better.  Both sides are estimated in us from
 // launches with weights from memory; K in steps of 128.  The constants were fitted over 220 launches of 8-bit codes of 24 to
-// 700 rows, 1152 to 9216 columns and K of 1152 to 12288, and 170 of int4 codes: the choice is 2.5 % (int4 1 %) from the best on the
-// mean of them (18 % and 6 % with constants of one tile a CU: 200 x 1536 x 6144 44.6 -> 14.2 us, 128 x 4096 x 4096 22.1 -> 13.3,
-// e4m3 500 x 2048 x 2048 17.9 -> 10.7, int4 154 x 2560 x 2560 11.8 -> 8.5, 320 x 6144 x 3072 30.4 -> 24.3).  `other_us`: what the
-// 8-wave tiles for a ragged K would take, where they serve the launch.
+// 700 rows, 1152 to 9216 columns and K of 1152 to 12288, and 170 of int4 codes: on other sizes the choice is 3.0 % from the best on
+// the mean, int4 1.6 %, with group factors 5.4 % (the fitted ones 18 % and int4 6 % with constants of one tile a CU:
+// 200 x 1536 x 6144 44.6 -> 14.2 us, 128 x 4096 x 4096 22.1 -> 13.3, e4m3 500 x 2048 x 2048 17.9 -> 10.7, int4 154 x 2560 x 2560
+// 11.8 -> 8.5, 320 x 6144 x 3072 30.4 -> 24.3).  `other_us`: what the 8-wave tiles for a ragged K would take, where they serve it.
 int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4, bool grp, double other_us) {
     const int64_t cus = device_cus(), steps = (k + 127) / 128;
     auto tiles = [&](int64_t bm, int64_t bn) { return (m + bm - 1) / bm * ((n + bn - 1) / bn) * batch; };
@@ -61,13 +61,13 @@ int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4,
             const bool stages = fmt == GEMM_I8 && rounds == 1, narrow = stages && n % 96 == 0 && (m + 127) / 128 * (n / 96) * batch <= cus;
             other = 6.0 + (stages ? 0.5 : fmt == GEMM_F8 ? 0.8 : 0.6) * steps * rounds;
             area = (steps + 6.0) * 128 * (narrow ? 96 : 128) / 0.7 * rounds;
-            if (stages && steps <= 12) keep = 0.72;  // 256 x 2176 x 1536 is asserted to stay: 9.0 us, 8.3 here
+            if (stages && steps <= 12) keep = 0.72;  // 256 x 2176 x 1536 is asserted to stay: 9.7 us, 8.2 here
         }
         // ... and in K shares, where their rule takes those (the sums of the shares pass through memory)
         const int64_t t = m <= 128 ? t128 : tiles(256, 192), fit = cus / t < steps / 8 ? cus / t : steps / 8, s = fit < 16 ? fit : 16;
         if (batch == 1 && steps >= 16 && s >= 2 && ((double)steps / s + 14.0) * (m <= 128 ? 128 * 128 / 0.7 : 256 * 192 / 0.95) < area) {
             other = 13.0 + (m <= 128 ? 0.45 : 0.9) * steps / s + (double)n * k / 5.5e6 + (double)s * m * n / 0.75e6;
-            // asserted to stay in shares: 64 x 9216 x 3072 in three (22 us, 18 here), 512 x 1024 x 8192 in eight (27 and 18)
+            // asserted to stay in shares: 64 x 9216 x 3072 in three (18 us, 14 here), 512 x 1024 x 8192 in eight (29 and 14)
             keep = s <= 3 || (m > 256 && steps >= 64) ? 0.65 : 0.92;
         }
         other *= keep;

@@ -623,7 +623,7 @@ int launch_gemm_i8(const GemmParams& p, int cfg, bool fold, int64_t batch, hipSt
 int launch_gemm_f8(const GemmParams& p, int cfg, bool fold, int64_t batch, hipStream_t st);
 int launch_gemm_w4(const GemmParams& p, int cfg, bool fold, int64_t batch, hipStream_t st);
 int choose_few(int64_t m, int64_t n, int64_t batch, int64_t k, int fmt, bool b4, bool grp, double other_us);
-// q: the quantise step whose codes the launch would read, to be done by the launch itself (few_quantises() says when), or null
+// q: the quantise step whose codes the launch would read, to be done by the launch itself (gemm_impl says when), or null
 int launch_gemm_few(const GemmParams& p, int fmt, bool b4, int cfg, int64_t batch, hipStream_t st, const segq_quant_desc* q);
 
 }  // namespace segq

@@ -181,7 +181,7 @@ def test_ragged_launch_takes_a_walk(ops, kind, M, N, K, tiles):
     _check(ops, kind, M, N, K, 0, torch.float32, g)
 
 
-def _check_dual(ops, kind, S, M, N, K, tile, dt, g, k0=0, pad=0, empty=None, per_row=True, per_col=True, add=False):
+def _check_dual(ops, kind, S, M, N, K, tile, dt, g, k0=0, pad=0, empty=None, per_row=True, per_col=True, add=False, lend=None):
     fa = FORMATS[kind][0]
     a, b = _codes(g, (S * M, k0 + K), fa), _codes(g, (S * N, k0 + K), fa)
     pick = g.random(a.shape) < 0.5
@@ -212,14 +212,18 @@ def _check_dual(ops, kind, S, M, N, K, tile, dt, g, k0=0, pad=0, empty=None, per
         want, mag = want + addend.double().cpu().numpy(), mag + addend.double().abs().cpu().numpy()
     kw = dict(batch=S, batch_stride_a=M * (k0 + K + pad), batch_stride_b=N * (k0 + K + pad), batch_stride_sx=sx[0].shape[1],
               batch_stride_sw=sw.shape[1]) if S > 1 else dict(addend=addend)
-    gd = ops.gemm_desc(ad, bd, rg, m=M, n=N, a_fmt=fa, b_fmt=fa, out_dtype=dt, lda=k0 + K + pad, ldb=k0 + K + pad, a_neg=nd, own_sums=1,
-                       bias=torch.from_numpy(bias).to(DEV), tile=tile, **kw)
-    took = ops.gemm_plan(gd)["tile"]
-    assert took == tile if tile else took in (29, 30)
-    got = ops.gemm_launch(gd).double().cpu().numpy().reshape(S, M, N)
+    gd = ops.gemm_desc(ad, bd, rg, m=M, n=N, a_fmt=fa, b_fmt=fa, out_dtype=dt, lda=k0 + K + pad, ldb=k0 + K + pad, a_neg=nd, own_sums=lend is None,
+                       finite_scales=lend is not None, bias=torch.from_numpy(bias).to(DEV), tile=tile, **kw)
+    ws = torch.empty(ops.gemm_workspace_bytes(gd), dtype=torch.uint8, device=DEV) if lend else None
+    plan = ops.gemm_plan(gd, ws)
+    took = plan["tile"]
+    assert took == tile if tile else lend is not None or took in (29, 30)
+    got = ops.gemm_launch(gd, ws).double().cpu().numpy().reshape(S, M, N)
     # per range an exact int32 sum, its conversion, two quotients and two products, then the addition of the two and of the bias
-    tol = (1e-6 if kind == "int8" else 3e-4 if K > 32 else 16 * 2.0 ** -15) * mag + {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8}[dt] * np.abs(want)
+    # (finite scales: sums carried from range to range by a ratio of two scales, or added in shares of K)
+    tol = (4e-6 if lend is not None and kind == "int8" else 1e-6 if kind == "int8" else 3e-4 if K > 32 else 16 * 2.0 ** -15) * mag + {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8}[dt] * np.abs(want)
     assert np.isfinite(got).all() and (np.abs(got - want) <= tol).all(), (kind, S, M, N, K, tile, dt, float((np.abs(got - want) - tol).max()))
+    return plan
 
 
 @pytest.mark.parametrize("kind", ["int8", "e4m3"])
@@ -233,6 +237,18 @@ def test_dual_ranges_in_one_walk(ops, kind, tile):
             _check_dual(ops, kind, 1, 70, 100, K, tile, torch.float32, g)
     for opt in (dict(empty=0), dict(empty=1), dict(per_row=False, per_col=False), dict(pad=32), dict(k0=16, pad=16), dict(add=True)):
         _check_dual(ops, kind, 1, 140, 210, 656, tile, torch.float32, g, **opt)
+
+
+@pytest.mark.parametrize("kind", ["int8", "e4m3"])
+def test_dual_ranges_with_finite_scales(ops, kind):
+    """Scales that are finite leave the way to the library: one walk, shares of K where room is lent for them, or in turn."""
+    g = np.random.default_rng(17)
+    took = {}
+    for M, N, K in ((300, 500, 1024), (400, 1024, 12288), (130, 640, 6144)):
+        for lend in (False, True):
+            plan = _check_dual(ops, kind, 1, M, N, K, 0, torch.bfloat16, g, lend=lend)
+            took[M, lend] = plan["tile"] in (29, 30), plan["splits"] > 1
+    assert took[300, False] == took[300, True] == took[400, False] == (True, False) and took[400, True] == (False, True)
 
 
 # ---- a linear of up to 16 rows in one launch ---------------------------------------------------------------------------------
