@@ -140,7 +140,10 @@ static Walk choose_ragged(int64_t m, int64_t n, int64_t batch, int64_t k, bool s
     auto rounds = [&](int cfg) { return (double)((tiles_of_cfg(cfg, m, n, batch) + cus - 1) / cus); };
     Walk w{FIRST_KT_CFG + 2, 4.2 + 0.72 * steps * rounds(FIRST_KT_CFG + 2)};
     const bool full = tiles_of_cfg(FIRST_KT_CFG + 1, m, n, batch) * 4 > cus * 3;
-    const double us192 = rounds(FIRST_KT_CFG + 1) * ((full ? 1.72 : 1.15) * steps + 9.0);
+    // (idle CUs, and at most two rounds of 128 x 128 tiles: 722 x 5554 x 2320 45 us on 256 x 192, 34 on 128 x 128 and 43 on the
+    // general kernel; 415 launches that go to 128 x 128 by this are 0.1 % from the best tile, 20 % with 1.15)
+    const bool two = tiles_of_cfg(FIRST_KT_CFG + 2, m, n, batch) <= 2 * cus;
+    const double us192 = rounds(FIRST_KT_CFG + 1) * ((full ? 1.72 : two ? 1.42 : 1.15) * steps + 9.0);
     if (us192 < w.us) w = Walk{FIRST_KT_CFG + 1, us192};
     const double us256 = rounds(FIRST_KT_CFG) * (2.0 * steps + 6.0);
     if (us256 < w.us) w = Walk{FIRST_KT_CFG, us256};

@@ -170,9 +170,9 @@ def test_ragged_end_of_k_scales_as_the_general_kernel(ops, tile, dt):
 
 @pytest.mark.parametrize("kind", ["int8", "e4m3"])
 @pytest.mark.parametrize("M,N,K,tiles", [(1300, 1500, 784, (26, 27, 28)), (2000, 2300, 1040, (26, 27, 28)), (748, 384, 208, (26, 27, 28)),
-                                         (748, 383, 208, (4,)), (869, 479, 160, (4,)), (2000, 2301, 1040, (26, 27, 28))])
+                                         (748, 383, 208, (4,)), (869, 479, 160, (4,)), (2000, 2301, 1040, (26, 27, 28)), (722, 5554, 2320, (28,)), (2100, 5550, 2320, (26, 27))])
 def test_ragged_launch_takes_a_walk(ops, kind, M, N, K, tiles):
-    """... unless K is short and the rows of the output start off the boundaries of whole stores."""
+    """... unless K is short and the rows of the output start off the boundaries of whole stores; on small tiles where they fill the CUs better."""
     g = np.random.default_rng(5)
     one = torch.ones(1, device=DEV)
     d = ops.gemm_desc(torch.empty(M, K, dtype=torch.uint8, device=DEV), torch.empty(N, K, dtype=torch.uint8, device=DEV), [ops.Range(0, K, one, one)],
