@@ -365,9 +365,9 @@ def linear(q, g, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     return out
 
 
-def linear_again(qd, gd, stream: int) -> None:
-    """``segq_linear`` on two descriptors that are complete, their workspace included; under the stream's lock."""
-    rc = L.lib().segq_linear(C.byref(qd), C.byref(gd), stream)
+def linear_again(q, g, stream: int) -> None:
+    """``segq_linear`` on two descriptors (by reference) that are complete, their workspace included; under the stream's lock."""
+    rc = L.lib().segq_linear(q, g, stream)
     if rc:
         L.check(rc)
 
@@ -473,20 +473,25 @@ def gemm_desc(a: torch.Tensor, b: torch.Tensor, ranges: Sequence[Range], *, m: i
         if group_dequant.dtype != torch.float32 or group_dequant.dim() != 2 or group_dequant.stride(1) != 1:
             raise RuntimeError("group_dequant is a float32 matrix (groups, n) with contiguous rows")
         d.group_dequant = group_dequant.data_ptr(); d.group_dequant_stride = group_dequant.stride(0)
+    k_alg = k_exec = 0
     for i, r in enumerate(ranges):
         kr = d.ranges[i]
         kr.k_begin = r.k_begin; kr.k_len = r.k_len; kr.a_sel = r.a_sel
         kr.sx_row_stride = r.sx_row_stride; kr.sw_col_stride = r.sw_col_stride
+        k_exec += r.k_len
+        if r.a_sel == 0 or r.a_sel == 2:
+            k_alg += r.k_len
         _need_cuda(r.sx, r.sw)
         for s in (r.sx, r.sw):
             if s is not None and s.dtype != torch.float32:
                 raise RuntimeError("scales must be float32")
         kr.sx = r.sx.data_ptr() if r.sx is not None else None
         kr.sw = r.sw.data_ptr() if r.sw is not None else None
-    d.ranges[0].own_sum = 1 if own_sums else 0
-    d.finite_scales = 1 if finite_scales else 0
-    info = dict(m=m, n=n, batch=batch, k_alg=sum(r.k_len for r in ranges if r.a_sel in (0, 2)),
-                k_exec=sum(r.k_len for r in ranges), a_fmt=a_fmt, b_fmt=b_fmt)
+    if own_sums:  # (a new descriptor is all zeros)
+        d.ranges[0].own_sum = 1
+    if finite_scales:
+        d.finite_scales = 1
+    info = dict(m=m, n=n, batch=batch, k_alg=k_alg, k_exec=k_exec, a_fmt=a_fmt, b_fmt=b_fmt)
     if oc is not None:
         out = (oc, oc_neg) if oc_neg is not None else oc
         info["codes_out"] = True

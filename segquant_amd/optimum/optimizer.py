@@ -17,6 +17,8 @@ algebra outside the kernel path and are not built.
 """
 from __future__ import annotations
 
+import ctypes as C
+
 import torch
 
 from .. import ops
@@ -595,12 +597,12 @@ class DefaultOptimizer(BaseOptimizer):
         if reuse is None or (stream and ops.capturing(stream)):
             return None
         out = torch.empty((*shape[:-1], hit["N"]), dtype=dtype, device=dev)
-        qd, gd, lock = reuse[0], reuse[1], reuse[4]
+        qd, gd, _, _, lock, q, g = reuse
         with lock:
             qd.x = x.data_ptr()
             qd.ldx = plan["K"]
             gd.out = out.data_ptr()
-            ops.linear_again(qd, gd, stream)
+            ops.linear_again(q, g, stream)
         return out
 
     def _relaunch(self, hit, x2, fresh=False):
@@ -620,7 +622,7 @@ class DefaultOptimizer(BaseOptimizer):
                 bufs.pop(next(iter(bufs)))  # streams come and go: keep the buffers of the last few
             reuse = bufs.get(stream)
             if reuse is not None:  # descriptors, codes and scales of the previous call on this stream
-                qd, gd, result, held, _ = reuse
+                qd, gd, result, held = reuse[:4]
                 qd.x = x2.data_ptr()
                 qd.ldx = ops.row_stride(x2)
                 gd.out = out.data_ptr()
@@ -656,6 +658,6 @@ class DefaultOptimizer(BaseOptimizer):
             for i, (which, s_) in enumerate(hit["sx_src"]):
                 gd.ranges[i].sx = base[which] + 4 * M * s_
         if stream is not None:
-            hit["buffers"][stream] = (qd, gd, result, held, ops.stream_lock[stream])
+            hit["buffers"][stream] = (qd, gd, result, held, ops.stream_lock[stream], C.byref(qd), C.byref(gd))
         keep = (x2, out, held)
         return (qd, result, hit["q"][1], keep), (gd, out, hit["g"][1], keep), ws
