@@ -167,6 +167,28 @@ static Walk choose_dual(int64_t m, int64_t n, int64_t batch, int64_t k) {
     return w;
 }
 
+// Group factors: us of rounds of the CUs x (steps x what a step takes + what a tile takes beside them), fitted to 14 shapes
+// (within 6 %).  Two workgroups of 128 x 128 share a CU; a last round of one per CU is quicker.  us with the int4 expansion,
+// 128 x 128 / 256 x 256 / 256 x 192 / 192 x 256:  8192 x 10240 x 1280 166 / 155 / 160 / 158;  8192 x 1280 x 5120 81 / 85 / 75 / 69;
+// 4096 x 12288 x 1536 117 / 108 / 117 / 128;  2048 x 10240 x 1280 50 / 59 / 53 / 53;  2048 x 1280 x 5120 37 / 83 / 70 / 65.
+// The big tiles have to be ahead by 3 %.  (256 x 128 and 128 x 256, by id: never the best by more than that.)
+static int choose_groups(int64_t m, int64_t n, int64_t steps, bool fold) {
+    if (fold) return FIRST_WIDE_CFG + 3;
+    const int64_t cus = device_cus(), t128 = tiles_of_cfg(FIRST_WIDE_CFG + 3, m, n, 1), rest = t128 % (2 * cus);
+    const double pair = 1.1 * steps + 4.5, alone = 0.78 * steps + 5.0;
+    double us = 0.97 * ((double)(t128 / (2 * cus)) * pair + (rest == 0 ? 0.0 : rest <= cus ? alone : pair));
+    int best = FIRST_WIDE_CFG + 3;
+    static const struct { int tile; double step, tail; } big[3] = {{0, 1.95, 10.0}, {6, 1.55, 8.0}, {7, 1.42, 7.5}};
+    for (const auto& b : big) {
+        const double t = (double)((tiles_of_cfg(FIRST_WIDE_CFG + b.tile, m, n, 1) + cus - 1) / cus) * (b.step * steps + b.tail);
+        if (t < us) {
+            us = t;
+            best = FIRST_WIDE_CFG + b.tile;
+        }
+    }
+    return best;
+}
+
 // Workgroups that could share the K steps of each of a launch's tiles (1: none).
 static int64_t k_shares(int64_t m, int64_t n, int64_t steps, int cfg) {
     const int64_t cus = device_cus(), t = tiles_of_cfg(cfg, m, n, 1);
@@ -544,10 +566,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     };
     if (d->tile == 0) {
         if (groups) {
-            // 128 x 128: at 126 registers two workgroups share a CU, and one's conversion (VALU) runs under
-            // the other's MFMAs; measured 8 % (8192 x 10240 x 1280) to 25 % (8192 x 1280 x 5120) ahead
-            // of 256 x 128 / 128 x 256, which are selectable by id
-            cfg = FIRST_WIDE_CFG + 3;
+            cfg = choose_groups(d->m, d->n, ktotal / 128, fold);
         } else {
             cfg = park ? choose_tile(d->m, d->n, d->batch, false, wide_ok, plain8) : -1;
             park = park && park_fits(cfg);
@@ -661,10 +680,10 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         // every 8-wave tile serves several ranges this way
     } else if (cfg >= FIRST_WIDE_CFG) {
         if (!wide_ok) return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: tile %d needs K ranges in multiples of 128", cfg + 1);
-        if (fold2 && cfg == FIRST_WIDE_CFG) cfg = FIRST_WIDE_CFG + 1;
-        if (groups && cfg == FIRST_WIDE_CFG) cfg = FIRST_WIDE_CFG + 1;
-        if (groups && cfg > FIRST_WIDE_CFG + 3)
-            return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: group factors run on tiles %d to %d", FIRST_WIDE_CFG + 2, FIRST_WIDE_CFG + 4);
+        if ((fold2 || (groups && fold)) && cfg == FIRST_WIDE_CFG) cfg = FIRST_WIDE_CFG + 1;
+        if (groups && cfg > FIRST_WIDE_CFG + 3 && (fold || (cfg != FIRST_WIDE_CFG + 6 && cfg != FIRST_WIDE_CFG + 7)))
+            return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: group factors run on tiles %d to %d, and with one range on %d and %d",
+                        FIRST_WIDE_CFG + 1, FIRST_WIDE_CFG + 4, FIRST_WIDE_CFG + 7, FIRST_WIDE_CFG + 8);
     } else if (groups) {
         return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: group factors run on tiles %d to %d", FIRST_WIDE_CFG + 2, FIRST_WIDE_CFG + 4);
     } else if (cfg >= FIRST_BIG_CFG) {

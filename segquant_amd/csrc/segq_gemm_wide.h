@@ -667,9 +667,17 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     // range, rescaled at range boundaries, scaled by 1/(sx sw) in the epilogue.
     // The group kernel runs the e4m3 schedule (whole-step fragments of 32 bytes,
     // refilled as the step lets go of them): both 64-byte K halves of an output
-    // block are multiplied back to back into a handful of int32 temporaries,
-    // which are converted at once, so no int32 accumulator set lives across
-    // steps and the 64 x 64 wave tile fits.
+    // block are multiplied back to back into int32 temporaries, so no int32
+    // accumulator set lives across steps.
+    // LAG (one range): a column block's temporaries wait while the next block is multiplied, and
+    // two of their values are converted and scaled behind every MFMA.  Bound by issue slots: an
+    // int8 MFMA holds the matrix pipe for 16 clocks and takes two of the four VALU slots in them, the
+    // four VALU instructions that belong to it the rest and more (25 to 27 clocks measured for an MFMA
+    // with four, 17 with two; v_cvt_f32_i32 and a subtraction cost the same).  Left to itself the compiler gathers
+    // a step's conversions at its end, behind the MFMAs of every wave, which two workgroups of 128 x 128
+    // per CU hide and one of a big tile does not: 8192 x 10240 x 1280 on 256 x 256 in LAG order 155 us with the
+    // int4 expansion, 128 x 128 165 to 167; 8192 x 1280 x 5120 on 192 x 256 69, 128 x 128 81 (256 x 128
+    // 100 in the compiler's order, 95 in this one).  With several ranges the big tiles spill: 128 x 128, converted at once.
     static_assert(!GRP || (!F8 && NS == 2), "group factors: int8, two stages");
     // int8 tiles above 256 x 256 run the whole-step schedule too: one set of 32-byte fragments
     // instead of two sets of 16-byte ones leaves room for their accumulators
@@ -1079,6 +1087,30 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     constexpr int RD_EVERY = (NMF >= 2 * NRD + 4) ? 2 : 1;
     constexpr int DM_EVERY = (NMF / NDM > 1) ? NMF / NDM : 1;
     static_assert(NRD * RD_EVERY <= NMF && NDM * DM_EVERY <= NMF, "more reads than MFMA slots");
+    // Group factors: int32 sums of a column block and, in LAG order, of the one before it, whose factors are gf
+    static_assert(!GRP || TN % 2 == 0, "group factors: two sets of temporaries in turn, also from one step to the next");
+    constexpr bool LAG = GRP && !FOLD;
+    v4i gt[2][GRP ? TM : 1];
+    v4f gf = v4f{0.f, 0.f, 0.f, 0.f};
+    if constexpr (GRP) {
+#pragma unroll
+        for (int b = 0; b < TM; ++b) gt[1][b] = acc_zero;
+    }
+    auto convert = [&](int a, int j) __attribute__((always_inline)) {  // piece j of 2 TM
+        if constexpr (GRP) {
+            const int b = j >> 1;
+#pragma unroll
+            for (int v = 2 * (j & 1); v < 2 * (j & 1) + 2; ++v) {
+                float t = __builtin_fmaf((float)gt[a & 1][b][v], gf[v], accf[a][b][v]);
+                if constexpr (LAG) asm volatile("" : "+v"(t));  // (keeps the conversion where it is written)
+                accf[a][b][v] = t;
+            }
+        }
+    };
+    auto convert_block = [&](int a) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 2 * TM; ++j) convert(a, j);
+    };
     // e4m3 schedule of one step.  On entry the activation fragments and weight
     // fragment 0 are in registers.  Column block a reads weight fragment a + 2
     // (block 0 also fragment 1), so after block TN - 3 every read of this step is
@@ -1091,30 +1123,30 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         constexpr bool MORE_ = decltype(more_c)::value;
         constexpr int NDM8 = A_IT + B_IT, TAIL = 2 * TM;  // DMA instructions over the tail's MFMAs
         const int nbuf = buf ^ 1;
-        // group mode: an output block is both K halves of the step into an int32 temporary
-        // (first MFMA with a zero C operand), converted and scaled by this step's factors at once
         auto lo4 = [](const v8i& f) __attribute__((always_inline)) { return v4i{f[0], f[1], f[2], f[3]}; };
         auto hi4 = [](const v8i& f) __attribute__((always_inline)) { return v4i{f[4], f[5], f[6], f[7]}; };
         const float* const gsrc = grw + cslot * BN + wn * WN + 4 * lgrp;
 #pragma unroll
         for (int a = 0; a < TN - 2; ++a) {
             if constexpr (GRP) {
-                v4i t[TM];
-                const v4f g = *reinterpret_cast<const v4f*>(gsrc + a * 16);
+                v4f g;
 #pragma unroll
                 for (int b = 0; b < TM; ++b) {
                     if (b == 0 && a == 0) frag8(buf, TM + 1);
                     if (b == (TM > 1 ? 1 : 0)) frag8(buf, TM + a + 2);
-                    t[b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo4(fb8[a]), lo4(fa8[b]), acc_zero, 0, 0, 0);
+                    gt[a & 1][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo4(fb8[a]), lo4(fa8[b]), acc_zero, 0, 0, 0);
+                    if constexpr (LAG) convert((a + TN - 1) % TN, b);
                     __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
                 for (int b = 0; b < TM; ++b) {
-                    t[b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi4(fb8[a]), hi4(fa8[b]), t[b], 0, 0, 0);
+                    gt[a & 1][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi4(fb8[a]), hi4(fa8[b]), gt[a & 1][b], 0, 0, 0);
+                    if constexpr (LAG) convert((a + TN - 1) % TN, TM + b);
+                    if (b == 0) g = *reinterpret_cast<const v4f*>(gsrc + a * 16);
                     __builtin_amdgcn_sched_barrier(0);
                 }
-#pragma unroll
-                for (int b = 0; b < TM; ++b) accf[a][b] += __builtin_convertvector(t[b], v4f) * g;
+                gf = g;
+                if constexpr (!LAG) convert_block(a);
             } else if constexpr (WS) {
                 // int8: the two 64-byte K halves of a block, TM MFMAs apart
 #pragma unroll
@@ -1148,11 +1180,12 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
 #pragma unroll
         for (int a = TN - 2; a < TN; ++a) {
             if constexpr (GRP) {
-                v4i t[TM];
-                const v4f g = *reinterpret_cast<const v4f*>(gsrc + a * 16);
+                v4f g;
 #pragma unroll
                 for (int b = 0; b < TM; ++b) {
-                    t[b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo4(fb8[a]), lo4(fa8[b]), acc_zero, 0, 0, 0);
+                    gt[a & 1][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo4(fb8[a]), lo4(fa8[b]), acc_zero, 0, 0, 0);
+                    if (LAG && !(a == TN - 1 && MORE_)) convert(a - 1, b);
+                    if (b == TM - 1) g = *reinterpret_cast<const v4f*>(gsrc + a * 16);
                     const int j = (a - (TN - 2)) * TM + b;
                     if constexpr (DMA_) {
 #pragma unroll
@@ -1163,15 +1196,20 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
                 }
 #pragma unroll
                 for (int b = 0; b < TM; ++b) {
-                    t[b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi4(fb8[a]), hi4(fa8[b]), t[b], 0, 0, 0);
+                    gt[a & 1][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi4(fb8[a]), hi4(fa8[b]), gt[a & 1][b], 0, 0, 0);
+                    if (LAG && !(a == TN - 1 && MORE_)) convert(a - 1, TM + b);
                     if constexpr (MORE_) {
                         if (a == TN - 2 && b == 0) frag8(nbuf, TM);  // next weight fragment 0: free since block 0
                         if (a == TN - 1) frag8(nbuf, b);              // next activation fragment b: this was its last reader
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
-#pragma unroll
-                for (int b = 0; b < TM; ++b) accf[a][b] += __builtin_convertvector(t[b], v4f) * g;
+                if (LAG && a == TN - 1 && MORE_) {  // under the next step's first fragment reads
+                    convert_block(a - 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                gf = g;
+                if constexpr (!LAG) convert_block(a);
             } else if constexpr (WS) {
 #pragma unroll
                 for (int b = 0; b < TM; ++b) {
@@ -1310,6 +1348,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     for (; s + NS < steps; ++s) step(std::true_type{}, std::true_type{});
     for (; s + 1 < steps; ++s) step(std::false_type{}, std::true_type{});
     if (s < steps) step(std::false_type{}, std::false_type{});
+    if constexpr (LAG) convert_block(TN - 1);
     if constexpr (ACCF) {
         if (dirty) fold(cr);
     }
@@ -1474,7 +1513,10 @@ int launch_wide(const GemmParams& p, int wcfg, bool fold, bool asel, int64_t bat
         if (p.grw) {  // group-wise factors (the host has checked: plain codes, K ranges in whole steps)
             if (asel || tail) return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: group factors need plain codes, and serve no low-rank branch");
             switch (wcfg) {
-                case 0: case 1:
+                case 0:
+                    if (!fold) return launch_pipe_instance<256, 256, 4, 2, FMT, false, 2, true>(p, batch, st);
+                    break;
+                case 1:
                     return fold ? launch_pipe_instance<256, 128, 4, 2, FMT, true, 2, true>(p, batch, st)
                                 : launch_pipe_instance<256, 128, 4, 2, FMT, false, 2, true>(p, batch, st);
                 case 2:
@@ -1483,8 +1525,15 @@ int launch_wide(const GemmParams& p, int wcfg, bool fold, bool asel, int64_t bat
                 case 3:
                     return fold ? launch_pipe_instance<128, 128, 4, 2, FMT, true, 2, true>(p, batch, st)
                                 : launch_pipe_instance<128, 128, 4, 2, FMT, false, 2, true>(p, batch, st);
+                case 6:
+                    if (!fold) return launch_pipe_instance<256, 192, 4, 2, FMT, false, 2, true>(p, batch, st);
+                    break;
+                case 7:
+                    if (!fold) return launch_pipe_instance<192, 256, 2, 4, FMT, false, 2, true>(p, batch, st);
+                    break;
             }
-            return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: group factors run on the 256x128, 128x256 and 128x128 tiles of eight waves");
+            return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: group factors run on the 256x128, 128x256 and 128x128 tiles of eight waves, and with one range on "
+                                              "256x256, 256x192 and 192x256");
         }
     }
 // a tile that exists with and without the tail / without only

@@ -704,6 +704,32 @@ def test_gemm_addend(ops, fmt, dt):
                  addend=add[0].contiguous().to(DEV))
 
 
+@pytest.mark.parametrize("M,N,K,tile", [(1, 4, 128, 11), (257, 260, 128, 18), (300, 500, 256, 11), (256, 192, 384, 17), (193, 513, 640, 18),
+                                        (511, 190, 1280, 17), (700, 514, 1280, 11), (8192, 1280, 384, 0), (8192, 10240, 1280, 0)])
+def test_group_factors_on_the_big_tiles(ops, M, N, K, tile):
+    """One range with group factors on 256 x 256, 256 x 192 and 192 x 256: every output is the same sum in the same order as on
+    128 x 128, so the same bits; and within the fp32 sums' rounding of the closed form.  tile 0: launches that the rule sends there."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a, w = _rand_codes((M, K), O.FMT_INT8, 5), _rand_codes((N, K), O.FMT_INT8, 6)
+    ad, wd = _to_dev_codes(a, O.FMT_INT8), _to_dev_codes(w, O.FMT_INT8)
+    sx, fac = torch.rand(M, generator=g) + 0.5, torch.rand(K // 128, N, generator=g) + 0.5
+    bias = torch.randn(N, generator=g)
+    rg = [ops.Range(0, K, sx.to(DEV), torch.ones(1, device=DEV), 0, 1, 0)]
+    kw = dict(m=M, n=N, a_fmt=O.FMT_INT8, b_fmt=O.FMT_INT8, lda=K, ldb=K, bias=bias.to(DEV), group_dequant=fac.to(DEV))
+    if tile == 0:
+        assert ops.gemm_plan(ops.gemm_desc(ad, wd, rg, out_dtype=torch.bfloat16, **kw))["tile"] in (11, 17, 18)
+    for dt in (torch.float32, torch.bfloat16):
+        out = ops.gemm(ad, wd, rg, out_dtype=dt, tile=tile, **kw)
+        assert torch.equal(out, ops.gemm(ad, wd, rg, out_dtype=dt, tile=14, **kw))
+        if M < 1000 and dt == torch.float32:
+            groups = [(a[:, k:k + 128].astype(np.int64) @ w[:, k:k + 128].astype(np.int64).T) * fac[k // 128].numpy().astype(np.float64)[None]
+                      for k in range(0, K, 128)]
+            want = sum(groups) / sx.numpy().astype(np.float64)[:, None] + bias.numpy()
+            # one rounding per group and three in the scaling, each 2^-24 of the largest partial sum, and the reciprocal's ulp
+            most = np.abs(np.cumsum(groups, axis=0)).max() / sx.min().item()
+            assert np.abs(_np(out).astype(np.float64) - want).max() <= (len(groups) + 5) * 2.0 ** -24 * most
+
+
 @pytest.mark.parametrize("fmt_w", [O.FMT_INT4, O.FMT_INT8])
 @pytest.mark.parametrize("dt", ["fp32", "bf16"])
 def test_group_wise_weight_scales(ops, fmt_w, dt):
