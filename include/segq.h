@@ -319,8 +319,9 @@ typedef struct segq_gemm_desc {
     const float* out_scale_neg; /* device or NULL */
     int32_t out_code_fmt;   /* SEGQ_CODE_I8 | SEGQ_CODE_E4M3 */
     int32_t finite_scales;  /* 0, or non-zero: the scales of all ranges are finite, and without own_sum the library
-                         * takes the faster way to sum them (two ranges over the same run of K, a and then a_neg,
-                         * can be multiplied in one walk of it, each with its own sums) */
+                         * takes the faster way to sum them (two ranges over the same run of K, one from a and one
+                         * from a_neg, can be multiplied in one walk of it, each with its own sums, and one more
+                         * range from a behind them; neither is parked) */
     segq_krange ranges[SEGQ_MAX_RANGES];
 } segq_gemm_desc;
 

@@ -234,6 +234,42 @@ static double quantise_in_gemm_us(const segq_quant_desc* q, int64_t tiles) {
     return rounds * (q->dynamic ? 0.9 : 0.1) + k * (rounds * (0.83 + (second ? 0.36 : 0.0) + (f32 ? second ? 0.44 : 0.12 : 0.0)) - 0.55);
 }
 
+struct MixPick {
+    int cfg, shares;
+    double us;
+};
+
+// Workspace of a launch in K shares on one of the MIX tiles: two tile-sized shares and a word per tile, or the partial results.
+static int64_t mix_bytes(int64_t m, int64_t n, int cfg, int shares) {
+    const int64_t tiles = tiles_of_cfg(cfg, m, n, 1);
+    if (shares == 2) return tiles * 2 * TILE_CFGS[cfg].bm * TILE_CFGS[cfg].bn * 4 + ((tiles * 4 + 255) & ~(int64_t)255);
+    return (shares * m * n * 4 + 255) & ~(int64_t)255;
+}
+
+// Tile and K shares of a DualScale pair and the plain range beside it (or none): us of rounds of the CUs, each so much per step,
+// the last one less the emptier it is, a launch of one round an eighth quicker (the clock), and what shares cost.  Fitted to 50
+// shapes: within 5 % of the best of three tiles and up to 12 shares on 45 of them, 12 % at most.  us, ranges in turn before / this,
+// int8 | e4m3:  9216 x 3072 x (3072 + 12288) 745 / 601 | 643 / 574;  4608 361 / 316 | 299 / 296;  2048 187 / 131 | 153 / 123;
+// 1024 119 / 79 | 82 / 74;  300 57 / 45 | 43 / 43;  4012 x 1536 x (1536 + 6144) 118 / 70 | 79 / 65;  366 42 / 27 | 31 / 27
+static MixPick choose_mix(int64_t m, int64_t n, int64_t steps, int64_t plain, int max_shares) {
+    static const struct { double full, few, tail; } fit[3] = {{1.80, 1.29, 7.0}, {1.57, 1.20, 7.0}, {1.25, 0.93, 6.5}};
+    const int64_t cus = device_cus();
+    const double e = (double)steps + 0.6 * (double)plain;
+    MixPick best{-1, 1, 1e30};
+    for (int i = 0; i < 3; ++i) {
+        const int64_t tiles = tiles_of_cfg(FIRST_MIX_CFG + i, m, n, 1);
+        for (int sh = 1; sh <= max_shares && (sh == 1 || (tiles * sh <= cus && e >= 8.0 * sh)); ++sh) {
+            const double full = (tiles * sh <= cus ? 0.92 : 1.0) * (fit[i].full * e / sh + fit[i].tail), few = fit[i].few * e / sh + fit[i].tail;
+            const double rest = (double)(tiles * sh % cus) / (double)cus;
+            double us = (double)(tiles * sh / cus) * full + (rest > 0.0 ? few + rest * rest * (full - few) : 0.0);
+            if (sh == 2) us += i == 2 ? 5.0 : 9.0;
+            else if (sh > 2) us += 4.0 + (double)m * n * sh / 0.8e6;
+            if (us < best.us) best = MixPick{FIRST_MIX_CFG + i, sh, us};
+        }
+    }
+    return best;
+}
+
 // int4 weight rows (two values per byte, even k in the low nibble) -> int8 rows.
 // One thread expands 16 packed bytes to 32 values.
 __global__ void __launch_bounds__(256) expand_i4_kernel(const uint8_t* src, int64_t ld_src, uint8_t* dst, int64_t ld_dst,
@@ -408,11 +444,11 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         const bool base = (i8 || f8) && !lowrank && !codes_out && !groups && d->split_k <= 1 && d->m * d->lda < (int64_t)1 << 32 && d->n * d->ldb < (int64_t)1 << 32;
         const bool one = base && d->n_ranges == 1 && r.a_sel < 2;
         const bool two = base && d->n_ranges == 2 && r.k_begin == s.k_begin && r.k_len == s.k_len && r.a_sel == 0 && s.a_sel == 1;
-        if (d->tile > FIRST_KT_CFG && d->tile <= NUM_TILE_CFG) {
+        if (d->tile > FIRST_KT_CFG && d->tile <= FIRST_MIX_CFG) {
             if (!(d->tile > FIRST_DUAL_CFG ? two : one))
                 return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: tiles %d to %d serve one range, tiles %d to %d two over the same run of K from a and a_neg, in plain "
                                                   "8-bit codes, without group factors, a low-rank branch, codes out or split_k",
-                            FIRST_KT_CFG + 1, FIRST_DUAL_CFG, FIRST_DUAL_CFG + 1, NUM_TILE_CFG);
+                            FIRST_KT_CFG + 1, FIRST_DUAL_CFG, FIRST_DUAL_CFG + 1, FIRST_MIX_CFG);
             walk.cfg = (int)d->tile - 1;
         } else if (d->tile == 0 && d->out_dtype != SEGQ_ACC) {
             if (one && r.k_len % 128) walk = choose_ragged(d->m, d->n, d->batch, r.k_len, osz == 4 && !vec_store);
@@ -425,6 +461,64 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
                 } else if (in_turn && lent && k_shares(d->m, d->n, steps, FIRST_WIDE_CFG + 6) > 2) {
                     walk.cfg = -1;  // a workspace lent to ranges summed on their own is lent for K shares
                 }
+            }
+        }
+    }
+    // ... or a DualScale pair with one plain range beside it (at any place), in whole steps
+    struct { int cfg = -1, shares = 1, pos = 0, neg = 1, plain = -1; } mix;
+    if (d->n_ranges == 2 || d->n_ranges == 3) {
+        bool ok = (i8 || f8) && !lowrank && !codes_out && !groups && d->batch == 1 && d->out_dtype != SEGQ_ACC &&
+                  d->m * d->lda < (int64_t)1 << 32 && d->n * d->ldb < (int64_t)1 << 32;
+        mix.neg = -1;
+        for (int i = 0; i < d->n_ranges; ++i) {
+            const segq_krange& r = d->ranges[i];
+            ok = ok && r.a_sel < 2 && r.k_begin % 128 == 0 && r.k_len % 128 == 0;
+            if (r.a_sel == 1) {
+                ok = ok && mix.neg < 0;
+                mix.neg = i;
+            }
+        }
+        mix.pos = -1;
+        for (int i = 0; ok && mix.neg >= 0 && i < d->n_ranges; ++i) {
+            const segq_krange &r = d->ranges[i], &s = d->ranges[mix.neg];
+            if (i == mix.neg) continue;
+            if (mix.pos < 0 && r.k_begin == s.k_begin && r.k_len == s.k_len) mix.pos = i;
+            else mix.plain = i;
+        }
+        ok = ok && mix.neg >= 0 && mix.pos >= 0;
+        const bool lent = ws && al(ws, 16);
+        auto shares_fit = [&](int c, int n_) { return lent && ws_bytes >= mix_bytes(d->m, d->n, c, n_); };
+        const int64_t steps = ok ? d->ranges[mix.neg].k_len / 128 : 0, plain = ok && mix.plain >= 0 ? d->ranges[mix.plain].k_len / 128 : 0;
+        if (d->tile > FIRST_MIX_CFG && d->tile <= NUM_TILE_CFG) {
+            if (!ok)
+                return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: tiles %d to %d serve two ranges over the same run of K from a and a_neg, and one plain range "
+                                                  "beside them, in plain 8-bit codes and whole steps of 128, one problem, without group factors, a low-rank "
+                                                  "branch or codes out", FIRST_MIX_CFG + 1, NUM_TILE_CFG);
+            mix.cfg = (int)d->tile - 1;
+            if (d->split_k > 1) {
+                mix.shares = (int)(d->split_k < steps + plain / 2 ? d->split_k : steps + plain / 2);  // (a step at least for each)
+                if (mix.shares > 1 && !shares_fit(mix.cfg, mix.shares)) return fail(SEGQ_ERR_ARG, "segq_gemm: workspace too small for split_k");
+            }
+        } else if (ok && d->tile == 0 && d->finite_scales && !d->ranges[0].own_sum && d->split_k <= 1 && (mix.plain >= 0 || steps > 4)) {
+            const bool share = lent && d->split_k != 1;
+            MixPick pick = choose_mix(d->m, d->n, steps, plain, share ? 16 : 1);
+            while (pick.shares > 1 && !shares_fit(pick.cfg, pick.shares)) pick = choose_mix(d->m, d->n, steps, plain, pick.shares - 1);
+            // Up to 128 rows the shares of a 128 x 128 tile are ahead: 32 x 1536 x (1536 + 6144) e4m3 18.7 us, here 23.4; 128 rows
+            // 22.0 and 25.1, int8 27.0 and 25.4.
+            bool take = d->m > 128 || !share || steps + plain < 32;
+            // The pair alone: against one walk of tiles 29 and 30, or the ranges in turn.  us, that / this: 2500 x 3072 x 12288 161 / 143,
+            // 600 x 2048 x 8192 44 / 34, 4608 x 3072 x 12288 int8 310 / 266; 4096 x 1536 x 6144 57 / 60, 2600 x 1152 x 4608 30 / 34.
+            if (mix.plain < 0) {
+                const double cus = device_cus(), t64 = (double)tiles_of_cfg(FIRST_DUAL_CFG + 1, d->m, d->n, 1) / cus, k = (double)steps;
+                const double now = walk.cfg < 0 ? in_turn_us(d->m, d->n, 2 * steps, f8, share)
+                                   : walk.cfg == FIRST_DUAL_CFG ? std::ceil((double)tiles_of_cfg(FIRST_DUAL_CFG, d->m, d->n, 1) / cus) * (1.1 * k + 5.0)
+                                   : t64 <= 1.0 ? 4.8 + 0.6 * k : 4.0 + t64 * (0.44 * k + 0.8);
+                take = take && pick.us < 0.95 * now;
+            }
+            if (take) {
+                walk.cfg = -1;
+                mix.cfg = pick.cfg;
+                mix.shares = pick.shares;
             }
         }
     }
@@ -524,6 +618,42 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         }
         return launch_gemm_few(p, f8 ? GEMM_F8 : GEMM_I8, w4, few, d->batch, st, q);
     }
+    // K shares in d's workspace: two that meet in the launch, or any number that a second kernel sums
+    auto launch_met = [&](int cfg, bool fold) -> int {
+        const TileCfg& c = TILE_CFGS[cfg];
+        p.splits = 2;
+        p.part = static_cast<float*>(d->workspace);
+        const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
+        p.arrived = reinterpret_cast<unsigned int*>(static_cast<uint8_t*>(d->workspace) + tiles * 2 * c.bm * c.bn * 4);
+        p.bsA = p.bsB = p.bsC = p.bsSx = p.bsSw = 0;  // blockIdx.y counts shares here, not problems
+        static unsigned int g_stamp = 0x5e690000u;
+        if (!p.dry) do p.stamp = __atomic_add_fetch(&g_stamp, 1u, __ATOMIC_RELAXED); while (p.stamp == 0u);  // 0 means "cleared"
+        return i8 ? launch_gemm_i8(p, cfg, fold, 2, st) : launch_gemm_f8(p, cfg, fold, 2, st);
+    };
+    auto launch_shares = [&](int cfg, bool fold, int splits) -> int {
+        p.splits = splits;
+        p.C = d->workspace;
+        p.ldc = d->n;
+        p.bsC = d->m * d->n;
+        p.bsA = p.bsB = p.bsSx = p.bsSw = 0;
+        p.out_dtype = SEGQ_F32;
+        p.bias = nullptr;
+        p.addend = nullptr;
+        p.vec_store = d->n % 4 == 0;
+        p.vec_store16 = 0;
+        const int rc = i8 ? launch_gemm_i8(p, cfg, fold, splits, st) : launch_gemm_f8(p, cfg, fold, splits, st);
+        if (rc != SEGQ_OK || p.dry) return rc;
+        const bool vec = d->n % 4 == 0 && d->ldo % 4 == 0 && al(d->out, 16);
+        const int64_t items = d->m * (vec ? d->n / 4 : d->n);
+        const dim3 grid((unsigned)((items + 255) / 256));
+        if (vec)
+            hipLaunchKernelGGL(splitk_reduce_kernel<true>, grid, dim3(256), 0, st, static_cast<const float*>(d->workspace), splits,
+                               d->m, d->n, d->bias, d->bias_dtype, d->out, d->out_dtype, d->ldo, d->addend, d->ld_addend);
+        else
+            hipLaunchKernelGGL(splitk_reduce_kernel<false>, grid, dim3(256), 0, st, static_cast<const float*>(d->workspace), splits,
+                               d->m, d->n, d->bias, d->bias_dtype, d->out, d->out_dtype, d->ldo, d->addend, d->ld_addend);
+        return check_launch("segq_gemm (split-K sum)");
+    };
     if (walk.cfg >= 0) {
         const TileCfg& c = TILE_CFGS[walk.cfg];
         const int64_t tm = (d->m + c.bm - 1) / c.bm, tn = (d->n + c.bn - 1) / c.bn;
@@ -536,6 +666,27 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
             p.dry = 1;
         }
         return i8 ? launch_gemm_i8(p, walk.cfg, false, d->batch, st) : launch_gemm_f8(p, walk.cfg, false, d->batch, st);
+    }
+    if (mix.cfg >= 0) {
+        const TileCfg& c = TILE_CFGS[mix.cfg];
+        p.tiles_m = (int32_t)((d->m + c.bm - 1) / c.bm);
+        p.tiles_n = (int32_t)((d->n + c.bn - 1) / c.bn);
+        if ((int64_t)p.tiles_m * p.tiles_n > 0x7fffffff) return fail(SEGQ_ERR_ARG, "segq_gemm: grid too large");
+        p.group_m = 8;
+        // the pair first, positive codes in front, then the plain range
+        const KRange pos = p.r[mix.pos], neg = p.r[mix.neg], plain = p.r[mix.plain >= 0 ? mix.plain : 0];
+        p.r[0] = pos;
+        p.r[1] = neg;
+        p.r[2] = plain;
+        if (plan) {
+            plan->bytes = mix.shares > 1 ? mix_bytes(d->m, d->n, mix.cfg, mix.shares) : 0;
+            plan->tile = mix.cfg + 1;
+            plan->splits = mix.shares;
+            p.dry = 1;
+        }
+        if (mix.shares == 2) return launch_met(mix.cfg, false);
+        if (mix.shares > 2) return launch_shares(mix.cfg, false, mix.shares);
+        return i8 ? launch_gemm_i8(p, mix.cfg, false, 1, st) : launch_gemm_f8(p, mix.cfg, false, 1, st);
     }
     const bool fold = d->n_ranges > 1;
     bool wide_ok = d->m * d->lda < (int64_t)1 << 32 && d->n * d->ldb < (int64_t)1 << 32;
@@ -743,40 +894,8 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         p.rot = (d->n_ranges > 1 && splits == 1 && f8 && !p.sep) ? 1 : 0;
     }
     if ((int64_t)p.tiles_m * p.tiles_n > 0x7fffffff || d->batch > 65535) return fail(SEGQ_ERR_ARG, "segq_gemm: grid too large");
-    if (meet(splits, cfg)) {
-        p.splits = 2;
-        p.part = static_cast<float*>(d->workspace);
-        const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
-        p.arrived = reinterpret_cast<unsigned int*>(static_cast<uint8_t*>(d->workspace) + tiles * 2 * c.bm * c.bn * 4);
-        p.bsA = p.bsB = p.bsC = p.bsSx = p.bsSw = 0;  // blockIdx.y counts shares here, not problems
-        static unsigned int g_stamp = 0x5e690000u;
-        if (!p.dry) do p.stamp = __atomic_add_fetch(&g_stamp, 1u, __ATOMIC_RELAXED); while (p.stamp == 0u);  // 0 means "cleared"
-        return i8 ? launch_gemm_i8(p, cfg, fold, 2, st) : launch_gemm_f8(p, cfg, fold, 2, st);
-    }
-    if (splits > 1) {
-        p.splits = splits;
-        p.C = d->workspace;
-        p.ldc = d->n;
-        p.bsC = d->m * d->n;
-        p.bsA = p.bsB = p.bsSx = p.bsSw = 0;
-        p.out_dtype = SEGQ_F32;
-        p.bias = nullptr;
-        p.addend = nullptr;
-        p.vec_store = d->n % 4 == 0;
-        p.vec_store16 = 0;
-        const int rc = i8 ? launch_gemm_i8(p, cfg, fold, splits, st) : launch_gemm_f8(p, cfg, fold, splits, st);
-        if (rc != SEGQ_OK || p.dry) return rc;
-        const bool vec = d->n % 4 == 0 && d->ldo % 4 == 0 && al(d->out, 16);
-        const int64_t items = d->m * (vec ? d->n / 4 : d->n);
-        const dim3 grid((unsigned)((items + 255) / 256));
-        if (vec)
-            hipLaunchKernelGGL(splitk_reduce_kernel<true>, grid, dim3(256), 0, st, static_cast<const float*>(d->workspace), splits,
-                               d->m, d->n, d->bias, d->bias_dtype, d->out, d->out_dtype, d->ldo, d->addend, d->ld_addend);
-        else
-            hipLaunchKernelGGL(splitk_reduce_kernel<false>, grid, dim3(256), 0, st, static_cast<const float*>(d->workspace), splits,
-                               d->m, d->n, d->bias, d->bias_dtype, d->out, d->out_dtype, d->ldo, d->addend, d->ld_addend);
-        return check_launch("segq_gemm (split-K sum)");
-    }
+    if (meet(splits, cfg)) return launch_met(cfg, fold);
+    if (splits > 1) return launch_shares(cfg, fold, splits);
     if (i8) return launch_gemm_i8(p, cfg, fold, d->batch, st);
     if (f8) return launch_gemm_f8(p, cfg, fold, d->batch, st);
     return launch_gemm_w4(p, cfg, fold, d->batch, st);

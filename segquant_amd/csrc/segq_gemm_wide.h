@@ -599,6 +599,52 @@ __device__ __forceinline__ void lowrank_accumulate(const GemmParams& p, v4f (&of
     }
 }
 
+// s_waitcnt immediate for "vmcnt(n) lgkmcnt(0)" on gfx9-family encodings
+constexpr int waitcnt_vm_lgkm0(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
+
+// Two workgroups share a tile.  Each leaves its share (of, in output units) in the workspace and counts itself in; the one that
+// finds the other counted adds that share to its own (a + b = b + a: the result does not depend on who came last) and
+// finishes the tile: true.  The two can sit on different XCDs, whose L2 caches do not see each other's lines, so the
+// shares are written through and read past the caches (agent scope: what the compiler emits for a relaxed agent-scope
+// atomic, but 16 bytes per lane: 1 KB contiguous per wave and instruction).  flag: a word of LDS that is read no more.
+// CH: blocks whose loads are in flight at once (registers: the sums are still live).
+template <int NT, int CH, int TN, int TM>
+__device__ __forceinline__ bool meet_share(const GemmParams& p, v4f (&of)[TN][TM], int tile_id, int my, int tid, int* flag) {
+    using v4u = __attribute__((ext_vector_type(4))) unsigned int;
+    constexpr int AGENT = 16;  // the cache-policy bit for agent scope
+    constexpr int SHARE = TN * TM * NT * 16;
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<uint8_t*>(p.part) + (int64_t)tile_id * 2 * SHARE, 0, 2 * SHARE, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < TN * TM; ++i)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, of[i / TM][i % TM]), rs, tid * 16, my * SHARE + i * NT * 16, AGENT);
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));  // this wave's stores have reached memory
+    __syncthreads();                                  // ... and so have the other waves'
+    if (tid == 0) {
+        // the launch's own stamp instead of a count: whatever the word held before (an earlier
+        // launch's stamp, or anything at all in a fresh workspace) reads as "nobody yet"
+        const unsigned before = __hip_atomic_exchange(p.arrived + tile_id, p.stamp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *flag = before == p.stamp;
+        // the second one clears the word: a replay of this very launch (a captured graph keeps
+        // the stamp it was recorded with) must find "nobody yet" again
+        if (before == p.stamp) __hip_atomic_store(p.arrived + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!*flag) return false;
+#pragma unroll
+    for (int c0 = 0; c0 < TN * TM; c0 += CH) {
+        v4u other[CH];
+#pragma unroll
+        for (int i = 0; i < CH; ++i)
+            if (c0 + i < TN * TM)
+                other[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, tid * 16, (1 - my) * SHARE + (c0 + i) * NT * 16, AGENT);
+#pragma unroll
+        for (int i = 0; i < CH; ++i)
+            if (c0 + i < TN * TM) of[(c0 + i) / TM][(c0 + i) % TM] += __builtin_bit_cast(v4f, other[i]);
+    }
+    return true;
+}
+
 // Software-pipelined variant for plain int8 operands (both straight to LDS) with
 // NS LDS stages.  Two stages are what is instantiated: on FLUX shapes three and
 // four stages measured slower (they cost a co-resident workgroup or buy nothing,
@@ -614,8 +660,6 @@ __device__ __forceinline__ void lowrank_accumulate(const GemmParams& p, v4f (&of
 //   wait own DMA and LDS reads, barrier
 //
 // so fragment reads never stand between an MFMA group and the one before it.
-// s_waitcnt immediate for "vmcnt(n) lgkmcnt(0)" on gfx9-family encodings
-constexpr int waitcnt_vm_lgkm0(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
 
 // 1 / x for the second register set of int8 ranges: v_rcp_f32 (1 ulp) and one Newton step, with which the sums lie as
 // close to the exact ones as with correctly rounded quotients, which the general kernel takes for the same launches when
@@ -635,15 +679,23 @@ template <int BM, int BN, int WGM, int WGN, int FMT, bool FOLD, int NS, bool GRP
           bool CODES = false,  // CODES: the epilogue writes the next linear's codes instead of floats (one range)
           bool SEP = false,    // SEP (e4m3, several ranges): a second register set, as int8 has it, instead of rescaling in place
           bool KT = false,     // KT: K ends anywhere in sixteens (one walk of K)
-          bool DUAL = false>   // DUAL: two ranges over one run of K, from the two code tensors, in one walk
+          bool DUAL = false,   // DUAL: two ranges over one run of K, from the two code tensors, in one walk
+          bool MIX = false>    // MIX (DUAL): whole steps of K, behind them those of a plain range, K shares
 __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmParams p) {
     static_assert(!CODES || (!FOLD && !GRP && !PARK && !FINISH), "codes out: plain operands, one range");
     static_assert(!KT || (!FOLD && !GRP && !PARK && !FINISH && !CODES && NS == 2), "a ragged end of K: one walk, two stages");
-    static_assert(!DUAL || KT, "DUAL instances take any K");
+    static_assert(!DUAL || KT != MIX, "DUAL instances take any K, or whole steps of it and a plain range");
+    static_assert(!MIX || (DUAL && !FOLD && !GRP && !PARK && !FINISH && !CODES && NS == 2), "MIX: one walk, two stages");
     // DUAL (DualScale's two ranges over the same K and the same weights): the tile's BM rows of LDS are BM / 2 rows of each
     // code tensor, the two halves of every wave's row blocks, so that a wave holds both sums of an output and a weight
     // tile is read once for both.  What two ranges in turn need a second register set for, these have as the second
     // half of their blocks, and each sum is scaled by its own range's scales at the end.
+    // MIX (an input segment in front of a DualScale one: attention output | GELU'd MLP state): the plain range is walked
+    // behind the two.  There the sums of both signs become one fp32 sum in output units, in the registers of the first, and
+    // the second's start again from zero with the plain range, whose rows take the second half of the tile's: half the MFMAs
+    // and fragment reads per step, two thirds of the DMA.  Three sums in two register sets: nothing is parked, no
+    // third set, no ratio of scales, weights read once.  Bound by the matrix cores' rate under the power limit: 9216 x 3072 x
+    // (3072 + 12288) int8 on 384 x 192 2.6 POP/s with both products (parked 2.1), e4m3 2.7 (rescaled in place 2.4).
     constexpr int OM = DUAL ? BM / 2 : BM;  // output rows of the tile
     constexpr int NW = WGM * WGN, NT = NW * 64;
     constexpr int WM = BM / WGM, WN = BN / WGN;
@@ -681,7 +733,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     static_assert(!GRP || (!F8 && NS == 2), "group factors: int8, two stages");
     // int8 tiles above 256 x 256 run the whole-step schedule too: one set of 32-byte fragments
     // instead of two sets of 16-byte ones leaves room for their accumulators
-    constexpr bool WS = !F8 && !GRP && BM * BN > 256 * 256;
+    constexpr bool WS = !F8 && !GRP && (BM * BN > 256 * 256 || MIX);
     constexpr bool S8 = F8 || GRP || WS;  // whole-step fragments
     //
     // PARK (int8, several ranges): no second register set at all.  When a range ends, its
@@ -772,8 +824,14 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
 #pragma unroll
     for (int i = 0; i < B_IT; ++i) b_goff[i] = (uint32_t)min(n0 + s_row + i * RPI, p.N - 1) * (uint32_t)p.ldb + s_lc * 16;
     const int w_lds = wave * 8 * BK;
-    static_assert(!DUAL || (RPI % WM == 0 && WM % 32 == 0), "a wave's eight rows of a pass come from one of the two tensors");
+    static_assert(!DUAL || ((MIX || RPI % WM == 0) && WM % 32 == 0), "a wave's eight rows of a pass come from one of the two tensors");
     const bool second = DUAL && (wave * 8) % WM >= WM / 2;
+    uint32_t seconds = 0;  // MIX: the passes whose rows are of the second tensor
+    if constexpr (MIX) {
+#pragma unroll
+        for (int i = 0; i < A_IT; ++i) seconds |= ((wave * 8 + i * RPI) % WM >= WM / 2 ? 1u : 0u) << i;
+    }
+    uint32_t wanted = seconds | (((1u << B_IT) - 1u) << A_IT);  // MIX: the passes that a step of the plain range loads, activations then weights
     // KT: pieces of a row past the end of K.  They are loaded from the step's first piece instead, which is there (a weight
     // row that holds a NaN gives NaN either way), and what they became in the activations is cleared before it is read.
     const int k_tail = KT ? (p.r[0].k1 - p.r[0].k0) % BK : 0;
@@ -794,9 +852,13 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     // a wave covers 8 rows of a pass, so whether it takes part in a partial last pass is wave-uniform
     const bool a_skip = A_TAIL != 0 && wave * 8 >= A_TAIL;
     const bool b_skip = B_TAIL != 0 && wave * 8 >= B_TAIL;
-    auto dma1 = [&](const uint8_t* ap, const uint8_t* bp, int buf, int i) {
+    auto dma1 = [&](const uint8_t* ap, const uint8_t* bp, int buf, int i, auto plain_c) {  // plain_c: a step of MIX's plain range
+        if constexpr (MIX && decltype(plain_c)::value) {
+            if (!((wanted >> i) & 1u)) return;
+        }
         if (i < A_IT) {
             if (i == A_IT - 1 && a_skip) return;
+            if constexpr (MIX && !decltype(plain_c)::value) ap += (seconds >> i) & 1u ? A2b - Ab : 0;
             load16_to_lds(ap + (KT ? a_goff[i] - back : a_goff[i]), As + buf * BM * BK + w_lds + i * RPI * BK);
         } else {
             if (i == A_IT + B_IT - 1 && b_skip) return;
@@ -816,9 +878,9 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
             else __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(nt * (full - 2)));
         }
     };
-    auto dma = [&](const uint8_t* ap, const uint8_t* bp, int buf) {
+    auto dma = [&](const uint8_t* ap, const uint8_t* bp, int buf, auto plain_c) {
 #pragma unroll
-        for (int i = 0; i < A_IT + B_IT; ++i) dma1(ap, bp, buf, i);
+        for (int i = 0; i < A_IT + B_IT; ++i) dma1(ap, bp, buf, i, plain_c);
     };
 
     acc_t acc[TN][TM];
@@ -962,11 +1024,26 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     // source of its activations stay in registers, so the range table is read
     // only when a cursor crosses into the next range.
     int steps = 0;
-    if constexpr (KT) steps = (p.r[0].k1 - p.r[0].k0 + BK - 1) / BK;
+    [[maybe_unused]] int n_dual = 0;  // MIX: how many of the steps are of the two ranges
+    if constexpr (MIX) {}
+    else if constexpr (KT) steps = (p.r[0].k1 - p.r[0].k0 + BK - 1) / BK;
     else
         for (int i = 0; i < p.nr; ++i) steps += (p.r[i].k1 - p.r[i].k0) / BK;
     int lr = 0, skip = 0;  // this workgroup's first step: `skip` steps into range lr
-    if (p.splits > 1) {
+    if constexpr (MIX) {  // a step of the plain range counts half of one of the two
+        const int d = (p.r[0].k1 - p.r[0].k0) / BK, all = 2 * d + (p.nr > 2 ? (p.r[2].k1 - p.r[2].k0) / BK : 0);
+        auto step_at = [&](int c) { return c < 2 * d ? c >> 1 : c - d; };
+        int first = 0;
+        steps = all - d;
+        if (p.splits > 1) {
+            first = step_at((int)((int64_t)all * zy / p.splits));
+            steps = step_at((int)((int64_t)all * (zy + 1) / p.splits)) - first;
+        }
+        n_dual = max(min(first + steps, d) - first, 0);
+        lr = first < d ? 0 : 2;
+        skip = first < d ? first : first - d;
+        r_last = 2;
+    } else if (p.splits > 1) {
         skip = (int)((int64_t)steps * zy / p.splits);
         steps = (int)((int64_t)steps * (zy + 1) / p.splits) - skip;
         while (lr + 1 < p.nr && skip >= (p.r[ph(lr)].k1 - p.r[ph(lr)].k0) / BK) {
@@ -979,12 +1056,20 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     }
     const int r_first = lr, k_first = p.r[ph(lr)].k0 + skip * BK;
     int lk = k_first, lk1 = p.r[ph(lr)].k1;
-    const uint8_t* la = (DUAL ? second : p.r[ph(lr)].a_sel == 1) ? A2b : Ab;
+    const uint8_t* la = (MIX ? false : DUAL ? second : p.r[ph(lr)].a_sel == 1) ? A2b : Ab;
+    [[maybe_unused]] const int k_plain = MIX && p.nr > 2 ? p.r[2].k0 : 0;
     if (KT && lk + BK > lk1) back = past_k ? s_lc * 16 : 0;
     auto advance_load = [&]() {
         lk += BK;
         if constexpr (KT) {
             if (lk + BK > lk1) back = past_k ? s_lc * 16 : 0;
+            return;
+        }
+        if constexpr (MIX) {  // (past the last step nothing more is loaded)
+            if (lk >= lk1) {
+                lk = k_plain;
+                lk1 = 0x7fffffff;
+            }
             return;
         }
         if (lk >= lk1) {
@@ -1000,8 +1085,9 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     // are fetched first of all, so that the wait for the first DMA covers them, and
     // parked in LDS behind the stages: the epilogue then starts without a round
     // trip to memory, and without the ~70 small loads per wave it would take there.
-    // (DUAL: [1/sx | 1/sw | bias] of the first range, as the epilogue reads them, then [1/sx | 1/sw] of the second)
-    constexpr int EPI_FLOATS = DUAL ? 2 * OM + 3 * BN : BM + 2 * BN, EPI_IT = (EPI_FLOATS + NT - 1) / NT;
+    // (DUAL: [1/sx | 1/sw | bias] of the first range, as the epilogue reads them, then [1/sx | 1/sw] of the second, MIX: and of
+    // the third, zeros where this workgroup has no step of it)
+    constexpr int EPI_FLOATS = MIX ? 3 * OM + 4 * BN : DUAL ? 2 * OM + 3 * BN : BM + 2 * BN, EPI_IT = (EPI_FLOATS + NT - 1) / NT;
     float* const epi = reinterpret_cast<float*>(smem + NS * (BM + BN) * BK);
     // group factors: a ring of four rows of BN floats behind the epilogue's vectors.  The row of
     // step s arrives with the step's operands and is read all through step s, at whose end the
@@ -1034,8 +1120,14 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
             if (p.bias) v = load_bias(p.bias, p.bias_dtype, min(n0 + e - OM - BN, p.N - 1));
         } else if (DUAL && e < 2 * OM + 2 * BN) {
             v = (p.r[1].sx + z * p.bsSx)[(int64_t)min(m0 + e - OM - 2 * BN, p.M - 1) * p.r[1].sx_rs];
-        } else if (DUAL && e < EPI_FLOATS) {
+        } else if (DUAL && e < 2 * OM + 3 * BN) {
             v = (p.r[1].sw + z * p.bsSw)[(int64_t)min(n0 + e - 2 * OM - 2 * BN, p.N - 1) * p.r[1].sw_cs];
+        } else if (MIX && steps == n_dual) {
+            v = __builtin_inff();
+        } else if (MIX && e < 3 * OM + 3 * BN) {
+            v = p.r[2].sx[(int64_t)min(m0 + e - 2 * OM - 3 * BN, p.M - 1) * p.r[2].sx_rs];
+        } else if (MIX && e < EPI_FLOATS) {
+            v = p.r[2].sw[(int64_t)min(n0 + e - 3 * OM - 3 * BN, p.N - 1) * p.r[2].sw_cs];
         }
         epi_val[i] = v;
     }
@@ -1045,7 +1137,8 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
 #pragma unroll
     for (int t = 0; t < NS; ++t) {
         if (t < steps) {
-            dma(la + lk, Bb + lk, t);
+            if (MIX && t >= n_dual) dma(la + lk, Bb + lk, t, std::true_type{});
+            else dma(la + lk, Bb + lk, t, std::false_type{});
             dma_g();
             advance_load();
             ++issued;
@@ -1056,7 +1149,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
 #pragma unroll
     for (int i = 0; i < EPI_IT; ++i) {
         const int e = i * NT + tid;
-        if constexpr (KT) {  // (quotients, as exact as the general kernel's, which such launches had)
+        if constexpr (KT || MIX) {  // (quotients, as exact as the general kernel's, which such launches had)
             if (e < EPI_FLOATS) epi[e] = (e < OM + BN || e >= OM + 2 * BN) ? 1.0f / epi_val[i] : epi_val[i];
         } else {
             if (e < EPI_FLOATS) epi[e] = (e < BM + BN && !ACCF) ? __builtin_amdgcn_rcpf(epi_val[i]) : epi_val[i];
@@ -1118,10 +1211,12 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     // registers this step is done with: next weight fragment 0, then each
     // activation fragment right behind the last MFMA that reads it, with the DMA
     // of step s + 2 spread over the same MFMAs.
-    auto step8 = [&](auto dma_c, auto more_c) __attribute__((always_inline)) {
+    // plain_c, dplain_c (MIX): this step, the one that it loads, is of the plain range: the second half of the row blocks only
+    auto step8 = [&](auto dma_c, auto more_c, auto plain_c, auto dplain_c) __attribute__((always_inline)) {
         constexpr bool DMA_ = decltype(dma_c)::value;
         constexpr bool MORE_ = decltype(more_c)::value;
-        constexpr int NDM8 = A_IT + B_IT, TAIL = 2 * TM;  // DMA instructions over the tail's MFMAs
+        constexpr int B0 = decltype(plain_c)::value ? TM / 2 : 0;      // the first row block
+        constexpr int NDM8 = A_IT + B_IT, TAIL = 2 * (TM - B0);  // DMA instructions over the tail's MFMAs
         const int nbuf = buf ^ 1;
         auto lo4 = [](const v8i& f) __attribute__((always_inline)) { return v4i{f[0], f[1], f[2], f[3]}; };
         auto hi4 = [](const v8i& f) __attribute__((always_inline)) { return v4i{f[4], f[5], f[6], f[7]}; };
@@ -1150,22 +1245,22 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
             } else if constexpr (WS) {
                 // int8: the two 64-byte K halves of a block, TM MFMAs apart
 #pragma unroll
-                for (int b = 0; b < TM; ++b) {
-                    if (b == 0 && a == 0) frag8(buf, TM + 1);
-                    if (b == (TM > 1 ? 1 : 0)) frag8(buf, TM + a + 2);
+                for (int b = B0; b < TM; ++b) {
+                    if (b == B0 && a == 0) frag8(buf, TM + 1);
+                    if (b == (TM > 1 ? B0 + 1 : 0)) frag8(buf, TM + a + 2);
                     if constexpr (!F8) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo4(fb8[a]), lo4(fa8[b]), acc[a][b], 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
-                for (int b = 0; b < TM; ++b) {
+                for (int b = B0; b < TM; ++b) {
                     if constexpr (!F8) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi4(fb8[a]), hi4(fa8[b]), acc[a][b], 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
 #pragma unroll
-                for (int b = 0; b < TM; ++b) {
-                    if (b == 0 && a == 0) frag8(buf, TM + 1);
-                    if (b == (TM > 1 ? 1 : 0)) frag8(buf, TM + a + 2);
+                for (int b = B0; b < TM; ++b) {
+                    if (b == B0 && a == 0) frag8(buf, TM + 1);
+                    if (b == (TM > 1 ? B0 + 1 : 0)) frag8(buf, TM + a + 2);
                     if constexpr (F8)
                         acc[a][b] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb8[a], fa8[b], acc[a][b], 0, 0, 0, 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
@@ -1189,7 +1284,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
                     const int j = (a - (TN - 2)) * TM + b;
                     if constexpr (DMA_) {
 #pragma unroll
-                        for (int i = j * NDM8 / TAIL; i < (j + 1) * NDM8 / TAIL; ++i) dma1(ap, bp, buf, i);
+                        for (int i = j * NDM8 / TAIL; i < (j + 1) * NDM8 / TAIL; ++i) dma1(ap, bp, buf, i, dplain_c);
                         if (j == TAIL - 1) dma_g();
                     }
                     __builtin_amdgcn_sched_barrier(0);
@@ -1212,36 +1307,36 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
                 if constexpr (!LAG) convert_block(a);
             } else if constexpr (WS) {
 #pragma unroll
-                for (int b = 0; b < TM; ++b) {
+                for (int b = B0; b < TM; ++b) {
                     if constexpr (!F8) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo4(fb8[a]), lo4(fa8[b]), acc[a][b], 0, 0, 0);
-                    const int j = (a - (TN - 2)) * TM + b;
+                    const int j = (a - (TN - 2)) * (TM - B0) + b - B0;
                     if constexpr (DMA_) {
 #pragma unroll
-                        for (int i = j * NDM8 / TAIL; i < (j + 1) * NDM8 / TAIL; ++i) dma1(ap, bp, buf, i);
+                        for (int i = j * NDM8 / TAIL; i < (j + 1) * NDM8 / TAIL; ++i) dma1(ap, bp, buf, i, dplain_c);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
-                for (int b = 0; b < TM; ++b) {
+                for (int b = B0; b < TM; ++b) {
                     if constexpr (!F8) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi4(fb8[a]), hi4(fa8[b]), acc[a][b], 0, 0, 0);
                     if constexpr (MORE_) {
-                        if (a == TN - 2 && b == 0) frag8(nbuf, TM);  // next weight fragment 0: free since block 0
+                        if (a == TN - 2 && b == B0) frag8(nbuf, TM);  // next weight fragment 0: free since block 0
                         if (a == TN - 1) frag8(nbuf, b);              // next activation fragment b: this was its last reader
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
 #pragma unroll
-                for (int b = 0; b < TM; ++b) {
+                for (int b = B0; b < TM; ++b) {
                     if constexpr (F8)
                         acc[a][b] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb8[a], fa8[b], acc[a][b], 0, 0, 0, 0, 0, 0);
-                    const int j = (a - (TN - 2)) * TM + b;
+                    const int j = (a - (TN - 2)) * (TM - B0) + b - B0;
                     if constexpr (DMA_) {
 #pragma unroll
-                        for (int i = j * NDM8 / TAIL; i < (j + 1) * NDM8 / TAIL; ++i) dma1(ap, bp, buf, i);
+                        for (int i = j * NDM8 / TAIL; i < (j + 1) * NDM8 / TAIL; ++i) dma1(ap, bp, buf, i, dplain_c);
                     }
                     if constexpr (MORE_) {
-                        if (a == TN - 2 && b == 0) frag8(nbuf, TM);  // next weight fragment 0: its registers were free since block 0
+                        if (a == TN - 2 && b == B0) frag8(nbuf, TM);  // next weight fragment 0: its registers were free since block 0
                         if (a == TN - 1) frag8(nbuf, b);              // next activation fragment b: this was its last reader
                     }
                     __builtin_amdgcn_sched_barrier(0);
@@ -1257,7 +1352,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         ck += BK;
         cslot = (cslot + 1) & 3;
         dirty = true;
-        if (!KT && ck >= ck1) {
+        if (!KT && !MIX && ck >= ck1) {
             if constexpr (FOLD) fold(cr);
             dirty = false;
             ++cr;
@@ -1313,7 +1408,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
             for (int b = 0; b < TM; ++b) {
                 const int i = a * TM + b;
                 if constexpr (DMA_) {
-                    if (i % DM_EVERY == DM_EVERY - 1 && i / DM_EVERY < NDM && !abl_dma) dma1(ap, bp, buf, i / DM_EVERY);
+                    if (i % DM_EVERY == DM_EVERY - 1 && i / DM_EVERY < NDM && !abl_dma) dma1(ap, bp, buf, i / DM_EVERY, std::false_type{});
                 }
                 if constexpr (MORE_) {
                     if (i % RD_EVERY == 0 && i / RD_EVERY < NRD && !abl_lds) frag1(nbuf, 0, i / RD_EVERY);
@@ -1341,10 +1436,39 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         buf = nbuf;
     };
     auto step = [&](auto dma_c, auto more_c) __attribute__((always_inline)) {
-        if constexpr (S8) step8(dma_c, more_c);
+        if constexpr (S8) step8(dma_c, more_c, std::false_type{}, std::false_type{});
         else step_i8(dma_c, more_c);
     };
     int s = 0;
+    if constexpr (MIX) {
+        constexpr std::true_type yes{};
+        constexpr std::false_type no{};
+        for (; s + 2 < n_dual; ++s) step8(yes, yes, no, no);
+        // from here on a step loads a plain one or, behind the last, none (what it reads of that goes nowhere)
+        for (; s < n_dual; ++s) {
+            if (s + 2 >= steps) wanted = 0;
+            step8(yes, yes, no, yes);
+        }
+        if (n_dual > 0) {  // the sums of both signs -> one, in output units
+            const float* const rx2 = epi + OM + 2 * BN;
+#pragma unroll
+            for (int a = 0; a < TN; ++a) {
+                const int n = wn * WN + a * 16 + 4 * lgrp;
+                const v4f w = *reinterpret_cast<const v4f*>(epi + OM + n), w2 = *reinterpret_cast<const v4f*>(rx2 + OM + n);
+#pragma unroll
+                for (int b = 0; b < TM / 2; ++b) {
+                    const int m = wm * (WM / 2) + b * 16 + lrow;
+                    acc[a][b] = __builtin_bit_cast(acc_t, __builtin_convertvector(acc[a][b], v4f) * epi[m] * w +
+                                                              __builtin_convertvector(acc[a][b + TM / 2], v4f) * rx2[m] * w2);
+                    acc[a][b + TM / 2] = acc_zero;
+                }
+            }
+        }
+        for (; s < steps; ++s) {
+            if (s + 2 >= steps) wanted = 0;
+            step8(yes, yes, yes, yes);
+        }
+    }
     for (; s + NS < steps; ++s) step(std::true_type{}, std::true_type{});
     for (; s + 1 < steps; ++s) step(std::false_type{}, std::true_type{});
     if (s < steps) step(std::false_type{}, std::false_type{});
@@ -1392,53 +1516,25 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (p.part) {
-            // Two workgroups share a tile.  Each leaves its share in the workspace and counts itself in;
-            // the one that finds the other counted adds that share to its own (a + b = b + a: the result
-            // does not depend on who came last) and finishes the tile.  The two can sit on different
-            // XCDs, whose L2 caches do not see each other's lines, so the shares are written through
-            // and read past the caches (agent scope: what the compiler emits for a relaxed agent-scope
-            // atomic, but 16 bytes per lane: 1 KB contiguous per wave and instruction).
-            using v4u = __attribute__((ext_vector_type(4))) unsigned int;
-            constexpr int AGENT = 16;  // the cache-policy bit for agent scope
-            constexpr int SHARE = BM * BN * 4;
-            const int my = zy;
-            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-                reinterpret_cast<uint8_t*>(p.part) + (int64_t)tile_id * 2 * SHARE, 0, 2 * SHARE, 0x00020000);
-#pragma unroll
-            for (int i = 0; i < TN * TM; ++i)
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, of[i / TM][i % TM]), rs, tid * 16, my * SHARE + i * NT * 16, AGENT);
-            __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));  // this wave's stores have reached memory
-            __syncthreads();                                  // ... and so have the other waves'
-            int* const flag = reinterpret_cast<int*>(epi);    // (1 / sx of row 0: no longer needed)
-            if (tid == 0) {
-                // the launch's own stamp instead of a count: whatever the word held before (an earlier
-                // launch's stamp, or anything at all in a fresh workspace) reads as "nobody yet"
-                const unsigned before = __hip_atomic_exchange(p.arrived + tile_id, p.stamp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                *flag = before == p.stamp;
-                // the second one clears the word: a replay of this very launch (a captured graph keeps
-                // the stamp it was recorded with) must find "nobody yet" again
-                if (before == p.stamp) __hip_atomic_store(p.arrived + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            __syncthreads();
-            if (!*flag) return;
-#pragma unroll
-            for (int c0 = 0; c0 < TN * TM; c0 += CH) {
-                v4u other[CH];
-#pragma unroll
-                for (int i = 0; i < CH; ++i)
-                    if (c0 + i < TN * TM)
-                        other[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, tid * 16, (1 - my) * SHARE + (c0 + i) * NT * 16, AGENT);
-#pragma unroll
-                for (int i = 0; i < CH; ++i)
-                    if (c0 + i < TN * TM) of[(c0 + i) / TM][(c0 + i) % TM] += __builtin_bit_cast(v4f, other[i]);
-            }
-        }
+        if (p.part && !meet_share<NT, CH>(p, of, tile_id, zy, tid, reinterpret_cast<int*>(epi))) return;
         if (p.lr_rank > 0) lowrank_accumulate<TM, TN>(p, of, m0 + wm * WM, n0 + wn * WN, lane);
         wide_epilogue<BM, BN, WGM, WGN, GEMM_F8, false, true>(p, of, of, smem, z, m0, n0, wave, lane, r_epi, epi);
         return;
     }
-    if constexpr (DUAL) {
+    if constexpr (MIX) {
+        v4f of[TN][TM / 2];
+        const float* const rx3 = epi + 2 * OM + 3 * BN;
+#pragma unroll
+        for (int a = 0; a < TN; ++a) {
+            const v4f w3 = *reinterpret_cast<const v4f*>(rx3 + OM + wn * WN + a * 16 + 4 * lgrp);
+#pragma unroll
+            for (int b = 0; b < TM / 2; ++b)
+                of[a][b] = __builtin_bit_cast(v4f, acc[a][b]) +
+                           __builtin_convertvector(acc[a][b + TM / 2], v4f) * rx3[wm * (WM / 2) + b * 16 + lrow] * w3;
+        }
+        if (p.part && !meet_share<NT, 8>(p, of, tile_id, zy, tid, reinterpret_cast<int*>(epi))) return;
+        wide_epilogue<OM, BN, WGM, WGN, GEMM_F8, false, true>(p, of, of, smem, z, m0, n0, wave, lane, 0, epi);
+    } else if constexpr (DUAL) {
         v4f of[TN][TM / 2];
         const float* const rx2 = epi + OM + 2 * BN;
 #pragma unroll
@@ -1476,11 +1572,11 @@ int launch_wide_instance(const GemmParams& p, int64_t batch, hipStream_t st) {
 
 // wide tile ids (after the generic ones): 256x256 | 256x128 | 128x256 | 128x128, eight waves each
 template <int BM, int BN, int WGM, int WGN, int FMT, bool FOLD, int NS, bool GRP = false, bool PARK = false, bool FINISH = false,
-          bool CODES = false, bool SEP = false, bool KT = false, bool DUAL = false>
+          bool CODES = false, bool SEP = false, bool KT = false, bool DUAL = false, bool MIX = false>
 int launch_pipe_instance(const GemmParams& p, int64_t batch, hipStream_t st) {
-    auto kern = gemm_pipe_kernel<BM, BN, WGM, WGN, FMT, FOLD, NS, GRP, PARK, FINISH, CODES, SEP, KT, DUAL>;
+    auto kern = gemm_pipe_kernel<BM, BN, WGM, WGN, FMT, FOLD, NS, GRP, PARK, FINISH, CODES, SEP, KT, DUAL, MIX>;
     // the stages, the epilogue's vectors, and the ring of group factors
-    constexpr int lds = NS * (BM + BN) * BK + (DUAL ? BM + 3 * BN : BM + 2 * BN) * 4 + (GRP ? 4 * BN * 4 : 0);
+    constexpr int lds = NS * (BM + BN) * BK + (MIX ? BM / 2 * 3 + 4 * BN : DUAL ? BM + 3 * BN : BM + 2 * BN) * 4 + (GRP ? 4 * BN * 4 : 0);
     if (p.dry) return SEGQ_OK;
     static unsigned long long attr_done = 0;
     if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), lds, &attr_done)) return rc;
@@ -1495,14 +1591,20 @@ int launch_walk(const GemmParams& p, int cfg, int64_t batch, hipStream_t st) {
     constexpr int WM = FMT == GEMM_F8 ? 4 : 2, WN = FMT == GEMM_F8 ? 2 : 4;  // (e4m3 wants three or more column blocks per wave)
 #define SEGQ_WALK(BM_, BN_, WGM_, WGN_, DUAL_) \
     return launch_pipe_instance<BM_, BN_, WGM_, WGN_, FMT, false, 2, false, false, false, false, false, true, DUAL_>(p, batch, st)
+#define SEGQ_MIX(BM_, BN_) \
+    return launch_pipe_instance<BM_, BN_, 4, 2, FMT, false, 2, false, false, false, false, false, false, true, true>(p, batch, st)
     switch (cfg) {
         case FIRST_KT_CFG: SEGQ_WALK(256, 256, 4, 2, false);
         case FIRST_KT_CFG + 1: SEGQ_WALK(256, 192, 4, 2, false);
         case FIRST_KT_CFG + 2: SEGQ_WALK(128, 128, WM, WN, false);
         case FIRST_DUAL_CFG: SEGQ_WALK(256, 192, 4, 2, true);
         case FIRST_DUAL_CFG + 1: SEGQ_WALK(128, 128, WM, WN, true);
+        case FIRST_MIX_CFG: SEGQ_MIX(384, 192);
+        case FIRST_MIX_CFG + 1: SEGQ_MIX(256, 256);
+        case FIRST_MIX_CFG + 2: SEGQ_MIX(256, 192);
     }
 #undef SEGQ_WALK
+#undef SEGQ_MIX
     return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: no kernel for tile %d", cfg + 1);
 }
 

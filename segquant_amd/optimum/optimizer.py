@@ -387,7 +387,7 @@ class DefaultOptimizer(BaseOptimizer):
         gdq = plan.get("group_dequant")
         add2 = None if addend is None else addend.reshape(M, N).contiguous()
         kw = dict(m=M, n=N, a_fmt=plan["fa"], b_fmt=plan["fw"], out_dtype=x.dtype, lda=K, ldb=ldb, bias=bias, a_neg=codes_neg,
-                  group_dequant=gdq, out_codes=out_codes, finite_scales=dual and S == 1)
+                  group_dequant=gdq, out_codes=out_codes, finite_scales=dual)
         g = None
         if "l2t" in plan:
             # the SVD optimiser's low-rank branch: inside the GEMM's epilogue where the library has a
@@ -562,7 +562,7 @@ class DefaultOptimizer(BaseOptimizer):
             if d_s:
                 ranges.append(ops.Range(k0, k1 - k0, neg[s_], plan["sw"], 1, rs, plan["sw_cs"]))
         g = ops.gemm_desc(codes, plan["w"], ranges, m=M, n=N, a_fmt=fa, b_fmt=plan["fw"], out_dtype=dt, lda=K,
-                          ldb=K // 2 if plan["fw"] == ops.FMT_INT4 else K, bias=bias, a_neg=codes_neg)
+                          ldb=K // 2 if plan["fw"] == ops.FMT_INT4 else K, bias=bias, a_neg=codes_neg, finite_scales=dual)
         int4 = plan["fw"] == ops.FMT_INT4
         ws = None
         if M >= 3072 or not int4:

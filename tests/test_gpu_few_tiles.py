@@ -251,6 +251,75 @@ def test_dual_ranges_with_finite_scales(ops, kind):
     assert took[300, False] == took[300, True] == took[400, False] == (True, False) and took[400, True] == (False, True)
 
 
+def _check_mix(ops, kind, M, N, K0, K1, tile, dt, g, shares=0, first=True, gap=0, empty=None, per_row=True, add=False, lend=True):
+    """DualScale's two ranges of K1 and a plain one of K0 (0: none; in front of or behind them in memory, `gap` apart)."""
+    fa = FORMATS[kind][0]
+    k0, k1 = (0, K0 + gap if K0 else gap) if first else (K1 + gap, 0)
+    K = max(k0 + K0, k1 + K1)
+    a, b = _codes(g, (M, K), fa), _codes(g, (N, K), fa)
+    neg = _codes(g, (M, K), fa)  # (outside the pair it holds what is never read)
+    pick = g.random((M, K1)) < 0.5
+    a[:, k1:k1 + K1][pick] = 0
+    neg[:, k1:k1 + K1][~pick] = 0
+    scale = lambda n: (g.random(n) * 30 + 10).astype(np.float32)
+    sx, sw = [scale(M if per_row else 1) for _ in range(3)], [scale(N), scale(N)]
+    if empty is not None:
+        (a if empty == 0 else neg)[:, k1:k1 + K1] = 0
+        sx[empty][:] = np.inf
+    parts = [(a, k1, K1, sx[0], sw[0]), (neg, k1, K1, sx[1], sw[0])] + ([(a, k0, K0, sx[2], sw[1])] if K0 else [])
+    bias = g.standard_normal(N).astype(np.float32)
+    want, mag = np.zeros((M, N)) + bias, np.zeros((M, N)) + np.abs(bias)
+    for c, k, n, s, w in parts:
+        av, bv = (O.code_values(t[:, k:k + n], fa).astype(np.float64) for t in (c, b))
+        den = s.astype(np.float64)[:, None] * w.astype(np.float64)[None, :]
+        want += av @ bv.T / den
+        mag += np.abs(av) @ np.abs(bv).T / den
+    up = lambda t: torch.from_numpy(t).to(DEV)
+    rg = [ops.Range(k, n, up(s), up(w), int(c is neg), int(per_row), 1) for c, k, n, s, w in parts]
+    if first and K0:
+        rg = rg[2:] + rg[:2]
+    addend = None
+    if add:
+        addend = torch.randn(M, N, device=DEV).to(dt)
+        want, mag = want + addend.double().cpu().numpy(), mag + addend.double().abs().cpu().numpy()
+    gd = ops.gemm_desc(_dev(a, fa), _dev(b, fa), rg, m=M, n=N, a_fmt=fa, b_fmt=fa, out_dtype=dt, lda=K, ldb=K, a_neg=_dev(neg, fa), finite_scales=True,
+                       bias=up(bias), addend=addend, tile=tile, split_k=shares)
+    # (a workspace that holds NaN: nothing of it is read before it is written)
+    ws = torch.full((ops.gemm_workspace_bytes(gd) // 4 + 4,), float("nan"), device=DEV).view(torch.uint8) if lend else None
+    plan = ops.gemm_plan(gd, ws)
+    assert plan["tile"] == tile if tile else plan["tile"] in (31, 32, 33)
+    assert not plan["parked"] and (not shares or plan["splits"] <= shares)
+    got = [ops.gemm_launch(gd, ws).double().cpu().numpy() for _ in range(2)]
+    # an exact int32 sum, its conversion, two quotients and two products per range and share (5 x 2^-24), the additions of up to
+    # three ranges, 16 shares, bias and addend (their running sums stay below mag, 21 x 2^-24); e4m3: the matrix cores' limited-width adder
+    tol = (1.6e-6 if kind == "int8" else 3e-4) * mag + {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dt] * np.abs(want)
+    assert np.isfinite(got[0]).all() and (np.abs(got[0] - want) <= tol).all(), (kind, M, N, K0, K1, tile, dt, float((np.abs(got[0] - want) - tol).max()))
+    assert (got[0] == got[1]).all()
+    return plan
+
+
+@pytest.mark.parametrize("kind", ["int8", "e4m3"])
+@pytest.mark.parametrize("tile", [31, 32, 33, 0])
+def test_dual_and_plain_ranges_in_one_walk(ops, kind, tile):
+    """Edges of the tiles; one, two and three steps of either kind (the loop loads two ahead); shares that begin or end in the
+    plain range; three ranges in any order; sides that hold nothing; rules that a workspace or none is given to."""
+    g = np.random.default_rng(tile + 2)
+    dts = (torch.float32, torch.bfloat16, torch.float16)
+    for i, (M, N, k0, k1) in enumerate(((1, 16, 1, 1), (64, 128, 2, 1), (193, 130, 1, 2), (129, 257, 3, 3), (192, 192, 2, 5), (300, 500, 7, 4), (257, 70, 5, 2))):
+        for lend in (False, True):
+            _check_mix(ops, kind, M, N, 128 * k0, 128 * k1, tile, dts[i % 3], g, first=bool(i % 2), lend=lend)
+    for opt in (dict(empty=0), dict(empty=1), dict(empty=2), dict(per_row=False), dict(gap=128), dict(gap=128, first=False), dict(add=True)):
+        _check_mix(ops, kind, 140, 210, 384, 640, tile, torch.float32, g, **opt)
+    if tile:
+        for i, shares in enumerate((2, 3, 5, 9)):  # of 18, 5 and 4 steps: whole ranges, one step, less
+            for k0, k1 in ((1024, 1280), (384, 256), (0, 512)):
+                _check_mix(ops, kind, 200, 300, k0, k1, tile, dts[i % 3], g, shares=shares, first=bool(i % 2), add=i == 1, empty=2 if i == 2 and k0 else None)
+    else:
+        # the library's shares: two that meet, more that a second kernel sums; the pair alone; up to 128 rows its own choice is another
+        for M, N, k0, k1, splits in ((1024, 3072, 512, 2048, (2, 3, 4)), (300, 640, 640, 4096, range(3, 17)), (600, 2048, 0, 8192, (3, 4, 5))):
+            assert _check_mix(ops, kind, M, N, k0, k1, 0, torch.bfloat16, g)["splits"] in splits
+
+
 # ---- a linear of up to 16 rows in one launch ---------------------------------------------------------------------------------
 @pytest.mark.parametrize("dt", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("kind,group", [("int8", False), ("e4m3", False), ("int4", False), ("int4", True)])
