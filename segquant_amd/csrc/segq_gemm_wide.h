@@ -1144,8 +1144,8 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
             ++issued;
         }
     }
-    if (issued == NS && !GRP) wait_dma(std::integral_constant<int, NS - 1>{});
-    else wait_dma(std::integral_constant<int, 0>{});  // (with group factors the waves' DMA counts differ)
+    if (issued == NS && !GRP && !(MIX && n_dual < NS)) wait_dma(std::integral_constant<int, NS - 1>{});
+    else wait_dma(std::integral_constant<int, 0>{});  // (with group factors and in plain steps the waves' DMA counts differ)
 #pragma unroll
     for (int i = 0; i < EPI_IT; ++i) {
         const int e = i * NT + tid;
