@@ -306,7 +306,8 @@ typedef struct segq_gemm_desc {
                          * by segq_quantize with pre_op and a static per-tensor scale.  With out_scale_neg set
                          * (DualScale) out_codes_neg is required: values >= 0 go to out_codes scaled by
                          * out_scale[0], the others to out_codes_neg scaled by out_scale_neg[0], the tensor not
-                         * taken holding code(0) (segquant/src/real_quant/quantizer.cuh:178-206).  out is
+                         * taken holding code(0) (segquant/src/real_quant/quantizer.cuh:178-206); where out_codes_neg
+                         * is out_codes, one tensor holds the codes of both (ranges of a_sel 2 and 3 read it).  out is
                          * ignored (may be NULL).  Needs plain int8 or e4m3 codes on both sides, one range with K
                          * a multiple of 128, batch == 1, out_dtype F16 or BF16; no split_k, group factors or
                          * low-rank branch (SEGQ_ERR_UNSUPPORTED otherwise).

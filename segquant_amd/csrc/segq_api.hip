@@ -443,7 +443,9 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         const segq_krange &r = d->ranges[0], &s = d->ranges[d->n_ranges - 1];
         const bool base = (i8 || f8) && !lowrank && !codes_out && !groups && d->split_k <= 1 && d->m * d->lda < (int64_t)1 << 32 && d->n * d->ldb < (int64_t)1 << 32;
         const bool one = base && d->n_ranges == 1 && r.a_sel < 2;
-        const bool two = base && d->n_ranges == 2 && r.k_begin == s.k_begin && r.k_len == s.k_len && r.a_sel == 0 && s.a_sel == 1;
+        const bool pair = base && d->n_ranges == 2 && r.k_begin == s.k_begin && r.k_len == s.k_len, two = pair && r.a_sel == 0 && s.a_sel == 1;
+        // (codes of both signs in one tensor: what two tensors would do, for the choice below)
+        const bool merged = pair && d->finite_scales && r.a_sel == 2 && s.a_sel == 3;
         if (d->tile > FIRST_KT_CFG && d->tile <= FIRST_MIX_CFG) {
             if (!(d->tile > FIRST_DUAL_CFG ? two : one))
                 return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: tiles %d to %d serve one range, tiles %d to %d two over the same run of K from a and a_neg, in plain "
@@ -452,7 +454,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
             walk.cfg = (int)d->tile - 1;
         } else if (d->tile == 0 && d->out_dtype != SEGQ_ACC) {
             if (one && r.k_len % 128) walk = choose_ragged(d->m, d->n, d->batch, r.k_len, osz == 4 && !vec_store);
-            if (two && (r.own_sum || d->finite_scales) && r.k_len > (r.k_len % 128 ? 256 : 512)) {
+            if ((two || merged) && (r.own_sum || d->finite_scales) && r.k_len > (r.k_len % 128 ? 256 : 512)) {
                 walk = choose_dual(d->m, d->n, d->batch, r.k_len);
                 const bool lent = d->split_k != 1 && ws && al(ws, 16), in_turn = r.k_len % 128 == 0 && d->batch == 1;
                 const int64_t steps = r.k_len / 64;  // of both ranges in turn
@@ -472,8 +474,8 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         mix.neg = -1;
         for (int i = 0; i < d->n_ranges; ++i) {
             const segq_krange& r = d->ranges[i];
-            ok = ok && r.a_sel < 2 && r.k_begin % 128 == 0 && r.k_len % 128 == 0;
-            if (r.a_sel == 1) {
+            ok = ok && r.k_begin % 128 == 0 && r.k_len % 128 == 0;
+            if (r.a_sel == 1 || r.a_sel == 3) {
                 ok = ok && mix.neg < 0;
                 mix.neg = i;
             }
@@ -482,8 +484,9 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         for (int i = 0; ok && mix.neg >= 0 && i < d->n_ranges; ++i) {
             const segq_krange &r = d->ranges[i], &s = d->ranges[mix.neg];
             if (i == mix.neg) continue;
-            if (mix.pos < 0 && r.k_begin == s.k_begin && r.k_len == s.k_len) mix.pos = i;
-            else mix.plain = i;
+            if (mix.pos < 0 && r.k_begin == s.k_begin && r.k_len == s.k_len && r.a_sel == s.a_sel - 1) mix.pos = i;
+            else if (r.a_sel == 0) mix.plain = i;
+            else ok = false;
         }
         ok = ok && mix.neg >= 0 && mix.pos >= 0;
         const bool lent = ws && al(ws, 16);
@@ -513,7 +516,8 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
                 const double now = walk.cfg < 0 ? in_turn_us(d->m, d->n, 2 * steps, f8, share)
                                    : walk.cfg == FIRST_DUAL_CFG ? std::ceil((double)tiles_of_cfg(FIRST_DUAL_CFG, d->m, d->n, 1) / cus) * (1.1 * k + 5.0)
                                    : t64 <= 1.0 ? 4.8 + 0.6 * k : 4.0 + t64 * (0.44 * k + 0.8);
-                take = take && pick.us < 0.95 * now;
+                // (one tensor: what the quantise step, which asks for this plan, then does not write)
+                take = take && pick.us < 0.95 * now + (d->ranges[0].a_sel == 2 ? (double)d->m * steps * 128 / 5e6 : 0.0);
             }
             if (take) {
                 walk.cfg = -1;
@@ -522,6 +526,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
             }
         }
     }
+    if (walk.cfg >= FIRST_DUAL_CFG && d->ranges[0].a_sel != 0) walk.cfg = -1;
     const int few = [&]() -> int {
         const int64_t reach = (int64_t)1 << 31;  // a tile's rows are addressed with 31 bits
         const segq_krange& r = d->ranges[0];

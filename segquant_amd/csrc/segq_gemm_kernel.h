@@ -584,9 +584,12 @@ template <int FMT, bool B4>
 int launch_wide(const GemmParams& p, int wcfg, bool fold, bool asel, int64_t batch, hipStream_t st);
 template <int FMT>
 int launch_walk(const GemmParams& p, int cfg, int64_t batch, hipStream_t st);
+int launch_mix_i8(const GemmParams& p, int cfg, int64_t batch, hipStream_t st);
+int launch_mix_f8(const GemmParams& p, int cfg, int64_t batch, hipStream_t st);
 
 template <int FMT, bool B4>
 int launch_format(const GemmParams& p, int cfg, bool fold, int64_t batch, hipStream_t st) {
+    if (cfg >= FIRST_MIX_CFG && !B4) return FMT == GEMM_I8 ? launch_mix_i8(p, cfg, batch, st) : launch_mix_f8(p, cfg, batch, st);
     if (cfg >= FIRST_KT_CFG) {
         if constexpr (!B4) return launch_walk<FMT>(p, cfg, batch, st);
         return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: tile %d needs plain 8-bit codes on both sides", cfg + 1);

@@ -81,7 +81,7 @@ __device__ __forceinline__ void codes_epilogue(const GemmParams& p, typename Acc
     const int lrow = lane & 15, lgrp = lane >> 4;
     const int m_base = m0 + wm * WM + lrow;
     const int n_base = n0 + wn * WN + 4 * lgrp;
-    const bool dual = p.oc_neg != nullptr;
+    const bool dual = p.oc_neg != nullptr, two = dual && p.oc_neg != p.oc;  // (the same tensor: codes of both signs in one)
     const float s_pos = p.oc_scale[0];
     const float s_neg = dual ? p.oc_scale_neg[0] : s_pos;
     const bool bf = p.out_dtype == SEGQ_BF16;
@@ -101,32 +101,34 @@ __device__ __forceinline__ void codes_epilogue(const GemmParams& p, typename Acc
             if ((16 * CH) % 64 != 0 && c >= 16 * CH) continue;
             const uint4 raw = *reinterpret_cast<const uint4*>(patch + row * RS + col * 16);
             const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+            const int mm = m0 + wm * WM + b * 16 + row;
+            const int n = n0 + wn * WN + col * 8;
+            if (mm >= p.M || n >= p.N) continue;
+            const int64_t e = (int64_t)mm * p.ldoc + n;
             float cp[8], cn[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const uint32_t h = (i & 1) ? (w[i >> 1] >> 16) : (w[i >> 1] & 0xffffu);
                 float t = bf ? bf16_bits_to_f32(h) : f16_bits_to_f32(h);
                 if (op != SEGQ_PRE_NONE) t = round_to(dt, act_value(op, t));
-                // x >= 0 takes the positive scale; the branch not taken holds code(0)
-                // (segquant/src/real_quant/quantizer.cuh:193-203).  One tensor: one scale for both signs.
-                cp[i] = dual ? (t >= 0.0f ? t * s_pos : 0.0f) : t * s_pos;
-                cn[i] = (t >= 0.0f) ? 0.0f : t * s_neg;
+                // x >= 0 takes the positive scale; in two tensors the branch not taken holds code(0)
+                // (segquant/src/real_quant/quantizer.cuh:193-203).  Without DualScale: one scale for both signs.
+                const bool pos = t >= 0.0f;
+                t *= pos ? s_pos : s_neg;
+                cp[i] = pos || !two ? t : 0.0f;
+                cn[i] = pos ? 0.0f : t;
             }
-            const int mm = m0 + wm * WM + b * 16 + row;
-            const int n = n0 + wn * WN + col * 8;
-            if (mm >= p.M || n >= p.N) continue;
-            const int64_t e = (int64_t)mm * p.ldoc + n;
             const uint2 vp = make_uint2(pack4_codes(fmt, cp[0], cp[1], cp[2], cp[3]), pack4_codes(fmt, cp[4], cp[5], cp[6], cp[7]));
             uint2 vn = make_uint2(0u, 0u);
-            if (dual) vn = make_uint2(pack4_codes(fmt, cn[0], cn[1], cn[2], cn[3]), pack4_codes(fmt, cn[4], cn[5], cn[6], cn[7]));
+            if (two) vn = make_uint2(pack4_codes(fmt, cn[0], cn[1], cn[2], cn[3]), pack4_codes(fmt, cn[4], cn[5], cn[6], cn[7]));
             if (p.oc_vec && n + 7 < p.N) {
                 *reinterpret_cast<uint2*>(ocp + e) = vp;
-                if (dual) *reinterpret_cast<uint2*>(ocn + e) = vn;
+                if (two) *reinterpret_cast<uint2*>(ocn + e) = vn;
             } else {
                 const uint64_t bp = ((uint64_t)vp.y << 32) | vp.x, bn = ((uint64_t)vn.y << 32) | vn.x;
                 for (int i = 0; i < 8 && n + i < p.N; ++i) {
                     ocp[e + i] = (uint8_t)(bp >> (8 * i));
-                    if (dual) ocn[e + i] = (uint8_t)(bn >> (8 * i));
+                    if (two) ocn[e + i] = (uint8_t)(bn >> (8 * i));
                 }
             }
         }
@@ -680,12 +682,14 @@ template <int BM, int BN, int WGM, int WGN, int FMT, bool FOLD, int NS, bool GRP
           bool SEP = false,    // SEP (e4m3, several ranges): a second register set, as int8 has it, instead of rescaling in place
           bool KT = false,     // KT: K ends anywhere in sixteens (one walk of K)
           bool DUAL = false,   // DUAL: two ranges over one run of K, from the two code tensors, in one walk
-          bool MIX = false>    // MIX (DUAL): whole steps of K, behind them those of a plain range, K shares
+          bool MIX = false,    // MIX (DUAL): whole steps of K, behind them those of a plain range, K shares
+          bool MERGE = false>  // MERGE (MIX): both signs in one code tensor, parted in registers
 __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmParams p) {
     static_assert(!CODES || (!FOLD && !GRP && !PARK && !FINISH), "codes out: plain operands, one range");
     static_assert(!KT || (!FOLD && !GRP && !PARK && !FINISH && !CODES && NS == 2), "a ragged end of K: one walk, two stages");
     static_assert(!DUAL || KT != MIX, "DUAL instances take any K, or whole steps of it and a plain range");
-    static_assert(!MIX || (DUAL && !FOLD && !GRP && !PARK && !FINISH && !CODES && NS == 2), "MIX: one walk, two stages");
+    static_assert(!MIX || (DUAL && !FOLD && !GRP && !PARK && !FINISH && !CODES && (NS == 2 || MERGE)), "MIX: one walk, two stages");
+    static_assert(!MERGE || MIX, "MERGE instances are MIX instances");
     // DUAL (DualScale's two ranges over the same K and the same weights): the tile's BM rows of LDS are BM / 2 rows of each
     // code tensor, the two halves of every wave's row blocks, so that a wave holds both sums of an output and a weight
     // tile is read once for both.  What two ranges in turn need a second register set for, these have as the second
@@ -696,13 +700,14 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     // and fragment reads per step, two thirds of the DMA.  Three sums in two register sets: nothing is parked, no
     // third set, no ratio of scales, weights read once.  Bound by the matrix cores' rate under the power limit: 9216 x 3072 x
     // (3072 + 12288) int8 on 384 x 192 2.6 POP/s with both products (parked 2.1), e4m3 2.7 (rescaled in place 2.4).
-    constexpr int OM = DUAL ? BM / 2 : BM;  // output rows of the tile
+    constexpr int OM = DUAL ? BM / 2 : BM;   // output rows of the tile
+    constexpr int AR = MERGE ? BM / 2 : BM;  // rows of activation codes in LDS
     constexpr int NW = WGM * WGN, NT = NW * 64;
     constexpr int WM = BM / WGM, WN = BN / WGN;
     constexpr int TM = WM / 16, TN = WN / 16;
     constexpr int RPI = NT / 8;                                  // rows one pass of all threads covers
-    constexpr int A_IT = (BM + RPI - 1) / RPI, B_IT = (BN + RPI - 1) / RPI;
-    constexpr int A_TAIL = BM % RPI, B_TAIL = BN % RPI;          // rows of a last, partial pass (0: none)
+    constexpr int A_IT = (AR + RPI - 1) / RPI, B_IT = (BN + RPI - 1) / RPI;
+    constexpr int A_TAIL = AR % RPI, B_TAIL = BN % RPI;          // rows of a last, partial pass (0: none)
     static_assert(A_TAIL % 8 == 0 && B_TAIL % 8 == 0 && WM % 16 == 0 && WN % 16 == 0, "tile does not divide over the waves");
     typedef typename AccT<FMT>::type acc_t;
     constexpr bool F8 = FMT == GEMM_F8;
@@ -762,10 +767,10 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     int r_last = p.nr - 1, r_begin = 0;  // (r_begin: the range its first step lies in)
 
     static_assert(NS >= 2 && (NS - 1) * (A_IT + B_IT) < 64, "vmcnt holds 6 bits");
-    static_assert(!S8 || (NS == 2 && TN >= 3), "the e4m3 schedule reads two weight fragments ahead in a two-stage ring");
+    static_assert(!S8 || ((NS == 2 || MERGE) && TN >= 3), "the e4m3 schedule reads two weight fragments ahead in a two-stage ring");
     extern __shared__ __align__(16) uint8_t smem[];
-    uint8_t* const As = smem;                  // [NS][BM][128]
-    uint8_t* const Bs = smem + NS * BM * BK;   // [NS][BN][128]
+    uint8_t* const As = smem;                  // [NS][AR][128]
+    uint8_t* const Bs = smem + NS * AR * BK;   // [NS][BN][128]
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -818,7 +823,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
 #pragma unroll
     for (int i = 0; i < A_IT; ++i) {
         int row = s_row + i * RPI;
-        if constexpr (DUAL) row = row / WM * (WM / 2) + row % (WM / 2);
+        if constexpr (DUAL && !MERGE) row = row / WM * (WM / 2) + row % (WM / 2);
         a_goff[i] = (uint32_t)min(m0 + row, p.M - 1) * (uint32_t)p.lda + s_lc * 16;
     }
 #pragma unroll
@@ -827,11 +832,11 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     static_assert(!DUAL || ((MIX || RPI % WM == 0) && WM % 32 == 0), "a wave's eight rows of a pass come from one of the two tensors");
     const bool second = DUAL && (wave * 8) % WM >= WM / 2;
     uint32_t seconds = 0;  // MIX: the passes whose rows are of the second tensor
-    if constexpr (MIX) {
+    if constexpr (MIX && !MERGE) {
 #pragma unroll
         for (int i = 0; i < A_IT; ++i) seconds |= ((wave * 8 + i * RPI) % WM >= WM / 2 ? 1u : 0u) << i;
     }
-    uint32_t wanted = seconds | (((1u << B_IT) - 1u) << A_IT);  // MIX: the passes that a step of the plain range loads, activations then weights
+    uint32_t wanted = MERGE ? ~0u : seconds | (((1u << B_IT) - 1u) << A_IT);  // MIX: the passes that a step of the plain range loads, activations then weights
     // KT: pieces of a row past the end of K.  They are loaded from the step's first piece instead, which is there (a weight
     // row that holds a NaN gives NaN either way), and what they became in the activations is cleared before it is read.
     const int k_tail = KT ? (p.r[0].k1 - p.r[0].k0) % BK : 0;
@@ -843,7 +848,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
 #pragma unroll
                 for (int i = 0; i < A_IT; ++i)
                     if (!(A_TAIL != 0 && i == A_IT - 1 && s_row >= A_TAIL))
-                        *reinterpret_cast<uint4*>(As + buf * BM * BK + (s_row + i * RPI) * BK + (tid & 7) * 16) = make_uint4(0, 0, 0, 0);
+                        *reinterpret_cast<uint4*>(As + buf * AR * BK + (s_row + i * RPI) * BK + (tid & 7) * 16) = make_uint4(0, 0, 0, 0);
             }
             __syncthreads();
         }
@@ -858,8 +863,8 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         }
         if (i < A_IT) {
             if (i == A_IT - 1 && a_skip) return;
-            if constexpr (MIX && !decltype(plain_c)::value) ap += (seconds >> i) & 1u ? A2b - Ab : 0;
-            load16_to_lds(ap + (KT ? a_goff[i] - back : a_goff[i]), As + buf * BM * BK + w_lds + i * RPI * BK);
+            if constexpr (MIX && !MERGE && !decltype(plain_c)::value) ap += (seconds >> i) & 1u ? A2b - Ab : 0;
+            load16_to_lds(ap + (KT ? a_goff[i] - back : a_goff[i]), As + buf * AR * BK + w_lds + i * RPI * BK);
         } else {
             if (i == A_IT + B_IT - 1 && b_skip) return;
             load16_to_lds(bp + (KT ? b_goff[i - A_IT] - back : b_goff[i - A_IT]), Bs + buf * BN * BK + w_lds + (i - A_IT) * RPI * BK);
@@ -898,7 +903,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
 
 
     const int f_sw = swz(lrow);
-    const int a_frag = (wm * WM + lrow) * BK;
+    const int a_frag = (wm * (MERGE ? WM / 2 : WM) + lrow) * BK;
     const int b_frag = (wn * WN + lrow) * BK;
     // int8: two fragment sets, one per 64-byte K half of a step.  e4m3: one set of
     // 32-byte fragments (the 16 x 16 x 128 MFMA eats a whole step), whose registers
@@ -914,7 +919,8 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         // instead costs a two-way bank conflict on every read).
         const int off0 = (lgrp ^ f_sw) << 4;
         const int off1 = ((4 + lgrp) ^ f_sw) << 4;
-        const uint8_t* src = (i < TM) ? As + buf * BM * BK + a_frag + i * 16 * BK : Bs + buf * BN * BK + b_frag + (i - TM) * 16 * BK;
+        // (MERGE: fragment i of the second half is read, as it stands)
+        const uint8_t* src = (i < TM) ? As + buf * AR * BK + a_frag + (MERGE ? i - TM / 2 : i) * 16 * BK : Bs + buf * BN * BK + b_frag + (i - TM) * 16 * BK;
         const v4i lo = *reinterpret_cast<const v4i*>(src + off0);
         const v4i hi = *reinterpret_cast<const v4i*>(src + off1);
         const v8i f = v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
@@ -923,12 +929,26 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
       }
     };
 
+    // MERGE: dwords [d0, d1) of a fragment of codes of both signs -> those of the positive ones and of the negative ones, the
+    // others zero: four VALU instructions per dword
+    auto part = [&](int i, int d0, int d1) __attribute__((always_inline)) {
+        if constexpr (MERGE) {
+#pragma unroll
+            for (int d = d0; d < d1; ++d) {
+                const uint32_t v = (uint32_t)fa8[i + TM / 2][d];
+                const uint32_t mask = __builtin_amdgcn_perm(v, v << 8, 0x0B090A08u);  // every byte's sign, eight times
+                fa8[i][d] = (int)(v & ~mask);
+                fa8[i + TM / 2][d] = (int)(v & mask);
+            }
+        }
+    };
+
     // K half h of the tile in buffer buf -> fragment slot h, one 16-byte read at a
     // time: reads 0 .. TM-1 are the activation fragments, TM .. TM+TN-1 the weights
     auto frag1 = [&](int buf, int h, int i) {
         if constexpr (!S8) {
             const int off = ((h * 4 + lgrp) ^ f_sw) << 4;
-            if (i < TM) fa[h][i] = *reinterpret_cast<const v4i*>(As + buf * BM * BK + a_frag + i * 16 * BK + off);
+            if (i < TM) fa[h][i] = *reinterpret_cast<const v4i*>(As + buf * AR * BK + a_frag + i * 16 * BK + off);
             else fb[h][i - TM] = *reinterpret_cast<const v4i*>(Bs + buf * BN * BK + b_frag + (i - TM) * 16 * BK + off);
         }
     };
@@ -1088,7 +1108,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     // (DUAL: [1/sx | 1/sw | bias] of the first range, as the epilogue reads them, then [1/sx | 1/sw] of the second, MIX: and of
     // the third, zeros where this workgroup has no step of it)
     constexpr int EPI_FLOATS = MIX ? 3 * OM + 4 * BN : DUAL ? 2 * OM + 3 * BN : BM + 2 * BN, EPI_IT = (EPI_FLOATS + NT - 1) / NT;
-    float* const epi = reinterpret_cast<float*>(smem + NS * (BM + BN) * BK);
+    float* const epi = reinterpret_cast<float*>(smem + NS * (AR + BN) * BK);
     // group factors: a ring of four rows of BN floats behind the epilogue's vectors.  The row of
     // step s arrives with the step's operands and is read all through step s, at whose end the
     // row of step s + 2 is already on its way
@@ -1137,14 +1157,14 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
 #pragma unroll
     for (int t = 0; t < NS; ++t) {
         if (t < steps) {
-            if (MIX && t >= n_dual) dma(la + lk, Bb + lk, t, std::true_type{});
+            if (MIX && !MERGE && t >= n_dual) dma(la + lk, Bb + lk, t, std::true_type{});
             else dma(la + lk, Bb + lk, t, std::false_type{});
             dma_g();
             advance_load();
             ++issued;
         }
     }
-    if (issued == NS && !GRP && !(MIX && n_dual < NS)) wait_dma(std::integral_constant<int, NS - 1>{});
+    if (issued == NS && !GRP && !(MIX && !MERGE && n_dual < NS)) wait_dma(std::integral_constant<int, NS - 1>{});
     else wait_dma(std::integral_constant<int, 0>{});  // (with group factors and in plain steps the waves' DMA counts differ)
 #pragma unroll
     for (int i = 0; i < EPI_IT; ++i) {
@@ -1161,7 +1181,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     }
     if constexpr (S8) {
 #pragma unroll
-        for (int i = 0; i <= TM; ++i) frag8(0, i);  // activations and the first weight fragment
+        for (int i = MERGE ? TM / 2 : 0; i <= TM; ++i) frag8(0, i);  // activations and the first weight fragment
     } else {
         frags(0, 0);
     }
@@ -1212,12 +1232,17 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     // activation fragment right behind the last MFMA that reads it, with the DMA
     // of step s + 2 spread over the same MFMAs.
     // plain_c, dplain_c (MIX): this step, the one that it loads, is of the plain range: the second half of the row blocks only
+    [[maybe_unused]] bool tail_left = false;  // three stages: there is a step behind the next one
     auto step8 = [&](auto dma_c, auto more_c, auto plain_c, auto dplain_c) __attribute__((always_inline)) {
         constexpr bool DMA_ = decltype(dma_c)::value;
         constexpr bool MORE_ = decltype(more_c)::value;
         constexpr int B0 = decltype(plain_c)::value ? TM / 2 : 0;      // the first row block
         constexpr int NDM8 = A_IT + B_IT, TAIL = 2 * (TM - B0);  // DMA instructions over the tail's MFMAs
-        const int nbuf = buf ^ 1;
+        // row blocks in the order of their MFMAs: MERGE has the negative codes' in front, so that the blocks that are read
+        // for the next step, theirs, are free half a column block earlier
+        auto nth = [](int j) __attribute__((always_inline)) { return MERGE && B0 == 0 ? (j + TM / 2) % TM : j; };
+        constexpr int H = MERGE && B0 == 0 ? TM / 2 : 0;  // fragments to be parted, in column block 0
+        const int nbuf = NS == 2 ? buf ^ 1 : buf + 1 == NS ? 0 : buf + 1;
         auto lo4 = [](const v8i& f) __attribute__((always_inline)) { return v4i{f[0], f[1], f[2], f[3]}; };
         auto hi4 = [](const v8i& f) __attribute__((always_inline)) { return v4i{f[4], f[5], f[6], f[7]}; };
         const float* const gsrc = grw + cslot * BN + wn * WN + 4 * lgrp;
@@ -1245,29 +1270,42 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
             } else if constexpr (WS) {
                 // int8: the two 64-byte K halves of a block, TM MFMAs apart
 #pragma unroll
-                for (int b = B0; b < TM; ++b) {
-                    if (b == B0 && a == 0) frag8(buf, TM + 1);
-                    if (b == (TM > 1 ? B0 + 1 : 0)) frag8(buf, TM + a + 2);
+                for (int j = B0; j < TM; ++j) {
+                    const int b = nth(j);
+                    if (j == B0 && a == 0) frag8(buf, TM + 1);
+                    if (j == (TM > 1 ? B0 + 1 : 0)) frag8(buf, TM + a + 2);
+                    if (a == 0 && H > 0) {  // low halves in front of their MFMAs, high ones among the positive codes'
+                        if (j == 0) part(0, 0, 4);
+                        if (j + 1 < H) part(j + 1, 0, 4);
+                        else if (j + 1 > H) part(j - H, 4, 8);
+                    }
                     if constexpr (!F8) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo4(fb8[a]), lo4(fa8[b]), acc[a][b], 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
-                for (int b = B0; b < TM; ++b) {
+                for (int j = B0; j < TM; ++j) {
+                    const int b = nth(j);
                     if constexpr (!F8) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi4(fb8[a]), hi4(fa8[b]), acc[a][b], 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
 #pragma unroll
-                for (int b = B0; b < TM; ++b) {
-                    if (b == B0 && a == 0) frag8(buf, TM + 1);
-                    if (b == (TM > 1 ? B0 + 1 : 0)) frag8(buf, TM + a + 2);
+                for (int j = B0; j < TM; ++j) {
+                    const int b = nth(j);
+                    if (j == B0 && a == 0) frag8(buf, TM + 1);
+                    if (j == (TM > 1 ? B0 + 1 : 0)) frag8(buf, TM + a + 2);
+                    if (a == 0 && H > 0) {
+                        if (j == 0) part(0, 0, 8);
+                        if (j + 1 < H) part(j + 1, 0, 8);
+                    }
                     if constexpr (F8)
                         acc[a][b] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb8[a], fa8[b], acc[a][b], 0, 0, 0, 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
         }
-        wait_dma(std::integral_constant<int, 0>{});
+        if (NS > 2 && (!decltype(dplain_c)::value || tail_left)) wait_dma(std::integral_constant<int, NS - 2>{});
+        else wait_dma(std::integral_constant<int, 0>{});
         __syncthreads();
         if constexpr (KT && MORE_ && !DMA_) clear_tail(nbuf);  // (two stages: the next step is the last)
         const uint8_t* const ap = la + lk;
@@ -1307,9 +1345,10 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
                 if constexpr (!LAG) convert_block(a);
             } else if constexpr (WS) {
 #pragma unroll
-                for (int b = B0; b < TM; ++b) {
+                for (int l = B0; l < TM; ++l) {
+                    const int b = nth(l);
                     if constexpr (!F8) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo4(fb8[a]), lo4(fa8[b]), acc[a][b], 0, 0, 0);
-                    const int j = (a - (TN - 2)) * (TM - B0) + b - B0;
+                    const int j = (a - (TN - 2)) * (TM - B0) + l - B0;
                     if constexpr (DMA_) {
 #pragma unroll
                         for (int i = j * NDM8 / TAIL; i < (j + 1) * NDM8 / TAIL; ++i) dma1(ap, bp, buf, i, dplain_c);
@@ -1317,27 +1356,29 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
                     __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
-                for (int b = B0; b < TM; ++b) {
+                for (int l = B0; l < TM; ++l) {
+                    const int b = nth(l);
                     if constexpr (!F8) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi4(fb8[a]), hi4(fa8[b]), acc[a][b], 0, 0, 0);
                     if constexpr (MORE_) {
-                        if (a == TN - 2 && b == B0) frag8(nbuf, TM);  // next weight fragment 0: free since block 0
-                        if (a == TN - 1) frag8(nbuf, b);              // next activation fragment b: this was its last reader
+                        if (a == TN - 2 && l == B0) frag8(nbuf, TM);  // next weight fragment 0: free since block 0
+                        if (a == TN - 1 && (!MERGE || b >= TM / 2)) frag8(nbuf, b);              // next activation fragment b: this was its last reader
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
 #pragma unroll
-                for (int b = B0; b < TM; ++b) {
+                for (int l = B0; l < TM; ++l) {
+                    const int b = nth(l);
                     if constexpr (F8)
                         acc[a][b] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb8[a], fa8[b], acc[a][b], 0, 0, 0, 0, 0, 0);
-                    const int j = (a - (TN - 2)) * (TM - B0) + b - B0;
+                    const int j = (a - (TN - 2)) * (TM - B0) + l - B0;
                     if constexpr (DMA_) {
 #pragma unroll
                         for (int i = j * NDM8 / TAIL; i < (j + 1) * NDM8 / TAIL; ++i) dma1(ap, bp, buf, i, dplain_c);
                     }
                     if constexpr (MORE_) {
-                        if (a == TN - 2 && b == B0) frag8(nbuf, TM);  // next weight fragment 0: its registers were free since block 0
-                        if (a == TN - 1) frag8(nbuf, b);              // next activation fragment b: this was its last reader
+                        if (a == TN - 2 && l == B0) frag8(nbuf, TM);  // next weight fragment 0: its registers were free since block 0
+                        if (a == TN - 1 && (!MERGE || b >= TM / 2)) frag8(nbuf, b);              // next activation fragment b: this was its last reader
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -1443,10 +1484,12 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     if constexpr (MIX) {
         constexpr std::true_type yes{};
         constexpr std::false_type no{};
-        for (; s + 2 < n_dual; ++s) step8(yes, yes, no, no);
+        const int alike = MERGE ? min(n_dual, steps - NS) : n_dual - NS;  // (plain steps are loaded like MERGE's others)
+        for (; s < alike; ++s) step8(yes, yes, no, no);
         // from here on a step loads a plain one or, behind the last, none (what it reads of that goes nowhere)
         for (; s < n_dual; ++s) {
-            if (s + 2 >= steps) wanted = 0;
+            if (s + NS >= steps) wanted = 0;
+            tail_left = s + 2 < steps;
             step8(yes, yes, no, yes);
         }
         if (n_dual > 0) {  // the sums of both signs -> one, in output units
@@ -1465,7 +1508,8 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
             }
         }
         for (; s < steps; ++s) {
-            if (s + 2 >= steps) wanted = 0;
+            if (s + NS >= steps) wanted = 0;
+            tail_left = s + 2 < steps;
             step8(yes, yes, yes, yes);
         }
     }
@@ -1572,11 +1616,12 @@ int launch_wide_instance(const GemmParams& p, int64_t batch, hipStream_t st) {
 
 // wide tile ids (after the generic ones): 256x256 | 256x128 | 128x256 | 128x128, eight waves each
 template <int BM, int BN, int WGM, int WGN, int FMT, bool FOLD, int NS, bool GRP = false, bool PARK = false, bool FINISH = false,
-          bool CODES = false, bool SEP = false, bool KT = false, bool DUAL = false, bool MIX = false>
+          bool CODES = false, bool SEP = false, bool KT = false, bool DUAL = false, bool MIX = false,
+          bool MERGE = false>
 int launch_pipe_instance(const GemmParams& p, int64_t batch, hipStream_t st) {
-    auto kern = gemm_pipe_kernel<BM, BN, WGM, WGN, FMT, FOLD, NS, GRP, PARK, FINISH, CODES, SEP, KT, DUAL, MIX>;
+    auto kern = gemm_pipe_kernel<BM, BN, WGM, WGN, FMT, FOLD, NS, GRP, PARK, FINISH, CODES, SEP, KT, DUAL, MIX, MERGE>;
     // the stages, the epilogue's vectors, and the ring of group factors
-    constexpr int lds = NS * (BM + BN) * BK + (MIX ? BM / 2 * 3 + 4 * BN : DUAL ? BM + 3 * BN : BM + 2 * BN) * 4 + (GRP ? 4 * BN * 4 : 0);
+    constexpr int lds = NS * ((MERGE ? BM / 2 : BM) + BN) * BK + (MIX ? BM / 2 * 3 + 4 * BN : DUAL ? BM + 3 * BN : BM + 2 * BN) * 4 + (GRP ? 4 * BN * 4 : 0);
     if (p.dry) return SEGQ_OK;
     static unsigned long long attr_done = 0;
     if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), lds, &attr_done)) return rc;
@@ -1591,19 +1636,30 @@ int launch_walk(const GemmParams& p, int cfg, int64_t batch, hipStream_t st) {
     constexpr int WM = FMT == GEMM_F8 ? 4 : 2, WN = FMT == GEMM_F8 ? 2 : 4;  // (e4m3 wants three or more column blocks per wave)
 #define SEGQ_WALK(BM_, BN_, WGM_, WGN_, DUAL_) \
     return launch_pipe_instance<BM_, BN_, WGM_, WGN_, FMT, false, 2, false, false, false, false, false, true, DUAL_>(p, batch, st)
-#define SEGQ_MIX(BM_, BN_) \
-    return launch_pipe_instance<BM_, BN_, 4, 2, FMT, false, 2, false, false, false, false, false, false, true, true>(p, batch, st)
     switch (cfg) {
         case FIRST_KT_CFG: SEGQ_WALK(256, 256, 4, 2, false);
         case FIRST_KT_CFG + 1: SEGQ_WALK(256, 192, 4, 2, false);
         case FIRST_KT_CFG + 2: SEGQ_WALK(128, 128, WM, WN, false);
         case FIRST_DUAL_CFG: SEGQ_WALK(256, 192, 4, 2, true);
         case FIRST_DUAL_CFG + 1: SEGQ_WALK(128, 128, WM, WN, true);
+    }
+#undef SEGQ_WALK
+    return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: no kernel for tile %d", cfg + 1);
+}
+
+// DualScale's two ranges in whole steps and a plain range or none behind them.  From one tensor of codes of both signs a stage is a
+// third smaller, which leaves room for a third one: 9216 x 3072 x (3072 + 12288) e4m3 192 x 192 566 us, two stages 561;
+// 128 x 192 600 and 630, 1024 rows in two shares 75 and 77; int8 level.
+template <int FMT>
+int launch_mix(const GemmParams& p, int cfg, int64_t batch, hipStream_t st) {
+#define SEGQ_MIX(BM_, BN_)                                                                                                                       \
+    return p.r[0].a_sel ? launch_pipe_instance<BM_, BN_, 4, 2, FMT, false, 3, false, false, false, false, false, false, true, true, true>(p, batch, st) \
+                        : launch_pipe_instance<BM_, BN_, 4, 2, FMT, false, 2, false, false, false, false, false, false, true, true>(p, batch, st)
+    switch (cfg) {
         case FIRST_MIX_CFG: SEGQ_MIX(384, 192);
         case FIRST_MIX_CFG + 1: SEGQ_MIX(256, 256);
         case FIRST_MIX_CFG + 2: SEGQ_MIX(256, 192);
     }
-#undef SEGQ_WALK
 #undef SEGQ_MIX
     return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: no kernel for tile %d", cfg + 1);
 }

@@ -231,8 +231,8 @@ class SegmentLinear(nn.Module):
         """``nxt(op(self(x)))`` for two chained linears (an MLP's fc1 -> activation -> fc2) with the
         activation codes of ``nxt`` written by this layer's GEMM epilogue: the epilogue adds the
         bias, rounds to the layer dtype, applies ``pre_op`` ("gelu_tanh" | "gelu" | "silu" | None),
-        rounds again, and encodes with the static activation scale(s) of ``nxt`` (two code tensors
-        for DualScale), bit for bit what ``nxt``'s quantise kernel would have made of the stored
+        rounds again, and encodes with the static activation scale(s) of ``nxt`` (one or two code
+        tensors for DualScale), bit for bit what ``nxt``'s quantise kernel would have made of the stored
         tensor.  Neither this layer's float output is written nor a quantise launch reads it back.
         Not in the reference, which runs the activation as a torch operator on the full-size tensor
         and quantises it in a launch of its own (backend/torch/layers/activations.py:52-57 in front
@@ -243,7 +243,7 @@ class SegmentLinear(nn.Module):
         if nxt.in_features != self.out_features:
             raise RuntimeError(f"forward_into: {self.out_features} outputs feed a layer with {nxt.in_features} inputs")
         if getattr(opt, "writes_codes", None) and opt.writes_codes(x) and getattr(nopt, "accepts_codes", None) and nopt.accepts_codes():
-            spec = nopt.code_spec(x.device, pre_op)
+            spec = nopt.code_spec(x.device, pre_op, x.numel() // x.shape[-1], x.dtype)
             q, g, ws = opt.fused_launches(x, self.bias_data if self.bias else None, out_codes=spec)
             if ops_mod().recording_launches():
                 ops_mod().quantize_launch(q)

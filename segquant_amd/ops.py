@@ -412,7 +412,7 @@ def gemm_desc(a: torch.Tensor, b: torch.Tensor, ranges: Sequence[Range], *, m: i
             raise RuntimeError("out_codes needs a float out_dtype, one problem and no out tensor")
         oc = torch.empty((m, n), dtype=code_dtype(out_codes["fmt"]), device=a.device)
         if out_codes.get("scale_neg") is not None:
-            oc_neg = torch.empty_like(oc)
+            oc_neg = oc if out_codes.get("one_tensor") else torch.empty_like(oc)
     elif out is None:
         out = torch.empty((batch, m, n) if batch > 1 else (m, n), dtype=tdt, device=a.device)
     d = L.GemmDesc()
@@ -493,7 +493,7 @@ def gemm_desc(a: torch.Tensor, b: torch.Tensor, ranges: Sequence[Range], *, m: i
         d.finite_scales = 1
     info = dict(m=m, n=n, batch=batch, k_alg=k_alg, k_exec=k_exec, a_fmt=a_fmt, b_fmt=b_fmt)
     if oc is not None:
-        out = (oc, oc_neg) if oc_neg is not None else oc
+        out = (oc, oc_neg) if oc_neg is not None and oc_neg is not oc else oc
         info["codes_out"] = True
     return d, out, info, (a, b, a_neg, bias, workspace, group_dequant, addend, lowrank, out, out_codes, list(ranges))
 
@@ -574,6 +574,26 @@ def _dual_in_two_tensors(tiles: int, K: int, int4: bool) -> bool:
     if K > (256 if K % 128 else 512):
         return True
     return K % 128 == 0 and tiles >= 32 and (tiles < 96 or K >= 512)
+
+
+def dual_in_one_tensor(M: int, N: int, K: int, segments, fmt: str, dtype: torch.dtype) -> bool:
+    """Whether the library has, and takes, a kernel that parts the signs of DualScale codes in registers: ``segments`` are
+    (begin, end, DualScale or not) along K, their scales finite.  The descriptor's addresses are made up, nothing is launched."""
+    d = L.GemmDesc()
+    d.a_fmt = d.b_fmt = _CODE[fmt]
+    d.out_dtype = _dt(dtype)
+    d.m, d.n, d.lda, d.ldb, d.ldo, d.batch, d.finite_scales = M, N, K, K, N, 1, 1
+    d.a = d.b = d.out = d.workspace = 4096
+    d.workspace_bytes = 1 << 60
+    kinds = [(k0, k1, sel) for k0, k1, dual in segments for sel in ((2, 3) if dual else (0,))]
+    if not 1 < len(kinds) <= 3 or K % 16 or any(k0 % 128 or k1 % 128 for k0, k1, _ in kinds):
+        return False
+    d.n_ranges = len(kinds)
+    for r, (k0, k1, sel) in zip(d.ranges, kinds):
+        r.k_begin, r.k_len, r.a_sel, r.sx, r.sw = k0, k1 - k0, sel, 4096, 4096
+    tile = C.c_int32(0)
+    L.check(L.lib().segq_gemm_plan(C.byref(d), C.byref(tile), None, None))
+    return tile.value > 30
 
 
 @functools.lru_cache(maxsize=256)

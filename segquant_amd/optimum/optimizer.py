@@ -365,24 +365,22 @@ class DefaultOptimizer(BaseOptimizer):
                 raise RuntimeError(f"static per-token scales were calibrated for {pos.shape[-1]} tokens, got {M}")
         kstride = M if per_tok else 1
         mask = sum(1 << i for i, d in enumerate(self.dual_segments) if d)
-        # DualScale: two code tensors (Xp, Xn).  Reading plain codes lets both
-        # operands stream straight into LDS; the single merged tensor would save a
-        # third of the quantise traffic but costs the GEMM ~50 % (sign selection in
-        # registers), measured on the 4608 x 15360 x 3072 shape.  (The operator, whose
-        # shapes can be short and small, has a rule: ops._dual_in_two_tensors.)
+        one = dual and self._one_code_tensor(plan, M, x.dtype)
+        two = dual and not one
         q = ops.quantize_desc(x2, plan["fa"], pos, neg, row_stride=1 if per_tok else 0,
                               kseg_bounds=bounds if S > 1 else None, kseg_stride=kstride, dual=dual,
-                              dual_kseg_mask=mask, dynamic=dyn, two_tensors=dual, pre_op=pre_op, gate=gate,
+                              dual_kseg_mask=mask, dynamic=dyn, two_tensors=two, pre_op=pre_op, gate=gate,
                               col_div=col_div, col_div_rounded=own_div)
-        codes, codes_neg = q[1] if dual else (q[1], None)
+        codes, codes_neg = q[1] if two else (q[1], None)
         ranges = []
         for s in range(S):
             k0, k1 = bounds[s], bounds[s + 1]
             rs = 1 if per_tok else 0
             sw_s = plan["sw_list"][s] if "sw_list" in plan else plan["sw"]  # smoothed layers: one weight scale per K segment
-            ranges.append(ops.Range(k0, k1 - k0, pos[s], sw_s, 0, rs, plan["sw_cs"]))
-            if dual and self.dual_segments[s]:
-                ranges.append(ops.Range(k0, k1 - k0, neg[s], sw_s, 1, rs, plan["sw_cs"]))
+            d_s = dual and self.dual_segments[s]
+            ranges.append(ops.Range(k0, k1 - k0, pos[s], sw_s, 2 if d_s and one else 0, rs, plan["sw_cs"]))
+            if d_s:
+                ranges.append(ops.Range(k0, k1 - k0, neg[s], sw_s, 3 if one else 1, rs, plan["sw_cs"]))
         ldb = K // 2 if plan["fw"] == ops.FMT_INT4 else K
         gdq = plan.get("group_dequant")
         add2 = None if addend is None else addend.reshape(M, N).contiguous()
@@ -440,7 +438,7 @@ class DefaultOptimizer(BaseOptimizer):
             if len(cache) >= _MAX_CACHED_TOKEN_COUNTS:
                 cache.pop(next(iter(cache)))
             cache[(M, x.dtype, None if bias is None else bias.data_ptr())] = dict(
-                q=(q[0], q[2]), g=(g[0], g[2]), need=0 if ws is None else need, dyn=dyn, dual=dual, S=S, M=M, N=N, sx_src=sx_src,
+                q=(q[0], q[2]), g=(g[0], g[2]), need=0 if ws is None else need, dyn=dyn, dual=dual, two=two, S=S, M=M, N=N, sx_src=sx_src,
                 code_shape=tuple(codes.shape), code_dtype=codes.dtype, out_dtype=x.dtype, static=(pos, neg, bias))
         return q, g, ws
 
@@ -457,11 +455,29 @@ class DefaultOptimizer(BaseOptimizer):
         fa = _FMT[self.kernel_type.split("A", 1)[1]]
         return bool(one_range and plain and not cal.dynamic and cal.axis is None and fa in (ops.FMT_INT8, ops.FMT_E4M3))
 
-    def code_spec(self, device, pre_op=None) -> dict:
-        """What a producing GEMM needs to write this layer's codes (``ops.gemm_desc(out_codes=...)``)."""
+    def code_spec(self, device, pre_op=None, rows=None, dtype=None) -> dict:
+        """What a producing GEMM needs to write this layer's codes (``ops.gemm_desc(out_codes=...)``): ``rows`` of them for
+        outputs of ``dtype``, or, without these, DualScale in two tensors."""
         plan = self._plan or self._build_plan(device)
         pos, neg = self._static_sx(plan, device)
-        return dict(fmt=plan["fa"], scale=pos[0], scale_neg=neg[0] if self.dual_scale else None, pre_op=pre_op)
+        one = self.dual_scale and rows is not None and self._one_code_tensor(plan, rows, dtype)
+        return dict(fmt=plan["fa"], scale=pos[0], scale_neg=neg[0] if self.dual_scale else None, pre_op=pre_op, one_tensor=one)
+
+    def _one_code_tensor(self, plan, M, dtype) -> bool:
+        """Whether DualScale codes go into one tensor, whose signs the GEMM parts in registers, or into two, which stream
+        straight into its matrix instructions: one where the library has the kernel for it (8-bit codes, whole steps
+        of K, at most one plain segment beside the DualScale one) and would take it.  Asked once per token count.
+        GEMM 9216 x 3072 x (3072 + 12288) two / one: int8 622 / 599 us, e4m3 596 / 567, 1024 rows 79 / 79 and 75 / 75; and the
+        quantise step writes one tensor less (9216 x 12288 GELU'd, 90 / 68 us)."""
+        known = plan.setdefault("one_tensor", {})
+        one = known.get((M, dtype))
+        if one is None:
+            bounds = plan["bounds"]
+            S = self.chunks if self.seg_mode == "input" else 1
+            segments = tuple((bounds[s], bounds[s + 1], bool(self.dual_segments[s])) for s in range(S))
+            one = known[M, dtype] = (plan["fa"] == plan["fw"] and plan["fa"] != ops.FMT_INT4 and plan.get("group_dequant") is None and
+                                     "l2t" not in plan and ops.dual_in_one_tensor(M, plan["N"], plan["K"], segments, plan["fa"], dtype))
+        return one
 
     def writes_codes(self, x: torch.Tensor) -> bool:
         """Whether this layer's GEMM has the epilogue that writes codes for ``x``: plain 8-bit codes on
@@ -482,9 +498,10 @@ class DefaultOptimizer(BaseOptimizer):
         K, N = plan["K"], plan["N"]
         M = codes.shape[0]
         pos, neg = self._static_sx(plan, codes.device)
-        ranges = [ops.Range(0, K, pos[0], plan["sw"], 0, 0, plan["sw_cs"])]
+        one = self.dual_scale and codes_neg is None
+        ranges = [ops.Range(0, K, pos[0], plan["sw"], 2 if one else 0, 0, plan["sw_cs"])]
         if self.dual_scale:
-            ranges.append(ops.Range(0, K, neg[0], plan["sw"], 1, 0, plan["sw_cs"]))
+            ranges.append(ops.Range(0, K, neg[0], plan["sw"], 3 if one else 1, 0, plan["sw_cs"]))
         g = ops.gemm_desc(codes, plan["w"], ranges, m=M, n=N, a_fmt=plan["fa"], b_fmt=plan["fw"], out_dtype=out_dtype, lda=K,
                           ldb=K // 2 if plan["fw"] == ops.FMT_INT4 else K, bias=bias, a_neg=codes_neg,
                           group_dequant=plan.get("group_dequant"), finite_scales=self.dual_scale)
@@ -550,17 +567,19 @@ class DefaultOptimizer(BaseOptimizer):
                 raise RuntimeError(f"static per-token scales were calibrated for {pos.shape[-1]} tokens, got {M}")
         fa = plan["fa"]
         codes = torch.empty((M, K), dtype=ops.code_dtype(fa), device=dev)
-        codes_neg = torch.empty_like(codes) if dual else None
+        one = dual and self._one_code_tensor(plan, M, dt)
+        two = dual and not one
+        codes_neg = torch.empty_like(codes) if two else None
         ranges = []
         rs = 1 if per_tok else 0
         for s_, x2 in enumerate(xs):
             k0, k1 = bounds[s_], bounds[s_ + 1]
             d_s = bool(dual and self.dual_segments[s_])
-            ops.quantize(x2, fa, pos[s_], neg[s_] if d_s else None, row_stride=rs, dual=d_s, dynamic=dyn, two_tensors=d_s,
-                         out=codes[:, k0:k1], out_neg=codes_neg[:, k0:k1] if d_s else None, pre_op=pre_ops[s_])
-            ranges.append(ops.Range(k0, k1 - k0, pos[s_], plan["sw"], 0, rs, plan["sw_cs"]))
+            ops.quantize(x2, fa, pos[s_], neg[s_] if d_s else None, row_stride=rs, dual=d_s, dynamic=dyn, two_tensors=d_s and two,
+                         out=codes[:, k0:k1], out_neg=codes_neg[:, k0:k1] if d_s and two else None, pre_op=pre_ops[s_])
+            ranges.append(ops.Range(k0, k1 - k0, pos[s_], plan["sw"], 2 if d_s and one else 0, rs, plan["sw_cs"]))
             if d_s:
-                ranges.append(ops.Range(k0, k1 - k0, neg[s_], plan["sw"], 1, rs, plan["sw_cs"]))
+                ranges.append(ops.Range(k0, k1 - k0, neg[s_], plan["sw"], 3 if one else 1, rs, plan["sw_cs"]))
         g = ops.gemm_desc(codes, plan["w"], ranges, m=M, n=N, a_fmt=fa, b_fmt=plan["fw"], out_dtype=dt, lda=K,
                           ldb=K // 2 if plan["fw"] == ops.FMT_INT4 else K, bias=bias, a_neg=codes_neg, finite_scales=dual)
         int4 = plan["fw"] == ops.FMT_INT4
@@ -640,7 +659,7 @@ class DefaultOptimizer(BaseOptimizer):
             gd.workspace, gd.workspace_bytes = ws.data_ptr(), ws.numel()
         held = [codes, hit["static"]]
         result = codes
-        if hit["dual"]:
+        if hit.get("two", hit["dual"]):
             codes_neg = torch.empty_like(codes)
             qd.codes_neg = gd.a_neg = codes_neg.data_ptr()
             held.append(codes_neg)

@@ -251,14 +251,18 @@ def test_dual_ranges_with_finite_scales(ops, kind):
     assert took[300, False] == took[300, True] == took[400, False] == (True, False) and took[400, True] == (False, True)
 
 
-def _check_mix(ops, kind, M, N, K0, K1, tile, dt, g, shares=0, first=True, gap=0, empty=None, per_row=True, add=False, lend=True):
-    """DualScale's two ranges of K1 and a plain one of K0 (0: none; in front of or behind them in memory, `gap` apart)."""
+def _check_mix(ops, kind, M, N, K0, K1, tile, dt, g, shares=0, first=True, gap=0, empty=None, per_row=True, add=False, lend=True,
+               merged=False):
+    """DualScale's two ranges of K1 and a plain one of K0 (0: none; in front of or behind them in memory, `gap` apart), from two
+    code tensors or from one of both signs."""
     fa = FORMATS[kind][0]
     k0, k1 = (0, K0 + gap if K0 else gap) if first else (K1 + gap, 0)
     K = max(k0 + K0, k1 + K1)
     a, b = _codes(g, (M, K), fa), _codes(g, (N, K), fa)
     neg = _codes(g, (M, K), fa)  # (outside the pair it holds what is never read)
-    pick = g.random((M, K1)) < 0.5
+    pick = a[:, k1:k1 + K1].view(np.uint8) >= 0x80 if merged else g.random((M, K1)) < 0.5
+    if merged:
+        neg[:, k1:k1 + K1] = a[:, k1:k1 + K1]
     a[:, k1:k1 + K1][pick] = 0
     neg[:, k1:k1 + K1][~pick] = 0
     scale = lambda n: (g.random(n) * 30 + 10).astype(np.float32)
@@ -275,14 +279,17 @@ def _check_mix(ops, kind, M, N, K0, K1, tile, dt, g, shares=0, first=True, gap=0
         want += av @ bv.T / den
         mag += np.abs(av) @ np.abs(bv).T / den
     up = lambda t: torch.from_numpy(t).to(DEV)
-    rg = [ops.Range(k, n, up(s), up(w), int(c is neg), int(per_row), 1) for c, k, n, s, w in parts]
+    rg = [ops.Range(k, n, up(s), up(w), int(c is neg) + (2 if merged and k == k1 else 0), int(per_row), 1) for c, k, n, s, w in parts]
+    if merged:
+        a = a.copy()
+        a[:, k1:k1 + K1] |= neg[:, k1:k1 + K1]
     if first and K0:
         rg = rg[2:] + rg[:2]
     addend = None
     if add:
         addend = torch.randn(M, N, device=DEV).to(dt)
         want, mag = want + addend.double().cpu().numpy(), mag + addend.double().abs().cpu().numpy()
-    gd = ops.gemm_desc(_dev(a, fa), _dev(b, fa), rg, m=M, n=N, a_fmt=fa, b_fmt=fa, out_dtype=dt, lda=K, ldb=K, a_neg=_dev(neg, fa), finite_scales=True,
+    gd = ops.gemm_desc(_dev(a, fa), _dev(b, fa), rg, m=M, n=N, a_fmt=fa, b_fmt=fa, out_dtype=dt, lda=K, ldb=K, a_neg=None if merged else _dev(neg, fa), finite_scales=True,
                        bias=up(bias), addend=addend, tile=tile, split_k=shares)
     # (a workspace that holds NaN: nothing of it is read before it is written)
     ws = torch.full((ops.gemm_workspace_bytes(gd) // 4 + 4,), float("nan"), device=DEV).view(torch.uint8) if lend else None
@@ -300,24 +307,43 @@ def _check_mix(ops, kind, M, N, K0, K1, tile, dt, g, shares=0, first=True, gap=0
 
 @pytest.mark.parametrize("kind", ["int8", "e4m3"])
 @pytest.mark.parametrize("tile", [31, 32, 33, 0])
-def test_dual_and_plain_ranges_in_one_walk(ops, kind, tile):
+@pytest.mark.parametrize("merged", [False, True])
+def test_dual_and_plain_ranges_in_one_walk(ops, kind, tile, merged):
     """Edges of the tiles; one, two and three steps of either kind (the loop loads two ahead); shares that begin or end in the
     plain range; three ranges in any order; sides that hold nothing; rules that a workspace or none is given to."""
     g = np.random.default_rng(tile + 2)
     dts = (torch.float32, torch.bfloat16, torch.float16)
     for i, (M, N, k0, k1) in enumerate(((1, 16, 1, 1), (64, 128, 2, 1), (193, 130, 1, 2), (129, 257, 3, 3), (192, 192, 2, 5), (300, 500, 7, 4), (257, 70, 5, 2))):
         for lend in (False, True):
-            _check_mix(ops, kind, M, N, 128 * k0, 128 * k1, tile, dts[i % 3], g, first=bool(i % 2), lend=lend)
+            _check_mix(ops, kind, M, N, 128 * k0, 128 * k1, tile, dts[i % 3], g, first=bool(i % 2), lend=lend, merged=merged)
     for opt in (dict(empty=0), dict(empty=1), dict(empty=2), dict(per_row=False), dict(gap=128), dict(gap=128, first=False), dict(add=True)):
-        _check_mix(ops, kind, 140, 210, 384, 640, tile, torch.float32, g, **opt)
+        _check_mix(ops, kind, 140, 210, 384, 640, tile, torch.float32, g, merged=merged, **opt)
     if tile:
         for i, shares in enumerate((2, 3, 5, 9)):  # of 18, 5 and 4 steps: whole ranges, one step, less
             for k0, k1 in ((1024, 1280), (384, 256), (0, 512)):
-                _check_mix(ops, kind, 200, 300, k0, k1, tile, dts[i % 3], g, shares=shares, first=bool(i % 2), add=i == 1, empty=2 if i == 2 and k0 else None)
+                _check_mix(ops, kind, 200, 300, k0, k1, tile, dts[i % 3], g, shares=shares, first=bool(i % 2), add=i == 1, empty=2 if i == 2 and k0 else None,
+                           merged=merged)
     else:
         # the library's shares: two that meet, more that a second kernel sums; the pair alone; up to 128 rows its own choice is another
         for M, N, k0, k1, splits in ((1024, 3072, 512, 2048, (2, 3, 4)), (300, 640, 640, 4096, range(3, 17)), (600, 2048, 0, 8192, (3, 4, 5))):
-            assert _check_mix(ops, kind, M, N, k0, k1, 0, torch.bfloat16, g)["splits"] in splits
+            assert _check_mix(ops, kind, M, N, k0, k1, 0, torch.bfloat16, g, merged=merged)["splits"] in splits
+
+
+@pytest.mark.parametrize("kind", ["int8", "e4m3"])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_codes_of_both_signs_written_by_the_gemm(ops, kind, dt):
+    """The epilogue that writes a DualScale layer's codes into one tensor against the quantise launch that does, bit for bit."""
+    g = np.random.default_rng(23)
+    fa = FORMATS[kind][0]
+    for M, N, K, op in ((130, 208, 256, "gelu_tanh"), (1, 16, 128, None), (257, 272, 384, "silu")):
+        a, b = _dev(_codes(g, (M, K), fa), fa), _dev(_codes(g, (N, K), fa), fa)
+        s = [torch.full((1,), v, device=DEV) for v in (900.0, 3.0, 40.0, 900.0)]
+        kw = dict(m=M, n=N, a_fmt=fa, b_fmt=fa, out_dtype=dt, lda=K, ldb=K, bias=torch.randn(N, device=DEV))
+        rg = [ops.Range(0, K, s[0], s[1])]
+        want = ops.quantize(ops.gemm(a, b, rg, tile=14, **kw), fa, s[2], s[3], dual=True, pre_op=op)
+        got = ops.gemm(a, b, rg, out_codes=dict(fmt=fa, scale=s[2], scale_neg=s[3], pre_op=op, one_tensor=True), **kw)
+        got = got[0] if isinstance(got, tuple) else got
+        assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
 
 
 # ---- a linear of up to 16 rows in one launch ---------------------------------------------------------------------------------
