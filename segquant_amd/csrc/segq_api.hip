@@ -516,8 +516,9 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
                 const double now = walk.cfg < 0 ? in_turn_us(d->m, d->n, 2 * steps, f8, share)
                                    : walk.cfg == FIRST_DUAL_CFG ? std::ceil((double)tiles_of_cfg(FIRST_DUAL_CFG, d->m, d->n, 1) / cus) * (1.1 * k + 5.0)
                                    : t64 <= 1.0 ? 4.8 + 0.6 * k : 4.0 + t64 * (0.44 * k + 0.8);
-                // (one tensor: what the quantise step, which asks for this plan, then does not write)
-                take = take && pick.us < 0.95 * now + (d->ranges[0].a_sel == 2 ? (double)d->m * steps * 128 / 5e6 : 0.0);
+                // (one tensor: with what the quantise step, which asks for this plan, then does not write.  Feed-forward of 4096
+                // rows, 1536 x 6144 e4m3 through the epilogue that writes codes: two tensors 125 us a pass, one 121)
+                take = take && pick.us < (d->ranges[0].a_sel == 2 ? now + (double)d->m * steps * 128 / 5e6 : 0.95 * now);
             }
             if (take) {
                 walk.cfg = -1;

@@ -576,9 +576,11 @@ def _dual_in_two_tensors(tiles: int, K: int, int4: bool) -> bool:
     return K % 128 == 0 and tiles >= 32 and (tiles < 96 or K >= 512)
 
 
-def dual_in_one_tensor(M: int, N: int, K: int, segments, fmt: str, dtype: torch.dtype) -> bool:
+@functools.lru_cache(maxsize=256)
+def dual_in_one_tensor(device: int, M: int, N: int, K: int, segments, fmt: str, dtype: torch.dtype) -> bool:
     """Whether the library has, and takes, a kernel that parts the signs of DualScale codes in registers: ``segments`` are
-    (begin, end, DualScale or not) along K, their scales finite.  The descriptor's addresses are made up, nothing is launched."""
+    (begin, end, DualScale or not) along K, their scales finite.  Asked of the library once per shape (and device): the
+    descriptor's addresses are made up, nothing is launched."""
     d = L.GemmDesc()
     d.a_fmt = d.b_fmt = _CODE[fmt]
     d.out_dtype = _dt(dtype)

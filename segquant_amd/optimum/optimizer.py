@@ -476,7 +476,7 @@ class DefaultOptimizer(BaseOptimizer):
             S = self.chunks if self.seg_mode == "input" else 1
             segments = tuple((bounds[s], bounds[s + 1], bool(self.dual_segments[s])) for s in range(S))
             one = known[M, dtype] = (plan["fa"] == plan["fw"] and plan["fa"] != ops.FMT_INT4 and plan.get("group_dequant") is None and
-                                     "l2t" not in plan and ops.dual_in_one_tensor(M, plan["N"], plan["K"], segments, plan["fa"], dtype))
+                                     "l2t" not in plan and ops.dual_in_one_tensor(plan["w"].device.index or 0, M, plan["N"], plan["K"], segments, plan["fa"], dtype))
         return one
 
     def writes_codes(self, x: torch.Tensor) -> bool:
