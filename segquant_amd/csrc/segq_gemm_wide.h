@@ -85,7 +85,7 @@ __device__ __forceinline__ void codes_epilogue(const GemmParams& p, typename Acc
     const float s_pos = p.oc_scale[0];
     const float s_neg = dual ? p.oc_scale_neg[0] : s_pos;
     const bool bf = p.out_dtype == SEGQ_BF16;
-    const int dt = p.out_dtype, fmt = p.oc_fmt, op = p.oc_pre;
+    const int fmt = p.oc_fmt, op = p.oc_pre;
     constexpr int RS = WN * 2 + 16;  // patch row stride in bytes; the 16 spreads the rows over the banks
     constexpr int CH = WN / 8;       // 8-element pieces per patch row
     __syncthreads();                 // the operand tiles are dead from here on
@@ -105,12 +105,27 @@ __device__ __forceinline__ void codes_epilogue(const GemmParams& p, typename Acc
             const int n = n0 + wn * WN + col * 8;
             if (mm >= p.M || n >= p.N) continue;
             const int64_t e = (int64_t)mm * p.ldoc + n;
-            float cp[8], cn[8];
+            float t8[8], cp[8], cn[8];
+            auto widen = [&](const uint32_t (&q)[4]) __attribute__((always_inline)) {
+                if (bf) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) t8[i] = __uint_as_float((i & 1) ? (q[i >> 1] & 0xffff0000u) : (q[i >> 1] << 16));
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) t8[i] = f16_bits_to_f32((i & 1) ? (q[i >> 1] >> 16) : (q[i >> 1] & 0xffffu));
+                }
+            };
+            widen(w);
+            if (op != SEGQ_PRE_NONE) {
+                act_values(op, t8);
+                uint32_t q[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) q[i] = bf ? pack2_bf16(t8[2 * i], t8[2 * i + 1]) : pack2_f16(t8[2 * i], t8[2 * i + 1]);
+                widen(q);
+            }
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const uint32_t h = (i & 1) ? (w[i >> 1] >> 16) : (w[i >> 1] & 0xffffu);
-                float t = bf ? bf16_bits_to_f32(h) : f16_bits_to_f32(h);
-                if (op != SEGQ_PRE_NONE) t = round_to(dt, act_value(op, t));
+                float t = t8[i];
                 // x >= 0 takes the positive scale; in two tensors the branch not taken holds code(0)
                 // (segquant/src/real_quant/quantizer.cuh:193-203).  Without DualScale: one scale for both signs.
                 const bool pos = t >= 0.0f;

@@ -199,28 +199,29 @@ __device__ __forceinline__ void f32_to_raw(const float (&v)[16], RawRun<DT>& r) 
     }
 }
 
-// r holds 16 elements of x at (row, col); on return it holds what is quantised:
+template <int DT>
+__device__ __forceinline__ void load_gate(const QuantParams& p, int64_t row, int64_t col, RawRun<DT>& g) {
+    const size_t esz = (DT == SEGQ_F32) ? 4 : 2;
+    if (p.gate) load_raw<DT>(static_cast<const uint8_t*>(p.gate) + (row * p.ldg + col) * esz, g);
+}
+
+// r holds 16 elements of x at (row, col), gr those of the gate if there is one; on return r holds what is quantised:
 // op(x), or x * op(gate), each operator's result rounded to the tensor's dtype
 template <int DT>
-__device__ __forceinline__ void pre_run(const QuantParams& p, int64_t row, int64_t col, RawRun<DT>& r) {
+__device__ __forceinline__ void pre_run(const QuantParams& p, int64_t col, RawRun<DT>& r, RawRun<DT>& gr) {
     float v[16];
     raw_to_f32<DT>(r, v);
     if (p.pre_op != SEGQ_PRE_NONE) {
         if (p.gate) {
-            const size_t esz = (DT == SEGQ_F32) ? 4 : 2;
-            RawRun<DT> gr;
-            load_raw<DT>(static_cast<const uint8_t*>(p.gate) + (row * p.ldg + col) * esz, gr);
             float g[16];
             raw_to_f32<DT>(gr, g);
-#pragma unroll
-            for (int i = 0; i < 16; ++i) g[i] = act_value(p.pre_op, g[i]);
+            act_values(p.pre_op, g);
             f32_to_raw<DT>(g, gr);
             raw_to_f32<DT>(gr, g);
 #pragma unroll
             for (int i = 0; i < 16; ++i) v[i] *= g[i];
         } else {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = act_value(p.pre_op, v[i]);
+            act_values(p.pre_op, v);
         }
         if (p.col_div) {  // the activation's result is rounded to the dtype before it is divided
             f32_to_raw<DT>(v, r);
@@ -246,7 +247,11 @@ template <int DT, bool PRE>
 __device__ __forceinline__ void load_run(const QuantParams& p, const uint8_t* xrow, int64_t row, int c, RawRun<DT>& r) {
     const size_t esz = (DT == SEGQ_F32) ? 4 : 2;
     load_raw<DT>(xrow + (size_t)c * 16 * esz, r);
-    if constexpr (PRE) pre_run<DT>(p, row, (int64_t)c << 4, r);
+    if constexpr (PRE) {
+        RawRun<DT> g;
+        load_gate<DT>(p, row, (int64_t)c << 4, g);
+        pre_run<DT>(p, (int64_t)c << 4, r, g);
+    }
 }
 
 // Maximum of two non-negative floats, taken on their encodings: non-negative floats are ordered
@@ -527,7 +532,9 @@ __global__ void __launch_bounds__(256) quant_static_kernel(const QuantParams p) 
     if constexpr (PRE) {
         RawRun<DT> r;
         load_raw<DT>(static_cast<const uint8_t*>(p.x) + (row * p.ldx + col) * esz, r);
-        pre_run<DT>(p, row, col, r);
+        RawRun<DT> g;
+        load_gate<DT>(p, row, col, g);
+        pre_run<DT>(p, col, r, g);
         raw_to_f32<DT>(r, x);
     } else {
         load16<DT>(static_cast<const uint8_t*>(p.x) + (row * p.ldx + col) * esz, x);
@@ -622,9 +629,9 @@ static int launch_quant(const QuantParams& p, hipStream_t st) {
         }
         // A run per thread wherever that many waves of many rows fit the chip at a time: rows of up to 4096 elements, longer
         // ones while there are at most three workgroups per CU.  One wave per row does its runs one after the other, with
-        // the activation function in front of each (bf16, x gelu(gate), us, wave per row / this: 400 x 5120 17.7 / 7.2, 1000 x
-        // 1280 9.0 / 6.7, 8192 x 2560 37.4 / 35.7; 8192 x 5120 61.7 / 94.8, where a workgroup's waves wait for each other
-        // with too few workgroups on the CU).  Rows of 8192 have all four runs of 256 threads (600 rows 9.0, this 9.9).
+        // the activation function in front of each (bf16, x gelu(gate), us, wave per row / this: 400 x 5120 17.7 / 6.0, 1000 x
+        // 1280 9.0 / 6.7, 8192 x 2560 37.4 / 27.5; 2048 x 5120 16.4 / 20.8, 8192 x 5120 49 / 75, where a workgroup's waves wait for
+        // each other with too few workgroups on the CU).  Rows of 8192 have all four runs of 256 threads (600 rows 9.0, this 9.9).
         // A wave per row is level with this or ahead of it where
         //  - the rows of the launch are resident at once that way, and the producer is short: 2048 x 3072 bf16 with column
         //    factors 9.6, this 10.3 (DualScale 11.9 and 13.3, 8192 rows 31.7 and 34.1); with an activation from ten rows per CU on;
@@ -646,8 +653,14 @@ static int launch_quant(const QuantParams& p, hipStream_t st) {
         } else if (longest <= 64 * 8 && longest % 256 != 0) {
             // rows a workgroup's 256 threads would share unevenly (320 runs: a quarter of the threads
             // with two, the rest with one) stay with one wave per row
-            if (p.dual) hipLaunchKernelGGL((quant_dynamic_wave_kernel<DT, FMT, 8, true, PRE>), wgrid, dim3(256), 0, st, p);
-            else hipLaunchKernelGGL((quant_dynamic_wave_kernel<DT, FMT, 8, false, PRE>), wgrid, dim3(256), 0, st, p);
+            // (six runs per lane where they do: 4096 x 5120 x gelu(gate) 27.4 us, eight 28.3)
+            if (longest <= 64 * 6) {
+                if (p.dual) hipLaunchKernelGGL((quant_dynamic_wave_kernel<DT, FMT, 6, true, PRE>), wgrid, dim3(256), 0, st, p);
+                else hipLaunchKernelGGL((quant_dynamic_wave_kernel<DT, FMT, 6, false, PRE>), wgrid, dim3(256), 0, st, p);
+            } else {
+                if (p.dual) hipLaunchKernelGGL((quant_dynamic_wave_kernel<DT, FMT, 8, true, PRE>), wgrid, dim3(256), 0, st, p);
+                else hipLaunchKernelGGL((quant_dynamic_wave_kernel<DT, FMT, 8, false, PRE>), wgrid, dim3(256), 0, st, p);
+            }
         } else {
             if (p.dual) hipLaunchKernelGGL((quant_dynamic_kernel<DT, FMT, 4, true, PRE>), bgrid, dim3(256), 0, st, p);
             else hipLaunchKernelGGL((quant_dynamic_kernel<DT, FMT, 4, false, PRE>), bgrid, dim3(256), 0, st, p);
