@@ -492,11 +492,11 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         const bool lent = ws && al(ws, 16);
         auto shares_fit = [&](int c, int n_) { return lent && ws_bytes >= mix_bytes(d->m, d->n, c, n_); };
         const int64_t steps = ok ? d->ranges[mix.neg].k_len / 128 : 0, plain = ok && mix.plain >= 0 ? d->ranges[mix.plain].k_len / 128 : 0;
-        if (d->tile > FIRST_MIX_CFG && d->tile <= NUM_TILE_CFG) {
+        if (d->tile > FIRST_MIX_CFG && d->tile <= FIRST_LR_CFG) {
             if (!ok)
                 return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: tiles %d to %d serve two ranges over the same run of K from a and a_neg, and one plain range "
                                                   "beside them, in plain 8-bit codes and whole steps of 128, one problem, without group factors, a low-rank "
-                                                  "branch or codes out", FIRST_MIX_CFG + 1, NUM_TILE_CFG);
+                                                  "branch or codes out", FIRST_MIX_CFG + 1, FIRST_LR_CFG);
             mix.cfg = (int)d->tile - 1;
             if (d->split_k > 1) {
                 mix.shares = (int)(d->split_k < steps + plain / 2 ? d->split_k : steps + plain / 2);  // (a step at least for each)
@@ -732,6 +732,9 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     }
     else if (d->tile >= 1 && d->tile <= NUM_TILE_CFG) cfg = d->tile - 1;
     else return fail(SEGQ_ERR_ARG, "segq_gemm: tile %d is not in 0..%d", d->tile, NUM_TILE_CFG);
+    if (cfg >= FIRST_MIX_CFG && (cfg < FIRST_LR_CFG || !lowrank || fold))
+        return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: tiles %d to %d serve a low-rank branch beside one range, %d to %d DualScale", FIRST_LR_CFG + 1, NUM_TILE_CFG,
+                    FIRST_MIX_CFG + 1, FIRST_LR_CFG);
     // Few tokens: when the 128 x 128 tiles do not even fill the CUs once, a workgroup has its CU to
     // itself and waits on HBM latency: the int8 kernel with four LDS stages keeps three K steps in
     // flight instead of one (256 x 9216 x 1536: 14.8 -> 12.9 us, 512 x 6144 x 3072: 25.5 -> 20.4 us)
@@ -892,7 +895,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     // tiles are numbered down groups of this many tile rows, so that the 32 tiles an XCD holds at a time
     // share few operand panels; 384-row tiles reach that with half as many rows (e4m3 4608 x 12288 x 3072
     // 140.7 -> 136.2 us; other heights between 2 and 16 measured the same or worse on the 4608-token shapes)
-    p.group_m = (cfg == FIRST_WIDE_CFG + 9) ? 4 : 8;
+    p.group_m = (cfg == FIRST_WIDE_CFG + 9 || cfg == FIRST_LR_CFG + 2) ? 4 : 8;
     {
         // e4m3 rescaled in place only (4608 x 15360 x 3072 in three ranges: 350 -> 338 us); int8, which parks its
         // sums at the boundaries, loses more to the XCDs reading different operand columns at a time than it gains

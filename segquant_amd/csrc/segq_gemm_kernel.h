@@ -535,13 +535,14 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_kernel(const GemmParams p)
 
 // ---- host-side launch of one (format, tile, fold) instance -------------------
 struct TileCfg { int bm, bn, wgm, wgn; };
-constexpr int NUM_TILE_CFG = 33;
+constexpr int NUM_TILE_CFG = 36;
 constexpr int FIRST_BIG_CFG = 8;    // two retired ids (a 4-wave 256 x 256 kernel that no shape profited from)
 constexpr int FIRST_WIDE_CFG = 10;  // the 8-wave kernels from here on (segq_gemm_wide.h)
 constexpr int FIRST_FEW_CFG = 21;   // tiles whose waves share K (segq_gemm_few.h)
 constexpr int FIRST_KT_CFG = 25;    // 8-wave tiles for one range with a ragged end of K
 constexpr int FIRST_DUAL_CFG = 28;  // ... and for DualScale's two ranges in one walk (rows of each code tensor x columns)
 constexpr int FIRST_MIX_CFG = 30;   // ... and a plain range behind the two (rows x columns of the output)
+constexpr int FIRST_LR_CFG = 33;    // the largest 8-wave tiles with the low-rank branch
 constexpr TileCfg TILE_CFGS[NUM_TILE_CFG] = {
     {256, 256, 2, 2}, {256, 128, 2, 2}, {128, 128, 2, 2}, {64, 128, 2, 2}, {128, 256, 2, 2},
     {256, 256, 2, 4}, {256, 256, 4, 2}, {256, 128, 4, 2}, {256, 256, 2, 2}, {256, 256, 2, 2},
@@ -549,7 +550,7 @@ constexpr TileCfg TILE_CFGS[NUM_TILE_CFG] = {
     {256, 192, 4, 2}, {192, 256, 2, 4}, {128, 128, 2, 4}, {384, 192, 4, 2}, {128, 96, 4, 2},
     {16, 32, 1, 1}, {16, 64, 1, 1}, {32, 32, 1, 1}, {32, 64, 1, 1},
     {256, 256, 4, 2}, {256, 192, 4, 2}, {128, 128, 2, 4}, {128, 192, 4, 2}, {64, 128, 2, 4},
-    {192, 192, 4, 2}, {128, 256, 4, 2}, {128, 192, 4, 2},
+    {192, 192, 4, 2}, {128, 256, 4, 2}, {128, 192, 4, 2}, {192, 288, 4, 2}, {288, 192, 2, 4}, {384, 192, 4, 2},
 };
 
 // Steps in flight of the general kernel's 64 x 128 and 128 x 128 tiles, one range (every other launch: one step ahead;

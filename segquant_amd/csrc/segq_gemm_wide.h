@@ -601,17 +601,26 @@ __device__ __forceinline__ void lowrank_accumulate(const GemmParams& p, v4f (&of
             const int64_t m = min(m_row0 + b * 16 + lrow, p.M - 1);
             tf[b] = *reinterpret_cast<const uint4*>(p.lr_t + m * p.lr_ldt + kk + lgrp * 8);
         }
+        // (half of the column blocks' loads at a time, in front of their products: one by one, every block waited for L2
+        // behind the block before it; all at once, registers)
+        constexpr int CH = (TN + 1) / 2;
 #pragma unroll
-        for (int a = 0; a < TN; ++a) {
-            const int64_t n = min(n_col0 + a * 16 + lrow, p.N - 1);
-            const uint4 lf = *reinterpret_cast<const uint4*>(p.lr_l2 + n * p.lr_ldl + kk + lgrp * 8);
+        for (int a0 = 0; a0 < TN; a0 += CH) {
+            uint4 lf[CH];
 #pragma unroll
-            for (int b = 0; b < TM; ++b) {
-                if (bf)
-                    of[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, lf), __builtin_bit_cast(v8bf, tf[b]), of[a][b], 0, 0, 0);
-                else
-                    of[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, lf), __builtin_bit_cast(v8h, tf[b]), of[a][b], 0, 0, 0);
+            for (int a = a0; a < TN && a < a0 + CH; ++a) {
+                const int64_t n = min(n_col0 + a * 16 + lrow, p.N - 1);
+                lf[a - a0] = *reinterpret_cast<const uint4*>(p.lr_l2 + n * p.lr_ldl + kk + lgrp * 8);
             }
+#pragma unroll
+            for (int a = a0; a < TN && a < a0 + CH; ++a)
+#pragma unroll
+                for (int b = 0; b < TM; ++b) {
+                    if (bf)
+                        of[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, lf[a - a0]), __builtin_bit_cast(v8bf, tf[b]), of[a][b], 0, 0, 0);
+                    else
+                        of[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, lf[a - a0]), __builtin_bit_cast(v8h, tf[b]), of[a][b], 0, 0, 0);
+                }
         }
     }
 }
@@ -1543,6 +1552,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         //  * a tile split in two along K: the two workgroups meet in the workspace (below);
         //  * low-rank branch (out += T L2): the product joins in fp32 on the matrix cores;
         // and the epilogue only adds the bias and the addend and rounds once.
+        constexpr bool MEET = BM % 128 == 0 ? BN != 192 || BM == 256 : BN == 256;  // (tail_tile() of the dispatch: no K shares on the largest)
         v4f of[TN][TM];
         [[maybe_unused]] const bool parked = r_begin < r_last;
         // blocks whose loads are in flight at once (registers: the sums are still live).  What is parked comes back in two
@@ -1575,7 +1585,9 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (p.part && !meet_share<NT, CH>(p, of, tile_id, zy, tid, reinterpret_cast<int*>(epi))) return;
+        if constexpr (MEET) {
+            if (p.part && !meet_share<NT, CH>(p, of, tile_id, zy, tid, reinterpret_cast<int*>(epi))) return;
+        }
         if (p.lr_rank > 0) lowrank_accumulate<TM, TN>(p, of, m0 + wm * WM, n0 + wn * WN, lane);
         wide_epilogue<BM, BN, WGM, WGN, GEMM_F8, false, true>(p, of, of, smem, z, m0, n0, wave, lane, r_epi, epi);
         return;
@@ -1674,6 +1686,10 @@ int launch_mix(const GemmParams& p, int cfg, int64_t batch, hipStream_t st) {
         case FIRST_MIX_CFG: SEGQ_MIX(384, 192);
         case FIRST_MIX_CFG + 1: SEGQ_MIX(256, 256);
         case FIRST_MIX_CFG + 2: SEGQ_MIX(256, 192);
+        // the three largest tiles of one range with the low-rank branch
+        case FIRST_LR_CFG: return launch_pipe_instance<192, 288, 4, 2, FMT, false, 2, false, false, true>(p, batch, st);
+        case FIRST_LR_CFG + 1: return launch_pipe_instance<288, 192, 2, 4, FMT, false, 2, false, false, true>(p, batch, st);
+        case FIRST_LR_CFG + 2: return launch_pipe_instance<384, 192, 4, 2, FMT, false, 2, false, false, true>(p, batch, st);
     }
 #undef SEGQ_MIX
     return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: no kernel for tile %d", cfg + 1);
@@ -1748,9 +1764,7 @@ int launch_wide(const GemmParams& p, int wcfg, bool fold, bool asel, int64_t bat
                             return launch_pipe_instance<128, 128, 2, 4, FMT, false, 4, false, false, false>(p, batch, st);
                         }
                         break;
-                    case 9:  // wave tiles of 96 x 96
-                        if (tail) break;
-                        return launch_pipe_instance<384, 192, 4, 2, FMT, false, 2, false, false, false>(p, batch, st);
+                    case 9: SEGQ_PIPE1(384, 192, 4, 2, false, false);  // wave tiles of 96 x 96
                     case 10:  // 128 x 96, five LDS stages: few tokens, more workgroups with four K steps in flight each
                         if constexpr (!F8W) {
                             if (tail) break;

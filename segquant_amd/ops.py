@@ -297,7 +297,7 @@ def gemm_workspace_bytes(g) -> int:
 TILE_SHAPES = {1: "256x256", 2: "256x128", 3: "128x128", 4: "64x128", 5: "128x256", 6: "256x256", 7: "256x256", 8: "256x128",
                11: "256x256", 12: "256x128", 13: "128x256", 14: "128x128", 15: "192x288", 16: "288x192", 17: "256x192", 18: "192x256", 19: "128x128", 20: "384x192", 21: "128x96",
                22: "16x32", 23: "16x64", 24: "32x32", 25: "32x64",
-               26: "256x256", 27: "256x192", 28: "128x128", 29: "128x192", 30: "64x128", 31: "192x192", 32: "128x256", 33: "128x192"}
+               26: "256x256", 27: "256x192", 28: "128x128", 29: "128x192", 30: "64x128", 31: "192x192", 32: "128x256", 33: "128x192", 34: "192x288", 35: "288x192", 36: "384x192"}
 
 
 def gemm_plan(g, workspace: Optional[torch.Tensor] = None) -> dict:
@@ -312,6 +312,20 @@ def gemm_plan(g, workspace: Optional[torch.Tensor] = None) -> dict:
     family = "gemm_few_kernel" if 22 <= tile.value <= 25 else "gemm_pipe_kernel" if tile.value >= 11 else "gemm_kernel"
     return dict(tile=tile.value, shape=TILE_SHAPES.get(tile.value, "?"), splits=splits.value, parked=bool(parked.value),
                 kernel=f"segq::{family}<{TILE_SHAPES.get(tile.value, '?').replace('x', ',')}>")
+
+
+def lowrank_tile(g) -> int:
+    """The tile on which the launch ``g`` takes a low-rank branch (0: the library's choice for it): the one it has without,
+    where that is one of the three largest and fills its rounds of the compute units, 4608 tokens say.  us, the library's
+    choice / this, rank 32, int8 | e4m3: 4608 x 12288 x 3072 178 / 161 | 180 / 150; 4608 x 9216 x 3072 133 / 125 | 132 / 120;
+    2304 x 12288 x 3072 88 / 85; rank 64, 4500 x 12000 x 3072 197 / 179; 2000 x 10240 x 2048, rounds filled to 77 %, 62 / 66."""
+    tile = gemm_plan(g)["tile"]
+    if tile not in (15, 16, 20):
+        return 0
+    rows, cols = map(int, TILE_SHAPES[tile].split("x"))
+    cus = torch.cuda.get_device_properties(g[1].device).multi_processor_count
+    tiles = -(-g[0].m // rows) * -(-g[0].n // cols)
+    return {15: 34, 16: 35, 20: 36}[tile] if tiles >= 0.9 * cus * -(-tiles // cus) else 0
 
 
 def gemm_launch(g, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -391,15 +391,18 @@ class DefaultOptimizer(BaseOptimizer):
             # the SVD optimiser's low-rank branch: inside the GEMM's epilogue where the library has a
             # kernel for it (16-bit dtypes, the 8-wave kernels), as a materialised (M, N) addend otherwise
             t_lr, l2t = self._lowrank_operands(plan, x2)
-            ok = plan.setdefault("lr_ok", {}).get((M, x.dtype))
+            key = (M, x.dtype)
+            ok, tiles = plan.setdefault("lr_ok", {}).get(key), plan.setdefault("lr_tile", {})
             if ok is None or ok:
                 try:
-                    g = ops.gemm_desc(codes, plan["w"], ranges, addend=add2, lowrank=(t_lr, l2t), **kw)
+                    if ok is None:
+                        tiles[key] = ops.lowrank_tile(ops.gemm_desc(codes, plan["w"], ranges, **kw)) if len(ranges) == 1 else 0
+                    g = ops.gemm_desc(codes, plan["w"], ranges, addend=add2, lowrank=(t_lr, l2t), tile=tiles[key], **kw)
                     if ok is None:
                         ops.gemm_plan(g)
                 except RuntimeError:
                     g = None
-                plan["lr_ok"][(M, x.dtype)] = g is not None
+                plan["lr_ok"][key] = g is not None
             if g is None:
                 low = t_lr @ l2t.t()
                 add2 = low if add2 is None else add2 + low

@@ -730,6 +730,31 @@ def test_group_factors_on_the_big_tiles(ops, M, N, K, tile):
             assert np.abs(_np(out).astype(np.float64) - want).max() <= (len(groups) + 5) * 2.0 ** -24 * most
 
 
+@pytest.mark.parametrize("fmt", [O.FMT_INT8, O.FMT_E4M3])
+@pytest.mark.parametrize("tile", [34, 35, 36])
+def test_low_rank_branch_on_the_largest_tiles(ops, fmt, tile):
+    """The low-rank branch on 192 x 288, 288 x 192 and 384 x 192, at their edges; refused without one and with several ranges."""
+    g = np.random.default_rng(tile)
+    for M, N, K, rank, dt in ((1, 16, 128, 32, "bf16"), (193, 290, 256, 64, "fp16"), (385, 191, 384, 96, "bf16"), (288, 384, 128, 32, "fp16")):
+        a, b = (g.integers(-128, 128, size=n).astype(np.int8) if fmt == O.FMT_INT8 else _e4m3_codes(g, n) for n in ((M, K), (N, K)))
+        sx, sw = ((g.random(n) * 50 + 20).astype(np.float32) for n in (M, N))
+        bias = torch.randn(N)
+        t_lr, l2t = ((torch.randn(n, rank) * 0.5).to(TDT[dt]) for n in (M, N))
+        base = O.code_values(a, fmt).astype(np.float64) @ O.code_values(b, fmt).astype(np.float64).T / (sx[:, None].astype(np.float64) * sw[None, :])
+        want = base + bias.double().numpy() + t_lr.double().numpy() @ l2t.double().numpy().T
+        up = lambda t: torch.from_numpy(t).to(DEV)
+        rg = [ops.Range(0, K, up(sx), up(sw), 0, 1, 1)]
+        kw = dict(m=M, n=N, a_fmt=fmt, b_fmt=fmt, out_dtype=TDT[dt], lda=K, ldb=K, bias=bias.to(DEV), tile=tile)
+        got = ops.gemm(up(a), up(b), rg, lowrank=(t_lr.to(DEV), l2t.to(DEV)), **kw).double().cpu().numpy()
+        # the output's one rounding; the fp32 sums (e4m3: the matrix cores' limited-width adder)
+        tol = {"bf16": 2.0 ** -8, "fp16": 2.0 ** -11}[dt] * np.abs(want) + (3e-4 if fmt == O.FMT_E4M3 else 1e-5) * np.abs(want).max()
+        assert (np.abs(got - want) <= tol).all(), (M, N, K, rank)
+    with pytest.raises(RuntimeError):
+        ops.gemm(up(a), up(b), rg, **kw)
+    with pytest.raises(RuntimeError):
+        ops.gemm(up(a), up(b), rg + rg, lowrank=(t_lr.to(DEV), l2t.to(DEV)), **kw)
+
+
 @pytest.mark.parametrize("fmt_w", [O.FMT_INT4, O.FMT_INT8])
 @pytest.mark.parametrize("dt", ["fp32", "bf16"])
 def test_group_wise_weight_scales(ops, fmt_w, dt):
