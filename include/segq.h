@@ -328,6 +328,12 @@ typedef struct segq_gemm_desc {
 
 int segq_gemm(const segq_gemm_desc* d, segq_stream_t stream);
 
+/* t[i][j] = sum over k of x[i][k] l1t[j][k], summed in fp32 and rounded once to dtype (SEGQ_F16 | SEGQ_BF16, of all three): the
+ * lowrank_t operand of segq_gemm from the layer's input and the transposed first factor (segquant/optimum/optimizer.py:698-722
+ * multiplies them with a library).  k a multiple of 64, r of 16; rows of x and l1t 16-byte aligned; strides in elements. */
+int segq_lowrank_rows(const void* x, int64_t ldx, const void* l1t, int64_t ld_l1t, void* t, int64_t ldt, int64_t m, int64_t k, int64_t r, int32_t dtype,
+                      segq_stream_t stream);
+
 /* Number of tile configurations accepted in segq_gemm_desc.tile (ids 1..count). */
 int segq_gemm_tile_count(void);
 

@@ -68,7 +68,7 @@ class GemmDesc(C.Structure):
 EXPORTS = (
     "segq_version", "segq_last_error", "segq_quantize", "segq_quantize_many", "segq_quantize_weights_scalar",
     "segq_quantize_weights_rows", "segq_quantize_weights_groups", "segq_repack_int4_cols_to_rows", "segq_gemm", "segq_gemm_tile_count", "segq_gemm_workspace_bytes", "segq_gemm_plan", "segq_linear", "segq_fake_e4m3",
-    "segq_gemm_noalloc", "segq_noalloc_scratch_bytes", "segq_init", "segq_device_info",
+    "segq_gemm_noalloc", "segq_noalloc_scratch_bytes", "segq_init", "segq_device_info", "segq_lowrank_rows",
 )
 
 _lib = None
@@ -112,6 +112,8 @@ def lib() -> C.CDLL:
     L.segq_repack_int4_cols_to_rows.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p]
     L.segq_gemm.argtypes = [C.POINTER(GemmDesc), C.c_void_p]
     L.segq_gemm_tile_count.restype = C.c_int
+    L.segq_lowrank_rows.argtypes = [C.c_void_p, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int32, C.c_void_p]
+    L.segq_lowrank_rows.restype = C.c_int
     L.segq_gemm_workspace_bytes.argtypes = [C.POINTER(GemmDesc), C.POINTER(C.c_int64)]
     L.segq_gemm_plan.argtypes = [C.POINTER(GemmDesc), C.POINTER(C.c_int32), C.POINTER(C.c_int32), C.POINTER(C.c_int32)]
     L.segq_gemm_plan.restype = C.c_int

@@ -51,6 +51,8 @@ int quantize_many_impl(const segq_quant_desc* descs, int32_t n, hipStream_t st);
 int fake_e4m3_impl(const void* x, void* out, int32_t dtype, int64_t numel, hipStream_t st);
 int quantize_groups_impl(const void* w, int32_t w_dtype, int64_t n, int64_t k, void* codes, int32_t fmt, const float* scales,
                          int64_t group, hipStream_t st);
+int lowrank_rows_impl(const void* x, int64_t ldx, const void* l1t, int64_t ldl, void* t, int64_t ldt, int64_t m, int64_t k, int64_t r, int32_t dtype,
+                      hipStream_t st);
 int repack_i4_impl(const void* colpacked, void* rowpacked, int64_t out, int64_t cols, hipStream_t st);
 
 static bool is_float_dtype(int t) { return t == SEGQ_F32 || t == SEGQ_F16 || t == SEGQ_BF16; }
@@ -1004,6 +1006,11 @@ int segq_quantize_weights_groups(const void* weights, int32_t w_dtype, int64_t n
 
 int segq_repack_int4_cols_to_rows(const void* colpacked, void* rowpacked, int64_t out, int64_t cols, segq_stream_t stream) {
     return repack_i4_impl(colpacked, rowpacked, out, cols, static_cast<hipStream_t>(stream));
+}
+
+int segq_lowrank_rows(const void* x, int64_t ldx, const void* l1t, int64_t ld_l1t, void* t, int64_t ldt, int64_t m, int64_t k, int64_t r, int32_t dtype,
+                      segq_stream_t stream) {
+    return lowrank_rows_impl(x, ldx, l1t, ld_l1t, t, ldt, m, k, r, dtype, static_cast<hipStream_t>(stream));
 }
 
 int segq_gemm(const segq_gemm_desc* d, segq_stream_t stream) { return gemm_impl(d, static_cast<hipStream_t>(stream)); }

@@ -314,6 +314,17 @@ def gemm_plan(g, workspace: Optional[torch.Tensor] = None) -> dict:
                 kernel=f"segq::{family}<{TILE_SHAPES.get(tile.value, '?').replace('x', ',')}>")
 
 
+def lowrank_rows(x: torch.Tensor, l1t: torch.Tensor, out: torch.Tensor) -> bool:
+    """``out = x @ l1t.t()`` for a low-rank branch (``segq_lowrank_rows``), or False, nothing launched, where the kernel does
+    not serve the sizes or the alignment."""
+    k, r = x.shape[1], l1t.shape[0]
+    if k % 64 or r % 16 or not x.is_cuda or x.stride(1) != 1 or row_stride(x) % 8 or x.data_ptr() % 16 or l1t.data_ptr() % 16:
+        return False
+    L.check(L.lib().segq_lowrank_rows(x.data_ptr(), row_stride(x), l1t.data_ptr(), k, out.data_ptr(), row_stride(out), x.shape[0], k, r, _dt(x.dtype),
+                                      _stream()))
+    return True
+
+
 def lowrank_tile(g) -> int:
     """The tile on which the launch ``g`` takes a low-rank branch (0: the library's choice for it): the one it has without,
     where that is one of the three largest and fills its rounds of the compute units, 4608 tokens say.  us, the library's

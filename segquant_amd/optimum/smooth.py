@@ -235,6 +235,7 @@ class SVDOptimizer(SmoothOptimizer):
         plan["l1s"] = l1                                                        # (k_i, r) each, fp32
         plan["l2t"] = torch.cat([self.l2s[i].to(device=device, dtype=torch.float32) for i in range(self.chunks)], dim=0).t().contiguous()  # (N, S r)
         # (cast here for every input dtype, as the divisors are)
+        plan["l1t_cast"] = {dt: [l.t().to(dt).contiguous() for l in l1] for dt in (torch.float16, torch.bfloat16)}
         plan["l12_cast"] = {dt: ([l.to(dt) for l in l1], plan["l2t"].to(dt).contiguous())
                             for dt in (torch.float32, torch.float16, torch.bfloat16)}
         return plan
@@ -247,5 +248,7 @@ class SVDOptimizer(SmoothOptimizer):
         bounds = plan["bounds"]
         t = torch.empty((x2.shape[0], r * self.chunks), dtype=dt, device=x2.device)
         for i in range(self.chunks):
-            torch.matmul(x2[:, bounds[i]:bounds[i + 1]], l1[i], out=t[:, i * r:(i + 1) * r])
+            part, out = x2[:, bounds[i]:bounds[i + 1]], t[:, i * r:(i + 1) * r]
+            if not (dt in plan["l1t_cast"] and ops.lowrank_rows(part, plan["l1t_cast"][dt][i], out)):
+                torch.matmul(part, l1[i], out=out)
         return t, l2t
