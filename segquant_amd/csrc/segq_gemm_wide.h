@@ -762,7 +762,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     static_assert(!GRP || (!F8 && NS == 2), "group factors: int8, two stages");
     // int8 tiles above 256 x 256 run the whole-step schedule too: one set of 32-byte fragments
     // instead of two sets of 16-byte ones leaves room for their accumulators
-    constexpr bool WS = !F8 && !GRP && (BM * BN > 256 * 256 || MIX);
+    constexpr bool WS = !F8 && !GRP && BM * BN > 256 * 256;
     constexpr bool S8 = F8 || GRP || WS;  // whole-step fragments
     //
     // PARK (int8, several ranges): no second register set at all.  When a range ends, its
@@ -955,16 +955,20 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
 
     // MERGE: dwords [d0, d1) of a fragment of codes of both signs -> those of the positive ones and of the negative ones, the
     // others zero: four VALU instructions per dword
-    auto part = [&](int i, int d0, int d1) __attribute__((always_inline)) {
-        if constexpr (MERGE) {
+    auto part_of = [](auto& pos, auto& neg, int d0, int d1) __attribute__((always_inline)) {
 #pragma unroll
-            for (int d = d0; d < d1; ++d) {
-                const uint32_t v = (uint32_t)fa8[i + TM / 2][d];
-                const uint32_t mask = __builtin_amdgcn_perm(v, v << 8, 0x0B090A08u);  // every byte's sign, eight times
-                fa8[i][d] = (int)(v & ~mask);
-                fa8[i + TM / 2][d] = (int)(v & mask);
-            }
+        for (int d = d0; d < d1; ++d) {
+            const uint32_t v = (uint32_t)neg[d];
+            const uint32_t mask = __builtin_amdgcn_perm(v, v << 8, 0x0B090A08u);  // every byte's sign, eight times
+            pos[d] = (int)(v & ~mask);
+            neg[d] = (int)(v & mask);
         }
+    };
+    auto part = [&](int i, int d0, int d1) __attribute__((always_inline)) {
+        if constexpr (MERGE && S8) part_of(fa8[i], fa8[i + TM / 2], d0, d1);
+    };
+    auto part1 = [&](int h, int d) __attribute__((always_inline)) {  // dword d of set h's
+        if constexpr (MERGE && !S8) part_of(fa[h][d / 4], fa[h][d / 4 + TM / 2], d % 4, d % 4 + 1);
     };
 
     // K half h of the tile in buffer buf -> fragment slot h, one 16-byte read at a
@@ -972,13 +976,13 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     auto frag1 = [&](int buf, int h, int i) {
         if constexpr (!S8) {
             const int off = ((h * 4 + lgrp) ^ f_sw) << 4;
-            if (i < TM) fa[h][i] = *reinterpret_cast<const v4i*>(As + buf * AR * BK + a_frag + i * 16 * BK + off);
+            if (i < TM) fa[h][i] = *reinterpret_cast<const v4i*>(As + buf * AR * BK + a_frag + (MERGE ? i - TM / 2 : i) * 16 * BK + off);
             else fb[h][i - TM] = *reinterpret_cast<const v4i*>(Bs + buf * BN * BK + b_frag + (i - TM) * 16 * BK + off);
         }
     };
     auto frags = [&](int buf, int h) {
 #pragma unroll
-        for (int i = 0; i < TM + TN; ++i) frag1(buf, h, i);
+        for (int i = MERGE ? TM / 2 : 0; i < TM + TN; ++i) frag1(buf, h, i);
     };
     const int m_base = m0 + wm * WM + lrow;
     const int n_base = n0 + wn * WN + 4 * lgrp;
@@ -1208,6 +1212,10 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         for (int i = MERGE ? TM / 2 : 0; i <= TM; ++i) frag8(0, i);  // activations and the first weight fragment
     } else {
         frags(0, 0);
+        if (MERGE && n_dual > 0) {
+#pragma unroll
+            for (int d = 0; d < TM / 2 * 4; ++d) part1(0, d);
+        }
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the loop head must see them as landed on every path
 
@@ -1220,10 +1228,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     int cr = r_first, ck = k_first, ck1 = p.r[ph(r_first)].k1;  // the tile being multiplied
     bool dirty = false;  // sums not yet folded into the second set (a split can end inside a range)
     int buf = 0;                                   // its buffer, s % NS
-    constexpr int NMF = TM * TN, NRD = TM + TN, NDM = A_IT + B_IT;
-    constexpr int RD_EVERY = (NMF >= 2 * NRD + 4) ? 2 : 1;
-    constexpr int DM_EVERY = (NMF / NDM > 1) ? NMF / NDM : 1;
-    static_assert(NRD * RD_EVERY <= NMF && NDM * DM_EVERY <= NMF, "more reads than MFMA slots");
+    constexpr int NDM = A_IT + B_IT;
     // Group factors: int32 sums of a column block and, in LAG order, of the one before it, whose factors are gf
     static_assert(!GRP || TN % 2 == 0, "group factors: two sets of temporaries in turn, also from one step to the next");
     constexpr bool LAG = GRP && !FOLD;
@@ -1256,7 +1261,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     // activation fragment right behind the last MFMA that reads it, with the DMA
     // of step s + 2 spread over the same MFMAs.
     // plain_c, dplain_c (MIX): this step, the one that it loads, is of the plain range: the second half of the row blocks only
-    [[maybe_unused]] bool tail_left = false;  // three stages: there is a step behind the next one
+    [[maybe_unused]] bool tail_left = false, next_dual = false;  // three stages: there is a step behind the next one; that one is of the pair
     auto step8 = [&](auto dma_c, auto more_c, auto plain_c, auto dplain_c) __attribute__((always_inline)) {
         constexpr bool DMA_ = decltype(dma_c)::value;
         constexpr bool MORE_ = decltype(more_c)::value;
@@ -1445,23 +1450,34 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
 #else
     constexpr bool abl_dma = false;
 #endif
-    auto step_i8 = [&](auto dma_c, auto more_c) __attribute__((always_inline)) {
+    // (plain_c, dplain_c: as in step8)
+    auto step_i8 = [&](auto dma_c, auto more_c, auto plain_c, auto dplain_c) __attribute__((always_inline)) {
         constexpr bool DMA_ = decltype(dma_c)::value;
         constexpr bool MORE_ = decltype(more_c)::value;
+        constexpr int B0 = decltype(plain_c)::value ? TM / 2 : 0;           // the first row block
+        constexpr int R0 = MERGE || decltype(plain_c)::value ? TM / 2 : 0;  // the first fragment that is read
+        constexpr int H = MERGE && B0 == 0 ? TM / 2 : 0;                    // fragments to be parted
+        constexpr int NM = (TM - B0) * TN, NR = TM + TN - R0;
+        constexpr int RDE = (NM >= 2 * NR + 4) ? 2 : 1;
+        constexpr int DME = (NM / NDM > 1) ? NM / NDM : 1;
+        static_assert(S8 || (NR * RDE <= NM && NDM * DME <= NM), "more reads than MFMA slots");
+        constexpr int P0 = NM - 4 * H;                                      // a dword per MFMA, the last of either half, behind its read
         const int nbuf = (buf + 1 == NS) ? 0 : buf + 1;
 #pragma unroll
         for (int a = 0; a < TN; ++a)
 #pragma unroll
-            for (int b = 0; b < TM; ++b) {
-                const int i = a * TM + b;
-                if (i % RD_EVERY == 0 && i / RD_EVERY < NRD && !abl_lds) frag1(buf, 1, i / RD_EVERY);
+            for (int b = B0; b < TM; ++b) {
+                const int i = a * (TM - B0) + b - B0;
+                if (i % RDE == 0 && i / RDE < NR && !abl_lds) frag1(buf, 1, R0 + i / RDE);
+                if (H > 0 && i >= P0) part1(1, i - P0);
                 if constexpr (!abl_mfma) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[0][a], fa[0][b], acc[a][b], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
             }
         // Tile s+1 must have landed (the NS-2 tiles issued after it may still be in
         // flight) and this wave's reads of tile s must be done, before anyone reads
         // tile s+1 or overwrites the buffer of tile s.
-        wait_dma(std::integral_constant<int, DMA_ ? NS - 2 : 0>{});
+        if (MIX && NS > 2 && decltype(dplain_c)::value && !tail_left) wait_dma(std::integral_constant<int, 0>{});
+        else wait_dma(std::integral_constant<int, DMA_ ? NS - 2 : 0>{});
         __syncthreads();
         if constexpr (KT && MORE_ && !DMA_) clear_tail(nbuf);  // (two stages: the next step is the last)
         // tile s+NS goes where tile s was: both its halves are in registers
@@ -1470,13 +1486,16 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
 #pragma unroll
         for (int a = 0; a < TN; ++a)
 #pragma unroll
-            for (int b = 0; b < TM; ++b) {
-                const int i = a * TM + b;
+            for (int b = B0; b < TM; ++b) {
+                const int i = a * (TM - B0) + b - B0;
                 if constexpr (DMA_) {
-                    if (i % DM_EVERY == DM_EVERY - 1 && i / DM_EVERY < NDM && !abl_dma) dma1(ap, bp, buf, i / DM_EVERY, std::false_type{});
+                    if (i % DME == DME - 1 && i / DME < NDM && !abl_dma) dma1(ap, bp, buf, i / DME, dplain_c);
                 }
                 if constexpr (MORE_) {
-                    if (i % RD_EVERY == 0 && i / RD_EVERY < NRD && !abl_lds) frag1(nbuf, 0, i / RD_EVERY);
+                    if (i % RDE == 0 && i / RDE < NR && !abl_lds) frag1(nbuf, 0, R0 + i / RDE);
+                }
+                if (H > 0 && i >= P0) {  // (of the next step, if that is one of the pair)
+                    if (!decltype(dplain_c)::value || next_dual) part1(0, i - P0);
                 }
                 if constexpr (!abl_mfma) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[1][a], fa[1][b], acc[a][b], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
@@ -1489,7 +1508,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         if constexpr (DMA_) advance_load();
         ck += BK;
         dirty = true;
-        if (!KT && ck >= ck1) {  // the range is complete: fold it, move to the next one
+        if (!KT && !MIX && ck >= ck1) {  // the range is complete: fold it, move to the next one
             if constexpr (PARK) park(cr);
             else if constexpr (FOLD) fold(cr);
             dirty = false;
@@ -1502,19 +1521,24 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     };
     auto step = [&](auto dma_c, auto more_c) __attribute__((always_inline)) {
         if constexpr (S8) step8(dma_c, more_c, std::false_type{}, std::false_type{});
-        else step_i8(dma_c, more_c);
+        else step_i8(dma_c, more_c, std::false_type{}, std::false_type{});
     };
     int s = 0;
     if constexpr (MIX) {
         constexpr std::true_type yes{};
         constexpr std::false_type no{};
-        const int alike = MERGE ? min(n_dual, steps - NS) : n_dual - NS;  // (plain steps are loaded like MERGE's others)
-        for (; s < alike; ++s) step8(yes, yes, no, no);
+        auto mstep = [&](auto plain_c, auto dplain_c) __attribute__((always_inline)) {
+            if constexpr (S8) step8(yes, yes, plain_c, dplain_c);
+            else step_i8(yes, yes, plain_c, dplain_c);
+        };
+        const int alike = MERGE ? min(n_dual - (S8 ? 0 : 1), steps - NS) : n_dual - NS;  // (plain steps are loaded like MERGE's others)
+        for (; s < alike; ++s) mstep(no, no);
         // from here on a step loads a plain one or, behind the last, none (what it reads of that goes nowhere)
         for (; s < n_dual; ++s) {
             if (s + NS >= steps) wanted = 0;
             tail_left = s + 2 < steps;
-            step8(yes, yes, no, yes);
+            next_dual = s + 1 < n_dual;
+            mstep(no, yes);
         }
         if (n_dual > 0) {  // the sums of both signs -> one, in output units
             const float* const rx2 = epi + OM + 2 * BN;
@@ -1534,7 +1558,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         for (; s < steps; ++s) {
             if (s + NS >= steps) wanted = 0;
             tail_left = s + 2 < steps;
-            step8(yes, yes, yes, yes);
+            mstep(yes, yes);
         }
     }
     for (; s + NS < steps; ++s) step(std::true_type{}, std::true_type{});
