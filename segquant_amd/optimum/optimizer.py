@@ -34,6 +34,16 @@ def _as_f32(v, device):
     return torch.tensor(v, dtype=torch.float32, device=device)
 
 
+def _lends_int4(plan, M: int) -> bool:
+    """Whether a layer with int4 weights lends the room to expand them to int8, once per launch.  Many tokens or a long K: the
+    GEMM is bound by the matrix cores, and the int8 kernels are ahead by more than the expansion; otherwise reading half the
+    weight bytes matters more.  us, unpacked in the GEMM / expanded: 3072 -> 9216, 1000 tokens 54 / 48, 2000 93 / 76, 700
+    33 / 40; 5120 -> 1280, 1500 tokens 41 / 29, 2500 42 / 30; 4096 -> 704, 2500 33 / 22; 2048 -> 4096, 2500 41 / 34, 2000
+    26 / 27; 1152 -> 6400, 2500 31 / 34, 3500 48 / 42.  Group-wise scales run on the int8 kernels only."""
+    K = plan["K"]
+    return plan.get("group_dequant") is not None or M >= 3072 or (M >= 1000 and K >= 3072) or M * K >= 2300 * 2048
+
+
 class BaseOptimizer:
     def __init__(self, seg_mode, chunks, chunksizes, weight_manager, input_calibrators, weight_calibrators,
                  real_quant=False, dual_scale=False, kernel_type=None, dual_segments=None):
@@ -410,16 +420,13 @@ class DefaultOptimizer(BaseOptimizer):
             g = ops.gemm_desc(codes, plan["w"], ranges, addend=add2, **kw)
         # Whether to lend the library a workspace is this layer's call; how much it could use is
         # the library's (segq_gemm_workspace_bytes), asked once per token count.
-        #  * int4 weights and many tokens: the GEMM is bound by the matrix cores, so the weights are
-        #    expanded to int8 once per launch and the int8 kernels run; with few tokens reading half
-        #    the weight bytes matters more (measured, K 1280, N 10240: 161 -> 119 us at 8192 tokens,
-        #    no gain at 2048).  Group-wise scales run on the int8 kernels only: always lend.
+        #  * int4 weights: _lends_int4.
         #  * 8-bit weights: always.  int8 with several ranges (K segments, DualScale) parks the
         #    finished ranges' sums there and keeps the big tiles (4608 x 15360 x 3072, three ranges:
         #    441 -> 383 us; 9216 tokens: 1044 -> 756 us); few tiles and a long K share the K steps of
         #    a tile between workgroups (1024 x 15360 x 3072: 162 -> 108 us int8, 135 -> 98 us e4m3).
         int4 = plan["fw"] == ops.FMT_INT4
-        lend = (M >= 3072 or gdq is not None) if int4 else True
+        lend = _lends_int4(plan, M) if int4 else True
         ws = None
         if lend:
             need = plan.setdefault("ws_need", {}).get(M)
@@ -510,7 +517,7 @@ class DefaultOptimizer(BaseOptimizer):
                           group_dequant=plan.get("group_dequant"), finite_scales=self.dual_scale)
         ws = None
         int4 = plan["fw"] == ops.FMT_INT4
-        if M >= 3072 or not int4 or plan.get("group_dequant") is not None:
+        if not int4 or _lends_int4(plan, M):
             need = plan.setdefault("ws_need", {}).get(M)
             if need is None:
                 need = plan["ws_need"][M] = ops.gemm_workspace_bytes(g)
@@ -587,7 +594,7 @@ class DefaultOptimizer(BaseOptimizer):
                           ldb=K // 2 if plan["fw"] == ops.FMT_INT4 else K, bias=bias, a_neg=codes_neg, finite_scales=dual)
         int4 = plan["fw"] == ops.FMT_INT4
         ws = None
-        if M >= 3072 or not int4:
+        if not int4 or _lends_int4(plan, M):
             need = plan.setdefault("ws_need", {}).get(M)
             if need is None:
                 need = plan["ws_need"][M] = ops.gemm_workspace_bytes(g)

@@ -531,3 +531,23 @@ def test_launch_cache_is_bounded_over_token_counts():
         got = layer(xs[:m])
         assert torch.equal(got, fresh.optimizer.forward_fused(xs[:m], fresh.bias_data, addend=None).view_as(got))
         assert len(layer.optimizer._plan["launches"]) <= opt_mod._MAX_CACHED_TOKEN_COUNTS
+
+
+@pytest.mark.parametrize("M,K,N", [(1500, 5120, 1280), (2500, 2048, 4096)])
+def test_int4_layer_expands_its_weights_from_where_that_pays(M, K, N):
+    """Rows of a launch that expands its int4 weights against the same rows in a smaller one, which unpacks them in the GEMM:
+    the same integers, scaled in fp32."""
+    from segquant_amd.layers.SegmentLinear import SegmentLinear
+    from segquant_amd.optimum.optimizer import _lends_int4
+    g = torch.Generator().manual_seed(M)
+    layer = SegmentLinear(K, N, bias=True, custom_weight_tensor=(torch.randn(N, K, generator=g) * 0.02).to(DEV),
+                          custom_bias_tensor=torch.randn(N, generator=g).to(DEV), input_quant_type="int8", weight_quant_type="int4",
+                          input_quant_args={"real_quant": True, "axis": -1, "dynamic": True}, weight_quant_args={"real_quant": True, "axis": 1}, device=DEV)
+    x = torch.randn(M, K, generator=g).to(DEV)
+    layer.calibrate(x)
+    layer.finish_calibrate()
+    out, few = layer(x), layer(x[:640])
+    plan = layer.optimizer._plan
+    assert _lends_int4(plan, M) and not _lends_int4(plan, 640) and plan["ws_need"][M] >= K * N and 640 not in plan["ws_need"]
+    # two hardware reciprocals, two products and the sum with the bias: 6 x 2^-24 of their magnitudes
+    assert ((out[:640] - few).abs() <= 6 * 2.0 ** -24 * (few.abs() + 2 * layer.bias_data.abs())).all()
