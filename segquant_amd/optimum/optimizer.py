@@ -337,7 +337,7 @@ class DefaultOptimizer(BaseOptimizer):
         plan = self._plan or self._build_plan(x.device)
         K, N = plan["K"], plan["N"]
         x2 = x.reshape(-1, K)
-        if "l2t" in plan:  # (the low-rank operand is a library product of this tensor)
+        if "l2t" in plan:  # (the low-rank operand is a product of this tensor)
             x2 = x2.contiguous()
         x2 = _readable_rows(x2)
         if col_div is not None and plan.get("col_div") is not None:
@@ -421,10 +421,9 @@ class DefaultOptimizer(BaseOptimizer):
         # Whether to lend the library a workspace is this layer's call; how much it could use is
         # the library's (segq_gemm_workspace_bytes), asked once per token count.
         #  * int4 weights: _lends_int4.
-        #  * 8-bit weights: always.  int8 with several ranges (K segments, DualScale) parks the
-        #    finished ranges' sums there and keeps the big tiles (4608 x 15360 x 3072, three ranges:
-        #    441 -> 383 us; 9216 tokens: 1044 -> 756 us); few tiles and a long K share the K steps of
-        #    a tile between workgroups (1024 x 15360 x 3072: 162 -> 108 us int8, 135 -> 98 us e4m3).
+        #  * 8-bit weights: always.  int8 with several ranges that no one walk of K serves parks the
+        #    finished ranges' sums there and keeps the big tiles; few tiles and a long K share the K steps of
+        #    a tile between workgroups (1024 x 15360 x 3072: 113 -> 79 us int8, 108 -> 75 us e4m3).
         int4 = plan["fw"] == ops.FMT_INT4
         lend = _lends_int4(plan, M) if int4 else True
         ws = None
