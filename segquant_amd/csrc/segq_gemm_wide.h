@@ -591,7 +591,9 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 template <int TM, int TN>
-__device__ __forceinline__ void lowrank_accumulate(const GemmParams& p, v4f (&of)[TN][TM], int m_row0, int n_col0, int lane) {
+__device__ __forceinline__ void lowrank_accumulate(const GemmParams& p, v4f (&of)[TN][TM], int m_row0, int n_col0, int lane,
+                                                   bool in_lds, const uint8_t* lds_t, const uint8_t* lds_l) {
+    // lds_t, lds_l: the wave's rows of the first 32 columns of T and L2T, 64 bytes each, if they are in LDS already
     const int lrow = lane & 15, lgrp = lane >> 4;
     const bool bf = p.out_dtype == SEGQ_BF16;
     for (int kk = 0; kk < p.lr_rank; kk += 32) {
@@ -599,7 +601,8 @@ __device__ __forceinline__ void lowrank_accumulate(const GemmParams& p, v4f (&of
 #pragma unroll
         for (int b = 0; b < TM; ++b) {
             const int64_t m = min(m_row0 + b * 16 + lrow, p.M - 1);
-            tf[b] = *reinterpret_cast<const uint4*>(p.lr_t + m * p.lr_ldt + kk + lgrp * 8);
+            if (in_lds && kk == 0) tf[b] = *reinterpret_cast<const uint4*>(lds_t + (b * 16 + lrow) * 64 + lgrp * 16);
+            else tf[b] = *reinterpret_cast<const uint4*>(p.lr_t + m * p.lr_ldt + kk + lgrp * 8);
         }
         // (half of the column blocks' loads at a time, in front of their products: one by one, every block waited for L2
         // behind the block before it; all at once, registers)
@@ -610,7 +613,8 @@ __device__ __forceinline__ void lowrank_accumulate(const GemmParams& p, v4f (&of
 #pragma unroll
             for (int a = a0; a < TN && a < a0 + CH; ++a) {
                 const int64_t n = min(n_col0 + a * 16 + lrow, p.N - 1);
-                lf[a - a0] = *reinterpret_cast<const uint4*>(p.lr_l2 + n * p.lr_ldl + kk + lgrp * 8);
+                if (in_lds && kk == 0) lf[a - a0] = *reinterpret_cast<const uint4*>(lds_l + (a * 16 + lrow) * 64 + lgrp * 16);
+                else lf[a - a0] = *reinterpret_cast<const uint4*>(p.lr_l2 + n * p.lr_ldl + kk + lgrp * 8);
             }
 #pragma unroll
             for (int a = a0; a < TN && a < a0 + CH; ++a)
@@ -1253,6 +1257,30 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
 #pragma unroll
         for (int j = 0; j < 2 * TM; ++j) convert(a, j);
     };
+    // Low-rank branch, one range: the first 32 columns of the tile's rows of T and L2T go into the stage that the last step but
+    // one is done with, and land under that step; they are read behind the last one.
+    // us, loaded there / this, int8: 4608 x 12288 x 3072 on 384 x 192 156 / 152, 4608 x 9216 122 / 120.5, 2304 x 12288 83 / 81,
+    // 300 x 3072 x 1536 12.0 / 11.4.
+    constexpr bool LRP = FINISH && !FOLD && !GRP && NS == 2;
+    [[maybe_unused]] int lr_buf = -1;
+    auto fetch_lr = [&](int buf) __attribute__((always_inline)) {
+        if constexpr (LRP) {
+            if (p.lr_rank > 0) {
+                const int r4 = lane >> 2, c = (lane & 3) * 8;  // four 16-byte pieces a row
+#pragma unroll
+                for (int i = 0; i < (BM + 127) / 128; ++i) {
+                    const int row = wave * 16 + i * 128;
+                    if (row < BM) load16_to_lds(reinterpret_cast<const uint8_t*>(p.lr_t + (int64_t)min(m0 + row + r4, p.M - 1) * p.lr_ldt + c), As + buf * AR * BK + row * 64);
+                }
+#pragma unroll
+                for (int i = 0; i < (BN + 127) / 128; ++i) {
+                    const int row = wave * 16 + i * 128;
+                    if (row < BN) load16_to_lds(reinterpret_cast<const uint8_t*>(p.lr_l2 + (int64_t)min(n0 + row + r4, p.N - 1) * p.lr_ldl + c), Bs + buf * BN * BK + row * 64);
+                }
+                lr_buf = buf;
+            }
+        }
+    };
     // e4m3 schedule of one step.  On entry the activation fragments and weight
     // fragment 0 are in registers.  Column block a reads weight fragment a + 2
     // (block 0 also fragment 1), so after block TN - 3 every read of this step is
@@ -1337,6 +1365,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         else wait_dma(std::integral_constant<int, 0>{});
         __syncthreads();
         if constexpr (KT && MORE_ && !DMA_) clear_tail(nbuf);  // (two stages: the next step is the last)
+        if constexpr (LRP && MORE_ && !DMA_) fetch_lr(buf);
         const uint8_t* const ap = la + lk;
         const uint8_t* const bp = Bb + lk;
 #pragma unroll
@@ -1480,6 +1509,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         else wait_dma(std::integral_constant<int, DMA_ ? NS - 2 : 0>{});
         __syncthreads();
         if constexpr (KT && MORE_ && !DMA_) clear_tail(nbuf);  // (two stages: the next step is the last)
+        if constexpr (LRP && MORE_ && !DMA_) fetch_lr(buf);
         // tile s+NS goes where tile s was: both its halves are in registers
         const uint8_t* const ap = la + lk;
         const uint8_t* const bp = Bb + lk;
@@ -1612,7 +1642,10 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
         if constexpr (MEET) {
             if (p.part && !meet_share<NT, CH>(p, of, tile_id, zy, tid, reinterpret_cast<int*>(epi))) return;
         }
-        if (p.lr_rank > 0) lowrank_accumulate<TM, TN>(p, of, m0 + wm * WM, n0 + wn * WN, lane);
+        if (p.lr_rank > 0) {
+            const int lb = max(lr_buf, 0);
+            lowrank_accumulate<TM, TN>(p, of, m0 + wm * WM, n0 + wn * WN, lane, LRP && lr_buf >= 0, As + lb * AR * BK + wm * WM * 64, Bs + lb * BN * BK + wn * WN * 64);
+        }
         wide_epilogue<BM, BN, WGM, WGN, GEMM_F8, false, true>(p, of, of, smem, z, m0, n0, wave, lane, r_epi, epi);
         return;
     }

@@ -328,8 +328,8 @@ def lowrank_rows(x: torch.Tensor, l1t: torch.Tensor, out: torch.Tensor) -> bool:
 def lowrank_tile(g) -> int:
     """The tile on which the launch ``g`` takes a low-rank branch (0: the library's choice for it): the one it has without,
     where that is one of the three largest and fills its rounds of the compute units, 4608 tokens say.  us, the library's
-    choice / this, rank 32, int8 | e4m3: 4608 x 12288 x 3072 178 / 161 | 180 / 150; 4608 x 9216 x 3072 133 / 125 | 132 / 120;
-    2304 x 12288 x 3072 88 / 85; rank 64, 4500 x 12000 x 3072 197 / 179; 2000 x 10240 x 2048, rounds filled to 77 %, 62 / 66."""
+    choice / this, rank 32, int8 | e4m3: 4608 x 12288 x 3072 175 / 152 | 172 / 143; 4608 x 9216 x 3072 125 / 120 | 125 / 118;
+    2304 x 12288 x 3072 85 / 81; rank 64, 4500 x 12000 x 3072 189 / 170; 2000 x 10240 x 2048, rounds filled to 77 %, 59 / 64."""
     tile = gemm_plan(g)["tile"]
     if tile not in (15, 16, 20):
         return 0
