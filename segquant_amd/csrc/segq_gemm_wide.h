@@ -585,15 +585,18 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_wide_kernel(const GemmPara
 // patch at (m_row0, n_col0).  `of` holds the de-quantised sums in output units in the lane layout
 // of the accumulators (four consecutive columns of one row per lane and block), which is also
 // the result layout of these MFMAs with L2T as the first operand.  Both fragments are 16 rows of
-// 32 contiguous 16-bit values: a lane reads the 16 bytes of its row at k + 8 lgrp straight from
-// memory (T and L2T are small and stay in the L2).
+// 32 contiguous 16-bit values: a lane reads the 16 bytes of its row at k + 8 lgrp, straight from
+// memory (T and L2T are small and stay in the L2) or, the first 32 columns with one range, from the K loop's LDS.
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
-template <int TM, int TN>
+// LDS: the kernel may have the wave's rows of the first 32 columns of both in LDS by then (in_lds), 64 bytes each at lds_t and lds_l.
+// (A template argument: instances that never have them there spilled more registers when the code merely did not take that
+// side, int8 parked 256 x 256 672 bytes a lane for 556, 192 x 256 208 for 132.)
+template <bool LDS, int TM, int TN>
 __device__ __forceinline__ void lowrank_accumulate(const GemmParams& p, v4f (&of)[TN][TM], int m_row0, int n_col0, int lane,
-                                                   bool in_lds, const uint8_t* lds_t, const uint8_t* lds_l) {
-    // lds_t, lds_l: the wave's rows of the first 32 columns of T and L2T, 64 bytes each, if they are in LDS already
+                                                   [[maybe_unused]] bool in_lds = false, [[maybe_unused]] const uint8_t* lds_t = nullptr,
+                                                   [[maybe_unused]] const uint8_t* lds_l = nullptr) {
     const int lrow = lane & 15, lgrp = lane >> 4;
     const bool bf = p.out_dtype == SEGQ_BF16;
     for (int kk = 0; kk < p.lr_rank; kk += 32) {
@@ -601,19 +604,20 @@ __device__ __forceinline__ void lowrank_accumulate(const GemmParams& p, v4f (&of
 #pragma unroll
         for (int b = 0; b < TM; ++b) {
             const int64_t m = min(m_row0 + b * 16 + lrow, p.M - 1);
-            if (in_lds && kk == 0) tf[b] = *reinterpret_cast<const uint4*>(lds_t + (b * 16 + lrow) * 64 + lgrp * 16);
+            if (LDS && in_lds && kk == 0) tf[b] = *reinterpret_cast<const uint4*>(lds_t + (b * 16 + lrow) * 64 + lgrp * 16);
             else tf[b] = *reinterpret_cast<const uint4*>(p.lr_t + m * p.lr_ldt + kk + lgrp * 8);
         }
         // (half of the column blocks' loads at a time, in front of their products: one by one, every block waited for L2
-        // behind the block before it; all at once, registers)
-        constexpr int CH = (TN + 1) / 2;
+        // behind the block before it; all at once, registers.  Two where the sums take half of the registers: with four the one-range
+        // int8 256 x 256 instance spilled 8 bytes a lane.)
+        constexpr int CH = TM * TN >= 32 ? 2 : (TN + 1) / 2;
 #pragma unroll
         for (int a0 = 0; a0 < TN; a0 += CH) {
             uint4 lf[CH];
 #pragma unroll
             for (int a = a0; a < TN && a < a0 + CH; ++a) {
                 const int64_t n = min(n_col0 + a * 16 + lrow, p.N - 1);
-                if (in_lds && kk == 0) lf[a - a0] = *reinterpret_cast<const uint4*>(lds_l + (a * 16 + lrow) * 64 + lgrp * 16);
+                if (LDS && in_lds && kk == 0) lf[a - a0] = *reinterpret_cast<const uint4*>(lds_l + (a * 16 + lrow) * 64 + lgrp * 16);
                 else lf[a - a0] = *reinterpret_cast<const uint4*>(p.lr_l2 + n * p.lr_ldl + kk + lgrp * 8);
             }
 #pragma unroll
@@ -1262,7 +1266,6 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
     // us, loaded there / this, int8: 4608 x 12288 x 3072 on 384 x 192 156 / 152, 4608 x 9216 122 / 120.5, 2304 x 12288 83 / 81,
     // 300 x 3072 x 1536 12.0 / 11.4.
     constexpr bool LRP = FINISH && !FOLD && !GRP && NS == 2;
-    [[maybe_unused]] int lr_buf = -1;
     auto fetch_lr = [&](int buf) __attribute__((always_inline)) {
         if constexpr (LRP) {
             if (p.lr_rank > 0) {
@@ -1277,7 +1280,6 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
                     const int row = wave * 16 + i * 128;
                     if (row < BN) load16_to_lds(reinterpret_cast<const uint8_t*>(p.lr_l2 + (int64_t)min(n0 + row + r4, p.N - 1) * p.lr_ldl + c), Bs + buf * BN * BK + row * 64);
                 }
-                lr_buf = buf;
             }
         }
     };
@@ -1643,8 +1645,12 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_pipe_kernel(const GemmPara
             if (p.part && !meet_share<NT, CH>(p, of, tile_id, zy, tid, reinterpret_cast<int*>(epi))) return;
         }
         if (p.lr_rank > 0) {
-            const int lb = max(lr_buf, 0);
-            lowrank_accumulate<TM, TN>(p, of, m0 + wm * WM, n0 + wn * WN, lane, LRP && lr_buf >= 0, As + lb * AR * BK + wm * WM * 64, Bs + lb * BN * BK + wn * WN * 64);
+            if constexpr (LRP) {
+                const int lb = steps & 1;  // the stage of the last step but one
+                lowrank_accumulate<true>(p, of, m0 + wm * WM, n0 + wn * WN, lane, steps > 1, As + lb * AR * BK + wm * WM * 64, Bs + lb * BN * BK + wn * WN * 64);
+            } else {
+                lowrank_accumulate<false>(p, of, m0 + wm * WM, n0 + wn * WN, lane);
+            }
         }
         wide_epilogue<BM, BN, WGM, WGN, GEMM_F8, false, true>(p, of, of, smem, z, m0, n0, wave, lane, r_epi, epi);
         return;
