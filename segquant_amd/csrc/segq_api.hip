@@ -508,9 +508,16 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
             const bool share = lent && d->split_k != 1;
             MixPick pick = choose_mix(d->m, d->n, steps, plain, share ? 16 : 1);
             while (pick.shares > 1 && !shares_fit(pick.cfg, pick.shares)) pick = choose_mix(d->m, d->n, steps, plain, pick.shares - 1);
-            // Up to 128 rows the shares of a 128 x 128 tile are ahead: 32 x 1536 x (1536 + 6144) e4m3 18.7 us, here 23.4; 128 rows
-            // 22.0 and 25.1, int8 27.0 and 25.4.
-            bool take = d->m > 128 || !share || steps + plain < 32;
+            // Up to 128 rows K shares of the ranges in turn are ahead, from where there are enough of them.  us a pass, that / this:
+            // 32 x 1536 x (1536 + 6144) e4m3 18.7 / 23.4, 128 rows 22.0 / 25.1, int8 27.0 / 25.4.  Beside a plain range e4m3 takes
+            // 128 x 128 tiles in three shares and more: 1 x 512 x (512 + 2048) 18.2 / 22.0, 128 rows 20.6 / 25.2, 1 x 4096 x (1024 +
+            // 1024) 15.7 / 21.7, 128 x 4096 x (1024 + 2816) 26.0 / 30.0; two shares 1 x 2048 x (512 + 1024) 29.7 / 19.9, and
+            // many outputs, whose shares are a trip through memory, 128 x 9216 x (384 + 1536) 27.6 / 24.2.  int8, which parks, has
+            // 256 x 192 tiles: 1 x 512 x (512 + 3072) 20.7 / 22.4, 32 x 512 x (1024 + 2816) 23.7 / 25.9, 64 rows 25.9 / 26.1, 128 x 768 x
+            // (768 + 3072) 27.0 / 26.4, 16 x 3072 24.7 / 24.0, 1 x 640 x (640 + 2560), which is not shared, 49.6 / 24.3.
+            const int64_t all = 2 * steps + plain;
+            const bool in_shares = steps + plain >= 32 || (mix.plain >= 0 && (f8 ? all >= 24 && d->m * d->n <= 540000 : all >= 52 && d->m <= 32 && d->n <= 1024));
+            bool take = d->m > 128 || !share || !in_shares;
             // The pair alone: against one walk of tiles 29 and 30, or the ranges in turn.  us, that / this: 2500 x 3072 x 12288 161 / 143,
             // 600 x 2048 x 8192 44 / 34, 4608 x 3072 x 12288 int8 310 / 266; 4096 x 1536 x 6144 57 / 60, 2600 x 1152 x 4608 30 / 34.
             if (mix.plain < 0) {

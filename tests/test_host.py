@@ -486,7 +486,7 @@ def test_smooth_and_svd_layers_on_the_fake_path_equal_the_oracle(opt_type, seg_m
                       opt_kwargs={"search_alpha_config": {"enable": True, "min": 0.1, "max": 0.9, "step": 0.1}}, device="cpu")
 
 
-def _plan(lib, m, n, ranges, fmt, out_dtype=2, lend=True, split_k=0, tile=0, lowrank=0):
+def _plan(lib, m, n, ranges, fmt, out_dtype=2, lend=True, split_k=0, tile=0, lowrank=0, finite=0):
     """segq_gemm_plan / segq_gemm_workspace_bytes on a descriptor of made-up (aligned, never
     dereferenced) device addresses: the library's decisions are host arithmetic and launch nothing.
     ranges: (k_begin, k_len, a_sel).  Returns (tile id, K shares, parked, workspace bytes)."""
@@ -498,7 +498,7 @@ def _plan(lib, m, n, ranges, fmt, out_dtype=2, lend=True, split_k=0, tile=0, low
     k = max(b + l for b, l, _ in ranges)
     d.m, d.n, d.lda, d.ldb, d.ldo, d.batch = m, n, k, k, n, 1
     d.a, d.a_neg, d.b, d.out, d.bias = 0x10000000, 0x20000000, 0x30000000, 0x40000000, 0x50000000
-    d.n_ranges, d.tile, d.split_k = len(ranges), tile, split_k
+    d.n_ranges, d.tile, d.split_k, d.finite_scales = len(ranges), tile, split_k, finite
     for i, (b, l, sel) in enumerate(ranges):
         d.ranges[i].k_begin, d.ranges[i].k_len, d.ranges[i].a_sel = b, l, sel
         d.ranges[i].sx_row_stride, d.ranges[i].sw_col_stride = 1, 1
@@ -555,6 +555,28 @@ def test_tile_and_share_choice_for_the_benchmark_shapes():
     assert t == 14 and s in (2, 3)
     # the low-rank branch moves to a tile that is built with it
     assert _plan(lib, 4608, 12288, one(3072), I8, lowrank=32)[:2] == (11, 1)
+
+
+@pytest.mark.parametrize("m, n, k0, k1, fmt, walk", [
+    # e4m3: K shares of the ranges in turn up to 128 rows where the three of them have 24 steps
+    (1, 512, 512, 2048, 1, False), (128, 768, 768, 3072, 1, False), (129, 768, 768, 3072, 1, True), (16, 4096, 1024, 1024, 1, False),
+    (16, 2048, 512, 1024, 1, True), (64, 9216, 384, 1536, 1, True), (32, 9216, 384, 1536, 1, False),
+    # int8: few rows and outputs, where the shares are not of smaller tiles than the walk's
+    (1, 512, 512, 3072, 0, False), (32, 1024, 512, 3072, 0, False), (33, 512, 512, 3072, 0, True), (16, 1152, 512, 3072, 0, True),
+    (16, 640, 640, 2560, 0, True),
+    (16, 1536, 1536, 6144, 0, False), (16, 1536, 1536, 6144, 1, False),
+])
+def test_few_rows_beside_a_plain_segment(m, n, k0, k1, fmt, walk):
+    """A DualScale segment behind a plain one and up to 128 rows: one walk of K, or the three ranges in turn in K shares."""
+    from segquant_amd import _lib as L
+    for pair in ((2, 3), (0, 1)):
+        tile, shares, _, need = _plan(L.lib(), m, n, [(0, k0, 0), (k0, k1, pair[0]), (k0, k1, pair[1])], fmt, finite=1)
+        if walk:
+            assert tile in (31, 32, 33)
+        elif pair == (0, 1):  # (codes of both signs in one tensor are not for the ranges in turn: layers that ask then have two)
+            assert tile < 31 and shares > 1 and need > 0
+        else:
+            assert tile < 31
 
 
 def test_plan_refuses_what_the_launch_would_refuse():
@@ -656,8 +678,9 @@ def test_any_own_sum_is_kept_apart_and_finite_scales_leave_the_way_open():
     assert plan(4096, 1536, 6144, finite=1) == plan(4096, 1536, 6144, own=1) != plan(4096, 1536, 6144)
 
 
-def _kernel_registers():
-    """Mangled kernel name -> vector registers per lane, from the metadata the compiler leaves in the library built here."""
+def _kernel_registers(what=".vgpr_count"):
+    """Mangled kernel name -> vector registers per lane, from the metadata the compiler leaves in the library built here
+    (".private_segment_fixed_size": bytes of scratch memory per lane)."""
     import struct
     msgpack = pytest.importorskip("msgpack")
     from segquant_amd import _lib
@@ -675,7 +698,7 @@ def _kernel_registers():
             if kind == 32:  # NT_AMDGPU_METADATA
                 start = note + 12 + (name + 3) // 4 * 4
                 for k in msgpack.unpackb(blob[start:start + size])["amdhsa.kernels"]:
-                    found[k[".name"]] = k[".vgpr_count"]
+                    found[k[".name"]] = k[what]
         at = blob.find(b"\x7fELF\x02\x01\x01\x40", at + 64)
     return found
 
@@ -686,3 +709,28 @@ def test_two_workgroups_of_the_general_kernel_share_a_compute_unit():
     regs = {k: v for k, v in _kernel_registers().items()
             if "gemm_kernelILi64ELi128E" in k or ("gemm_kernelILi128ELi128E" in k and re.match(r".*ILi128ELi128ELi2ELi2ELi\dELb\dELb0E", k))}
     assert len(regs) >= 9 and max(regs.values()) <= 256, regs
+
+
+def _pipe(bm, bn, wm, wn, fmt, fold, park, finish):
+    flags = "".join(f"Lb{int(f)}E" for f in (False, park, finish) + (False,) * 6)
+    return f"_ZN4segq16gemm_pipe_kernelILi{bm}ELi{bn}ELi{wm}ELi{wn}ELi{fmt}ELb{int(fold)}ELi2E{flags}EEvNS_10GemmParamsE"
+
+
+@pytest.mark.parametrize("tile, fmt, fold, park, registers, scratch", [
+    # several ranges of int8, parked: they have the low-rank branch, and nothing of its way through LDS
+    ((256, 256, 4, 2), 0, True, True, 256, 556),
+    ((256, 192, 4, 2), 0, True, True, 256, 140),
+    ((192, 256, 2, 4), 0, True, True, 256, 132),
+    ((256, 128, 4, 2), 0, True, True, 224, 0),
+    # several ranges of e4m3: two workgroups share a compute unit
+    ((128, 128, 4, 2), 1, True, False, 128, 0),
+    # one range
+    ((256, 256, 4, 2), 0, False, False, 256, 0),
+    ((256, 256, 4, 2), 1, False, False, 256, 16),
+    ((384, 192, 4, 2), 0, False, False, 256, 12),
+    ((384, 192, 4, 2), 1, False, False, 256, 12),
+])
+def test_instances_that_finish_in_output_units(tile, fmt, fold, park, registers, scratch):
+    """What an instance loses in registers costs resident waves, or a trip through scratch memory in every workgroup."""
+    name = _pipe(*tile, fmt, fold, park, True)
+    assert _kernel_registers()[name] <= registers and _kernel_registers(".private_segment_fixed_size")[name] <= scratch
