@@ -321,8 +321,11 @@ typedef struct segq_gemm_desc {
     int32_t out_code_fmt;   /* SEGQ_CODE_I8 | SEGQ_CODE_E4M3 */
     int32_t finite_scales;  /* 0, or non-zero: the scales of all ranges are finite, and without own_sum the library
                          * takes the faster way to sum them (two ranges over the same run of K, one from a and one
-                         * from a_neg, can be multiplied in one walk of it, each with its own sums, and one more
-                         * range from a behind them; neither is parked) */
+                         * from a_neg, or of a_sel 2 and 3, can be multiplied in one walk of it, each with its own sums,
+                         * and one more range of a_sel 0 behind them; neither is parked).  Ranges of a_sel 2 and 3 go
+                         * there wherever they can: their other kernel is far behind.  With a_neg set beside them
+                         * (it is not read) they go there only where that is the best of both forms, so that a caller who
+                         * has not written the codes yet can ask segq_gemm_plan: a tile from 31 on is for one tensor */
     segq_krange ranges[SEGQ_MAX_RANGES];
 } segq_gemm_desc;
 

@@ -508,6 +508,8 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
             const bool share = lent && d->split_k != 1;
             MixPick pick = choose_mix(d->m, d->n, steps, plain, share ? 16 : 1);
             while (pick.shares > 1 && !shares_fit(pick.cfg, pick.shares)) pick = choose_mix(d->m, d->n, steps, plain, pick.shares - 1);
+            // (Codes of both signs in one tensor have no other way than this but the general kernel, far behind it: the lines below are
+            // for two tensors, and for the caller that may still make two of them, a_neg.)
             // Up to 128 rows K shares of the ranges in turn are ahead, from where there are enough of them.  us a pass, that / this:
             // 32 x 1536 x (1536 + 6144) e4m3 18.7 / 23.4, 128 rows 22.0 / 25.1, int8 27.0 / 25.4.  Beside a plain range e4m3 takes
             // 128 x 128 tiles in three shares and more: 1 x 512 x (512 + 2048) 18.2 / 22.0, 128 rows 20.6 / 25.2, 1 x 4096 x (1024 +
@@ -517,6 +519,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
             // (768 + 3072) 27.0 / 26.4, 16 x 3072 24.7 / 24.0, 1 x 640 x (640 + 2560), which is not shared, 49.6 / 24.3.
             const int64_t all = 2 * steps + plain;
             const bool in_shares = steps + plain >= 32 || (mix.plain >= 0 && (f8 ? all >= 24 && d->m * d->n <= 540000 : all >= 52 && d->m <= 32 && d->n <= 1024));
+            const bool part = d->ranges[mix.pos].a_sel == 2;
             bool take = d->m > 128 || !share || !in_shares;
             // The pair alone: against one walk of tiles 29 and 30, or the ranges in turn.  us, that / this: 2500 x 3072 x 12288 161 / 143,
             // 600 x 2048 x 8192 44 / 34, 4608 x 3072 x 12288 int8 310 / 266; 4096 x 1536 x 6144 57 / 60, 2600 x 1152 x 4608 30 / 34.
@@ -527,9 +530,16 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
                                    : t64 <= 1.0 ? 4.8 + 0.6 * k : 4.0 + t64 * (0.44 * k + 0.8);
                 // (one tensor: with what the quantise step, which asks for this plan, then does not write.  Feed-forward of 4096
                 // rows, 1536 x 6144 e4m3 through the epilogue that writes codes: two tensors 125 us a pass, one 121)
-                take = take && pick.us < (d->ranges[0].a_sel == 2 ? now + (double)d->m * steps * 128 / 5e6 : 0.95 * now);
+                double most = part ? now + (double)d->m * steps * 128 / 5e6 : 0.95 * now;
+                // Where the two estimates meet these are short of what the launches take: int8 beside whole tiles of 128 x 192 with fewer than
+                // twice as many rows as columns, so that what one tensor saves is not the most of what is loaded (1552 x 3008 x 5760
+                // 58.4 us a pass, here 64.7; of 28 such shapes 27 were slower here, by 3 % in the middle; 4096 x 1536 x 6144 76.2 / 74.5), and three
+                // or four shares of a short K beside one round of 64 x 128 (605 x 1088 x 3968 27.2 / 30.9, 800 x 1152 x 4608 32.1 / 33.9).
+                if (i8 && walk.cfg == FIRST_DUAL_CFG && d->m < 2 * d->n) most = 0.92 * now;
+                if (walk.cfg == FIRST_DUAL_CFG + 1 && t64 <= 1.0 && pick.shares > 2 && steps < 40) most = 0.85 * now;
+                take = take && pick.us < most;
             }
-            if (take) {
+            if (take || (part && !d->a_neg)) {
                 walk.cfg = -1;
                 mix.cfg = pick.cfg;
                 mix.shares = pick.shares;

@@ -610,7 +610,7 @@ def dual_in_one_tensor(device: int, M: int, N: int, K: int, segments, fmt: str, 
     d.a_fmt = d.b_fmt = _CODE[fmt]
     d.out_dtype = _dt(dtype)
     d.m, d.n, d.lda, d.ldb, d.ldo, d.batch, d.finite_scales = M, N, K, K, N, 1, 1
-    d.a = d.b = d.out = d.workspace = 4096
+    d.a = d.a_neg = d.b = d.out = d.workspace = 4096  # (a_neg: there may be two tensors)
     d.workspace_bytes = 1 << 60
     kinds = [(k0, k1, sel) for k0, k1, dual in segments for sel in ((2, 3) if dual else (0,))]
     if not 1 < len(kinds) <= 3 or K % 16 or any(k0 % 128 or k1 % 128 for k0, k1, _ in kinds):

@@ -486,7 +486,7 @@ def test_smooth_and_svd_layers_on_the_fake_path_equal_the_oracle(opt_type, seg_m
                       opt_kwargs={"search_alpha_config": {"enable": True, "min": 0.1, "max": 0.9, "step": 0.1}}, device="cpu")
 
 
-def _plan(lib, m, n, ranges, fmt, out_dtype=2, lend=True, split_k=0, tile=0, lowrank=0, finite=0):
+def _plan(lib, m, n, ranges, fmt, out_dtype=2, lend=True, split_k=0, tile=0, lowrank=0, finite=0, neg=True):
     """segq_gemm_plan / segq_gemm_workspace_bytes on a descriptor of made-up (aligned, never
     dereferenced) device addresses: the library's decisions are host arithmetic and launch nothing.
     ranges: (k_begin, k_len, a_sel).  Returns (tile id, K shares, parked, workspace bytes)."""
@@ -497,7 +497,7 @@ def _plan(lib, m, n, ranges, fmt, out_dtype=2, lend=True, split_k=0, tile=0, low
     d.out_dtype = d.bias_dtype = out_dtype  # 2: bf16
     k = max(b + l for b, l, _ in ranges)
     d.m, d.n, d.lda, d.ldb, d.ldo, d.batch = m, n, k, k, n, 1
-    d.a, d.a_neg, d.b, d.out, d.bias = 0x10000000, 0x20000000, 0x30000000, 0x40000000, 0x50000000
+    d.a, d.a_neg, d.b, d.out, d.bias = 0x10000000, 0x20000000 if neg else 0, 0x30000000, 0x40000000, 0x50000000
     d.n_ranges, d.tile, d.split_k, d.finite_scales = len(ranges), tile, split_k, finite
     for i, (b, l, sel) in enumerate(ranges):
         d.ranges[i].k_begin, d.ranges[i].k_len, d.ranges[i].a_sel = b, l, sel
@@ -577,6 +577,25 @@ def test_few_rows_beside_a_plain_segment(m, n, k0, k1, fmt, walk):
             assert tile < 31 and shares > 1 and need > 0
         else:
             assert tile < 31
+        if pair == (2, 3):
+            assert _plan(L.lib(), m, n, [(0, k0, 0), (k0, k1, 2), (k0, k1, 3)], fmt, finite=1, neg=False)[0] in (31, 32, 33)
+
+
+@pytest.mark.parametrize("m, n, k, fmt, walk", [
+    # int8 beside whole tiles of 128 x 192 that walk K once on two tensors
+    (1552, 3008, 5760, 0, False), (2812, 1856, 6656, 0, False), (2834, 1664, 2048, 0, False), (2834, 1664, 2048, 1, True),
+    (4096, 1536, 6144, 0, True),
+    # three or four shares of a short K beside one round of 64 x 128
+    (605, 1088, 3968, 0, False), (500, 768, 3072, 1, False), (800, 1152, 4608, 1, False), (500, 1152, 4608, 1, True),
+    (605, 1088, 5120, 0, True), (1000, 1280, 5120, 0, True),
+])
+def test_pair_alone_in_one_walk(m, n, k, fmt, walk):
+    """DualScale without another segment: one tensor (or, of two, the same walk) only where it is ahead of two tensors."""
+    from segquant_amd import _lib as L
+    plan = lambda sel, **kw: _plan(L.lib(), m, n, [(0, k, sel), (0, k, sel + 1)], fmt, finite=1, **kw)
+    assert (plan(2)[0] >= 31) == walk and (walk or plan(0)[0] < 31)
+    # codes that are in one tensor already go there anyway, whatever is lent
+    assert all(plan(2, neg=False, lend=lend)[0] in (31, 32, 33) for lend in (True, False))
 
 
 def test_plan_refuses_what_the_launch_would_refuse():
