@@ -156,6 +156,17 @@ class OptimizerRegistry:
 _MAX_CACHED_TOKEN_COUNTS = 8  # (token count, dtype, bias) entries a layer keeps launch descriptors and buffers for
 
 
+def _lent(plan, g, M, dtype, form=None):
+    """Workspace bytes that the library would use for ``g``, asked once for what the answer depends on: the rows, whether the
+    outputs have 16 bits, and ``form``, what else sets the launch apart from a plain one of as many rows."""
+    known = plan.setdefault("ws_need", {})
+    key = M if form is None and dtype != torch.float32 else (M, dtype == torch.float32, form)
+    need = known.get(key)
+    if need is None:
+        need = known[key] = ops.gemm_workspace_bytes(g)
+    return need
+
+
 def _readable_rows(x2: torch.Tensor) -> torch.Tensor:
     """``x2`` (rows, K) if the quantise kernel can read it where it lies, a contiguous copy otherwise.
     A column slice of a wider tensor (one half of a gated projection, a part of a fused qkv) is read in
@@ -419,7 +430,7 @@ class DefaultOptimizer(BaseOptimizer):
         if g is None:
             g = ops.gemm_desc(codes, plan["w"], ranges, addend=add2, **kw)
         # Whether to lend the library a workspace is this layer's call; how much it could use is
-        # the library's (segq_gemm_workspace_bytes), asked once per token count.
+        # the library's (segq_gemm_workspace_bytes), asked once per token count, dtype and kind of launch.
         #  * int4 weights: _lends_int4.
         #  * 8-bit weights: always.  int8 with several ranges that no one walk of K serves parks the
         #    finished ranges' sums there and keeps the big tiles; few tiles and a long K share the K steps of
@@ -428,9 +439,8 @@ class DefaultOptimizer(BaseOptimizer):
         lend = _lends_int4(plan, M) if int4 else True
         ws = None
         if lend:
-            need = plan.setdefault("ws_need", {}).get(M)
-            if need is None:
-                need = plan["ws_need"][M] = ops.gemm_workspace_bytes(g)
+            # (codes out and a low-rank branch in the epilogue rule out K shares, which the same rows have without them)
+            need = _lent(plan, g, M, x.dtype, "codes out" if out_codes is not None else "low rank" if g[0].lowrank_rank else None)
             if need:
                 ws = ops.int4_workspace(x.device, need)
         if plain:
@@ -517,9 +527,7 @@ class DefaultOptimizer(BaseOptimizer):
         ws = None
         int4 = plan["fw"] == ops.FMT_INT4
         if not int4 or _lends_int4(plan, M):
-            need = plan.setdefault("ws_need", {}).get(M)
-            if need is None:
-                need = plan["ws_need"][M] = ops.gemm_workspace_bytes(g)
+            need = _lent(plan, g, M, out_dtype, "two tensors" if codes_neg is not None else None)
             if need:
                 ws = ops.int4_workspace(codes.device, need)
         out = ops.gemm_launch(g, ws)
@@ -594,9 +602,7 @@ class DefaultOptimizer(BaseOptimizer):
         int4 = plan["fw"] == ops.FMT_INT4
         ws = None
         if not int4 or _lends_int4(plan, M):
-            need = plan.setdefault("ws_need", {}).get(M)
-            if need is None:
-                need = plan["ws_need"][M] = ops.gemm_workspace_bytes(g)
+            need = _lent(plan, g, M, dt)
             if need:
                 ws = ops.int4_workspace(dev, need)
         out = ops.gemm_launch(g, ws)

@@ -1,6 +1,7 @@
 """What a layer keeps between calls, on the host: descriptors filled for CPU buffers, nothing launched."""
 import threading
 import time
+import types
 
 import pytest
 import torch
@@ -131,3 +132,35 @@ def test_calls_that_share_no_buffers_take_no_lock(layer, monkeypatch):
                              ({"K": K, "launches": {}}, {"pre_op": "gelu"}, False), ({"K": K, "launches": {}}, {"addend": x}, False)):
         layer._plan = plan
         assert layer.forward_fused(x, **kw) is locked
+
+
+def _fused_layer(layer, monkeypatch, rows, k, n, l2t=None):
+    """The layer's fused route on CPU tensors (never read: nothing is launched), with a plan for int8 codes; what it lends."""
+    lent = []
+    monkeypatch.setattr(ops, "_need_cuda", lambda *ts: None)
+    monkeypatch.setattr(ops, "int4_workspace", lambda device, need: lent.append(need) or torch.empty(1, dtype=torch.uint8))
+    one = torch.ones(1)
+    layer.chunks, layer.seg_mode, layer.dual_scale, layer.dual_segments = 1, "weight", False, [False]
+    layer.input_calibrators = [types.SimpleNamespace(dynamic=False)]
+    layer._plan = dict(fa="int8", fw="int8", w=torch.empty(n, k, dtype=torch.int8), sw=one, sw_cs=0, bounds=[0, k], N=n, K=k, sx=(one[None], None))
+    if l2t is not None:
+        layer._plan["l2t"] = l2t
+        layer._lowrank_operands = lambda plan, x2: (torch.empty(rows, l2t.shape[1], dtype=x2.dtype), l2t.to(x2.dtype))
+    return lent
+
+
+def test_a_launch_without_shares_leaves_those_of_other_launches_their_workspace(layer, monkeypatch):
+    """256 x 3072 x 12288 is shared along K, but not with codes out or with a low-rank branch in the epilogue: whichever comes
+    first, every launch is lent what it can use itself."""
+    rows, k, n = 256, 12288, 3072
+    x = torch.empty(rows, k, dtype=torch.bfloat16)
+    spec = dict(fmt="int8", scale=torch.ones(1))
+    for calls in (("codes", "plain"), ("plain", "codes")):
+        lent = _fused_layer(layer, monkeypatch, rows, k, n)
+        for call in calls:
+            ws = layer.fused_launches(x, out_codes=spec if call == "codes" else None)[2]
+            assert (ws is None) == (call == "codes")
+        assert len(lent) == 1 and lent[0] > 0
+    lent = _fused_layer(layer, monkeypatch, rows, k, n, l2t=torch.empty(n, 32))
+    assert layer.fused_launches(x)[2] is None  # the branch is in the epilogue
+    assert layer.fused_launches(x.float())[2] is not None and lent[0] > 0  # 32-bit outputs have it as an addend
