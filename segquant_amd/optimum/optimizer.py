@@ -156,6 +156,18 @@ class OptimizerRegistry:
 _MAX_CACHED_TOKEN_COUNTS = 8  # (token count, dtype, bias) entries a layer keeps launch descriptors and buffers for
 
 
+_MAX_ANSWERS = 256  # ... and keeps the library's answers for
+
+
+def _keep(table, key, value):
+    """``table[key] = value`` in a table of answers that can be asked for again: a full one is emptied, so that a layer fed with
+    ever-changing token counts does not grow."""
+    if len(table) >= _MAX_ANSWERS:
+        table.clear()
+    table[key] = value
+    return value
+
+
 def _lent(plan, g, M, dtype, form=None):
     """Workspace bytes that the library would use for ``g``, asked once for what the answer depends on: the rows, whether the
     outputs have 16 bits, and ``form``, what else sets the launch apart from a plain one of as many rows."""
@@ -163,7 +175,7 @@ def _lent(plan, g, M, dtype, form=None):
     key = M if form is None and dtype != torch.float32 else (M, dtype == torch.float32, form)
     need = known.get(key)
     if need is None:
-        need = known[key] = ops.gemm_workspace_bytes(g)
+        need = _keep(known, key, ops.gemm_workspace_bytes(g))
     return need
 
 
@@ -413,17 +425,19 @@ class DefaultOptimizer(BaseOptimizer):
             # kernel for it (16-bit dtypes, the 8-wave kernels), as a materialised (M, N) addend otherwise
             t_lr, l2t = self._lowrank_operands(plan, x2)
             key = (M, x.dtype)
-            ok, tiles = plan.setdefault("lr_ok", {}).get(key), plan.setdefault("lr_tile", {})
+            known, tiles = plan.setdefault("lr_ok", {}), plan.setdefault("lr_tile", {})
+            ok, tile = known.get(key), tiles.get(key)
             if ok is None or ok:
                 try:
-                    if ok is None:
-                        tiles[key] = ops.lowrank_tile(ops.gemm_desc(codes, plan["w"], ranges, **kw)) if len(ranges) == 1 else 0
-                    g = ops.gemm_desc(codes, plan["w"], ranges, addend=add2, lowrank=(t_lr, l2t), tile=tiles[key], **kw)
+                    if tile is None:
+                        tile = _keep(tiles, key, ops.lowrank_tile(ops.gemm_desc(codes, plan["w"], ranges, **kw)) if len(ranges) == 1 else 0)
+                    g = ops.gemm_desc(codes, plan["w"], ranges, addend=add2, lowrank=(t_lr, l2t), tile=tile, **kw)
                     if ok is None:
                         ops.gemm_plan(g)
                 except RuntimeError:
                     g = None
-                plan["lr_ok"][key] = g is not None
+                if ok is None:
+                    _keep(known, key, g is not None)
             if g is None:
                 low = t_lr @ l2t.t()
                 add2 = low if add2 is None else add2 + low
@@ -494,8 +508,8 @@ class DefaultOptimizer(BaseOptimizer):
             bounds = plan["bounds"]
             S = self.chunks if self.seg_mode == "input" else 1
             segments = tuple((bounds[s], bounds[s + 1], bool(self.dual_segments[s])) for s in range(S))
-            one = known[M, dtype] = (plan["fa"] == plan["fw"] and plan["fa"] != ops.FMT_INT4 and plan.get("group_dequant") is None and
-                                     "l2t" not in plan and ops.dual_in_one_tensor(plan["w"].device.index or 0, M, plan["N"], plan["K"], segments, plan["fa"], dtype))
+            one = _keep(known, (M, dtype), plan["fa"] == plan["fw"] and plan["fa"] != ops.FMT_INT4 and plan.get("group_dequant") is None and
+                        "l2t" not in plan and ops.dual_in_one_tensor(plan["w"].device.index or 0, M, plan["N"], plan["K"], segments, plan["fa"], dtype))
         return one
 
     def writes_codes(self, x: torch.Tensor) -> bool:

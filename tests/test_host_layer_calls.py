@@ -164,3 +164,23 @@ def test_a_launch_without_shares_leaves_those_of_other_launches_their_workspace(
     lent = _fused_layer(layer, monkeypatch, rows, k, n, l2t=torch.empty(n, 32))
     assert layer.fused_launches(x)[2] is None  # the branch is in the epilogue
     assert layer.fused_launches(x.float())[2] is not None and lent[0] > 0  # 32-bit outputs have it as an addend
+
+
+def test_answers_kept_per_token_count_are_bounded(layer, monkeypatch):
+    """A layer fed with ever-changing token counts keeps no more of the library's answers than a fixed number."""
+    k, n, most = 128, 256, opt_mod._MAX_ANSWERS
+    counts = range(1, 2 * most + 3)
+    monkeypatch.setattr(ops, "lowrank_tile", lambda g: 0)
+    _fused_layer(layer, monkeypatch, 0, k, n)
+    layer._lowrank_operands = lambda plan, x2: (torch.empty(x2.shape[0], 32, dtype=x2.dtype), torch.empty(n, 32, dtype=x2.dtype))
+    layer._plan["l2t"] = torch.empty(n, 32)
+    for m in counts:
+        layer.fused_launches(torch.empty(m, k, dtype=torch.bfloat16))
+    layer.dual_segments = [True]
+    plan = {k_: v for k_, v in layer._plan.items() if k_ != "l2t"}
+    monkeypatch.setattr(ops, "dual_in_one_tensor", lambda *a: True)
+    for m in counts:
+        assert layer._one_code_tensor(plan, m, torch.bfloat16) is True
+    for table in (layer._plan["lr_ok"], layer._plan["lr_tile"], layer._plan["ws_need"], plan["one_tensor"]):
+        assert 0 < len(table) <= most
+    assert layer._plan["lr_ok"][counts[-1], torch.bfloat16] is True  # (a full table starts anew: the newest is there)
