@@ -65,6 +65,10 @@ class BaseOptimizer:
         self.scale_tensor = None
         self._plan = None
 
+    def __setstate__(self, state):
+        # a plan belongs to the build of the package, and to the device, that made it: loaded and copied layers make their own
+        self.__dict__.update(state, _plan=None)
+
     def _stack(self, calibrators, attr):
         dev = self.weight_manager.device()
 

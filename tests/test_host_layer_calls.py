@@ -1,4 +1,6 @@
 """What a layer keeps between calls, on the host: descriptors filled for CPU buffers, nothing launched."""
+import copy
+import pickle
 import threading
 import time
 import types
@@ -7,7 +9,8 @@ import pytest
 import torch
 
 from segquant_amd import ops
-from segquant_amd.optimum import optimizer as opt_mod
+from segquant_amd.optimum import optimizer as opt_mod, smooth  # noqa: F401 (registers the smoothing optimisers)
+from segquant_amd.optimum.optimizer import OptimizerRegistry
 
 M, N, K = 4, 8, 16
 
@@ -184,3 +187,13 @@ def test_answers_kept_per_token_count_are_bounded(layer, monkeypatch):
     for table in (layer._plan["lr_ok"], layer._plan["lr_tile"], layer._plan["ws_need"], plan["one_tensor"]):
         assert 0 < len(table) <= most
     assert layer._plan["lr_ok"][counts[-1], torch.bfloat16] is True  # (a full table starts anew: the newest is there)
+
+
+@pytest.mark.parametrize("again", [lambda o: pickle.loads(pickle.dumps(o)), copy.deepcopy])
+def test_a_loaded_layer_makes_a_plan_of_its_own(again):
+    """A layer saved after its first call has a plan in the file, of the version that saved it: one from before the transposed
+    low-rank factors has none of them, and the layer must not look for them there."""
+    opt = object.__new__(OptimizerRegistry.get("svd"))
+    opt.__dict__.update(low_rank=32, chunks=1, _plan=dict(K=K, N=N, l2t=torch.empty(N, 32), l12_cast={}))
+    loaded = again(opt)
+    assert loaded._plan is None and (loaded.low_rank, loaded.chunks) == (32, 1) and opt._plan is not None
