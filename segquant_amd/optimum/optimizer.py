@@ -172,11 +172,11 @@ def _keep(table, key, value):
     return value
 
 
-def _lent(plan, g, M, dtype, form=None):
-    """Workspace bytes that the library would use for ``g``, asked once for what the answer depends on: the rows, whether the
-    outputs have 16 bits, and ``form``, what else sets the launch apart from a plain one of as many rows."""
+def _lent(plan, g, M, form=None):
+    """Workspace bytes that the library would use for ``g``, asked once for what the answer depends on: the rows, and ``form``,
+    what sets the launch apart from a plain one of as many rows (the output's type does not: only ragged K has a rule on it)."""
     known = plan.setdefault("ws_need", {})
-    key = M if form is None and dtype != torch.float32 else (M, dtype == torch.float32, form)
+    key = M if form is None else (M, form)
     need = known.get(key)
     if need is None:
         need = _keep(known, key, ops.gemm_workspace_bytes(g))
@@ -448,7 +448,7 @@ class DefaultOptimizer(BaseOptimizer):
         if g is None:
             g = ops.gemm_desc(codes, plan["w"], ranges, addend=add2, **kw)
         # Whether to lend the library a workspace is this layer's call; how much it could use is
-        # the library's (segq_gemm_workspace_bytes), asked once per token count, dtype and kind of launch.
+        # the library's (segq_gemm_workspace_bytes), asked once per token count and kind of launch.
         #  * int4 weights: _lends_int4.
         #  * 8-bit weights: always.  int8 with several ranges that no one walk of K serves parks the
         #    finished ranges' sums there and keeps the big tiles; few tiles and a long K share the K steps of
@@ -458,7 +458,7 @@ class DefaultOptimizer(BaseOptimizer):
         ws = None
         if lend:
             # (codes out and a low-rank branch in the epilogue rule out K shares, which the same rows have without them)
-            need = _lent(plan, g, M, x.dtype, "codes out" if out_codes is not None else "low rank" if g[0].lowrank_rank else None)
+            need = _lent(plan, g, M, "codes out" if out_codes is not None else "low rank" if g[0].lowrank_rank else None)
             if need:
                 ws = ops.int4_workspace(x.device, need)
         if plain:
@@ -545,7 +545,7 @@ class DefaultOptimizer(BaseOptimizer):
         ws = None
         int4 = plan["fw"] == ops.FMT_INT4
         if not int4 or _lends_int4(plan, M):
-            need = _lent(plan, g, M, out_dtype, "two tensors" if codes_neg is not None else None)
+            need = _lent(plan, g, M, "two tensors" if codes_neg is not None else None)
             if need:
                 ws = ops.int4_workspace(codes.device, need)
         out = ops.gemm_launch(g, ws)
@@ -620,7 +620,7 @@ class DefaultOptimizer(BaseOptimizer):
         int4 = plan["fw"] == ops.FMT_INT4
         ws = None
         if not int4 or _lends_int4(plan, M):
-            need = _lent(plan, g, M, dt)
+            need = _lent(plan, g, M)
             if need:
                 ws = ops.int4_workspace(dev, need)
         out = ops.gemm_launch(g, ws)
