@@ -316,7 +316,9 @@ def gemm_plan(g, workspace: Optional[torch.Tensor] = None) -> dict:
 
 def lowrank_rows(x: torch.Tensor, l1t: torch.Tensor, out: torch.Tensor) -> bool:
     """``out = x @ l1t.t()`` for a low-rank branch (``segq_lowrank_rows``), or False, nothing launched, where the kernel does
-    not serve the sizes or the alignment."""
+    not serve the sizes or the alignment, or a derivative is wanted (torch's product into ``out`` refuses that)."""
+    if (x.requires_grad and torch.is_grad_enabled()) or torch.autograd.forward_ad._current_level >= 0:
+        return False
     k, r = x.shape[1], l1t.shape[0]
     if k % 64 or r % 16 or not x.is_cuda or x.stride(1) != 1 or row_stride(x) % 8 or x.data_ptr() % 16 or l1t.data_ptr() % 16:
         return False

@@ -774,6 +774,21 @@ def test_low_rank_rows(ops, dt):
         assert not ops.lowrank_rows(wide[:, 1:1 + K], l1t, out[:, :r]) and not ops.lowrank_rows(wide[:, :K + 8], l1t, out[:, :r])
 
 
+def test_low_rank_rows_leave_derivatives_to_the_product_that_refuses_them(ops):
+    """A layer's low-rank operand is a product into a tensor that is there: torch refuses to differentiate that, and the kernel
+    must not take the call and lose the gradient without a word."""
+    x, l1t = (torch.randn(n, 128, dtype=torch.bfloat16, device=DEV) for n in (20, 32))
+    out = torch.empty(20, 32, dtype=torch.bfloat16, device=DEV)
+    with torch.autograd.forward_ad.dual_level():
+        assert not ops.lowrank_rows(x, l1t, out)
+    x.requires_grad_()
+    assert not ops.lowrank_rows(x, l1t, out)
+    with pytest.raises(RuntimeError):
+        torch.matmul(x, l1t.t(), out=out)
+    with torch.no_grad():
+        assert ops.lowrank_rows(x, l1t, out)
+
+
 @pytest.mark.parametrize("fmt_w", [O.FMT_INT4, O.FMT_INT8])
 @pytest.mark.parametrize("dt", ["fp32", "bf16"])
 def test_group_wise_weight_scales(ops, fmt_w, dt):
