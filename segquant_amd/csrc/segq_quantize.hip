@@ -199,6 +199,13 @@ __device__ __forceinline__ void f32_to_raw(const float (&v)[16], RawRun<DT>& r) 
     }
 }
 
+// What stands in front of the codes: nothing, column divisors, or an activation function and, if given, divisors behind it.
+// 16-bit inputs have instances for divisors alone: the function's registers (bf16, rows of 8192 and more: 191 for 162) cost them
+// the third workgroup per CU.  us, one instance / two, dynamic: bf16 4608 x 12288 63 / 47, 4096 x 8192 40 / 32, 4608 x 5120 26.1 / 23.1,
+// 8192 x 1280 14.8 / 13.7, fp16 4608 x 12288 51 / 44; static, bf16 9216 x 12288 86 / 83.  fp32 stays with the one: static 9216 x 12288
+// 117 / 129, dynamic 4608 x 16384 81 / 85, 2048 x 4096 12.6 / 13.6.
+enum { PRE_RUN_NONE, PRE_RUN_DIV, PRE_RUN_ACT };
+
 template <int DT>
 __device__ __forceinline__ void load_gate(const QuantParams& p, int64_t row, int64_t col, RawRun<DT>& g) {
     const size_t esz = (DT == SEGQ_F32) ? 4 : 2;
@@ -207,11 +214,11 @@ __device__ __forceinline__ void load_gate(const QuantParams& p, int64_t row, int
 
 // r holds 16 elements of x at (row, col), gr those of the gate if there is one; on return r holds what is quantised:
 // op(x), or x * op(gate), each operator's result rounded to the tensor's dtype
-template <int DT>
+template <int DT, int PRE>
 __device__ __forceinline__ void pre_run(const QuantParams& p, int64_t col, RawRun<DT>& r, RawRun<DT>& gr) {
     float v[16];
     raw_to_f32<DT>(r, v);
-    if (p.pre_op != SEGQ_PRE_NONE) {
+    if (PRE == PRE_RUN_ACT && p.pre_op != SEGQ_PRE_NONE) {
         if (p.gate) {
             float g[16];
             raw_to_f32<DT>(gr, g);
@@ -228,7 +235,7 @@ __device__ __forceinline__ void pre_run(const QuantParams& p, int64_t col, RawRu
             raw_to_f32<DT>(r, v);
         }
     }
-    if (p.col_div) {
+    if (PRE == PRE_RUN_DIV || p.col_div) {
         // x / s as torch's in-place div_ in the tensor's dtype: an IEEE fp32 division, rounded to the dtype
         const float4* q = reinterpret_cast<const float4*>(p.col_div + col);
 #pragma unroll
@@ -243,14 +250,14 @@ __device__ __forceinline__ void pre_run(const QuantParams& p, int64_t col, RawRu
 
 // With a fused activation the run kept in registers is the activation's output
 // (already in the tensor's dtype, so repacking it loses nothing).
-template <int DT, bool PRE>
+template <int DT, int PRE>
 __device__ __forceinline__ void load_run(const QuantParams& p, const uint8_t* xrow, int64_t row, int c, RawRun<DT>& r) {
     const size_t esz = (DT == SEGQ_F32) ? 4 : 2;
     load_raw<DT>(xrow + (size_t)c * 16 * esz, r);
-    if constexpr (PRE) {
+    if constexpr (PRE != PRE_RUN_NONE) {
         RawRun<DT> g;
-        load_gate<DT>(p, row, (int64_t)c << 4, g);
-        pre_run<DT>(p, (int64_t)c << 4, r, g);
+        if constexpr (PRE == PRE_RUN_ACT) load_gate<DT>(p, row, (int64_t)c << 4, g);
+        pre_run<DT, PRE>(p, (int64_t)c << 4, r, g);
     }
 }
 
@@ -288,7 +295,7 @@ __device__ __forceinline__ float wave_max(float v) {  // of non-negative values 
 // One workgroup per row.  All loads of the row are issued before anything is computed; up to
 // CACHE runs per thread stay in registers in packed form between the reduction and the encode,
 // longer rows are read again (they hit in L2).  CACHE 1: a run per thread (up to eight waves).
-template <int DT, int FMT, int CACHE, bool DUAL, bool PRE>
+template <int DT, int FMT, int CACHE, bool DUAL, int PRE>
 __global__ void __launch_bounds__(CACHE == 4 ? 256 : 512) quant_dynamic_kernel(const QuantParams p) {
     __shared__ float red[2][8];
     const int nt = CACHE == 4 ? 256 : blockDim.x, nw = nt >> 6;
@@ -375,7 +382,7 @@ __global__ void __launch_bounds__(CACHE == 4 ? 256 : 512) quant_dynamic_kernel(c
 // For rows of up to 64 * CPL runs: the whole row is in flight at once, the
 // maximum is reduced with cross-lane shuffles only, and four rows share a
 // workgroup without ever synchronising.
-template <int DT, int FMT, int CPL, bool DUAL, bool PRE>
+template <int DT, int FMT, int CPL, bool DUAL, int PRE>
 __global__ void __launch_bounds__(256) quant_dynamic_wave_kernel(const QuantParams p) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -515,7 +522,7 @@ __global__ void __launch_bounds__(64) quant_dynamic_row_many_kernel(const QuantB
 
 
 // ---- static scales ---------------------------------------------------------
-template <int DT, int FMT, bool PRE>
+template <int DT, int FMT, int PRE>
 __global__ void __launch_bounds__(256) quant_static_kernel(const QuantParams p) {
     const int64_t cpr = p.cols >> 4;  // runs of 16 per row
     const int64_t run = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -529,12 +536,12 @@ __global__ void __launch_bounds__(256) quant_static_kernel(const QuantParams p) 
     const float s_neg = dual ? p.scale_neg[si] : s_pos;
     const size_t esz = (DT == SEGQ_F32) ? 4 : 2;
     float x[16];
-    if constexpr (PRE) {
+    if constexpr (PRE != PRE_RUN_NONE) {
         RawRun<DT> r;
         load_raw<DT>(static_cast<const uint8_t*>(p.x) + (row * p.ldx + col) * esz, r);
         RawRun<DT> g;
-        load_gate<DT>(p, row, col, g);
-        pre_run<DT>(p, col, r, g);
+        if constexpr (PRE == PRE_RUN_ACT) load_gate<DT>(p, row, col, g);
+        pre_run<DT, PRE>(p, col, r, g);
         raw_to_f32<DT>(r, x);
     } else {
         load16<DT>(static_cast<const uint8_t*>(p.x) + (row * p.ldx + col) * esz, x);
@@ -605,13 +612,13 @@ __global__ void __launch_bounds__(256) fake_e4m3_kernel(const void* x, void* out
 }
 
 // ---- host side ---------------------------------------------------------------
-template <int DT, int FMT, bool PRE>
+template <int DT, int FMT, int PRE>
 static int launch_quant(const QuantParams& p, hipStream_t st) {
     if (p.dynamic) {
         int longest = 0;  // runs of 16 in the longest column segment
         for (int i = 0; i < p.n_kseg; ++i) longest = longest > (p.kb[i + 1] - p.kb[i]) / 16 ? longest : (p.kb[i + 1] - p.kb[i]) / 16;
         const dim3 wgrid((unsigned)((p.rows + 3) / 4)), bgrid((unsigned)p.rows);
-        if constexpr (!PRE) {
+        if constexpr (PRE == PRE_RUN_NONE) {
             if (p.n_kseg == 1 && longest <= 64 * 8 && (!p.dual || (p.dual_mask & 1u))) {
                 const dim3 rgrid((unsigned)p.rows), one_wave(64);
 #define SEGQ_ROW(CPL_)                                                                                              \
@@ -672,12 +679,21 @@ static int launch_quant(const QuantParams& p, hipStream_t st) {
     return check_launch("segq_quantize");
 }
 
+template <int DT, int FMT>
+static int launch_quant_pre(const QuantParams& p, hipStream_t st) {
+    if (!p.pre_op && !p.col_div) return launch_quant<DT, FMT, PRE_RUN_NONE>(p, st);
+    if constexpr (DT != SEGQ_F32) {
+        if (!p.pre_op) return launch_quant<DT, FMT, PRE_RUN_DIV>(p, st);
+    }
+    return launch_quant<DT, FMT, PRE_RUN_ACT>(p, st);
+}
+
 template <int DT>
 static int launch_quant_fmt(const QuantParams& p, hipStream_t st) {
     switch (p.fmt) {
-        case SEGQ_CODE_I8: return (p.pre_op || p.col_div) ? launch_quant<DT, SEGQ_CODE_I8, true>(p, st) : launch_quant<DT, SEGQ_CODE_I8, false>(p, st);
-        case SEGQ_CODE_E4M3: return (p.pre_op || p.col_div) ? launch_quant<DT, SEGQ_CODE_E4M3, true>(p, st) : launch_quant<DT, SEGQ_CODE_E4M3, false>(p, st);
-        case SEGQ_CODE_I4: return (p.pre_op || p.col_div) ? launch_quant<DT, SEGQ_CODE_I4, true>(p, st) : launch_quant<DT, SEGQ_CODE_I4, false>(p, st);
+        case SEGQ_CODE_I8: return launch_quant_pre<DT, SEGQ_CODE_I8>(p, st);
+        case SEGQ_CODE_E4M3: return launch_quant_pre<DT, SEGQ_CODE_E4M3>(p, st);
+        case SEGQ_CODE_I4: return launch_quant_pre<DT, SEGQ_CODE_I4>(p, st);
     }
     return fail(SEGQ_ERR_ARG, "segq_quantize: unknown code_fmt %d", p.fmt);
 }

@@ -84,3 +84,22 @@ def test_segments_equal_their_own_launches(dt, widths, dual):
             assert torch.equal(p.view(torch.int32), pos[s].view(torch.int32)) and (not dual or torch.equal(n.view(torch.int32), neg[s].view(torch.int32))), (dt, widths, rows, s)
             for g, w in zip(got if dual else (got,), want if dual else (want,)):
                 assert torch.equal(g[:, c0:c1], w), (dt, widths, rows, s)
+
+
+@pytest.mark.parametrize("dual", [False, True])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("cols", [16, 5136, 7184, 8192, 12304, 16400])
+def test_divisors_alone_equal_a_division_in_front(cols, dt, dual):
+    """A wave, a workgroup with four runs a thread, and a row that is longer than those; scales of the row and given ones.  The
+    division is one of fp32 rounded to the type, as torch's, so codes and scales are equal bit for bit."""
+    from segquant_amd import ops
+    rows = 3 * torch.cuda.get_device_properties(0).multi_processor_count + 1
+    x, div = torch.randn(rows, cols, device=DEV).to(dt), (torch.rand(cols, device=DEV) * 4 + 0.05).to(dt)
+    x[0], x[1, 3], x[2, cols - 1] = 0, float("nan"), float("inf")
+    for dynamic in (True, False):
+        out = []
+        for t, kw in ((x, dict(col_div=div)), (x / div, {})):
+            pos, neg = torch.full((rows,), 30.0, device=DEV), torch.full((rows,), 50.0, device=DEV)
+            codes = ops.quantize(t, "int8", pos, neg if dual else None, row_stride=1, dynamic=dynamic, dual=dual, two_tensors=dual, **kw)
+            out.append(list(codes if dual else (codes,)) + [s.view(torch.int32) for s in (pos, neg)])
+        assert all(torch.equal(p, q) for p, q in zip(*out)), (dt, cols, dual, dynamic)

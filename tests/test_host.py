@@ -753,3 +753,12 @@ def test_instances_that_finish_in_output_units(tile, fmt, fold, park, registers,
     """What an instance loses in registers costs resident waves, or a trip through scratch memory in every workgroup."""
     name = _pipe(*tile, fmt, fold, park, True)
     assert _kernel_registers()[name] <= registers and _kernel_registers(".private_segment_fixed_size")[name] <= scratch
+
+
+@pytest.mark.parametrize("dtype", [1, 2])
+def test_column_divisors_alone_are_rid_of_the_activation_functions_registers(dtype):
+    """Long rows of 16-bit inputs divided by column factors: three workgroups a compute unit, which takes at most 168 registers."""
+    for fmt in range(3):
+        for dual in range(2):
+            name = f"_ZN4segq20quant_dynamic_kernelILi{dtype}ELi{fmt}ELi4ELb{dual}ELi1EEEvNS_11QuantParamsE"
+            assert _kernel_registers()[name] <= 168 and _kernel_registers(".private_segment_fixed_size")[name] == 0
