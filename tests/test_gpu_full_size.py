@@ -241,11 +241,11 @@ LAYER_CASES = [(1, None, torch.float32), (2, None, torch.bfloat16), (3, None, to
 def test_full_size_layers_against_the_oracle(config, M, dtype):
     """SegmentLinear at the benchmark's own sizes with the library's own tile choice and the layer's
     own workspace lending: configuration 1 (256 tokens, whole output), configuration 2 (4096 tokens:
-    fc1 on the two-workgroup 128 x 128 kernel, fc2 DualScale in two code tensors), configuration 3
+    fc1 in two rounds of 256 x 192, fc2 DualScale, both signs in one code tensor and one walk), configuration 3
     (4608 tokens, per-token dynamic scales, the three FLUX linears on their own tiles), configuration 4
     (8192 and 2048 tokens: the row quantiser at K = 1280 / 5120, int4 weights expanded into the lent
     workspace, one factor per group of 128 input channels) and configuration 5
-    at 9216 and 1024 tokens (int8 parked, e4m3 rescaled in place, split K), on row and column bands
+    at 9216 and 1024 tokens (DualScale and the plain segment in one walk, whole and in two K shares), on row and column bands
     against the closed form built by the oracle from the layer's codes and scales
     (element-wise: one rounding to the output dtype plus the accumulation's own error)."""
     from _layer_oracle import _np32, oracle_layer_output
@@ -281,7 +281,7 @@ def test_full_size_layers_against_the_oracle(config, M, dtype):
 
 
 @pytest.mark.parametrize("rank", [32, 64])
-def test_full_size_svd_layer_low_rank_in_the_epilogue(rank):
+def test_full_size_svd_layer_low_rank_in_the_epilogue(rank, monkeypatch):
     """Configuration 3's mlp_up (4608 x 3072 -> 12288, int8, per-token dynamic activations,
     per-channel weights, bf16) as an svd layer: SmoothQuant division in the quantise kernel, the
     rank-r branch added by the GEMM's epilogue.  Row and column bands against the oracle's closed
@@ -291,9 +291,14 @@ def test_full_size_svd_layer_low_rank_in_the_epilogue(rank):
     M, K, N = 4608, 3072, 12288
     layer, xd, _ = _smooth_layer("svd", "int8", "weight", 1, M, K, N, torch.bfloat16, True, axis=True, rank=rank, seed=9)
     assert layer.optimizer.fused_available()
+    from segquant_amd import ops
+    rows_kernel, served = ops.lowrank_rows, []
+    monkeypatch.setattr(ops, "lowrank_rows", lambda *a: served.append(rows_kernel(*a)) or served[-1])
     out = layer(xd)
     plan = layer.optimizer._plan
     assert plan["lr_ok"][(M, torch.bfloat16)] is True  # the epilogue branch ran, not the materialised addend
+    assert plan["lr_tile"][(M, torch.bfloat16)] == 36  # ... on 384 x 192, whose three rounds are full
+    assert served == [True]                            # T came from this library's kernel
     got = _np32(out).astype(np.float64)
     x_np = _np32(xd)
     rows, cols = _bands(M, N)

@@ -755,23 +755,39 @@ def test_low_rank_branch_on_the_largest_tiles(ops, fmt, tile):
         ops.gemm(up(a), up(b), rg + rg, lowrank=(t_lr.to(DEV), l2t.to(DEV)), **kw)
 
 
+def _check_low_rank_rows(ops, M, K, r, dt, tg):
+    """T = x L1 with x and T as slices of wider tensors, whose other columns stay as they are."""
+    wide = torch.randn(M, K + 40, generator=tg).to(TDT[dt]).to(DEV)
+    x, l1t = wide[:, 8:8 + K], torch.randn(r, K, generator=tg).to(TDT[dt]).to(DEV)
+    out = torch.full((M, r + 24), 7.0, dtype=TDT[dt], device=DEV)
+    assert ops.lowrank_rows(x, l1t, out[:, 8:8 + r])
+    want = x.double() @ l1t.double().t()
+    mag = x.double().abs() @ l1t.double().abs().t()
+    # fp32 sums of K exact products, the output's one rounding
+    tol = K * 2.0 ** -24 * mag + {"bf16": 2.0 ** -8, "fp16": 2.0 ** -11}[dt] * want.abs()
+    assert ((out[:, 8:8 + r].double() - want).abs() <= tol).all(), (M, K, r)
+    assert (out[:, :8] == 7.0).all() and (out[:, 8 + r:] == 7.0).all()
+    return wide, l1t, out
+
+
 @pytest.mark.parametrize("dt", ["bf16", "fp16"])
 def test_low_rank_rows(ops, dt):
     """T = x L1: row tiles, K from one 64-wide unit to several per wave with a remainder, 16 to 160 columns, x and T as slices of
     wider tensors; what the kernel does not serve is left to the caller."""
     tg = torch.Generator().manual_seed(5)
     for M, K, r in ((1, 64, 16), (16, 448, 32), (17, 512, 64), (130, 576, 96), (33, 1600, 48), (300, 3072, 32), (40, 3136, 160), (5, 2048, 128)):
-        wide = torch.randn(M, K + 40, generator=tg).to(TDT[dt]).to(DEV)
-        x, l1t = wide[:, 8:8 + K], torch.randn(r, K, generator=tg).to(TDT[dt]).to(DEV)
-        out = torch.full((M, r + 24), 7.0, dtype=TDT[dt], device=DEV)
-        assert ops.lowrank_rows(x, l1t, out[:, 8:8 + r])
-        want = x.double() @ l1t.double().t()
-        mag = x.double().abs() @ l1t.double().abs().t()
-        # fp32 sums of K exact products, the output's one rounding
-        tol = K * 2.0 ** -24 * mag + {"bf16": 2.0 ** -8, "fp16": 2.0 ** -11}[dt] * want.abs()
-        assert ((out[:, 8:8 + r].double() - want).abs() <= tol).all(), (M, K, r)
-        assert (out[:, :8] == 7.0).all() and (out[:, 8 + r:] == 7.0).all()
+        wide, l1t, out = _check_low_rank_rows(ops, M, K, r, dt, tg)
         assert not ops.lowrank_rows(wide[:, 1:1 + K], l1t, out[:, :r]) and not ops.lowrank_rows(wide[:, :K + 8], l1t, out[:, :r])
+
+
+@pytest.mark.parametrize("dt", ["bf16", "fp16"])
+@pytest.mark.parametrize("K, r", [(64, 16), (1856, 16), (192, 32), (3136, 96), (64, 64), (1088, 128)])
+def test_low_rank_rows_of_many_rows(ops, dt, K, r):
+    """Both sides of 16 rows per compute unit, where workgroups go from 16 rows to 32: 16, 32 and 64 columns each, K of less than a
+    stage and with a remainder."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for M in (16 * cus, 16 * cus + 1, 16 * cus + 31):
+        _check_low_rank_rows(ops, M, K, r, dt, torch.Generator().manual_seed(M + K))
 
 
 def test_low_rank_rows_leave_derivatives_to_the_product_that_refuses_them(ops):

@@ -259,41 +259,110 @@ def test_repeated_forwards_reuse_descriptors_and_buffers(config, M):
         assert codes1.data_ptr() != codes2.data_ptr()
 
 
-@pytest.mark.parametrize("config,M", [(1, None), (2, None), (4, 2048), (5, 1024)])
-def test_layer_forward_replays_from_a_captured_graph(config, M):
-    """The layer's forward recorded into a HIP graph (the quantise and GEMM launches, the expansion
-    of int4 weights, the sum of K shares; config 2's fc2 is two K shares that meet inside the launch,
-    config 5 at 1024 tokens four shares and parked ranges) and replayed four times, with the input
-    rewritten, other eager launches and synchronisations between the replays: every replay must
-    equal the eager forward on the data then in the input buffer, bit for bit."""
-    from segquant_amd import workloads as W
-    for spec in W.config_linears(config, M=M):
-        layer, x = W.build_layer(spec, device=DEV, real_quant=True)
-        gen = torch.Generator().manual_seed(17)
-        variants = [x.to(spec.x_dtype).to(DEV)] + [
-            (x * (torch.rand(x.shape[1], generator=gen) + 0.5)).to(spec.x_dtype).to(DEV) for _ in range(3)]
-        eager = [layer(v).clone() for v in variants]
-        static_in = variants[0].clone()
-        side = torch.cuda.Stream()
-        side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side):  # buffers, workspaces and kernel attributes of this stream exist before the capture
-            for _ in range(2):
-                layer(static_in)
-        torch.cuda.current_stream().wait_stream(side)
+def _replays_from_a_captured_graph(spec):
+    """A layer's forward recorded into a HIP graph and replayed five times, with the input rewritten, other eager launches and
+    synchronisations between the replays: every replay must equal the eager forward on the data then in the input buffer, bit
+    for bit.  Returns the plan of its GEMM: tile, K shares, parked."""
+    from segquant_amd import ops, workloads as W
+    layer, x = W.build_layer(spec, device=DEV, real_quant=True)
+    gen = torch.Generator().manual_seed(17)
+    variants = [x.to(spec.x_dtype).to(DEV)] + [
+        (x * (torch.rand(x.shape[1], generator=gen) + 0.5)).to(spec.x_dtype).to(DEV) for _ in range(3)]
+    q, g, ws = layer.optimizer.fused_launches(variants[0], layer.bias_data, fresh=True)
+    plan = ops.gemm_plan(g, ws)
+    eager = [layer(v).clone() for v in variants]
+    static_in = variants[0].clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):  # buffers, workspaces and kernel attributes of this stream exist before the capture
+        for _ in range(2):
+            layer(static_in)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        static_out = layer(static_in)
+    for i in (0, 1, 2, 3, 1):
+        static_in.copy_(variants[i])
+        graph.replay()
         torch.cuda.synchronize()
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, stream=side):
-            static_out = layer(static_in)
-        for i in (0, 1, 2, 3, 1):
-            static_in.copy_(variants[i])
-            graph.replay()
-            torch.cuda.synchronize()
-            assert torch.equal(static_out, eager[i]), (spec.name, i)
-            again = layer(variants[(i + 1) % 4])  # the program's own eager work between replays
-            torch.cuda.synchronize()
-            assert torch.equal(again, eager[(i + 1) % 4]), (spec.name, i)
-        del graph, layer
-        torch.cuda.empty_cache()
+        assert torch.equal(static_out, eager[i]), (spec.name, i)
+        again = layer(variants[(i + 1) % 4])  # the program's own eager work between replays
+        torch.cuda.synchronize()
+        assert torch.equal(again, eager[(i + 1) % 4]), (spec.name, i)
+    del graph, layer
+    torch.cuda.empty_cache()
+    return plan["tile"], plan["splits"], bool(plan["parked"])
+
+
+@pytest.mark.parametrize("config,M,plans", [
+    (1, None, [(21, 1, False)]),
+    (2, None, [(17, 1, False), (33, 1, False)]),                     # fc2: one walk from one code tensor
+    (4, 2048, [(14, 1, False)] * 3),
+    (5, 1024, [(33, 2, False)] * 2),                                 # two shares that meet inside the launch
+])
+def test_layer_forward_replays_from_a_captured_graph(config, M, plans):
+    """The quantise and GEMM launches, the expansion of int4 weights, K shares that meet."""
+    from segquant_amd import workloads as W
+    assert [_replays_from_a_captured_graph(spec) for spec in W.config_linears(config, M=M)] == plans
+
+
+@pytest.mark.parametrize("config,M,change,plan", [
+    (2, 1024, {}, (33, 4, False)),                                   # four shares that a second kernel sums
+    (5, 1024, dict(dual_segments=[], gelu_segments=[]), (17, 4, True)),   # two plain segments of int8: parked, four shares
+    (5, 1000, dict(dual_segments=[], gelu_segments=[], K=6144, N=6144, chunksizes=[3072, 3072]), (17, 2, True)),  # ... two that meet
+    (5, 4608, dict(dual_segments=[], gelu_segments=[]), (16, 1, True)),
+])
+def test_captured_shares_and_parked_ranges(config, M, change, plan):
+    import dataclasses
+    from segquant_amd import workloads as W
+    spec = W.config_linears(config, M=M)[1 if config == 2 else 0]
+    assert _replays_from_a_captured_graph(dataclasses.replace(spec, **change)) == plan
+
+
+@pytest.mark.parametrize("fmt", ["int8", "fpe4m3"])
+def test_dual_scale_layers_keep_their_codes_in_one_tensor(fmt):
+    """Where the layer says so it does: first call, relaunch, the parts of the input, and codes written by another layer; and the
+    same layers held to two tensors give the same sums."""
+    import dataclasses
+    from segquant_amd import workloads as W
+
+    def held_to_two(layer, rows):
+        plan = layer.optimizer._plan or layer.optimizer._build_plan(torch.device(DEV))
+        plan.setdefault("one_tensor", {})[rows, torch.bfloat16] = False
+
+    def close(got, want):
+        # int32 sums are the same; e4m3 products meet in the matrix cores' limited-width adder in another order
+        err = (got.float() - want.float()).abs()
+        return bool((err <= 2.0 ** -7 * want.float().abs() + (0 if fmt == "int8" else 3e-4) * want.float().abs().max()).all())
+
+    rows = 1024
+    spec = [s for s in W.config_linears(5, M=rows) if s.act == fmt][0]
+    layer, x = W.build_layer(spec, device=DEV, real_quant=True)
+    two, _ = W.build_layer(spec, device=DEV, real_quant=True, x=x)
+    held_to_two(two, rows)
+    xd = x.to(spec.x_dtype).to(DEV)
+    out, again, other = layer(xd), layer(xd), two(xd)
+    hit, = layer.optimizer._plan["launches"].values()
+    hit2, = two.optimizer._plan["launches"].values()
+    assert layer.optimizer._plan["one_tensor"] == {(rows, spec.x_dtype): True} and (hit["two"], hit2["two"]) == (False, True)
+    assert torch.equal(out, again) and torch.equal(two(xd), other) and close(out, other)
+    halves = [xd[:, :3072], xd[:, 3072:]]
+    assert torch.equal(layer.forward_parts(halves), out) and torch.equal(two.forward_parts(halves), other)
+
+    s1, s2 = (dataclasses.replace(s, act=fmt, weight=fmt) for s in W.config_linears(2, M=rows))
+    fc1, x = W.build_layer(s1, device=DEV, real_quant=True)
+    xd = x.to(torch.bfloat16).to(DEV)
+    h = torch.nn.functional.gelu(fc1(xd), approximate="tanh")
+    fc2, _ = W.build_layer(s2, device=DEV, real_quant=True, x=h.float().cpu())
+    two, _ = W.build_layer(s2, device=DEV, real_quant=True, x=h.float().cpu())
+    held_to_two(two, rows)
+    for nxt, one in ((fc2, True), (two, False)):
+        spec = nxt.optimizer.code_spec(torch.device(DEV), "gelu_tanh", rows, torch.bfloat16)
+        codes = fc1.optimizer.fused_launches(xd, fc1.bias_data, out_codes=spec)[1][1]
+        assert spec["one_tensor"] is one and isinstance(codes, tuple) is not one
+    got = fc1.forward_into(fc2, xd, pre_op="gelu_tanh")
+    assert torch.equal(got, fc2(fc1(xd), pre_op="gelu_tanh")) and close(got, fc1.forward_into(two, xd, pre_op="gelu_tanh"))
 
 
 @pytest.mark.parametrize("fmt", ["int8", "fpe4m3"])
@@ -488,7 +557,7 @@ def test_one_layer_serves_every_float_input_dtype(config):
 @pytest.mark.parametrize("fmt", ["fpe4m3", "int8"])
 def test_chained_linears_write_the_next_layers_codes(fmt):
     """Config 2's MLP pair (fc1 -> GELU(tanh) -> fc2 with DualScale) through ``forward_into``: fc1's GEMM
-    epilogue writes fc2's two code tensors.  Bit for bit the result of the three launches it
+    epilogue writes fc2's codes (of both signs in one tensor or in two, as fc2 asks).  Bit for bit the result of the three launches it
     replaces (fc1's GEMM writing bf16, fc2's quantise kernel with the GELU fused, fc2's GEMM), which
     the other tests pin against the oracle; and pairs the epilogue does not serve (an fp32 input)
     take the two ordinary forwards."""

@@ -486,10 +486,11 @@ def test_smooth_and_svd_layers_on_the_fake_path_equal_the_oracle(opt_type, seg_m
                       opt_kwargs={"search_alpha_config": {"enable": True, "min": 0.1, "max": 0.9, "step": 0.1}}, device="cpu")
 
 
-def _plan(lib, m, n, ranges, fmt, out_dtype=2, lend=True, split_k=0, tile=0, lowrank=0, finite=0, neg=True):
+def _plan(lib, m, n, ranges, fmt, out_dtype=2, lend=True, split_k=0, tile=0, lowrank=0, finite=0, neg=True, short=0, groups=False):
     """segq_gemm_plan / segq_gemm_workspace_bytes on a descriptor of made-up (aligned, never
     dereferenced) device addresses: the library's decisions are host arithmetic and launch nothing.
-    ranges: (k_begin, k_len, a_sel).  Returns (tile id, K shares, parked, workspace bytes)."""
+    ranges: (k_begin, k_len, a_sel); short: bytes that the lent workspace falls short of what the library
+    asks for.  Returns (tile id, K shares, parked, workspace bytes)."""
     import ctypes as C
     from segquant_amd import _lib as L
     d = L.GemmDesc()
@@ -505,10 +506,12 @@ def _plan(lib, m, n, ranges, fmt, out_dtype=2, lend=True, split_k=0, tile=0, low
         d.ranges[i].sx, d.ranges[i].sw = 0x60000000, 0x70000000
     if lowrank:
         d.lowrank_t, d.lowrank_l2t, d.lowrank_rank, d.ld_lowrank_t, d.ld_lowrank_l2t = 0x80000000, 0x90000000, lowrank, lowrank, lowrank
+    if groups:
+        d.group_dequant, d.group_dequant_stride = 0xB0000000, n
     need = C.c_int64(-1)
     assert lib.segq_gemm_workspace_bytes(C.byref(d), C.byref(need)) == 0, lib.segq_last_error()
     if lend:
-        d.workspace, d.workspace_bytes = 0xA0000000, max(need.value, 16)
+        d.workspace, d.workspace_bytes = 0xA0000000, max(need.value, 16) - short
     t, s, p = C.c_int32(0), C.c_int32(0), C.c_int32(0)
     assert lib.segq_gemm_plan(C.byref(d), C.byref(t), C.byref(s), C.byref(p)) == 0, lib.segq_last_error()
     return t.value, s.value, p.value, need.value
@@ -517,7 +520,8 @@ def _plan(lib, m, n, ranges, fmt, out_dtype=2, lend=True, split_k=0, tile=0, low
 def test_tile_and_share_choice_for_the_benchmark_shapes():
     """What the library picks (tile id, K shares, parking) for the shapes of the five benchmark
     configurations and for a few-token shape, with a workspace of the size it asks for and without
-    one.  Pure host arithmetic: no GPU, nothing launched.  (256 CUs are assumed when there is no
+    one.  The DualScale rows are without finite_scales, as a caller of the C interface may have them
+    (layers set it: the next test).  Pure host arithmetic: no GPU, nothing launched.  (256 CUs are assumed when there is no
     device to ask.)"""
     import ctypes as C
     from segquant_amd import _lib as L
@@ -555,6 +559,43 @@ def test_tile_and_share_choice_for_the_benchmark_shapes():
     assert t == 14 and s in (2, 3)
     # the low-rank branch moves to a tile that is built with it
     assert _plan(lib, 4608, 12288, one(3072), I8, lowrank=32)[:2] == (11, 1)
+
+
+def test_plans_of_the_layers_dual_scale_shapes():
+    """What a layer's descriptors get, scales known to be finite, from two code tensors and from one: tile, K shares, nothing
+    parked, the exact workspace, none, and one byte less than asked for."""
+    from segquant_amd import _lib as L
+    lib = L.lib()
+    for fmt in (0, 1):
+        for sel in (0, 2):
+            plan = lambda m, n, rg, **kw: _plan(lib, m, n, rg, fmt, finite=1, neg=sel == 0, **kw)
+            pair = lambda k0, k: [(k0, k, sel), (k0, k, sel + 1)]
+            c5, fc2 = [(0, 3072, 0)] + pair(3072, 12288), pair(0, 6144)
+            # 8 x 16 tiles of 128 x 192, two shares that meet: both of every tile, and a word for each
+            need = 128 * 2 * 128 * 192 * 4 + 128 * 4
+            assert plan(1024, 3072, c5) == (33, 2, 0, need)
+            assert plan(1024, 3072, c5, short=1)[:3] == plan(1024, 3072, c5, lend=False)[:3] == (33, 1, 0)
+            assert plan(1024, 3072, c5, split_k=1)[:3] == (33, 1, 0)
+            assert plan(4608, 3072, c5) == (32, 1, 0, 0) and plan(9216, 3072, c5) == (31, 1, 0, 0)
+            # more than two shares: as many partial results, which a second kernel sums
+            assert plan(1024, 1536, fc2) == (33, 4, 0, 4 * 1024 * 1536 * 4)
+            # (two tensors: one walk of 64 x 128 is ahead of three shares)
+            assert plan(1024, 1536, fc2, short=1)[:3] == ((30, 1, 0) if sel == 0 else (33, 3, 0))
+            # whole rounds of 128 x 192 (the two-tensor kernel has its own): nothing shared
+            assert plan(4096, 1536, fc2) == ((29 if sel == 0 else 33), 1, 0, 0)
+            # not known to be finite: the ranges in turn
+            assert sel or _plan(lib, 1024, 3072, c5, fmt) == (17, 4, 1 - fmt, 4 * 1024 * 3072 * 4 + (1 - fmt) * 4 * 1024 * 3072 * 4)
+
+
+def test_tile_of_group_factors():
+    """One range: two workgroups of 128 x 128 a compute unit, or one of a big tile where that is ahead; several: 128 x 128."""
+    from segquant_amd import _lib as L
+    plan = lambda m, n, rg: _plan(L.lib(), m, n, rg, 0, groups=True)[:3]
+    one = lambda k: [(0, k, 0)]
+    assert plan(8192, 10240, one(1280)) == plan(4096, 12288, one(1536)) == (11, 1, 0)
+    assert plan(8192, 1280, one(5120)) == (18, 1, 0)
+    assert plan(2048, 10240, one(1280)) == plan(2048, 1280, one(5120)) == plan(1, 16, one(128)) == (14, 1, 0)
+    assert plan(8192, 10240, [(0, 640, 0), (640, 640, 0)]) == (14, 1, 0)
 
 
 @pytest.mark.parametrize("m, n, k0, k1, fmt, walk", [
