@@ -169,20 +169,28 @@ static Walk choose_dual(int64_t m, int64_t n, int64_t batch, int64_t k) {
     return w;
 }
 
-// Group factors: us of rounds of the CUs x (steps x what a step takes + what a tile takes beside them), fitted to 14 shapes
-// (within 6 %).  Two workgroups of 128 x 128 share a CU; a last round of one per CU is quicker.  us with the int4 expansion,
-// 128 x 128 / 256 x 256 / 256 x 192 / 192 x 256:  8192 x 10240 x 1280 166 / 155 / 160 / 158;  8192 x 1280 x 5120 81 / 85 / 75 / 69;
-// 4096 x 12288 x 1536 117 / 108 / 117 / 128;  2048 x 10240 x 1280 50 / 59 / 53 / 53;  2048 x 1280 x 5120 37 / 83 / 70 / 65.
-// The big tiles have to be ahead by 3 %.  (256 x 128 and 128 x 256, by id: never the best by more than that.)
-static int choose_groups(int64_t m, int64_t n, int64_t steps, bool fold) {
-    if (fold) return FIRST_WIDE_CFG + 3;
-    const int64_t cus = device_cus(), t128 = tiles_of_cfg(FIRST_WIDE_CFG + 3, m, n, 1), rest = t128 % (2 * cus);
-    const double pair = 1.1 * steps + 4.5, alone = 0.78 * steps + 5.0;
-    double us = 0.97 * ((double)(t128 / (2 * cus)) * pair + (rest == 0 ? 0.0 : rest <= cus ? alone : pair));
+// Group factors: us, of what the outputs take (x: rounds of the CUs that they would be without ragged tiles) and of the rounds that
+// the tiles take, per step and beside the steps; fp32 outputs are bound by their stores as well, and a tile with ragged columns
+// takes longer than whole ones.  Fitted to 1379 shapes of 200 to 8192 rows (rms 5 to 7 %).  Two workgroups of 128 x 128 share
+// a CU and flow on from round to round, so their rounds count by halves.  A big tile has to be ahead by more than the fit is off where
+// it matters, fp32 by more: of the shapes 20 are then slower than 128 x 128 by 2 % (at most 11 %), and all 2 to 3 % faster in the mean (52
+// and 21 % with rounds alone in the sum).  us, 128 x 128 / 256 x 256 / 256 x 192 / 192 x 256:  8192 x 10240 x 1280 166 / 155 / 160 / 158;
+// 8192 x 1280 x 5120 81 / 85 / 75 / 69;  4096 x 12288 x 1536 117 / 108 / 117 / 128;  2048 x 10240 x 1280 50 / 59 / 53 / 53;  2048 x 1280 x 5120 37 / 83 /
+// 70 / 65;  4774 x 7680 x 384 35 / 45 / 36 / 42;  6105 x 6912 x 2176 fp32 141 / 151 / 151 / 161.
+// (256 x 128 and 128 x 256, by id: never the best by more than 3 %.)
+static int choose_groups(int64_t m, int64_t n, int64_t k_steps, bool fold, bool f32) {
+    const int64_t cus = device_cus(), t128 = tiles_of_cfg(FIRST_WIDE_CFG + 3, m, n, 1);
+    if (fold || 8 * t128 <= 5 * cus) return FIRST_WIDE_CFG + 3;
+    const double s = (double)k_steps, outs = (double)m * (double)n / (double)cus, f = f32 ? 1.0 : 0.0;
+    const double x128 = outs / (2 * 128 * 128), half = 0.5 * (double)((t128 + cus - 1) / cus);
+    double us = (f32 ? 0.94 : 0.985) * ((0.37 * s + 3.32 + 3.76 * f) * x128 + (0.84 * s + 0.27) * half + 5.3);
     int best = FIRST_WIDE_CFG + 3;
-    static const struct { int tile; double step, tail; } big[3] = {{0, 1.95, 10.0}, {6, 1.55, 8.0}, {7, 1.42, 7.5}};
+    static const struct { int tile; double x_step, x, x_f32, step, tail, ragged; } big[3] = {
+        {0, 0.63, 0.71, 7.58, 1.56, 9.14, 2.5}, {6, 0.36, 0.0, 5.16, 1.24, 8.47, 1.18}, {7, 0.42, 0.0, 5.83, 1.11, 8.66, 1.09}};
     for (const auto& b : big) {
-        const double t = (double)((tiles_of_cfg(FIRST_WIDE_CFG + b.tile, m, n, 1) + cus - 1) / cus) * (b.step * steps + b.tail);
+        const TileCfg& c = TILE_CFGS[FIRST_WIDE_CFG + b.tile];
+        const double x = outs / (c.bm * c.bn), rounds = (double)((tiles_of_cfg(FIRST_WIDE_CFG + b.tile, m, n, 1) + cus - 1) / cus);
+        const double t = (b.x_step * s + b.x + b.x_f32 * f) * x + (b.step * s + b.tail) * rounds + (n % c.bn ? b.ragged * (1.0 + f) : 0.0);
         if (t < us) {
             us = t;
             best = FIRST_WIDE_CFG + b.tile;
@@ -742,7 +750,7 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
     };
     if (d->tile == 0) {
         if (groups) {
-            cfg = choose_groups(d->m, d->n, ktotal / 128, fold);
+            cfg = choose_groups(d->m, d->n, ktotal / 128, fold, d->out_dtype == SEGQ_F32);
         } else {
             cfg = park ? choose_tile(d->m, d->n, d->batch, false, wide_ok, plain8) : -1;
             park = park && park_fits(cfg);
