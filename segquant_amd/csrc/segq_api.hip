@@ -169,6 +169,51 @@ static Walk choose_dual(int64_t m, int64_t n, int64_t batch, int64_t k) {
     return w;
 }
 
+// K shares of the steps of `cfg`'s tiles, and the tile that takes them (cfg and 1: none).
+// Whole tiles would leave more than a tenth of the CUs idle: look for a big tile and a
+// number of shares that fill them.  Measured (us, random codes, 256 CUs):
+//   1024 x 3072, K 13824 twice (DualScale):  e4m3  256x192 x4 99 | 256x256 x5 130 | 128x128 176
+//                                            int8  256x192 x4 108 | 256x256 x4 125 | 128x128 184
+//   4096 x 1536, K 6144 twice:               e4m3  256x192 x2 85 | 256x256 x2 94 | 256x128 123
+// The choice minimises rounds x (K steps per share + fixed cost) x tile area / efficiency:
+// about 6 steps' worth of prologue and epilogue per workgroup, 8 more for the shares' trip
+// through memory; big tiles get more out of every byte they stream.
+struct Shares {
+    int cfg, n;
+};
+
+static Shares choose_shares(int64_t m, int64_t n, int64_t total_steps, int cfg, bool big_ok, bool sep, bool parks) {
+    const int64_t cus = device_cus();
+    Shares pick{cfg, 1};
+    if (total_steps < 16 || tiles_of_cfg(cfg, m, n, 1) * 10 >= cus * 9) return pick;
+    auto eff = [](int c) {
+        const int area = TILE_CFGS[c].bm * TILE_CFGS[c].bn;
+        return c < FIRST_WIDE_CFG ? 0.5 : area >= 256 * 256 ? 1.0 : area >= 256 * 192 ? 0.95 : area >= 256 * 128 ? 0.85 : 0.7;
+    };
+    auto cost = [&](int c, int64_t s_) {
+        const int64_t wgs = tiles_of_cfg(c, m, n, 1) * s_;
+        return (double)((wgs + cus - 1) / cus) * ((double)total_steps / s_ + 6.0 + (s_ > 1 ? 8.0 : 0.0)) *
+               TILE_CFGS[c].bm * TILE_CFGS[c].bn / eff(c);
+    };
+    // (the 128 x 128 tile joins for very few tokens: 64 x 9216 x 3072 in two or three shares
+    // 19 us against 25 us whole)
+    const int cands[4] = {FIRST_WIDE_CFG + 6, FIRST_WIDE_CFG, FIRST_WIDE_CFG + 7, FIRST_WIDE_CFG + 3};
+    double best = cost(cfg, 1);
+    for (int i = 0; i < (big_ok ? 4 : sep ? 2 : 1); ++i) {
+        const int c = big_ok ? cands[i] : FIRST_WIDE_CFG + (i == 0 ? 1 : 3);
+        if (c == FIRST_WIDE_CFG + 3 && (m > 128 || parks)) continue;
+        int64_t s_ = cus / tiles_of_cfg(c, m, n, 1);
+        if (s_ > total_steps / 8) s_ = total_steps / 8;
+        if (s_ > 16) s_ = 16;
+        if (s_ < 2) continue;
+        if (cost(c, s_) < best) {
+            best = cost(c, s_);
+            pick = Shares{c, (int)s_};
+        }
+    }
+    return pick;
+}
+
 // Group factors: us, of what the outputs take (x: rounds of the CUs that they would be without ragged tiles) and of the rounds that
 // the tiles take, per step and beside the steps; fp32 outputs are bound by their stores as well, and a tile with ragged columns
 // takes longer than whole ones.  Fitted to 1379 shapes of 200 to 8192 rows (rms 5 to 7 %).  Two workgroups of 128 x 128 share
@@ -278,6 +323,36 @@ static MixPick choose_mix(int64_t m, int64_t n, int64_t steps, int64_t plain, in
         }
     }
     return best;
+}
+
+// e4m3, DualScale beside a plain range.  One walk multiplies a step of the plain range on half of its rows' registers; the ranges in turn,
+// rescaled in place, have their tiles whole for it and walk the pair twice.  us of both, for steps and output tiles in whole
+// rounds and beside them, fitted to 1169 shapes of 129 to 9216 rows (rms 6 % and 5 %).  us, one walk / in turn: 1479 x 6336 x (3328 + 256)
+// 62 / 45;  8950 x 1408 x (3072 + 256) fp32 77 / 56;  7940 x 4736 x (3328 + 640) fp32 245 / 203;  472 x 7424 x (3200 + 512) 32 / 26;  425 x 1280 x (256 + 256)
+// 11.1 / 9.9;  4608 x 3072 x (3072 + 12288) 296 / 299.  Of the shapes 234 were slower by 2 % or more on the one walk, by up to 39 %; with this line 30 are, by up to 24 %.
+// (int8 parks in turn: of 155 shapes two were slower on the one walk, by 4 %.)
+static double mix_beside_us(int64_t m, int64_t n, int64_t steps, int64_t plain, const MixPick& pick, bool f32) {
+    if (pick.shares > 1) return pick.us;
+    static const struct { double xs, xp, rs, rp, x, r, one, x_f32; } fit[3] = {
+        {0.35, 0.61, 1.11, 0.37, 0.0, 9.6, 1.1, 4.5}, {0.49, 0.43, 0.84, 0.54, 0.4, 7.3, 2.9, 4.25}, {0.08, 0.12, 0.81, 0.61, 1.2, 5.3, 2.5, 4.65}};
+    const auto& w = fit[pick.cfg - FIRST_MIX_CFG];
+    const TileCfg& c = TILE_CFGS[pick.cfg];
+    const double cus = (double)device_cus(), s = (double)steps, p = (double)plain;
+    const double x = (double)m * (double)n / (cus * c.bm * c.bn), r = std::ceil((double)tiles_of_cfg(pick.cfg, m, n, 1) / cus);
+    return (w.xs * s + w.xp * p + w.x + (f32 ? w.x_f32 : 0.0)) * x + (w.rs * s + w.rp * p + w.r) * r + w.one;
+}
+
+static double beside_in_turn_us(int64_t m, int64_t n, int64_t all_steps, int cfg, bool f32) {
+    static const struct { double xs, rs, x, r, one, x_f32; } fit[4] = {
+        {0.0, 1.7, 4.5, 0.0, 7.1, 0.0}, {0.0, 1.15, 4.1, 0.52, 6.7, 3.9}, {0.3, 0.59, 0.0, 11.3, 0.0, 3.1}, {0.56, 0.8, 3.6, 10.1, 1.3, 6.5}};
+    const TileCfg& c = TILE_CFGS[cfg];
+    const int area = c.bm * c.bn;
+    if (area > 192 * 288 || cfg >= NUM_TILE_CFG) return 1e30;
+    const auto& w = fit[area <= 64 * 128 ? 0 : area <= 128 * 128 ? 1 : area <= 256 * 128 ? 2 : 3];
+    // (two workgroups of the smaller tiles share a CU and flow on from round to round: rounds by halves)
+    const double cus = (double)device_cus(), room = area <= 128 * 128 ? 2.0 * cus : cus, part = area <= 128 * 128 ? 2.0 : 1.0;
+    const double x = (double)m * (double)n / (room * area), r = std::ceil(part * (double)tiles_of_cfg(cfg, m, n, 1) / room) / part;
+    return (w.xs * (double)all_steps + w.x + (f32 ? w.x_f32 : 0.0)) * x + (w.rs * (double)all_steps + w.r) * r + w.one;
 }
 
 // int4 weight rows (two values per byte, even k in the low nibble) -> int8 rows.
@@ -547,6 +622,14 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
                 if (walk.cfg == FIRST_DUAL_CFG + 1 && t64 <= 1.0 && pick.shares > 2 && steps < 40) most = 0.85 * now;
                 take = take && pick.us < most;
             }
+            // Beside a plain range, e4m3: where whole tiles in turn are ahead (not those that would be shared along K: one walk is).
+            // One tensor: with what the quantise step then does not write.
+            if (mix.plain >= 0 && f8) {
+                const int turn = choose_tile(d->m, d->n, 1, false, true, true, all, true);
+                const bool whole = !share || choose_shares(d->m, d->n, all, turn, true, false, false).n == 1;
+                const double more = part ? (double)d->m * steps * 128 / 5e6 : 0.0;
+                if (whole && beside_in_turn_us(d->m, d->n, all, turn, osz == 4) + more < 1.03 * mix_beside_us(d->m, d->n, steps, plain, pick, osz == 4)) take = false;
+            }
             if (take || (part && !d->a_neg)) {
                 walk.cfg = -1;
                 mix.cfg = pick.cfg;
@@ -806,42 +889,14 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
         if (can) {
             int want = 1, scfg = cfg;
             const bool big_ok = !fold2 || park;  // the 256 x 256 tile, or 256 x 128 with a second register set
-            const int64_t cus = device_cus();
             auto tiles_of = [&](int c) { return ((d->m + TILE_CFGS[c].bm - 1) / TILE_CFGS[c].bm) * ((d->n + TILE_CFGS[c].bn - 1) / TILE_CFGS[c].bn); };
             if (d->split_k > 1) {
                 want = (int)(d->split_k < total_steps ? d->split_k : total_steps);
                 if (d->tile == 0) scfg = big_ok ? FIRST_WIDE_CFG : FIRST_WIDE_CFG + 1;
-            } else if (d->tile == 0 && total_steps >= 16 && tiles_of(cfg) * 10 < cus * 9) {
-                // Whole tiles would leave more than a tenth of the CUs idle: look for a big tile and a
-                // number of shares that fill them.  Measured (us, random codes, 256 CUs):
-                //   1024 x 3072, K 13824 twice (DualScale):  e4m3  256x192 x4 99 | 256x256 x5 130 | 128x128 176
-                //                                            int8  256x192 x4 108 | 256x256 x4 125 | 128x128 184
-                //   4096 x 1536, K 6144 twice:               e4m3  256x192 x2 85 | 256x256 x2 94 | 256x128 123
-                // The choice minimises rounds x (K steps per share + fixed cost) x tile area / efficiency:
-                // about 6 steps' worth of prologue and epilogue per workgroup, 8 more for the shares' trip
-                // through memory; big tiles get more out of every byte they stream.
-                auto eff = [](int c) {
-                    const int area = TILE_CFGS[c].bm * TILE_CFGS[c].bn;
-                    return c < FIRST_WIDE_CFG ? 0.5 : area >= 256 * 256 ? 1.0 : area >= 256 * 192 ? 0.95 : area >= 256 * 128 ? 0.85 : 0.7;
-                };
-                auto cost = [&](int c, int64_t s_) {
-                    const int64_t wgs = tiles_of(c) * s_;
-                    return (double)((wgs + cus - 1) / cus) * ((double)total_steps / s_ + 6.0 + (s_ > 1 ? 8.0 : 0.0)) *
-                           TILE_CFGS[c].bm * TILE_CFGS[c].bn / eff(c);
-                };
-                // (the 128 x 128 tile joins for very few tokens: 64 x 9216 x 3072 in two or three shares
-                // 19 us against 25 us whole)
-                const int cands[4] = {FIRST_WIDE_CFG + 6, FIRST_WIDE_CFG, FIRST_WIDE_CFG + 7, FIRST_WIDE_CFG + 3};
-                double best = cost(cfg, 1);
-                for (int i = 0; i < (big_ok ? 4 : p.sep ? 2 : 1); ++i) {
-                    const int c = big_ok ? cands[i] : FIRST_WIDE_CFG + (i == 0 ? 1 : 3);
-                    if (c == FIRST_WIDE_CFG + 3 && (d->m > 128 || (i8 && fold))) continue;
-                    int64_t s_ = cus / tiles_of(c);
-                    if (s_ > total_steps / 8) s_ = total_steps / 8;
-                    if (s_ > 16) s_ = 16;
-                    if (s_ < 2) continue;
-                    if (cost(c, s_) < best) { best = cost(c, s_); scfg = c; want = (int)s_; }
-                }
+            } else if (d->tile == 0) {
+                const Shares pick = choose_shares(d->m, d->n, total_steps, cfg, big_ok, p.sep, i8 && fold);
+                scfg = pick.cfg;
+                want = pick.n;
             }
             const TileCfg& t = TILE_CFGS[scfg];
             const int64_t tiles = tiles_of(scfg);

@@ -576,7 +576,8 @@ def test_plans_of_the_layers_dual_scale_shapes():
             assert plan(1024, 3072, c5) == (33, 2, 0, need)
             assert plan(1024, 3072, c5, short=1)[:3] == plan(1024, 3072, c5, lend=False)[:3] == (33, 1, 0)
             assert plan(1024, 3072, c5, split_k=1)[:3] == (33, 1, 0)
-            assert plan(4608, 3072, c5) == (32, 1, 0, 0) and plan(9216, 3072, c5) == (31, 1, 0, 0)
+            # (level with the ranges in turn in e4m3, which go to it for the codes that are then not written twice)
+            assert plan(4608, 3072, c5) == ((16 if fmt and sel == 0 else 32), 1, 0, 0) and plan(9216, 3072, c5) == (31, 1, 0, 0)
             # more than two shares: as many partial results, which a second kernel sums
             assert plan(1024, 1536, fc2) == (33, 4, 0, 4 * 1024 * 1536 * 4)
             # (two tensors: one walk of 64 x 128 is ahead of three shares)
@@ -623,6 +624,21 @@ def test_few_rows_beside_a_plain_segment(m, n, k0, k1, fmt, walk):
             assert tile < 31
         if pair == (2, 3):
             assert _plan(L.lib(), m, n, [(0, k0, 0), (k0, k1, 2), (k0, k1, 3)], fmt, finite=1, neg=False)[0] in (31, 32, 33)
+
+
+@pytest.mark.parametrize("m, n, k0, k1, dt, walk", [
+    # a plain range that is the most of K: whole tiles in turn
+    (1479, 6336, 3328, 256, 2, False), (8950, 1408, 3072, 256, 0, False), (7940, 4736, 3328, 640, 0, False), (472, 7424, 3200, 512, 1, False),
+    (425, 1280, 256, 256, 2, False), (5187, 1792, 3072, 384, 0, False),
+    # the pair, or tiles that would be shared along K
+    (4608, 3072, 3072, 12288, 2, True), (1024, 3072, 3072, 12288, 2, True), (901, 640, 5248, 128, 0, True), (3965, 1088, 640, 384, 1, True),
+])
+def test_e4m3_pair_beside_a_long_plain_segment(m, n, k0, k1, dt, walk):
+    """One walk, whatever the order of the ranges, or the ranges in turn; int8, which would park there, always walks once."""
+    from segquant_amd import _lib as L
+    plan = lambda fmt, **kw: _plan(L.lib(), m, n, kw.pop("rg"), fmt, out_dtype=dt, finite=1, **kw)[0] > 30
+    for a, b, c in (((0, k0, 0), (k0, k1, 2), (k0, k1, 3)), ((0, k1, 2), (0, k1, 3), (k1, k0, 0))):
+        assert plan(1, rg=[a, b, c]) == walk and plan(1, rg=[a, b, c], neg=False) and plan(0, rg=[a, b, c])
 
 
 @pytest.mark.parametrize("m, n, k, fmt, walk", [
