@@ -927,7 +927,8 @@ static int gemm_impl(const segq_gemm_desc* d, hipStream_t st, GemmPlan* plan = n
             return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: group factors run on tiles %d to %d, and with one range on %d and %d",
                         FIRST_WIDE_CFG + 1, FIRST_WIDE_CFG + 4, FIRST_WIDE_CFG + 7, FIRST_WIDE_CFG + 8);
     } else if (groups) {
-        return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: group factors run on tiles %d to %d", FIRST_WIDE_CFG + 2, FIRST_WIDE_CFG + 4);
+        return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: group factors run on tiles %d to %d, and with one range on %d and %d", FIRST_WIDE_CFG + 1,
+                    FIRST_WIDE_CFG + 4, FIRST_WIDE_CFG + 7, FIRST_WIDE_CFG + 8);
     } else if (cfg >= FIRST_BIG_CFG) {
         if (!wide_ok || w4 || fold)
             return fail(SEGQ_ERR_UNSUPPORTED, "segq_gemm: tile %d needs one range, 8-bit weights and K in multiples of 128", cfg + 1);

@@ -65,8 +65,7 @@ __device__ __forceinline__ void act_values(int op, float (&v)[N]) {
 __device__ __forceinline__ int q_i8(float v) { return (int)rintf(fminf(fmaxf(v, -128.0f), 127.0f)); }
 __device__ __forceinline__ int q_i4(float v) { return (int)rintf(fminf(fmaxf(v, -8.0f), 7.0f)); }
 
-// e4m3 with saturation to +-448 (fminf/fmaxf drop a NaN operand, so NaN is
-// patched afterwards: it encodes as 0x7F whatever its sign).
+// Saturation to e4m3's +-448 for the round trip through it.  fminf/fmaxf drop a NaN operand: the callers put it back.
 __device__ __forceinline__ float sat_e4m3(float v) { return fminf(fmaxf(v, -448.0f), 448.0f); }
 
 // Four codes.  v_maximum3 / v_minimum3 let a NaN through the clamp and the conversion makes it 0x7F or 0xFF; the sign of such

@@ -10,8 +10,9 @@
 //    and nothing in the loop consumes a loaded value, so the loads of step k+1
 //    really overlap the MFMAs of step k.  The LDS side of such a load is
 //    lane-linear, so the bank swizzle is applied to the global address instead.
-//  * Activations that need sign selection (merged DualScale codes) and int4
-//    weights go through registers; their transform is branch-free.
+//  * int4 weights, and DualScale codes of both signs in one tensor on the tiles that
+//    cannot part them behind LDS (MERGE, below, does), go through registers on their
+//    way there; their transform is branch-free.
 //  * Epilogue through LDS for 16-bit outputs: each lane owns 4 consecutive
 //    columns of 16 different rows, which as direct stores are 32-byte pieces of
 //    16 lines per instruction (measured 1.7 TB/s); transposed through a private
@@ -679,11 +680,12 @@ __device__ __forceinline__ bool meet_share(const GemmParams& p, v4f (&of)[TN][TM
     return true;
 }
 
-// Software-pipelined variant for plain int8 operands (both straight to LDS) with
-// NS LDS stages.  Two stages are what is instantiated: on FLUX shapes three and
+// Software-pipelined variant for plain 8-bit operands (both straight to LDS) with
+// NS LDS stages.  Two are what nearly all instances have: on FLUX shapes three and
 // four stages measured slower (they cost a co-resident workgroup or buy nothing,
 // the global -> LDS path being throughput- rather than latency-bound: ~31 of a
-// measured ~55 B/clk/CU).  The K step is split at its one barrier:
+// measured ~55 B/clk/CU).  MERGE instances have three (launch_mix), launches of few
+// tiles four and five (128 x 128 and 128 x 96, int8).  The K step is split at its one barrier:
 //
 //   barrier (tile s landed, tile s-1 fully in registers)
 //     DMA tile s+1 into the buffer of tile s-1      <- a whole step of latency cover
@@ -1738,8 +1740,9 @@ int launch_walk(const GemmParams& p, int cfg, int64_t batch, hipStream_t st) {
 }
 
 // DualScale's two ranges in whole steps and a plain range or none behind them.  From one tensor of codes of both signs a stage is a
-// third smaller, which leaves room for a third one: 9216 x 3072 x (3072 + 12288) e4m3 192 x 192 566 us, two stages 561;
-// 128 x 192 600 and 630, 1024 rows in two shares 75 and 77; int8 level.
+// third smaller, which leaves room for a third one.  us, three stages / two, e4m3: 9216 x 3072 x (3072 + 12288) on 128 x 192 600 / 630,
+// 1024 rows in two shares 75 / 77; on 192 x 192, whose wave tiles load less per MFMA, 566 / 561; int8 level.  All three tiles have
+// three: what that costs the largest lies within what runs of one card differ by.
 template <int FMT>
 int launch_mix(const GemmParams& p, int cfg, int64_t batch, hipStream_t st) {
 #define SEGQ_MIX(BM_, BN_)                                                                                                                       \

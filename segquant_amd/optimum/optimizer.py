@@ -452,7 +452,8 @@ class DefaultOptimizer(BaseOptimizer):
         #  * int4 weights: _lends_int4.
         #  * 8-bit weights: always.  int8 with several ranges that no one walk of K serves parks the
         #    finished ranges' sums there and keeps the big tiles; few tiles and a long K share the K steps of
-        #    a tile between workgroups (1024 x 15360 x 3072: 113 -> 79 us int8, 108 -> 75 us e4m3).
+        #    a tile between workgroups (one walk of 1024 x 15360 x 3072, whole / in two shares, operands in the
+        #    caches: int8 105 / 81 us, e4m3 101 / 72).
         int4 = plan["fw"] == ops.FMT_INT4
         lend = _lends_int4(plan, M) if int4 else True
         ws = None
@@ -504,7 +505,8 @@ class DefaultOptimizer(BaseOptimizer):
         """Whether DualScale codes go into one tensor, whose signs the GEMM parts in registers, or into two, which stream
         straight into its matrix instructions: one where the library has the kernel for it (8-bit codes, whole steps
         of K, at most one plain segment beside the DualScale one) and would take it.  Asked once per token count.
-        GEMM 9216 x 3072 x (3072 + 12288) two / one: int8 622 / 599 us, e4m3 596 / 567, 1024 rows 79 / 79 and 75 / 75; and the
+        GEMM 9216 x 3072 x (3072 + 12288), one walk from two / one, operands in the caches: int8 622 / 599 us, e4m3 596 / 567, 1024 rows
+        79 / 79 and 75 / 75; and the
         quantise step writes one tensor less (9216 x 12288 GELU'd, 90 / 68 us)."""
         known = plan.setdefault("one_tensor", {})
         one = known.get((M, dtype))
