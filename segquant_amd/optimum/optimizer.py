@@ -44,6 +44,9 @@ def _lends_int4(plan, M: int) -> bool:
     return plan.get("group_dequant") is not None or M >= 3072 or (M >= 1000 and K >= 3072) or M * K >= 2300 * 2048
 
 
+_PLAN_VERSION = 1  # of what a plan holds: saved with it, raised when that changes
+
+
 class BaseOptimizer:
     def __init__(self, seg_mode, chunks, chunksizes, weight_manager, input_calibrators, weight_calibrators,
                  real_quant=False, dual_scale=False, kernel_type=None, dual_segments=None):
@@ -66,8 +69,11 @@ class BaseOptimizer:
         self._plan = None
 
     def __setstate__(self, state):
-        # a plan belongs to the build of the package, and to the device, that made it: loaded and copied layers make their own
-        self.__dict__.update(state, _plan=None)
+        # a plan of another version of the package may lack what this one looks for: such a layer makes its own.  One of this
+        # version stays with its copy, whose first call may be one that a graph records
+        self.__dict__.update(state)
+        if self._plan is not None and self._plan.get("version") != _PLAN_VERSION:
+            self._plan = None
 
     def _stack(self, calibrators, attr):
         dev = self.weight_manager.device()
@@ -292,7 +298,7 @@ class DefaultOptimizer(BaseOptimizer):
                 bounds = [0]
                 for c in self.chunksizes:
                     bounds.append(bounds[-1] + c)
-            self._plan = dict(fa=fa, fw=fw, w=wcodes, sw=torch.ones(1, dtype=torch.float32, device=device), sw_cs=0,
+            self._plan = dict(version=_PLAN_VERSION, fa=fa, fw=fw, w=wcodes, sw=torch.ones(1, dtype=torch.float32, device=device), sw_cs=0,
                               bounds=bounds, N=N, K=K, group_dequant=(1.0 / per_row).t().contiguous().to(device))
             return self._plan
         wscales = [_as_f32(c.scale, dev).reshape(-1) for c in self.weight_calibrators]
@@ -308,7 +314,7 @@ class DefaultOptimizer(BaseOptimizer):
             bounds = [0]
             for c in self.chunksizes:
                 bounds.append(bounds[-1] + c)
-        self._plan = dict(fa=fa, fw=fw, w=wcodes, sw=sw_vec.contiguous().to(device),
+        self._plan = dict(version=_PLAN_VERSION, fa=fa, fw=fw, w=wcodes, sw=sw_vec.contiguous().to(device),
                           sw_cs=1 if sw_vec.numel() > 1 else 0, bounds=bounds, N=N, K=K)
         return self._plan
 

@@ -32,7 +32,7 @@ from __future__ import annotations
 import torch
 
 from .. import ops
-from .optimizer import BaseOptimizer, DefaultOptimizer, OptimizerRegistry, _as_f32, _FMT
+from .optimizer import BaseOptimizer, DefaultOptimizer, OptimizerRegistry, _as_f32, _FMT, _PLAN_VERSION
 
 
 @OptimizerRegistry.register("smooth")
@@ -159,7 +159,7 @@ class SmoothOptimizer(DefaultOptimizer):
         # rounded here for every input dtype, not on the first call that brings one: that call may be on another
         # stream than the next, or under a capture, which would leave the later calls a tensor without contents
         casts = {dt: ops.rounded_col_div(col_div, dt) for dt in (torch.float32, torch.float16, torch.bfloat16)}
-        self._plan = dict(fa=fa, fw=fw, w=wcodes, sw=sw_list[0], sw_list=sw_list, sw_cs=1 if sw_list[0].numel() > 1 else 0,
+        self._plan = dict(version=_PLAN_VERSION, fa=fa, fw=fw, w=wcodes, sw=sw_list[0], sw_list=sw_list, sw_cs=1 if sw_list[0].numel() > 1 else 0,
                           bounds=bounds, N=N, K=K, col_div=col_div, col_div_cast=casts)
         return self._plan
 

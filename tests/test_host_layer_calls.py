@@ -197,3 +197,17 @@ def test_a_loaded_layer_makes_a_plan_of_its_own(again):
     opt.__dict__.update(low_rank=32, chunks=1, _plan=dict(K=K, N=N, l2t=torch.empty(N, 32), l12_cast={}))
     loaded = again(opt)
     assert loaded._plan is None and (loaded.low_rank, loaded.chunks) == (32, 1) and opt._plan is not None
+
+
+@pytest.mark.parametrize("again", [lambda o: pickle.loads(pickle.dumps(o)), copy.deepcopy])
+def test_a_copy_of_a_planned_layer_is_ready_for_a_capture(again):
+    """A plan that is made while a graph is recorded holds tensors without contents until the graph runs: the copy of a layer that
+    has one keeps it."""
+    opt = object.__new__(OptimizerRegistry.get("smooth"))
+    one = torch.ones(N)
+    opt.__dict__.update(chunks=1, seg_mode="weight", chunksizes=[N], kernel_type="Wint8Aint8", s=[torch.ones(K)], _plan=None,
+                        weight_manager=types.SimpleNamespace(out_features=N, in_features=K, weight_tensor=torch.zeros(N, K, dtype=torch.int8)),
+                        weight_calibrators=[types.SimpleNamespace(scale=one)])
+    opt._build_plan(torch.device("cpu"))
+    loaded = again(opt)
+    assert loaded._plan is not None and loaded._plan is not opt._plan and torch.equal(loaded._plan["w"], opt._plan["w"])
